@@ -278,10 +278,10 @@ int ngpu_iterate(ngpu_t *h, const ngpu_iter_in_t *in, ngpu_iter_out_t *out);
 int ngpu_set_graph(ngpu_t *h, int32_t on);
 
 /* Launch shape, the knobs of the autotuner (neci_stable_amd/autotune.py):
-   blocks of the chunked kernels (prepass, attempt scan, radix passes; 64 to
-   16 per compute unit), blocks of the grid-stride kernels (spawn, merge and
-   annihilation, insert, statistics; 64 to 64 per compute unit), elements
-   per thread of a radix tile (2, 4 or 8), lanes per heat-bath single attempt
+   blocks of the chunked kernels (prepass, attempt scan; 64 to 16 per compute
+   unit), blocks of the grid-stride kernels (spawn, insert, statistics; 64 to
+   64 per compute unit), elements per thread of a radix tile (2, 4 or 8; the
+   sorts of the core space's set-up), lanes per heat-bath single attempt
    (4, 8 or 16) and blocks of the merge-annihilation kernel (64 to 64 per
    compute unit).  0 keeps a value.  Results do not
    depend on the shape (the kernels' outputs are independent of how work is
@@ -382,8 +382,8 @@ int ngpu_get_check_counts(ngpu_t *h, int64_t *counts, int32_t n);
    lib/timing.F90:122-188).  Each stage is timed from the start of its first
    kernel to the end of its last.  Stages: 0 prepass (initiator, proj-E, death),
    1 attempt scan (2 kernels), 2 spawn (all attempts; molecular: doubles, singles
-   queued), 3 queued singles, 4 sort (all radix passes), 5 merge (empty: fused
-   into 6), 6 merge and annihilation, 7 insert, 8 hash statistics, 9 the core
+   queued), 3 queued singles, 4 sort and 5 merge (empty: the spawning kernels
+   bin their records, 6 merges the bins), 6 merge and annihilation, 7 insert, 8 hash statistics, 9 the core
    Hamiltonian's H.v (semistochastic projection).  Stages 0, 2, 3, 6, 7, 8 and
    9 are one kernel each.  on is a bit mask of the stages to time
    (bit s for stage s; 0 switches timing off); each timed stage adds two events

@@ -1,12 +1,11 @@
 """Launch-shape autotuner.
 
 The engine's kernels split their work over a number of blocks fixed at launch
-and the radix sort ranks tiles of a fixed number of elements per thread
 (ngpu_set_launch_shape); the heat-bath singles run 4, 8 or 16 lanes per
 attempt.  The best values depend on the walker count and the system, so they
-are measured on the running calculation: one knob at a time (radix tile, the
-chunked kernels' blocks, the grid-stride kernels' blocks, the lanes per
-single attempt, then the merge-annihilation kernel's blocks), each candidate
+are measured on the running calculation: one knob at a time (the chunked
+kernels' blocks, the grid-stride kernels' blocks, the lanes per single
+attempt, then the merge-annihilation kernel's blocks), each candidate
 timed over a few iterations of the driver (or of a batch, for the engines of
 one launch group), the fastest kept.  The walker dynamics do not depend on
 the shape, so tuning while the calculation runs changes nothing but its
@@ -30,11 +29,10 @@ def tune_engines(engines, run, steps=20, warm=5, repeats=2, log=None):
     base = engines[0].launch_shape()
     cu = base["n_cu"]
     knobs = [
-        ("radix_items", [2, 4, 8]),
         ("chunk_blocks", [2 * cu, 4 * cu, 8 * cu]),
         ("grid_blocks", [3 * cu, 4 * cu, 8 * cu]),
         ("single_lanes", [4, 8, 16]),
-        ("merge_blocks", [2 * cu, 3 * cu, 4 * cu]),
+        ("merge_blocks", [3 * cu, 4 * cu, 5 * cu]),
     ]
     best = {k: base[k] for k in ("chunk_blocks", "grid_blocks", "radix_items", "single_lanes", "merge_blocks")}
     trials = []

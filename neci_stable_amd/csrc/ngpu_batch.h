@@ -2,8 +2,8 @@
 // chain covers every engine of a batch group.
 //
 // A group is a set of engines whose chains use the same kernel instances
-// (words per determinant, replica layout, generator, sort path and its
-// passes, spawn-record precision, core precision, launch knobs).  Each engine
+// (words per determinant, replica layout, generator, spawn-record precision,
+// core precision, launch knobs).  Each engine
 // keeps its own walker table, hash, spawn buffers, counters and statistics;
 // an EngDev in device memory describes them, and each launch kind gives every
 // engine a contiguous share of the launch's blocks.  A block finds its engine
@@ -17,17 +17,13 @@ namespace ngpu {
 
 // launch kinds of a batch chain and how each engine's share is sized
 enum {
-  kLkChunk = 0,  // chunked kernels: prepass, attempt scan, radix histogram and scatter
+  kLkChunk = 0,  // chunked kernels: prepass, attempt scan
   kLkGrid,       // grid-stride kernels: spawns, insert, statistics
   kLkMerge,      // merge and annihilation
   kLkCore,       // core gather and apply (one element per thread)
   kLkCoreRow,    // core H.v (one row per wave)
   kLkKinds
 };
-// kinds with a fixed number of blocks per engine: the radix digit scan and
-// the segment sort (one block per 8-bit digit), the end of the iteration (1)
-constexpr int kDigitBlocks = 256;
-
 // One engine of a batch group as its kernels see it.
 struct EngDev {
   DevSys s;
@@ -41,14 +37,9 @@ struct EngDev {
   int64_t* blk_rm;
   int64_t* tile_p;
   int64_t tcap;
-  uint64_t* sp_rec;
-  uint32_t* rk;
+  Bins bins;
   int64_t scap;
   int64_t* sq;
-  uint64_t* sk[2];
-  uint32_t* si[2];
-  uint32_t* hist;
-  uint32_t* digit_tot;
   uint64_t* n_key;
   double* n_sgn;
   uint32_t* n_flag;
@@ -89,112 +80,31 @@ __global__ void __launch_bounds__(kBlock) km_scan_apply(const EngDev* __restrict
   Grid g;
   const EngDev& a = eng_of(ed, map, kLkChunk, g);
   k_scan_apply_body<W>(g, a.s, a.wk, a.att_cnt, a.att_off, a.blk_part, a.blk_rm, a.pinfo, a.cnt, a.s.S, a.tile_p,
-                       a.tcap);
+                       a.tcap, a.bins);
 }
 
 template <int W, int R, int G>
-__global__ void __launch_bounds__(kBlock) km_spawn(const EngDev* __restrict__ ed, const uint16_t* __restrict__ map,
-                                                   int ranked) {
+__global__ void __launch_bounds__(kBlock) km_spawn(const EngDev* __restrict__ ed, const uint16_t* __restrict__ map) {
   Grid g;
   const EngDev& a = eng_of(ed, map, kLkGrid, g);
-  k_spawn_body<W, R, G>(g, a.s, a.wk, a.cnt, a.part, a.att_off, a.tile_p, a.tcap, a.pinfo, a.sp_rec,
-                        ranked ? a.rk : nullptr, a.scap, a.sq, a.prm);
+  k_spawn_body<W, R, G>(g, a.s, a.wk, a.cnt, a.part, a.att_off, a.tile_p, a.tcap, a.pinfo, a.bins,
+                        a.scap, a.sq, a.prm);
 }
 
 template <int W, int R, int PL, int G>
 __global__ void __launch_bounds__(kBlock) km_spawn_singles(const EngDev* __restrict__ ed,
-                                                           const uint16_t* __restrict__ map, int ranked) {
+                                                           const uint16_t* __restrict__ map) {
   Grid g;
   const EngDev& a = eng_of(ed, map, kLkGrid, g);
-  k_spawn_singles_body<W, R, PL, G>(g, a.s, a.wk, a.cnt, a.part, a.pinfo, a.sp_rec, ranked ? a.rk : nullptr, a.scap,
-                                    a.sq, a.prm);
+  k_spawn_singles_body<W, R, PL, G>(g, a.s, a.wk, a.cnt, a.part, a.pinfo, a.bins, a.scap, a.sq, a.prm);
 }
 
-// radix pass p of the word sort: the first pass reads the keys inside the
-// spawn records (first = 1) or the 64-bit rank keys in sk[cur] (first = 2,
-// the rank path's partition pass), later passes the previous pass's output
-// (ping-pong cur)
-template <typename K, int NW, bool FLIP, int IT, int DB>
-__global__ void __launch_bounds__(kBlock) km_radix_hist_words(const EngDev* __restrict__ ed,
-                                                              const uint16_t* __restrict__ map, int first, int cur,
-                                                              int word, int shift) {
-  Grid g;
-  const EngDev& a = eng_of(ed, map, kLkChunk, g);
-  const K* kin = first == 1 ? (const K*)a.sp_rec : (const K*)a.sk[cur];
-  const int kstride = first == 1 ? a.s.rec_words : NW;
-  k_radix_hist_body<K, NW, FLIP, IT, DB>(g, kin, kstride, &a.cnt->n_spawned, a.scap, word, shift, a.hist);
-}
-
-template <typename K, int NW, bool FLIP, int IT, int DB>
-__global__ void __launch_bounds__(kBlock) km_radix_scatter_words(const EngDev* __restrict__ ed,
-                                                                 const uint16_t* __restrict__ map, int first,
-                                                                 int cur, int word, int shift) {
-  Grid g;
-  const EngDev& a = eng_of(ed, map, kLkChunk, g);
-  const K* kin = first == 1 ? (const K*)a.sp_rec : (const K*)a.sk[cur];
-  const int kstride = first == 1 ? a.s.rec_words : NW;
-  const uint32_t* iin = first ? nullptr : a.si[cur];
-  k_radix_scatter_body<K, NW, FLIP, IT, DB>(g, kin, kstride, iin, (K*)a.sk[cur ^ 1], a.si[cur ^ 1], &a.cnt->n_spawned,
-                                            a.scap, word, shift, a.hist, a.digit_tot);
-}
-
-// the 64-bit rank path's keys of the spawned list into sk[0] (the partition
-// pass's input) with the histogram of their top byte
-template <int IT>
-__global__ void __launch_bounds__(kBlock) km_rank64_hist(const EngDev* __restrict__ ed,
-                                                         const uint16_t* __restrict__ map, int bits) {
-  Grid g;
-  const EngDev& a = eng_of(ed, map, kLkChunk, g);
-  k_rank64_hist_body<IT, kSegBits>(g, a.sp_rec, a.s.rec_words, &a.cnt->n_spawned, a.scap, a.s.binom64,
-                                     a.s.nbasis, a.s.nel1, bits, a.sk[0], a.hist);
-}
-
-// the colex-rank sort: top-byte pass over the ranks the spawn kernels wrote
-template <int IT>
-__global__ void __launch_bounds__(kBlock) km_radix_hist_ranks(const EngDev* __restrict__ ed,
+template <int W, int R>
+__global__ void __launch_bounds__(kBlock, R <= 2 && W == 1 ? 5 : 1) km_merge_annihilate(const EngDev* __restrict__ ed,
                                                               const uint16_t* __restrict__ map) {
   Grid g;
-  const EngDev& a = eng_of(ed, map, kLkChunk, g);
-  k_radix_hist_body<uint32_t, 1, false, IT, kSegBits>(g, a.rk, 1, &a.cnt->n_spawned, a.scap, 0, 32 - kSegBits,
-                                                   a.hist);
-}
-template <int IT>
-__global__ void __launch_bounds__(kBlock) km_radix_scatter_ranks(const EngDev* __restrict__ ed,
-                                                                 const uint16_t* __restrict__ map) {
-  Grid g;
-  const EngDev& a = eng_of(ed, map, kLkChunk, g);
-  k_radix_scatter_body<uint32_t, 1, false, IT, kSegBits>(g, a.rk, 1, nullptr, (uint32_t*)a.sk[1], a.si[1],
-                                                         &a.cnt->n_spawned, a.scap, 0, 32 - kSegBits, a.hist,
-                                                         a.digit_tot);
-}
-
-// one block per digit of every engine: engine blockIdx / digits
-__global__ void __launch_bounds__(kBlock) km_radix_scan(const EngDev* __restrict__ ed, int digits) {
-  const EngDev& a = ed[blockIdx.x / digits];
-  const Grid g{(int64_t)(blockIdx.x % digits), digits};
-  k_radix_scan_body(g, a.hist, a.nb[kLkChunk], a.digit_tot);
-}
-__global__ void __launch_bounds__(kSegThreads) km_seg_sort(const EngDev* __restrict__ ed) {
-  const EngDev& a = ed[blockIdx.x / kSegs];
-  const Grid g{(int64_t)(blockIdx.x % kSegs), kSegs};
-  k_seg_sort_body<uint32_t>(g, (uint32_t*)a.sk[1], a.si[1], (uint32_t*)a.sk[0], a.si[0], a.digit_tot,
-                            (32 - kSegBits + 7) / 8);
-}
-// the 64-bit rank path's kSegs segments per engine: sk[1] -> sk[0],
-// npass bytes below the top digit
-__global__ void __launch_bounds__(kSegThreads) km_seg_sort64(const EngDev* __restrict__ ed, int npass) {
-  const EngDev& a = ed[blockIdx.x / kSegs];
-  const Grid g{(int64_t)(blockIdx.x % kSegs), kSegs};
-  k_seg_sort_body<uint64_t>(g, a.sk[1], a.si[1], a.sk[0], a.si[0], a.digit_tot, npass);
-}
-
-template <int W, int R, typename K, int NW>
-__global__ void __launch_bounds__(kBlock) km_merge_annihilate(const EngDev* __restrict__ ed,
-                                                              const uint16_t* __restrict__ map, int cur) {
-  Grid g;
   const EngDev& a = eng_of(ed, map, kLkMerge, g);
-  k_merge_annihilate_body<W, R, K, NW>(g, a.s, a.wk, a.cnt, a.part, (const K*)a.sk[cur], a.si[cur], a.sp_rec, a.scap,
-                                       a.n_key, a.n_sgn, a.n_flag, a.prm);
+  k_merge_body<W, R, false>(g, a.s, a.wk, a.cnt, a.part, a.bins, a.n_key, a.n_sgn, a.n_flag, &a.cnt->n_new, a.prm);
 }
 
 template <int R>

@@ -200,28 +200,16 @@ struct ngpu_engine {
   double* core_y = nullptr;
   // spawns, sort, merge, new
   int64_t scap = 0;
-  uint64_t* sp_rec = nullptr;  // spawned list, kRecWords words per record
-  uint64_t* sk[2] = {nullptr, nullptr};
-  uint32_t* si[2] = {nullptr, nullptr};
-  uint32_t* hist = nullptr;
+  Bins bins{};                 // spawned records by determinant hash
+  uint32_t* hist = nullptr;    // radix sort of the set-up paths
   uint32_t* digit_tot = nullptr;
-  // sort by 32-bit colex rank when every determinant has one
-  bool rank_sort = false;
-  int rank_bits = 0;
-  uint32_t* d_binom = nullptr;  // C(p, i) at [p*(nel+1)+i]
-  uint32_t* rk = nullptr;       // ranks of the spawned list
-  // one-word determinants with C(nbasis, nel) < 2^64 whose colex rank needs
-  // fewer bytes than the word: the spawn sort partitions on the top byte of
-  // the (spread) 64-bit rank, then sorts each segment (k_seg_sort64)
-  bool rank64 = false;
-  int rank64_bits = 0;
-  uint64_t* d_binom64 = nullptr;  // C(p, i) at [p*(nel+1)+i], 64 bits
   int64_t* sq = nullptr;  // queued single-excitation attempts
   // merged spawned list, kept only for the explicit-list entry point
   uint64_t* u_key = nullptr;
   double* u_sgn = nullptr;
   uint32_t* u_flag = nullptr;
   unsigned long long* u_count = nullptr;
+  uint64_t* l_rec = nullptr;  // its input list, dense records
   uint64_t* n_key = nullptr;
   double* n_sgn = nullptr;
   uint32_t* n_flag = nullptr;
@@ -288,11 +276,7 @@ struct BatchGroup {
   int gen = 0;              // kGenHubbard, kGenPchb or kGenUniform
   bool singles = false;     // queued heat-bath singles (PCHB generator)
   int lanes = 4, pl = 4;    // heat-bath singles: lanes per attempt, orbitals per lane
-  int items = 4;            // radix tile: elements per thread
-  bool rank_sort = false;
-  bool rank64 = false;                      // the 64-bit rank partition sort
-  int rank64_bits = 0;
-  std::vector<std::pair<int, int>> passes;  // (word, shift) of the word-key sort
+  int items = 4;            // launch-shape knob of the set-up sorts
   bool core = false, core_fp32 = false;
   // every engine of the group has the same core determinants: one projection
   // over the interleaved vectors X, Y of ccols columns (kernels in ngpu_batch.h)
@@ -369,11 +353,13 @@ __global__ void k_begin_iter(ngpu_iter_out_t* out, double* part, Counters* cnt, 
 // accumulation into the cycle sums (ENumCyc, HFCyc, NoBorn, ... are cycle
 // accumulators in the reference too)
 __device__ __forceinline__ void end_iter_body(ngpu_iter_out_t* out, double* part, ngpu_iter_out_t* cyc, Counters* cnt,
-                                              int64_t scap, int64_t cap, int64_t hash_entries, const IterParams* prm) {
+                                              int64_t scap, int64_t cap, int64_t hash_entries, const IterParams* prm,
+                                              uint32_t* scount) {
   // halted: the output block keeps the failing iteration's statistics and
   // error, and nothing is added to the cycle
   if (cnt->halt) return;
   __shared__ unsigned long long n_unique;
+  for (uint32_t i = threadIdx.x; i < kSpill; i += blockDim.x) scount[i] = 0;
   if (threadIdx.x < kWave) {
     // the spread per-block counts, one line per lane, summed across the wave
     const int l = threadIdx.x;
@@ -434,9 +420,12 @@ __device__ __forceinline__ void end_iter_body(ngpu_iter_out_t* out, double* part
       cnt->halt = cnt->err;
       cnt->err_iter = prm->iter;
     }
+    cnt->prev_spawned = (unsigned long long)out->n_spawned;
+    cnt->prev_attempts = cnt->n_attempts;
     // the counters the next iteration appends to start from zero (the chain
     // has no separate reset launch)
     cnt->n_spawned = 0;
+    cnt->n_ovf = 0;
     cnt->n_singles = 0;
     cnt->n_new = 0;
     cnt->n_fail = 0;
@@ -445,13 +434,15 @@ __device__ __forceinline__ void end_iter_body(ngpu_iter_out_t* out, double* part
   }
 }
 __global__ void k_end_iter(ngpu_iter_out_t* out, double* part, ngpu_iter_out_t* cyc, Counters* cnt,
-                           int64_t scap, int64_t cap, int64_t hash_entries, const IterParams* prm) {
-  end_iter_body(out, part, cyc, cnt, scap, cap, hash_entries, prm);
+                           int64_t scap, int64_t cap, int64_t hash_entries, const IterParams* prm,
+                           uint32_t* scount) {
+  end_iter_body(out, part, cyc, cnt, scap, cap, hash_entries, prm, scount);
 }
 // the end of the iteration of every engine of a batch group: one block each
 __global__ void km_end_iter(const EngDev* __restrict__ ed) {
   const EngDev& a = ed[blockIdx.x];
-  end_iter_body(a.dout, a.part, a.dcyc, a.cnt, a.scap, a.wk.cap, a.wk.L * (int64_t)kBucketEntries, a.prm);
+  end_iter_body(a.dout, a.part, a.dcyc, a.cnt, a.scap, a.wk.cap, a.wk.L * (int64_t)kBucketEntries, a.prm,
+                a.bins.scount);
 }
 
 __global__ void k_reset_cycle(ngpu_iter_out_t* cyc) {
@@ -521,104 +512,22 @@ std::vector<std::pair<int, int>> word_passes(const ngpu_t* h) {
   return p;
 }
 
-// sort of the spawned list (stage 4) then the merge of equal determinants
-// fused with their annihilation into the walker list (stage 6; stage 5, the
-// merge alone, is empty since the fusion); ranked: the spawn kernels already
-// wrote each record's colex rank
-// the rank path: one stable pass on the keys' top byte, then one block per
-// top-byte segment sorts it by the low 24 bits (k_seg_sort); the sorted
-// (key, spawn index) pairs end in buffer 0
-template <int W, int R, int IT>
-int sort_ranks(ngpu_t* h, bool ranked) {
-  const unsigned long long* n_ptr = &h->cnt->n_spawned;
-  constexpr int kTop = 32 - kSegBits;  // the partition digit's shift
-  if (ranked)
-    launch(h, 4, -1, k_radix_hist<uint32_t, 1, false, IT, kSegBits>, dim3(h->nb_chunk), dim3(kBlock),
-           (const uint32_t*)h->rk, 1, n_ptr, h->scap, 0, kTop, h->hist);
-  else
-    launch(h, 4, -1, k_rank_hist<W, IT, kSegBits>, dim3(h->nb_chunk), dim3(kBlock), (const uint64_t*)h->sp_rec,
-           n_ptr, h->scap, h->ds.rec_words, (const uint32_t*)h->d_binom, h->sys.nel + 1, h->rk, h->hist, kTop);
-  launch(h, -1, -1, k_radix_scan, dim3(kSegs), dim3(kBlock), h->hist, h->nb_chunk, h->digit_tot);
-  launch(h, -1, -1, k_radix_scatter<uint32_t, 1, false, IT, kSegBits>, dim3(h->nb_chunk), dim3(kBlock),
-         (const uint32_t*)h->rk, 1, (const uint32_t*)nullptr, (uint32_t*)h->sk[1], h->si[1], n_ptr, h->scap, 0, kTop,
-         (const uint32_t*)h->hist, (const uint32_t*)h->digit_tot);
-  launch(h, -1, 4, k_seg_sort, dim3(kSegs), dim3(kSegThreads), (uint32_t*)h->sk[1], h->si[1], (uint32_t*)h->sk[0],
-         h->si[0], (const uint32_t*)h->digit_tot);
-  return 0;
+// blocks of the merge: a wave per bin, no more waves than there can be bins
+int merge_blocks(const ngpu_t* h) {
+  const int nb = h->nb_merge ? h->nb_merge : h->nb_grid;
+  return (int)std::min<int64_t>(nb, ((int64_t)h->bins.maxb + kBlock / kWave - 1) / (kBlock / kWave));
 }
 
-template <int W, int R, int IT>
-void sort_and_merge_it(ngpu_t* h, bool ranked, bool list_out) {
-  const unsigned long long* n_ptr = &h->cnt->n_spawned;
-  if (h->rank_sort) {
-    const int cur = sort_ranks<W, R, IT>(h, ranked);
-    if (list_out)
-      launch(h, -1, -1, k_merge_list<W, R, uint32_t, 1>, dim3(h->nb_grid), dim3(kBlock), h->ds, h->cnt,
-             (const uint32_t*)h->sk[cur], (const uint32_t*)h->si[cur], (const uint64_t*)h->sp_rec, h->scap, h->u_key,
-             h->u_sgn, h->u_flag, h->u_count);
-    launch(h, 6, 6, k_merge_annihilate<W, R, uint32_t, 1>, dim3(h->nb_merge ? h->nb_merge : h->nb_grid), dim3(kBlock), h->ds, h->wk, h->cnt,
-           h->dpart, (const uint32_t*)h->sk[cur], (const uint32_t*)h->si[cur], (const uint64_t*)h->sp_rec, h->scap,
-           h->n_key, h->n_sgn, h->n_flag, (const IterParams*)h->dparams);
-    return;
-  }
-  if (h->rank64) {
-    // the 64-bit rank keys (spread over the top byte) into sk[0], one stable
-    // pass on the top byte into sk[1], then each top-byte segment sorted by
-    // the bytes below it (k_seg_sort64) back into sk[0]
-    const int bits = h->rank64_bits;
-    launch(h, 4, -1, k_rank64_hist<IT, kSegBits>, dim3(h->nb_chunk), dim3(kBlock), (const uint64_t*)h->sp_rec,
-           h->ds.rec_words, n_ptr, h->scap, (const uint64_t*)h->d_binom64, h->sys.nbasis, h->sys.nel + 1, bits,
-           h->sk[0], h->hist);
-    launch(h, -1, -1, k_radix_scan, dim3(kSegs), dim3(kBlock), h->hist, h->nb_chunk, h->digit_tot);
-    launch(h, -1, -1, k_radix_scatter<uint64_t, 1, false, IT, kSegBits>, dim3(h->nb_chunk), dim3(kBlock),
-           (const uint64_t*)h->sk[0], 1, (const uint32_t*)nullptr, h->sk[1], h->si[1], n_ptr, h->scap, 0,
-           bits - kSegBits, (const uint32_t*)h->hist, (const uint32_t*)h->digit_tot);
-    launch(h, -1, 4, k_seg_sort64, dim3(kSegs), dim3(kSegThreads), h->sk[1], h->si[1], h->sk[0], h->si[0],
-           (const uint32_t*)h->digit_tot, (bits - kSegBits + 7) / 8);
-    if (list_out)
-      launch(h, -1, -1, k_merge_list<W, R, uint64_t, W>, dim3(h->nb_grid), dim3(kBlock), h->ds, h->cnt,
-             (const uint64_t*)h->sk[0], (const uint32_t*)h->si[0], (const uint64_t*)h->sp_rec, h->scap, h->u_key,
-             h->u_sgn, h->u_flag, h->u_count);
-    launch(h, 6, 6, k_merge_annihilate<W, R, uint64_t, W>, dim3(h->nb_merge ? h->nb_merge : h->nb_grid),
-           dim3(kBlock), h->ds, h->wk, h->cnt, h->dpart, (const uint64_t*)h->sk[0], (const uint32_t*)h->si[0],
-           (const uint64_t*)h->sp_rec, h->scap, h->n_key, h->n_sgn, h->n_flag, (const IterParams*)h->dparams);
-    return;
-  }
-  // determinant keys in ilut_lt order: least significant word first
-  const std::vector<std::pair<int, int>> passes = word_passes(h);
-  int cur = 0;
-  const uint64_t* kin = h->sp_rec;
-  int kstride = h->ds.rec_words;  // the first pass reads the keys inside the records
-  const uint32_t* iin = nullptr;
-  for (size_t p = 0; p < passes.size(); ++p) {
-    int out = (int)(p & 1);
-    bool first = p == 0, last = p + 1 == passes.size();
-    launch(h, first ? 4 : -1, -1, k_radix_hist<uint64_t, W, W == 2, IT, 8>, dim3(h->nb_chunk), dim3(kBlock), kin,
-           kstride, n_ptr, h->scap, passes[p].first, passes[p].second, h->hist);
-    launch(h, -1, -1, k_radix_scan, dim3(256), dim3(kBlock), h->hist, h->nb_chunk, h->digit_tot);
-    launch(h, -1, last ? 4 : -1, k_radix_scatter<uint64_t, W, W == 2, IT, 8>, dim3(h->nb_chunk), dim3(kBlock), kin, kstride, iin,
-           h->sk[out], h->si[out], n_ptr, h->scap, passes[p].first, passes[p].second, (const uint32_t*)h->hist,
-           (const uint32_t*)h->digit_tot);
-    kin = h->sk[out];
-    kstride = W;
-    iin = h->si[out];
-    cur = out;
-  }
-  if (list_out)
-    launch(h, -1, -1, k_merge_list<W, R, uint64_t, W>, dim3(h->nb_grid), dim3(kBlock), h->ds, h->cnt,
-           (const uint64_t*)h->sk[cur], (const uint32_t*)h->si[cur], (const uint64_t*)h->sp_rec, h->scap, h->u_key,
-           h->u_sgn, h->u_flag, h->u_count);
-  launch(h, 6, 6, k_merge_annihilate<W, R, uint64_t, W>, dim3(h->nb_merge ? h->nb_merge : h->nb_grid), dim3(kBlock), h->ds, h->wk, h->cnt,
-         h->dpart, (const uint64_t*)h->sk[cur], (const uint32_t*)h->si[cur], (const uint64_t*)h->sp_rec, h->scap,
-         h->n_key, h->n_sgn, h->n_flag, (const IterParams*)h->dparams);
-}
-
-// the sort with the engine's tile size (elements per thread of a radix tile)
+// merge of equal determinants of the spawned list, fused with their
+// annihilation into the walker list (stage 6; stages 4 and 5, the sort and
+// the merge alone, are empty)
 template <int W, int R>
-void sort_and_merge(ngpu_t* h, bool ranked, bool list_out) {
-  if (h->radix_items == 2) sort_and_merge_it<W, R, 2>(h, ranked, list_out);
-  else if (h->radix_items == 8) sort_and_merge_it<W, R, 8>(h, ranked, list_out);
-  else sort_and_merge_it<W, R, 4>(h, ranked, list_out);
+void merge(ngpu_t* h, bool list_out) {
+  if (list_out)
+    launch(h, -1, -1, k_merge_list<W, R>, dim3(merge_blocks(h)), dim3(kBlock), h->ds, h->wk, h->cnt, h->bins, h->u_key,
+           h->u_sgn, h->u_flag, h->u_count);
+  launch(h, 6, 6, k_merge_annihilate<W, R>, dim3(merge_blocks(h)), dim3(kBlock), h->ds, h->wk, h->cnt, h->dpart,
+         h->bins, h->n_key, h->n_sgn, h->n_flag, (const IterParams*)h->dparams);
 }
 
 // semistochastic projection of the core amplitudes (before spawning)
@@ -650,14 +559,14 @@ void annihilation_chain(ngpu_t* h, bool with_core, bool list_out = false) {
     launch(h, -1, -1, k_core_apply<R>, dim3((int)std::min<int64_t>((h->ncore + kBlock - 1) / kBlock, h->nb_grid)),
            dim3(kBlock), h->ds, h->wk, (const Counters*)h->cnt, (const int64_t*)h->core_slot, (const double*)h->core_y,
            h->ncore, h->dpart);
-  sort_and_merge<W, R>(h, with_core, list_out);  // spawns of the iteration chain carry their ranks
+  merge<W, R>(h, list_out);
   launch(h, 7, 7, k_insert<W, R>, dim3(h->nb_grid), dim3(kBlock), h->ds, h->wk, h->cnt,
          (const uint64_t*)h->n_key, (const double*)h->n_sgn, (const uint32_t*)h->n_flag,
          (const unsigned long long*)&h->cnt->n_new);
   launch(h, 8, 8, k_stats<W, R>, dim3(h->nb_grid), dim3(kBlock), h->ds, h->wk, h->cnt, h->dpart,
          (const IterParams*)h->dparams);
   launch(h, -1, -1, k_end_iter, dim3(1), dim3(kBlock), h->dout, h->dpart, h->dcyc, h->cnt,
-         h->scap, h->wk.cap, h->wk.L * (int64_t)kBucketEntries, (const IterParams*)h->dparams);
+         h->scap, h->wk.cap, h->wk.L * (int64_t)kBucketEntries, (const IterParams*)h->dparams, h->bins.scount);
   if (h->checks) check_chain<W>(h, with_core);
 }
 
@@ -675,14 +584,14 @@ void iterate_chain(ngpu_t* h) {
   if (h->ncore) core_projection<R>(h);
   launch(h, 1, 1, k_scan_apply<W>, dim3(h->nb_chunk), dim3(kBlock), h->ds, h->wk, (const int32_t*)h->att_cnt,
          h->att_off, (const int64_t*)h->blk_part, (const int64_t*)h->blk_rm, (const uint8_t*)h->pinfo, h->cnt,
-         h->S, h->tile_p, h->tcap);
+         h->S, h->tile_p, h->tcap, h->bins);
   const int gen = gen_of(h);
   auto spawn = gen == kGenHubbard ? k_spawn<W, R, kGenHubbard>
              : gen == kGenUniform ? k_spawn<W, R, kGenUniform>
              : gen == kGenPchbW ? k_spawn<W, R, kGenPchbW> : k_spawn<W, R, kGenPchb>;
   launch(h, 2, 2, spawn, dim3(h->nb_grid), dim3(kBlock), h->ds, h->wk, h->cnt, h->dpart,
-         (const int64_t*)h->att_off, (const int64_t*)h->tile_p, h->tcap, (const uint8_t*)h->pinfo, h->sp_rec,
-         h->rank_sort ? h->rk : nullptr, h->scap, h->sq, (const IterParams*)h->dparams);
+         (const int64_t*)h->att_off, (const int64_t*)h->tile_p, h->tcap, (const uint8_t*)h->pinfo, h->bins,
+         h->scap, h->sq, (const IterParams*)h->dparams);
   if (h->sys.model == NGPU_MODEL_MOLECULAR && !h->ds.uniform) {
     const int nsp = h->sys.nbasis / 2;
     // G lanes per attempt, PL >= nsp / G orbitals per lane
@@ -697,7 +606,7 @@ void iterate_chain(ngpu_t* h) {
               : nsp <= 32 ? k_spawn_singles<W, R, 8, 4> : nsp <= 40 ? k_spawn_singles<W, R, 10, 4>
               : k_spawn_singles<W, R, 16, 4>;
     launch_lds(h, 3, 3, kern, dim3(h->nb_grid), dim3(kBlock), lds, h->ds, h->wk, h->cnt, h->dpart,
-               (const uint8_t*)h->pinfo, h->sp_rec, h->rank_sort ? h->rk : nullptr, h->scap, (const int64_t*)h->sq,
+               (const uint8_t*)h->pinfo, h->bins, h->scap, (const int64_t*)h->sq,
                (const IterParams*)h->dparams);
   }
   annihilation_chain<W, R>(h, true);
@@ -1087,7 +996,10 @@ int ngpu_create(ngpu_t** out, const ngpu_sys_t* sys) {
   }
   h->nb_chunk = std::max(256, 4 * prop.multiProcessorCount);
   h->nb_grid = std::max(512, 4 * prop.multiProcessorCount);
-  h->nb_merge = std::max(384, 3 * prop.multiProcessorCount);
+  // what the merge's registers keep resident: five blocks of one-word keys
+  // per compute unit (94 VGPRs), four of two-word keys (121).  Past that, a
+  // last partial round: 126 against 84 us at 1.3e6 spawns with one block too many
+  h->nb_merge = std::max(512, (h->W == 1 ? 5 : 4) * prop.multiProcessorCount);
   h->n_cu = std::max(1, prop.multiProcessorCount);
   h->max_chunk = 16 * h->n_cu;  // buffers sized by the chunk count allow up to this many blocks
   int rc = NGPU_OK;
@@ -1120,57 +1032,22 @@ int ngpu_create(ngpu_t** out, const ngpu_sys_t* sys) {
   // spawn capacity (beyond it the spawn kernel searches the offsets itself)
   h->tcap = (4 * scap) / kBlock + 2;
   fail(dalloc(&h->tile_p, (size_t)h->tcap));
-  fail(dalloc(&h->sp_rec, (size_t)scap * kRecWords));
-  for (int q = 0; q < 2; ++q) {
-    fail(dalloc(&h->sk[q], (size_t)scap * W));
-    fail(dalloc(&h->si[q], (size_t)scap));
+  {
+    // one bin per kBinFill expected records, at most one per 64 of the
+    // capacity; their regions hold the whole capacity and 16 records' slack
+    // each, so that even lists near it spill little
+    Bins& bn = h->bins;
+    bn.maxb = (uint32_t)std::max<int64_t>(1, std::min<int64_t>(scap / 64, 1 << 20));
+    bn.cap = scap + 16 * (int64_t)bn.maxb;
+    bn.words = std::max<uint32_t>(bn.maxb, (uint32_t)std::min<int64_t>(32 * (int64_t)bn.maxb, 1 << 19));
+    bn.spill_cap = (uint32_t)(scap / 2 / kSpill + 1);
+    fail(dalloc(&bn.rec, (size_t)bn.cap * kRecWords));
+    fail(dalloc(&bn.spill, (size_t)bn.spill_cap * kSpill * kRecWords));
+    fail(dalloc(&bn.ovf, (size_t)scap * kRecWords));
+    fail(dalloc(&bn.count, (size_t)bn.words));
+    fail(dalloc(&bn.scount, (size_t)kSpill));
   }
   fail(dalloc(&h->hist, (size_t)h->max_chunk * kRadixBins));
-  {
-    // C(nbasis, nel) decides the sort key; the table holds C(p, i) for the
-    // colex rank of a determinant (p < nbasis, i <= nel)
-    const int nb = sys->nbasis, ne = sys->nel;
-    std::vector<unsigned __int128> c((size_t)(nb + 1) * (ne + 1), 0);
-    for (int p = 0; p <= nb; ++p) {
-      c[(size_t)p * (ne + 1)] = 1;
-      for (int i = 1; i <= ne && i <= p; ++i) {
-        unsigned __int128 v = c[(size_t)(p - 1) * (ne + 1) + i - 1] + c[(size_t)(p - 1) * (ne + 1) + i];
-        c[(size_t)p * (ne + 1) + i] = v > ((unsigned __int128)1 << 64) ? ((unsigned __int128)1 << 64) : v;
-      }
-    }
-    unsigned __int128 total = c[(size_t)nb * (ne + 1) + ne];
-    if (total <= ((unsigned __int128)1 << 32) && nb * (ne + 1) <= kBinomLds) {
-      h->rank_sort = true;
-      while (h->rank_bits < 32 && ((unsigned __int128)1 << h->rank_bits) < total) ++h->rank_bits;
-      if (h->rank_bits == 0) h->rank_bits = 1;
-      std::vector<uint32_t> b((size_t)nb * (ne + 1));
-      for (int p = 0; p < nb; ++p)
-        for (int i = 0; i <= ne; ++i) b[(size_t)p * (ne + 1) + i] = (uint32_t)c[(size_t)p * (ne + 1) + i];
-      fail(dalloc(&h->d_binom, b.size()));
-      if (rc == NGPU_OK) fail(hipMemcpy(h->d_binom, b.data(), b.size() * 4, hipMemcpyHostToDevice));
-      h->ds.binom = h->d_binom;
-      h->ds.nel1 = sys->nel + 1;
-      fail(dalloc(&h->rk, (size_t)scap));
-    } else if (h->W == 1 && total < ((unsigned __int128)1 << 64) && nb * (ne + 1) <= kBinom64Lds) {
-      int bits = 1;
-      while (bits < 64 && ((unsigned __int128)1 << bits) < total) ++bits;
-      if ((bits + 7) / 8 < (nb + 7) / 8) {
-        h->rank64 = true;
-        h->rank64_bits = bits;
-        // entries above the total belong to no determinant's rank
-        std::vector<uint64_t> b((size_t)nb * (ne + 1));
-        for (int p = 0; p < nb; ++p)
-          for (int i = 0; i <= ne; ++i) {
-            unsigned __int128 v = c[(size_t)p * (ne + 1) + i];
-            b[(size_t)p * (ne + 1) + i] = v < total ? (uint64_t)v : 0;
-          }
-        fail(dalloc(&h->d_binom64, b.size()));
-        if (rc == NGPU_OK) fail(hipMemcpy(h->d_binom64, b.data(), b.size() * 8, hipMemcpyHostToDevice));
-        h->ds.binom64 = h->d_binom64;
-        h->ds.nel1 = sys->nel + 1;
-      }
-    }
-  }
   fail(dalloc(&h->digit_tot, (size_t)kRadixBins));
   fail(dalloc(&h->sq, (size_t)scap * 2));  // (parent pair, attempt number)
   int64_t ncap = std::max<int64_t>(scap, cap);
@@ -1188,6 +1065,8 @@ int ngpu_create(ngpu_t** out, const ngpu_sys_t* sys) {
   if (rc == NGPU_OK) {
     fail(hipMemsetAsync(wk.htab, 0xFF, (size_t)wk.L * 8 * W * sizeof(uint64_t), h->stream));
     fail(hipMemsetAsync(h->cnt, 0, sizeof(Counters), h->stream));
+    fail(hipMemsetAsync(h->bins.count, 0, (size_t)h->bins.words * 4, h->stream));
+    fail(hipMemsetAsync(h->bins.scount, 0, kSpill * 4, h->stream));
     fail(hipMemsetAsync(h->dout, 0, sizeof(ngpu_iter_out_t), h->stream));
     fail(hipMemsetAsync(h->dpart, 0, sizeof(double) * kStatCopies * kStatStride, h->stream));
     fail(hipMemsetAsync(h->dcyc, 0, sizeof(ngpu_iter_out_t), h->stream));
@@ -1231,9 +1110,9 @@ int ngpu_destroy(ngpu_t* h) {
   if (h->batch) return NGPU_ERR_STATE;  // ngpu_batch_destroy first
   if (h->stream) (void)hipStreamSynchronize(h->stream);
   void* ptrs[] = {h->wk.keys, h->wk.st, h->wk.diagH, h->wk.offdiagH, h->wk.freeq,
-                  h->wk.htab, h->att_cnt, h->att_off, h->pinfo, h->blk_part, h->blk_rm, h->sp_rec,
-                  h->sk[0], h->sk[1], h->si[0], h->si[1], h->hist, h->digit_tot, h->sq, h->n_key,
-                  h->n_sgn, h->n_flag, h->u_key, h->u_sgn, h->u_flag, h->u_count, h->cnt, h->dout, h->dpart, h->dcyc, h->own_params, h->d_rh, h->d_nbr, h->d_tmat, h->d_umat, h->d_jk, h->d_jk0, h->d_fref, h->d_chk, h->d_binom, h->d_binom64, h->rk, h->tile_p, h->core_keys, h->core_slot, h->core_rowptr, h->core_cols,
+                  h->wk.htab, h->att_cnt, h->att_off, h->pinfo, h->blk_part, h->blk_rm, h->bins.rec,
+                  h->bins.spill, h->bins.ovf, h->bins.count, h->bins.scount, h->l_rec, h->hist, h->digit_tot, h->sq, h->n_key,
+                  h->n_sgn, h->n_flag, h->u_key, h->u_sgn, h->u_flag, h->u_count, h->cnt, h->dout, h->dpart, h->dcyc, h->own_params, h->d_rh, h->d_nbr, h->d_tmat, h->d_umat, h->d_jk, h->d_jk0, h->d_fref, h->d_chk, h->tile_p, h->core_keys, h->core_slot, h->core_rowptr, h->core_cols,
                   h->core_vals, h->core_x, h->core_y, h->d_ab_tab,
                   h->d_ab_prob, h->d_ab_ok, h->d_j_tab, h->d_j_prob, h->d_j_ok, h->d_ab_tgt, h->d_i_tab, h->d_i_prob,
                   h->d_a_tab, h->d_a_prob, h->d_a_ok, h->d_b_tab, h->d_b_prob, h->d_b_ok};
@@ -1620,8 +1499,7 @@ int ngpu_upload_walkers(ngpu_t* h, const int64_t* rows, int64_t n) {
 
 extern "C++" {
 namespace {
-// ascending (key, index) radix sort of n elements with the spawn sort's
-// kernels: (word, shift) passes, the first reading kin (stride kstride) and
+// ascending (key, index) radix sort of n elements: (word, shift) passes, the first reading kin (stride kstride) and
 // iin (nullptr: the identity), ping-ponging through kb[2], ib[2]; returns the
 // buffer pair holding the result
 template <typename K, int NW, bool FLIP, int IT>
@@ -1644,14 +1522,6 @@ int radix_sort_pairs_in(ngpu_t* h, const K* kin, int kstride, const uint32_t* ii
   }
   return cur;
 }
-// the same in the engine's spawn-sort buffers (n <= the spawn capacity)
-template <typename K, int NW, bool FLIP, int IT>
-int radix_sort_pairs(ngpu_t* h, const K* kin, int kstride, const uint32_t* iin,
-                     const std::vector<std::pair<int, int>>& passes, const unsigned long long* n_ptr, int64_t n) {
-  K* kb[2] = {(K*)h->sk[0], (K*)h->sk[1]};
-  return radix_sort_pairs_in<K, NW, FLIP, IT>(h, kin, kstride, iin, passes, n_ptr, n, kb, h->si);
-}
-
 // ---- the core Hamiltonian from its connections ----
 // Two determinants with excitation level <= 2 share nel - 2 electrons.  Each
 // core determinant is listed once under every (nel - 2)-electron subset of
@@ -2155,28 +2025,36 @@ int most_populated_impl(ngpu_t* h, int64_t target, std::vector<uint64_t>& out) {
   }
   out.clear();
   if (n == 0) return NGPU_OK;
-  if (n > h->scap) return NGPU_ERR_SPAWN_FULL;  // the sort runs in the spawn-sort buffers
+  if (n > h->scap) return NGPU_ERR_SPAWN_FULL;  // the selection sorts at most a spawned list's length
   HIP_OK(hipMemcpy(counts.p, hc.data(), (size_t)ntiles * 8, hipMemcpyHostToDevice));
   hipLaunchKernelGGL(k_mp_write, dim3((unsigned)ntiles), dim3(kBlock), 0, h->stream, h->wk, (const Counters*)h->cnt,
                      W, h->S, (const int64_t*)counts.p, ckeys.p, wkey.p);
   const unsigned long long nn = (unsigned long long)n;
   HIP_OK(hipMemcpyAsync(n_dev.p, &nn, 8, hipMemcpyHostToDevice, h->stream));
   // determinant order first (the tie order), then weight (stable)
-  int cur = radix_sort_pairs<uint64_t, W, W == 2, 4>(h, ckeys.p, W, nullptr, word_passes(h), n_dev.p, n);
+  DevBuf<uint64_t> sk0, sk1;
+  DevBuf<uint32_t> si0, si1;
+  HIP_OK(sk0.alloc((size_t)n * W));
+  HIP_OK(sk1.alloc((size_t)n * W));
+  HIP_OK(si0.alloc((size_t)n));
+  HIP_OK(si1.alloc((size_t)n));
+  uint64_t* const kb[2] = {sk0.p, sk1.p};
+  uint32_t* const ib[2] = {si0.p, si1.p};
+  int cur = radix_sort_pairs_in<uint64_t, W, W == 2, 4>(h, ckeys.p, W, nullptr, word_passes(h), n_dev.p, n, kb, ib);
   hipLaunchKernelGGL(k_mp_gather, dim3(grid_for(n)), dim3(kBlock), 0, h->stream, (const uint64_t*)wkey.p,
-                     (const uint32_t*)h->si[cur], n, wperm.p);
+                     (const uint32_t*)ib[cur], n, wperm.p);
   std::vector<std::pair<int, int>> wp;
   for (int sh = 0; sh < 64; sh += 8) wp.push_back({0, sh});
-  const uint32_t* perm = h->si[cur];
+  const uint32_t* perm = ib[cur];
   // the weight passes must not overwrite the permutation they read first
   if (cur == 0) {
-    HIP_OK(hipMemcpyAsync(h->si[1], h->si[0], (size_t)n * 4, hipMemcpyDeviceToDevice, h->stream));
-    perm = h->si[1];
+    HIP_OK(hipMemcpyAsync(ib[1], ib[0], (size_t)n * 4, hipMemcpyDeviceToDevice, h->stream));
+    perm = ib[1];
   }
-  cur = radix_sort_pairs<uint64_t, 1, false, 4>(h, wperm.p, 1, perm, wp, n_dev.p, n);
+  cur = radix_sort_pairs_in<uint64_t, 1, false, 4>(h, wperm.p, 1, perm, wp, n_dev.p, n, kb, ib);
   const int64_t k = std::min(target, n);
   std::vector<uint32_t> idx((size_t)k);
-  HIP_OK(hipMemcpyAsync(idx.data(), h->si[cur], (size_t)k * 4, hipMemcpyDeviceToHost, h->stream));
+  HIP_OK(hipMemcpyAsync(idx.data(), ib[cur], (size_t)k * 4, hipMemcpyDeviceToHost, h->stream));
   std::vector<uint64_t> all((size_t)n * W);
   HIP_OK(hipMemcpyAsync(all.data(), ckeys.p, all.size() * 8, hipMemcpyDeviceToHost, h->stream));
   HIP_OK(hipStreamSynchronize(h->stream));
@@ -2670,10 +2548,6 @@ BatchGroup group_of(const ngpu_t* h) {
   g.lanes = h->single_lanes;
   g.pl = singles_pl(h->single_lanes, h->sys.nbasis / 2);
   g.items = h->radix_items;
-  g.rank_sort = h->rank_sort;
-  g.rank64 = h->rank64;
-  g.rank64_bits = h->rank64_bits;
-  if (!g.rank_sort) g.passes = word_passes(h);
   g.core = h->ncore > 0;
   g.core_fp32 = h->core_fp32;
   g.rec_words = h->ds.rec_words;
@@ -2682,9 +2556,7 @@ BatchGroup group_of(const ngpu_t* h) {
 
 bool same_group(const BatchGroup& a, const BatchGroup& b) {
   return a.W == b.W && a.S == b.S && a.gen == b.gen && a.lanes == b.lanes && a.pl == b.pl && a.items == b.items &&
-         a.rank_sort == b.rank_sort && a.rank64 == b.rank64 && a.rank64_bits == b.rank64_bits &&
-         a.passes == b.passes && a.core == b.core && a.core_fp32 == b.core_fp32 &&
-         a.rec_words == b.rec_words;
+         a.core == b.core && a.core_fp32 == b.core_fp32 && a.rec_words == b.rec_words;
 }
 
 void free_group(BatchGroup& g) {
@@ -2714,16 +2586,9 @@ EngDev eng_dev(const ngpu_t* h) {
   e.blk_rm = h->blk_rm;
   e.tile_p = h->tile_p;
   e.tcap = h->tcap;
-  e.sp_rec = h->sp_rec;
-  e.rk = h->rk;
+  e.bins = h->bins;
   e.scap = h->scap;
   e.sq = h->sq;
-  for (int q = 0; q < 2; ++q) {
-    e.sk[q] = h->sk[q];
-    e.si[q] = h->si[q];
-  }
-  e.hist = h->hist;
-  e.digit_tot = h->digit_tot;
   e.n_key = h->n_key;
   e.n_sgn = h->n_sgn;
   e.n_flag = h->n_flag;
@@ -2776,7 +2641,7 @@ int build_groups(ngpu_batch* b) {
       int nb[kLkKinds];
       nb[kLkChunk] = std::min(scaled(h->nb_chunk), h->max_chunk);
       nb[kLkGrid] = scaled(h->nb_grid);
-      nb[kLkMerge] = scaled(h->nb_merge ? h->nb_merge : h->nb_grid);
+      nb[kLkMerge] = std::min(scaled(h->nb_merge ? h->nb_merge : h->nb_grid), merge_blocks(h));
       nb[kLkCore] = (int)std::max<int64_t>(1, std::min<int64_t>((h->ncore + kBlock - 1) / kBlock, h->nb_grid));
       nb[kLkCoreRow] = (int)std::max<int64_t>(
           1, std::min<int64_t>((h->ncore + kBlock / kWave - 1) / (kBlock / kWave), 8 * (int64_t)h->nb_grid));
@@ -2847,61 +2712,17 @@ void glaunch(ngpu_t* h0, int open, int close, F kern, int nblocks, int threads, 
   launch_lds(h0, open, close, kern, dim3((unsigned)nblocks), dim3((unsigned)threads), lds, args...);
 }
 
-template <int W, int R, int IT>
-void group_sort_merge(BatchGroup& g) {
-  ngpu_t* h0 = g.hs[0];
-  const int E = (int)g.hs.size();
-  const EngDev* ed = g.d_ed;
-  int cur = 0;
-  if (g.rank_sort) {
-    glaunch(h0, 4, -1, km_radix_hist_ranks<IT>, g.tot[kLkChunk], kBlock, 0, ed, (const uint16_t*)g.d_map[kLkChunk]);
-    glaunch(h0, -1, -1, km_radix_scan, E * kSegs, kBlock, 0, ed, kSegs);
-    glaunch(h0, -1, -1, km_radix_scatter_ranks<IT>, g.tot[kLkChunk], kBlock, 0, ed,
-            (const uint16_t*)g.d_map[kLkChunk]);
-    glaunch(h0, -1, 4, km_seg_sort, E * kSegs, kSegThreads, 0, ed);
-    glaunch(h0, 6, 6, km_merge_annihilate<W, R, uint32_t, 1>, g.tot[kLkMerge], kBlock, 0, ed,
-            (const uint16_t*)g.d_map[kLkMerge], 0);
-    return;
-  }
-  if (g.rank64) {
-    // 64-bit rank keys into sk[0], the top-byte partition into sk[1], the
-    // segments sorted back into sk[0]
-    const int bits = g.rank64_bits;
-    glaunch(h0, 4, -1, km_rank64_hist<IT>, g.tot[kLkChunk], kBlock, 0, ed, (const uint16_t*)g.d_map[kLkChunk], bits);
-    glaunch(h0, -1, -1, km_radix_scan, E * kSegs, kBlock, 0, ed, kSegs);
-    glaunch(h0, -1, -1, km_radix_scatter_words<uint64_t, 1, false, IT, kSegBits>, g.tot[kLkChunk], kBlock, 0, ed,
-            (const uint16_t*)g.d_map[kLkChunk], 2, 0, 0, bits - kSegBits);
-    glaunch(h0, -1, 4, km_seg_sort64, E * kSegs, kSegThreads, 0, ed, (bits - kSegBits + 7) / 8);
-    glaunch(h0, 6, 6, km_merge_annihilate<W, R, uint64_t, W>, g.tot[kLkMerge], kBlock, 0, ed,
-            (const uint16_t*)g.d_map[kLkMerge], 0);
-    return;
-  }
-  const int np = (int)g.passes.size();
-  for (int p = 0; p < np; ++p) {
-    const int in = (p & 1) ^ 1;  // pass p writes sk[p & 1]
-    const int first = p == 0 ? 1 : 0;  // the first pass reads the records' words
-    glaunch(h0, p == 0 ? 4 : -1, -1, km_radix_hist_words<uint64_t, W, W == 2, IT, 8>, g.tot[kLkChunk], kBlock, 0,
-            ed, (const uint16_t*)g.d_map[kLkChunk], first, in, g.passes[p].first, g.passes[p].second);
-    glaunch(h0, -1, -1, km_radix_scan, E * kDigitBlocks, kBlock, 0, ed, kDigitBlocks);
-    glaunch(h0, -1, p + 1 == np ? 4 : -1, km_radix_scatter_words<uint64_t, W, W == 2, IT, 8>, g.tot[kLkChunk], kBlock,
-            0, ed, (const uint16_t*)g.d_map[kLkChunk], first, in, g.passes[p].first, g.passes[p].second);
-    cur = p & 1;
-  }
-  glaunch(h0, 6, 6, km_merge_annihilate<W, R, uint64_t, W>, g.tot[kLkMerge], kBlock, 0, ed,
-          (const uint16_t*)g.d_map[kLkMerge], cur);
-}
-
 template <int W, int R, int G>
 void group_spawn(BatchGroup& g) {
   glaunch(g.hs[0], 2, 2, km_spawn<W, R, G>, g.tot[kLkGrid], kBlock, 0, (const EngDev*)g.d_ed,
-          (const uint16_t*)g.d_map[kLkGrid], g.rank_sort ? 1 : 0);
+          (const uint16_t*)g.d_map[kLkGrid]);
 }
 
 template <int W, int R, int PL, int GL>
 void group_singles(BatchGroup& g, int nsp) {
   const size_t lds = 2 * sizeof(double) * (size_t)(kBlock / GL) * nsp;  // weights and running sums
   glaunch(g.hs[0], 3, 3, km_spawn_singles<W, R, PL, GL>, g.tot[kLkGrid], kBlock, lds, (const EngDev*)g.d_ed,
-          (const uint16_t*)g.d_map[kLkGrid], g.rank_sort ? 1 : 0);
+          (const uint16_t*)g.d_map[kLkGrid]);
 }
 
 template <int W, int R>
@@ -2956,9 +2777,7 @@ void group_chain_wr(BatchGroup& g) {
             (const double*)g.d_Y, g.ccols);
   else if (g.core)
     glaunch(h0, -1, -1, km_core_apply<R>, g.tot[kLkCore], kBlock, 0, ed, (const uint16_t*)m[kLkCore]);
-  if (g.items == 2) group_sort_merge<W, R, 2>(g);
-  else if (g.items == 8) group_sort_merge<W, R, 8>(g);
-  else group_sort_merge<W, R, 4>(g);
+  glaunch(h0, 6, 6, km_merge_annihilate<W, R>, g.tot[kLkMerge], kBlock, 0, ed, (const uint16_t*)m[kLkMerge]);
   glaunch(h0, 7, 7, km_insert<W, R>, g.tot[kLkGrid], kBlock, 0, ed, (const uint16_t*)m[kLkGrid]);
   glaunch(h0, 8, 8, km_stats<W, R>, g.tot[kLkGrid], kBlock, 0, ed, (const uint16_t*)m[kLkGrid]);
   glaunch(h0, -1, -1, km_end_iter, (int)g.hs.size(), kBlock, 0, ed);
@@ -3428,6 +3247,7 @@ int ngpu_annihilate(ngpu_t* h, uint32_t iter, const int64_t* sdet, const double*
     HIP_OK(hipMalloc((void**)&h->u_sgn, (size_t)h->scap * S * 8));
     HIP_OK(hipMalloc((void**)&h->u_flag, (size_t)h->scap * 4));
     HIP_OK(hipMalloc((void**)&h->u_count, 8));
+    HIP_OK(hipMalloc((void**)&h->l_rec, (size_t)h->scap * kRecWords * 8));
   }
   if (n) {
     const int rw = h->ds.rec_words;
@@ -3447,12 +3267,18 @@ int ngpu_annihilate(ngpu_t* h, uint32_t iter, const int64_t* sdet, const double*
         r[3] = sinfo[i];
       }
     }
-    HIP_OK(hipMemcpy(h->sp_rec, rec.data(), rec.size() * 8, hipMemcpyHostToDevice));
+    HIP_OK(hipMemcpy(h->l_rec, rec.data(), rec.size() * 8, hipMemcpyHostToDevice));
   }
   hipLaunchKernelGGL(k_begin_iter, dim3(1), dim3(kBlock), 0, h->stream, h->dout, h->dpart, h->cnt, h->dparams,
                      IterParams{}, 0);
   hipLaunchKernelGGL(k_set_count, dim3(1), dim3(1), 0, h->stream, &h->cnt->n_spawned, (unsigned long long)n);
   hipLaunchKernelGGL(k_set_count, dim3(1), dim3(1), 0, h->stream, h->u_count, 0ull);
+  hipLaunchKernelGGL(k_set_bins, dim3(1), dim3(1), 0, h->stream, h->cnt, h->bins, n);
+  if (n) {
+    auto kern = W == 1 ? k_bin_list<1> : k_bin_list<2>;
+    hipLaunchKernelGGL(kern, dim3(grid_for(n)), dim3(kBlock), 0, h->stream, h->ds, h->cnt, (const uint64_t*)h->l_rec, n,
+                       h->bins);
+  }
   bool p = h->prof;
   h->prof = false;
   // an explicit list carries no deterministic projection

@@ -8,11 +8,11 @@
 //   k_scan_apply exclusive scan of attempt counts -> attempt offsets; the
 //                freed slots into the free queue; the hash refill of a rebuild
 //   k_spawn      per attempt: parent by binary search, excitation, H_ij,
-//                stochastic rounding, LDS-staged append of spawn records;
-//                heat-bath singles are queued for k_spawn_singles
-//   k_radix_*    stable LSD radix sort of (colex rank or ilut_lt key, spawn index)
-//   k_merge_annihilate per run of equal keys: CompressSpawnedList /
-//                FindResidualParticle, then hash lookup, add/abort/remove
+//                stochastic rounding, spawn records staged in LDS and written
+//                into the bins of their determinants' hashes; heat-bath
+//                singles are queued for k_spawn_singles
+//   k_merge_annihilate per bin: CompressSpawnedList / FindResidualParticle in
+//                LDS, then hash lookup, add/abort/remove
 //   k_insert     new dets: slot from the free queue, bucketed open-addressing insert
 //   k_stats      per slot: occupied-threshold rounding, TotParts, norm, HF pop
 //   (k_end_iter in the engine: slot and hash bookkeeping, statistics sums)
@@ -80,11 +80,20 @@ struct alignas(256) Counters {
   unsigned int halt;
   unsigned int err_iter;
   unsigned long long n_rebuilds;  // walker-hash rebuilds since creation
+  // the iteration's spawn bins (set by the attempt scan): their number, the
+  // records each holds, and the log2 distance of their counters in words
+  unsigned int nbins;
+  unsigned int bin_cap;
+  unsigned int bin_shift;
+  // spawned records and attempts of the previous iteration: the expected
+  // number of records sizes the bins (speed only, results do not depend on it)
+  unsigned long long prev_spawned, prev_attempts;
   alignas(256) unsigned long long free_tail;
   alignas(256) unsigned long long n_spawned;
   alignas(256) unsigned long long n_singles;  // queued single-excitation attempts
   alignas(256) unsigned long long n_unique;
   alignas(256) unsigned long long n_new;
+  alignas(256) unsigned long long n_ovf;      // spawned records past their bin's end
   // per-block counts of tombstone entries taken by inserts, spread over
   // kSpread lines (one add per block)
   struct alignas(256) Spread { unsigned long long v; };
@@ -291,24 +300,27 @@ __device__ inline void free_flush(const Walk& wk, Counters* cnt, FreeStage* fs, 
 
 // hash lookup: returns slot or -1.  Entries of a bucket fill in order and
 // become empty only when the table is rebuilt, so the first empty entry ends
-// the probe sequence.
+// the probe sequence.  A bucket's slots and keys are loaded together (16-byte
+// loads of one line) and compared in registers: one round trip per bucket.
 template <int W>
 __device__ inline int64_t hash_lookup(const Walk& wk, const uint64_t* key, int64_t home, Counters* cnt) {
   int64_t b = home;
   int64_t maxp = wk.L < kMaxProbe ? wk.L : kMaxProbe;
   for (int64_t probe = 0; probe < maxp; ++probe) {
     const uint64_t* bk = wk.htab + (size_t)b * 8 * W;
-    const int32_t* sl = (const int32_t*)(bk + 4 * W);
+    const int4 sl = *(const int4*)(bk + 4 * W);
+    ulonglong2 k[2 * W];
+#pragma unroll
+    for (int q = 0; q < 2 * W; ++q) k[q] = ((const ulonglong2*)bk)[q];
+    const int32_t slot[kBucketEntries] = {sl.x, sl.y, sl.z, sl.w};
 #pragma unroll
     for (int e = 0; e < kBucketEntries; ++e) {
-      int32_t s = sl[e];
+      const int32_t s = slot[e];
       if (s == kSlotEmpty) return -1;
-      if (s >= 0) {
-        bool eq = true;
-#pragma unroll
-        for (int w = 0; w < W; ++w) eq = eq && (bk[e * W + w] == key[w]);
-        if (eq) return s;
-      }
+      bool eq;
+      if constexpr (W == 1) eq = ((e & 1) ? k[e / 2].y : k[e / 2].x) == key[0];
+      else eq = k[e].x == key[0] && k[e].y == key[1];
+      if (s >= 0 && eq) return s;
     }
     b = (b + 1 == wk.L) ? 0 : b + 1;
   }
@@ -369,6 +381,66 @@ __device__ inline void hash_refill_part(const Grid& g, const DevSys& s, const Wa
     if (hp < 0) atomicOr(&cnt->err, 1u << NGPU_ERR_HASH_FULL);
     else wk.hpos(slot) = hp;
   }
+}
+
+// ----------------------------------------------------------- spawn bins
+// The spawning kernels write each record straight into one of nbins bins,
+// chosen by a hash of its determinant, so equal determinants meet in one bin
+// and one wave merges a bin in LDS: no sort and no gather stands between
+// spawning and annihilation.  A record takes its place with one atomic on its
+// bin's counter; the counters are spread over as many cache lines as their
+// array has (an address, and so a line, takes one atomic in about 12 ns, and
+// scattered ones run at 25 G/s).  A bin that is full (one determinant spawned
+// very often, or a spawned list near its capacity) sends its further records
+// to one of kSpill spill areas, a full area to the overflow list; the wave of
+// a bin that spilled searches them for its own.  Order within a bin is the
+// order of arrival: the merge's sums do not depend on it beyond FP64 rounding.
+constexpr uint32_t kSpill = 1024;
+struct Bins {
+  uint64_t* rec;     // cap records, bin_cap to each bin
+  uint64_t* spill;   // kSpill areas of spill_cap records, area b % kSpill for bin b
+  uint64_t* ovf;     // overflow list (the spawn capacity)
+  uint32_t* count;   // records of bin b at [b << bin_shift], emptied by the merge
+  uint32_t* scount;  // records sent to each area, emptied at the iteration's end
+  int64_t cap;
+  uint32_t spill_cap;
+  uint32_t maxb;     // most bins
+  uint32_t words;    // length of count
+};
+// records per bin aimed at: a wave merges up to 64 in one pass over its lanes
+constexpr int kBinFill = 44;
+
+__device__ inline void set_bins(Counters* cnt, const Bins& b, double expect) {
+  double nb = expect * (1.0 / kBinFill) + 1.0;
+  const uint32_t n = nb < (double)b.maxb ? (uint32_t)nb : b.maxb;
+  uint32_t sh = 0;
+  while (sh < 5 && ((uint64_t)n << (sh + 1)) <= b.words) ++sh;
+  const int64_t c = b.cap / n;
+  cnt->nbins = n;
+  cnt->bin_cap = (uint32_t)(c < 0x7FFFFFFF ? c : 0x7FFFFFFF);
+  cnt->bin_shift = sh;
+}
+
+// hash of a determinant: the high word picks the bin, its fraction inside the
+// bin the first slot of the merge's table
+template <int W>
+__device__ inline uint32_t bin_hash(const uint64_t* d) {
+  uint64_t h = d[0] * 0x9E3779B97F4A7C15ull;
+  if constexpr (W == 2) {
+    h += (d[1] ^ (d[1] >> 29)) * 0xBF58476D1CE4E5B9ull;
+    h = (h ^ (h >> 31)) * 0x94D049BB133111EBull;
+  }
+  return (uint32_t)(h >> 32);
+}
+__device__ inline uint32_t bin_of(uint32_t h, uint32_t nb) { return (uint32_t)(((uint64_t)h * nb) >> 32); }
+
+// where the record with place pos of bin b goes
+__device__ inline uint64_t* bin_record(Counters* cnt, const Bins& bins, uint32_t b, uint32_t pos, uint32_t cap,
+                                       int rec_words) {
+  if (pos < cap) return bins.rec + ((size_t)b * cap + pos) * rec_words;
+  const uint32_t a = b % kSpill, p = atomicAdd(&bins.scount[a], 1u);
+  if (p < bins.spill_cap) return bins.spill + ((size_t)a * bins.spill_cap + p) * rec_words;
+  return bins.ovf + (size_t)atomicAdd(&cnt->n_ovf, 1ull) * rec_words;
 }
 
 __device__ inline void chunk_of(const Grid& g, int64_t n, int64_t& begin, int64_t& end) {
@@ -605,7 +677,7 @@ __global__ void __launch_bounds__(kBlock) k_prepass(DevSys s, Walk wk, Counters*
 // a rebuild is due, also the refill of the walker hash that the prepass
 // cleared, before any lookup of the iteration.
 template <int W>
-__device__ __forceinline__ void k_scan_apply_body(const Grid& g_, const DevSys& s, const Walk& wk, const int32_t* att_cnt, int64_t* att_off, const int64_t* part, const int64_t* part_rm, const uint8_t* pinfo, Counters* cnt, int S, int64_t* tile_p, int64_t tcap) {
+__device__ __forceinline__ void k_scan_apply_body(const Grid& g_, const DevSys& s, const Walk& wk, const int32_t* att_cnt, int64_t* att_off, const int64_t* part, const int64_t* part_rm, const uint8_t* pinfo, Counters* cnt, int S, int64_t* tile_p, int64_t tcap, const Bins& bins) {
   if (cnt->halt) return;
   __shared__ int64_t red[kBlock / kWave];
   int64_t nslots = (int64_t)cnt->nslots;
@@ -684,11 +756,14 @@ __device__ __forceinline__ void k_scan_apply_body(const Grid& g_, const DevSys& 
     cnt->n_attempts = (unsigned long long)run;
     cnt->free_tail = tail0 + (unsigned long long)run_rm;
     cnt->rm_pre = (unsigned long long)run_rm;
+    // spawns expected at the previous iteration's rate per attempt
+    set_bins(cnt, bins, cnt->prev_attempts ? (double)run * ((double)cnt->prev_spawned / (double)cnt->prev_attempts)
+                                           : 0.5 * (double)run);
   }
 }
 template <int W>
-__global__ void __launch_bounds__(kBlock) k_scan_apply(DevSys s, Walk wk, const int32_t* att_cnt, int64_t* att_off, const int64_t* part, const int64_t* part_rm, const uint8_t* pinfo, Counters* cnt, int S, int64_t* tile_p, int64_t tcap) {
-  k_scan_apply_body<W>(hw_grid(), s, wk, att_cnt, att_off, part, part_rm, pinfo, cnt, S, tile_p, tcap);
+__global__ void __launch_bounds__(kBlock) k_scan_apply(DevSys s, Walk wk, const int32_t* att_cnt, int64_t* att_off, const int64_t* part, const int64_t* part_rm, const uint8_t* pinfo, Counters* cnt, int S, int64_t* tile_p, int64_t tcap, Bins bins) {
+  k_scan_apply_body<W>(hw_grid(), s, wk, att_cnt, att_off, part, part_rm, pinfo, cnt, S, tile_p, tcap, bins);
 }
 
 // ------------------------------------------------------------- spawning
@@ -736,69 +811,79 @@ __device__ inline uint32_t rec_info(const DevSys& s, const uint64_t* r) {
   return s.spawn_fp32 ? (uint32_t)(r[W] >> 32) : (uint32_t)r[3];
 }
 
-// the spawn sort's 32-bit key is the colex rank times this odd constant: a
-// bijection of 32-bit values that spreads the keys' top byte evenly
-constexpr uint32_t kRankMul = 0x9E3779B1u;
-
-// colex rank of a determinant: sum over its i-th occupied orbital (bit p,
-// ascending) of C(p, i); injective on determinants of nel electrons
 template <int W>
-__device__ inline uint32_t colex_rank(const uint32_t* binom, int nel1, const uint64_t* d) {
-  uint32_t r = 0;
-  int c = 0;
-#pragma unroll
-  for (int w = 0; w < W; ++w) {
-    uint64_t x = d[w];
-    while (x) {
-      int p = 64 * w + ctz64(x);
-      x &= x - 1;
-      ++c;
-      r += binom[p * nel1 + c];
+__device__ inline void rec_store(const DevSys& s, uint64_t* r, const uint64_t* key, double val, uint32_t info) {
+  if (s.spawn_fp32) {  // the value is already FP32-representable (attempt_create)
+    const uint64_t last = ((uint64_t)info << 32) | __float_as_uint((float)val);
+    if constexpr (W == 1) {
+      *(ulonglong2*)r = ulonglong2{key[0], last};
+    } else {
+      r[0] = key[0];
+      r[1] = key[1];
+      r[2] = last;
     }
+  } else {
+    *(ulonglong2*)r = ulonglong2{key[0], W == 2 ? key[W - 1] : 0ull};
+    *(ulonglong2*)(r + 2) = ulonglong2{(uint64_t)__double_as_longlong(val), (uint64_t)info};
   }
-  return r;
+}
+// the mark of a record that found the merge's table full (the info word's top bit)
+constexpr uint32_t kInfoLeft = 1u << 31;
+template <int W>
+__device__ inline void rec_mark(const DevSys& s, uint64_t* r, bool on) {
+  const int w = s.spawn_fp32 ? W : 3;
+  const uint64_t bit = s.spawn_fp32 ? 1ull << 63 : (uint64_t)kInfoLeft;
+  r[w] = on ? r[w] | bit : r[w] & ~bit;
 }
 
-// binomial table of the colex rank, staged in LDS by the spawn kernels (the
-// engine ranks only when nbasis*(nel+1) fits)
-constexpr int kBinomLds = 512;
-struct BinomLds {
-  uint32_t c[kBinomLds];
-  __device__ void load(const DevSys& s, const uint32_t* rk) {
-    if (rk)
-      for (int i = threadIdx.x; i < s.nbasis * s.nel1; i += blockDim.x) c[i] = s.binom[i];
-    __syncthreads();
-  }
-};
-
-// block-wide: drain staged spawns into the spawned list when due; with rk,
-// also each spawn's colex rank (the first sort key) at the same index
+// block-wide: drain staged spawns into their bins when due.  A thread's
+// counter atomics are all issued before the first of its records is written.
 template <int W>
-__device__ inline void spawn_flush(SpawnStage<W>* ss, Counters* cnt, uint64_t* sp_rec, int64_t scap, bool force,
-                                   bool& overflow, const DevSys& s, const BinomLds& bl, uint32_t* rk) {
+__device__ inline void spawn_flush(SpawnStage<W>* ss, Counters* cnt, const Bins& bins, int64_t scap, bool force,
+                                   bool& overflow, const DevSys& s) {
   uint32_t n;
   unsigned long long base;
   if (!stage_flush_begin(&ss->st, &cnt->n_spawned, kSpawnStage, force, n, base)) return;
-  for (uint32_t i = threadIdx.x; i < n; i += blockDim.x) {
-    unsigned long long d = base + i;
-    if (d < (unsigned long long)scap) {
-      uint64_t* r = sp_rec + d * (unsigned long long)s.rec_words;
+  const uint32_t nb = cnt->nbins, cap = cnt->bin_cap, sh = cnt->bin_shift;
+  constexpr int kPer = (kSpawnStage + kBlock - 1) / kBlock;
+  uint32_t bin[kPer], pos[kPer];
 #pragma unroll
-      for (int w = 0; w < W; ++w) r[w] = ss->key[i * W + w];
-      if (s.spawn_fp32) {  // the value is already FP32-representable (attempt_create)
-        r[W] = ((uint64_t)ss->info[i] << 32) | __float_as_uint((float)ss->val[i]);
+  for (int j = 0; j < kPer; ++j) {
+    const uint32_t i = threadIdx.x + j * kBlock;
+    pos[j] = 0xFFFFFFFFu;
+    bin[j] = 0;
+    if (i < n) {
+      if (base + i < (unsigned long long)scap) {
+        bin[j] = bin_of(bin_hash<W>(ss->key + i * W), nb);
+        pos[j] = atomicAdd(&bins.count[(size_t)bin[j] << sh], 1u);
       } else {
-        if (W == 1) r[1] = 0;
-        r[2] = (uint64_t)__double_as_longlong(ss->val[i]);
-        r[3] = ss->info[i];
+        overflow = true;
       }
-      if (rk) rk[d] = colex_rank<W>(bl.c, s.nel1, ss->key + i * W) * kRankMul;
-    } else {
-      overflow = true;
+    }
+  }
+#pragma unroll
+  for (int j = 0; j < kPer; ++j) {
+    const uint32_t i = threadIdx.x + j * kBlock;
+    if (pos[j] != 0xFFFFFFFFu) {
+      uint64_t* r = bin_record(cnt, bins, bin[j], pos[j], cap, s.rec_words);
+      rec_store<W>(s, r, ss->key + i * W, ss->val[i], ss->info[i]);
     }
   }
   stage_flush_end(&ss->st);
 }
+
+// an explicit spawned list (n dense records) into the bins
+template <int W>
+__global__ void __launch_bounds__(kBlock) k_bin_list(DevSys s, Counters* cnt, const uint64_t* list, int64_t n, Bins bins) {
+  const uint32_t nb = cnt->nbins, cap = cnt->bin_cap, sh = cnt->bin_shift;
+  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
+    const uint64_t* q = list + i * s.rec_words;
+    const uint32_t bin = bin_of(bin_hash<W>(q), nb), pos = atomicAdd(&bins.count[(size_t)bin << sh], 1u);
+    uint64_t* r = bin_record(cnt, bins, bin, pos, cap, s.rec_words);
+    for (int w = 0; w < s.rec_words; ++w) r[w] = q[w];
+  }
+}
+__global__ void k_set_bins(Counters* cnt, Bins bins, int64_t n) { set_bins(cnt, bins, (double)n); }
 
 __device__ inline void queue_flush(QueueStage* qs, Counters* cnt, int64_t* sq, int64_t scap, bool force,
                                    bool& overflow) {
@@ -967,14 +1052,12 @@ __device__ inline void spawn_attempt(const DevSys& s, const Walk& wk, Counters* 
 // singles (the heat-bath list is ~20x longer per attempt) go to a queue so that
 // waves do not idle on a few long lanes
 template <int W, int R, int G>
-__device__ __forceinline__ void k_spawn_body(const Grid& g_, const DevSys& s, const Walk& wk, Counters* cnt, double* part, const int64_t* att_off, const int64_t* tile_p, int64_t tcap, const uint8_t* pinfo, uint64_t* sp_rec, uint32_t* rk, int64_t scap, int64_t* sq, const IterParams* prm) {
+__device__ __forceinline__ void k_spawn_body(const Grid& g_, const DevSys& s, const Walk& wk, Counters* cnt, double* part, const int64_t* att_off, const int64_t* tile_p, int64_t tcap, const uint8_t* pinfo, const Bins& bins, int64_t scap, int64_t* sq, const IterParams* prm) {
   if (cnt->halt) return;
   const double tau = prm->tau;
   const uint32_t iter = prm->iter;
   __shared__ double acc_lds[kStatStride];
   __shared__ SpawnStage<W> ss;
-  __shared__ BinomLds bl;
-  bl.load(s, rk);
   __shared__ QueueStage qs;
   BlockStats bs{acc_lds};
   bs.zero();
@@ -1033,18 +1116,18 @@ __device__ __forceinline__ void k_spawn_body(const Grid& g_, const DevSys& s, co
       k = (uint32_t)(a - att_off[p]);
     }
     spawn_attempt<W, R, G>(s, wk, cnt, bs, acc, pinfo, act, p, k, mode, &ss, &qs, tau, iter);
-    spawn_flush<W>(&ss, cnt, sp_rec, scap, false, overflow, s, bl, rk);
+    spawn_flush<W>(&ss, cnt, bins, scap, false, overflow, s);
     if (mode == 1) queue_flush(&qs, cnt, sq, scap, false, overflow);
   }
-  spawn_flush<W>(&ss, cnt, sp_rec, scap, true, overflow, s, bl, rk);
+  spawn_flush<W>(&ss, cnt, bins, scap, true, overflow, s);
   if (mode == 1) queue_flush(&qs, cnt, sq, scap, true, overflow);
   if (overflow) atomicOr(&cnt->err, 1u << NGPU_ERR_SPAWN_FULL);
   acc.done(bs, mode);
   bs.flush(part, g_.b);
 }
 template <int W, int R, int G>
-__global__ void __launch_bounds__(kBlock) k_spawn(DevSys s, Walk wk, Counters* cnt, double* part, const int64_t* att_off, const int64_t* tile_p, int64_t tcap, const uint8_t* pinfo, uint64_t* sp_rec, uint32_t* rk, int64_t scap, int64_t* sq, const IterParams* prm) {
-  k_spawn_body<W, R, G>(hw_grid(), s, wk, cnt, part, att_off, tile_p, tcap, pinfo, sp_rec, rk, scap, sq, prm);
+__global__ void __launch_bounds__(kBlock) k_spawn(DevSys s, Walk wk, Counters* cnt, double* part, const int64_t* att_off, const int64_t* tile_p, int64_t tcap, const uint8_t* pinfo, Bins bins, int64_t scap, int64_t* sq, const IterParams* prm) {
+  k_spawn_body<W, R, G>(hw_grid(), s, wk, cnt, part, att_off, tile_p, tcap, pinfo, bins, scap, sq, prm);
 }
 
 // Queued single excitations (molecular, heat-bath singles), G lanes per
@@ -1112,15 +1195,13 @@ __device__ inline void hb_corr(uint64_t x, int base, const double* row, int nsp,
 // PL: spatial orbitals per lane (nsp <= G*PL); dynamic LDS holds the
 // (kBlock/G)*nsp values of the block's attempts
 template <int W, int R, int PL, int G>
-__device__ __forceinline__ void k_spawn_singles_body(const Grid& g_, const DevSys& s, const Walk& wk, Counters* cnt, double* part, const uint8_t* pinfo, uint64_t* sp_rec, uint32_t* rk, int64_t scap, const int64_t* sq, const IterParams* prm) {
+__device__ __forceinline__ void k_spawn_singles_body(const Grid& g_, const DevSys& s, const Walk& wk, Counters* cnt, double* part, const uint8_t* pinfo, const Bins& bins, int64_t scap, const int64_t* sq, const IterParams* prm) {
   if (cnt->halt) return;
   constexpr int kGroups = kBlock / G;
   const double tau = prm->tau;
   const uint32_t iter = prm->iter;
   __shared__ double acc_lds[kStatStride];
   __shared__ SpawnStage<W> ss;
-  __shared__ BinomLds bl;
-  bl.load(s, rk);
   // per group: the signed H(src -> b) of its attempt, then their running sums
   extern __shared__ double hv_dyn[];
   BlockStats bs{acc_lds};
@@ -1273,32 +1354,23 @@ __device__ __forceinline__ void k_spawn_singles_body(const Grid& g_, const DevSy
         ss.info[idx] = info;
       }
     }
-    spawn_flush<W>(&ss, cnt, sp_rec, scap, false, overflow, s, bl, rk);  // its barriers also order the reuse of hv
+    spawn_flush<W>(&ss, cnt, bins, scap, false, overflow, s);  // its barriers also order the reuse of hv
   }
-  spawn_flush<W>(&ss, cnt, sp_rec, scap, true, overflow, s, bl, rk);
+  spawn_flush<W>(&ss, cnt, bins, scap, true, overflow, s);
   if (overflow) atomicOr(&cnt->err, 1u << NGPU_ERR_SPAWN_FULL);
   acc.done(bs, 2);
   bs.flush(part, g_.b);
 }
 template <int W, int R, int PL, int G>
-__global__ void __launch_bounds__(kBlock) k_spawn_singles(DevSys s, Walk wk, Counters* cnt, double* part, const uint8_t* pinfo, uint64_t* sp_rec, uint32_t* rk, int64_t scap, const int64_t* sq, const IterParams* prm) {
-  k_spawn_singles_body<W, R, PL, G>(hw_grid(), s, wk, cnt, part, pinfo, sp_rec, rk, scap, sq, prm);
+__global__ void __launch_bounds__(kBlock) k_spawn_singles(DevSys s, Walk wk, Counters* cnt, double* part, const uint8_t* pinfo, Bins bins, int64_t scap, const int64_t* sq, const IterParams* prm) {
+  k_spawn_singles_body<W, R, PL, G>(hw_grid(), s, wk, cnt, part, pinfo, bins, scap, sq, prm);
 }
 
 // ---------------------------------------------------------- radix sort
 // Stable LSD radix sort, 8-bit digits, reduce-then-scan: per-block digit
 // histograms, a per-digit scan over blocks, stable block-local scatter.  The
-// merge only needs equal determinants to be adjacent (and, within a run, the
-// spawn order, which a stable sort keeps), so the sort key may be any
-// injective function of the determinant.  When C(nbasis, nel) < 2^32 the key
-// is the determinant's 32-bit colex rank (sum over its i-th occupied bit at
-// position p of C(p, i)) times an odd constant; for one-word determinants
-// with C(nbasis, nel) < 2^64 whose rank is shorter than the word, the 64-bit
-// rank times an odd constant modulo 2^bits.  Both are sorted by one pass on
-// their top digit and a per-segment sort (k_seg_sort, k_seg_sort64).
-// Otherwise the key is the determinant itself, ordered as ilut_lt orders it,
-// in LSD passes.
-constexpr int kRadixBins = 1024;  // bins of the widest digit (10 bits)
+// set-up paths sort with it (the core space's selection and its connections).
+constexpr int kRadixBins = 256;  // digit values
 // radix tiles: IT elements per thread, IT*kBlock per tile (IT = 2, 4 or 8,
 // chosen per engine at run time)
 
@@ -1346,73 +1418,6 @@ __device__ __forceinline__ void k_radix_hist_body(const Grid& g_, const K* keys,
 template <typename K, int NW, bool FLIP, int IT, int DB>
 __global__ void __launch_bounds__(kBlock) k_radix_hist(const K* keys, int kstride, const unsigned long long* n_ptr, int64_t ncap, int word, int shift, uint32_t* hist) {
   k_radix_hist_body<K, NW, FLIP, IT, DB>(hw_grid(), keys, kstride, n_ptr, ncap, word, shift, hist);
-}
-
-// sort key of each spawned record's determinant: its colex rank
-// (binom[p*(nel+1)+i] = C(p, i)) times kRankMul, fused with the histogram of
-// the digit at shift
-template <int W, int IT, int DB>
-__device__ __forceinline__ void k_rank_hist_body(const Grid& g_, const uint64_t* keys, const unsigned long long* n_ptr, int64_t ncap, int rstride, const uint32_t* binom, int nel1, uint32_t* rank, uint32_t* hist, int shift) {
-  constexpr int RB = 1 << DB;
-  __shared__ uint32_t h[RB];
-  for (int i = threadIdx.x; i < RB; i += blockDim.x) h[i] = 0;
-  __syncthreads();
-  int64_t n = (int64_t)*n_ptr;
-  if (n > ncap) n = ncap;
-  int64_t begin, end;
-  radix_chunk<IT>(g_, n, begin, end);
-  for (int64_t i = begin + threadIdx.x; i < end; i += blockDim.x) {
-    uint32_t r = colex_rank<W>(binom, nel1, keys + i * rstride) * kRankMul;
-    rank[i] = r;
-    atomicAdd(&h[(r >> shift) & (RB - 1u)], 1u);
-  }
-  __syncthreads();
-  for (int d = threadIdx.x; d < RB; d += blockDim.x) hist[(size_t)d * g_.nb + g_.b] = h[d];
-}
-template <int W, int IT, int DB>
-__global__ void __launch_bounds__(kBlock) k_rank_hist(const uint64_t* keys, const unsigned long long* n_ptr, int64_t ncap, int rstride, const uint32_t* binom, int nel1, uint32_t* rank, uint32_t* hist, int shift) {
-  k_rank_hist_body<W, IT, DB>(hw_grid(), keys, n_ptr, ncap, rstride, binom, nel1, rank, hist, shift);
-}
-
-// the 64-bit colex-rank sort of one-word determinants (C(nbasis, nel) <
-// 2^64, the rank shorter than the word): each record's key, its colex rank
-// (binom[p*nel1 + i] = C(p, i) in 64 bits, staged in LDS) times an odd
-// constant modulo 2^bits (a bijection of bits-bit values that spreads the
-// ranks, which cluster, evenly over the top byte), written to rank[i] and
-// fused with the histogram of the top byte (the digit at shift = bits - 8).
-// The partition pass on that byte then leaves 256 segments for k_seg_sort64.
-constexpr int kBinom64Lds = 64 * 33;
-constexpr uint64_t kRank64Mul = 0x9E3779B97F4A7C15ull;
-template <int IT, int DB>
-__device__ __forceinline__ void k_rank64_hist_body(const Grid& g_, const uint64_t* rec, int rstride, const unsigned long long* n_ptr, int64_t ncap, const uint64_t* binom, int nbasis, int nel1, int bits, uint64_t* rank, uint32_t* hist) {
-  constexpr int RB = 1 << DB;
-  __shared__ uint32_t h[RB];
-  __shared__ uint64_t bt[kBinom64Lds];
-  for (int i = threadIdx.x; i < RB; i += blockDim.x) h[i] = 0;
-  for (int i = threadIdx.x; i < nbasis * nel1; i += blockDim.x) bt[i] = binom[i];
-  __syncthreads();
-  const uint64_t mask = bits >= 64 ? ~0ull : ((1ull << bits) - 1ull);
-  const int shift = bits - DB;
-  int64_t n = (int64_t)*n_ptr;
-  if (n > ncap) n = ncap;
-  int64_t begin, end;
-  radix_chunk<IT>(g_, n, begin, end);
-  for (int64_t i = begin + threadIdx.x; i < end; i += blockDim.x) {
-    uint64_t x = rec[i * rstride], r = 0;
-    for (int c = 1; x; ++c) {
-      r += bt[ctz64(x) * nel1 + c];
-      x &= x - 1;
-    }
-    r = (r * kRank64Mul) & mask;
-    rank[i] = r;
-    atomicAdd(&h[(uint32_t)(r >> shift) & (RB - 1u)], 1u);
-  }
-  __syncthreads();
-  for (int d = threadIdx.x; d < RB; d += blockDim.x) hist[(size_t)d * g_.nb + g_.b] = h[d];
-}
-template <int IT, int DB>
-__global__ void __launch_bounds__(kBlock) k_rank64_hist(const uint64_t* rec, int rstride, const unsigned long long* n_ptr, int64_t ncap, const uint64_t* binom, int nbasis, int nel1, int bits, uint64_t* rank, uint32_t* hist) {
-  k_rank64_hist_body<IT, DB>(hw_grid(), rec, rstride, n_ptr, ncap, binom, nbasis, nel1, bits, rank, hist);
 }
 
 // one block per digit: exclusive scan of that digit's per-block counts
@@ -1569,438 +1574,440 @@ __global__ void __launch_bounds__(kBlock) k_radix_scatter(const K* kin, int kstr
   k_radix_scatter_body<K, NW, FLIP, IT, DB>(hw_grid(), kin, kstride, iin, kout, iout, n_ptr, ncap, word, shift, hist, digit_tot);
 }
 
-// ------------------------------------------------------- partition sort
-// Sort of 32-bit keys in two launches after one stable radix pass on the
-// keys' top byte: that pass leaves segment b (the keys whose top byte is b)
-// contiguous and in input order, and block b of k_seg_sort sorts segment b
-// by the low 24 bits with three stable 8-bit passes, so the whole list ends
-// sorted and stable.  The passes run in LDS for segments of up to kSegCap
-// keys and through global memory (the input buffers serve as scratch) for
-// larger ones.  The keys are colex ranks times an odd constant (a bijection
-// of 32-bit values), so the top byte spreads the keys evenly over segments.
-// Both rank paths partition on a 9-bit top digit (512 segments) and sort up
-// to 2048 keys of a segment in LDS, so that two (64-bit keys) or three
-// (32-bit keys) 1024-thread blocks fit a compute unit.
-constexpr int kSegCap = 2048;
-constexpr int kSegBits = 9;  // top digit of the rank partitions
-constexpr int kSegs = 1 << kSegBits;
-
-constexpr int kSegThreads = 1024;  // threads of a k_seg_sort block
-constexpr int kSegWaves = kSegThreads / kWave;
-
-struct SegScratch {
-  uint32_t cnt[256];  // digit counts, then each digit's next position
-  uint32_t wcnt[kSegWaves][256];
-};
-
-// exclusive scan of the 256 digit counts by the first wave (4 per lane)
-__device__ inline void seg_scan_counts(SegScratch* sc) {
-  if (threadIdx.x < kWave) {
-    const int l = threadIdx.x;
-    uint32_t c0 = sc->cnt[4 * l], c1 = sc->cnt[4 * l + 1], c2 = sc->cnt[4 * l + 2], c3 = sc->cnt[4 * l + 3];
-    uint32_t s = c0 + c1 + c2 + c3, x = s;
-#pragma unroll
-    for (int o = 1; o < kWave; o <<= 1) {
-      uint32_t y = __shfl_up(x, o);
-      if (l >= o) x += y;
-    }
-    uint32_t pre = x - s;
-    sc->cnt[4 * l] = pre;
-    sc->cnt[4 * l + 1] = pre + c0;
-    sc->cnt[4 * l + 2] = pre + c0 + c1;
-    sc->cnt[4 * l + 3] = pre + c0 + c1 + c2;
-  }
-}
-
-// one stable 8-bit pass, src -> dst (LDS or global), in tiles of one key per
-// thread: ballots rank the keys of a digit within each wave, the waves'
-// counts in LDS order the waves.  Every thread of the block calls it.
-template <typename K>
-__device__ inline void seg_pass(const K* sk, const uint32_t* si, K* dk, uint32_t* di, int64_t n, int shift,
-                                SegScratch* sc) {
-  const int wv = threadIdx.x / kWave;
-  const uint64_t ltmask = lanemask_lt();
-  for (int t = threadIdx.x; t < 256; t += blockDim.x) sc->cnt[t] = 0;
-  for (int t = threadIdx.x; t < kSegWaves * 256; t += blockDim.x) (&sc->wcnt[0][0])[t] = 0;
-  __syncthreads();
-  for (int64_t i = threadIdx.x; i < n; i += blockDim.x) atomicAdd(&sc->cnt[(uint32_t)(sk[i] >> shift) & 255u], 1u);
-  __syncthreads();
-  seg_scan_counts(sc);
-  __syncthreads();
-  for (int64_t t0 = 0; t0 < n; t0 += blockDim.x) {
-    const int64_t i = t0 + threadIdx.x;
-    const bool valid = i < n;
-    const K k = valid ? sk[i] : (K)0;
-    const uint32_t v = valid ? si[i] : 0u;
-    const uint32_t d = (uint32_t)(k >> shift) & 255u;
-    uint64_t peers = __ballot(valid);
-#pragma unroll
-    for (int bit = 0; bit < 8; ++bit) {
-      uint64_t m = __ballot(valid && ((d >> bit) & 1u));
-      peers &= ((d >> bit) & 1u) ? m : ~m;
-    }
-    const int rank = popc64(peers & ltmask);
-    if (valid && rank == 0) sc->wcnt[wv][d] = (uint32_t)popc64(peers);
-    __syncthreads();
-    if (valid) {
-      uint32_t o = sc->cnt[d] + (uint32_t)rank;
-      for (int q = 0; q < wv; ++q) o += sc->wcnt[q][d];
-      dk[o] = k;
-      di[o] = v;
-    }
-    __syncthreads();
-    for (int t = threadIdx.x; t < 256; t += blockDim.x) {
-      uint32_t add = 0;
-      for (int q = 0; q < kSegWaves; ++q) {
-        add += sc->wcnt[q][t];
-        sc->wcnt[q][t] = 0;
-      }
-      sc->cnt[t] += add;
-    }
-    __syncthreads();
-  }
-}
-
-// block b sorts segment b (one block of kSegThreads per segment) by the npass
-// bytes below the top digit; digit_tot holds the segment sizes, the counts of
-// the top-digit pass.  Keys of 32 bits (colex rank times an odd constant,
-// three passes) or 64 bits (the 64-bit rank path).
-template <typename K>
-__device__ __forceinline__ void k_seg_sort_body(const Grid& g_, K* kin, uint32_t* iin, K* kout, uint32_t* iout, const uint32_t* digit_tot, int npass) {
-  constexpr int CAP = kSegCap;
-  __shared__ K ka[CAP], kb[CAP];
-  __shared__ uint32_t ia[CAP], ib[CAP];
-  __shared__ SegScratch sc;
-  __shared__ int64_t seg[2];
-  __shared__ int64_t wsum[kSegWaves];
-  {  // this segment's start: the sizes of the segments before it
-    int64_t v = 0;
-    for (int b = threadIdx.x; b < (int)g_.b; b += blockDim.x) v += digit_tot[b];
-#pragma unroll
-    for (int o = kWave / 2; o > 0; o >>= 1) v += __shfl_xor(v, o);
-    if (lane_id() == 0) wsum[threadIdx.x / kWave] = v;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-      int64_t st = 0;
-      for (int q = 0; q < kSegWaves; ++q) st += wsum[q];
-      seg[0] = st;
-      seg[1] = digit_tot[g_.b];
-    }
-    __syncthreads();
-  }
-  const int64_t start = seg[0], n = seg[1];
-  if (n == 0) return;  // block-uniform
-  K *gk = kin + start, *ok = kout + start;
-  uint32_t *gi = iin + start, *oi = iout + start;
-  if (n <= CAP) {
-    for (int64_t i = threadIdx.x; i < n; i += blockDim.x) {
-      ka[i] = gk[i];
-      ia[i] = gi[i];
-    }
-    __syncthreads();
-    K *sk = ka, *dk = kb;
-    uint32_t *si = ia, *di = ib;
-    for (int p = 0; p < npass; ++p) {
-      seg_pass<K>(sk, si, dk, di, n, 8 * p, &sc);
-      K* tk = sk; sk = dk; dk = tk;
-      uint32_t* ti = si; si = di; di = ti;
-    }
-    for (int64_t i = threadIdx.x; i < n; i += blockDim.x) {
-      ok[i] = sk[i];
-      oi[i] = si[i];
-    }
-  } else {  // through global memory, the input serving as scratch
-    K *sk = gk, *dk = ok;
-    uint32_t *si = gi, *di = oi;
-    for (int p = 0; p < npass; ++p) {
-      seg_pass<K>(sk, si, dk, di, n, 8 * p, &sc);
-      K* tk = sk; sk = dk; dk = tk;
-      uint32_t* ti = si; si = di; di = ti;
-    }
-    if (sk != ok) {  // an even number of passes ended in the input
-      for (int64_t i = threadIdx.x; i < n; i += blockDim.x) {
-        ok[i] = sk[i];
-        oi[i] = si[i];
-      }
-    }
-  }
-}
-__global__ void __launch_bounds__(kSegThreads) k_seg_sort(uint32_t* kin, uint32_t* iin, uint32_t* kout, uint32_t* iout, const uint32_t* digit_tot) {
-  k_seg_sort_body<uint32_t>(hw_grid(), kin, iin, kout, iout, digit_tot, (32 - kSegBits + 7) / 8);
-}
-__global__ void __launch_bounds__(kSegThreads) k_seg_sort64(uint64_t* kin, uint32_t* iin, uint64_t* kout, uint32_t* iout, const uint32_t* digit_tot, int npass) {
-  k_seg_sort_body<uint64_t>(hw_grid(), kin, iin, kout, iout, digit_tot, npass);
-}
-
 // ------------------------------------------------------------- merging
-// LDS stage of a determinant list (key, S signs, flag): the merged spawns and
-// the new determinants
+// CompressSpawnedList (Annihilation.F90:249-515) + FindResidualParticle
+// (:551-634), then AnnihilateSpawnedParts (:965-1352): one wave per spawn bin
+// merges the bin's records by determinant in an LDS table, then looks each
+// determinant up in the walker hash.
+//
+// The time goes into random accesses of the walker table (a bucket line and a
+// state row per determinant), so the point is to have many in flight and
+// nothing else in their way: waves share no barrier, a bin's records are read
+// as one contiguous run, and equal determinants meet in LDS instead of in a
+// serial run-length loop over gathered records.  Measured against the sort of
+// (key, index) pairs and the merge of its runs that it replaced (us per
+// iteration, sort + merge before, now): 14e/30o, 1.34e6 spawns 124 + 115, 85;
+// 10e/20o, 5.0e5 spawns 48 + 45, 38; 18-site chain, 5.1e5 spawns 109 + 101,
+// 39; two-word 26e/40o, 3.0e5 spawns 213 + 41, 39; 1400 spawns 36 + 14, 10.
+// Writing the bins costs the spawning kernels 5 to 20 us of that.
+
+// One wave's table of the determinants of a bin.  It is left empty by the
+// lanes that take the merged determinants out.
 template <int W, int R>
-struct ListStage {
-  static constexpr int kCap = R == 1 ? 768 : 256;
-  Stage st;
-  uint64_t key[kCap * W];
-  double sgn[kCap * R];
-  uint32_t flag[kCap];
+struct MergeTab {
+  static constexpr int kSize = R <= 2 ? 128 : 64;
+  uint64_t key[kSize * W];
+  double sum[kSize * R];
+  uint32_t tag[kSize];   // bits 0-15 initiator flags, kTag* bits
+  uint8_t list[kSize];   // the slots in use, in order of arrival
+};
+// an empty slot's key: one-word determinants have at most 63 orbitals
+constexpr unsigned long long kTabEmpty = ~0ull;
+constexpr uint32_t kTagMulti = 1u << 16;  // more than one record
+constexpr uint32_t kTagTaken = 1u << 17;  // two-word keys: claimed,
+constexpr uint32_t kTagKey = 1u << 18;    // then key written
+
+// a determinant list (key, S signs, flag) and a list of freed slots, staged
+// per wave; each list's place in memory is reserved once per flush.  Rows of
+// many signs are not staged: they would take the LDS of the wave's table.
+template <int W, int R>
+struct WaveStage {
+  static constexpr int kCap = R <= 2 ? 128 : 0;
+  uint64_t key[kCap ? kCap * W : 1];
+  double sgn[kCap ? kCap * R : 1];
+  uint32_t flag[kCap ? kCap : 1];
+  int32_t freed[128];
 };
 
+// the staged determinants (n of them, wave-uniform) to the list at base
 template <int W, int R>
-__device__ inline int list_push(ListStage<W, R>* ls, bool pred, const uint64_t* key, const double* sg,
-                                uint32_t flag, int S) {
-  int i = stage_push(pred, &ls->st);
-  if (pred) {
+__device__ inline void wave_list_write(const WaveStage<W, R>* ws, int n, unsigned long long base, uint64_t* okey,
+                                       double* osgn, uint32_t* oflag, int S) {
+  for (int i = lane_id(); i < n; i += kWave) {
+    const unsigned long long d = base + (unsigned long long)i;
 #pragma unroll
-    for (int w = 0; w < W; ++w) ls->key[i * W + w] = key[w];
-    for (int r = 0; r < S; ++r) ls->sgn[i * R + r] = sg[r];
-    ls->flag[i] = flag;
+    for (int w = 0; w < W; ++w) okey[d * W + w] = ws->key[i * W + w];
+    for (int r = 0; r < S; ++r) osgn[d * S + r] = ws->sgn[i * R + r];
+    oflag[d] = ws->flag[i];
   }
-  return i;
 }
-
 template <int W, int R>
-__device__ inline void list_flush(ListStage<W, R>* ls, unsigned long long* gctr, uint64_t* okey, double* osgn,
-                                  uint32_t* oflag, int S, bool force) {
-  uint32_t n;
-  unsigned long long base;
-  if (!stage_flush_begin(&ls->st, gctr, ListStage<W, R>::kCap, force, n, base)) return;
-  for (uint32_t i = threadIdx.x; i < n; i += blockDim.x) {
-    unsigned long long d = base + i;
-#pragma unroll
-    for (int w = 0; w < W; ++w) okey[d * W + w] = ls->key[i * W + w];
-    for (int r = 0; r < S; ++r) osgn[d * S + r] = ls->sgn[i * R + r];
-    oflag[d] = ls->flag[i];
-  }
-  stage_flush_end(&ls->st);
+__device__ inline void wave_free_write(const Walk& wk, const WaveStage<W, R>* ws, int n, unsigned long long base) {
+  for (int i = lane_id(); i < n; i += kWave)
+    wk.freeq[(base + (unsigned long long)i) % (unsigned long long)wk.cap] = ws->freed[i];
+}
+__device__ inline unsigned long long wave_reserve(unsigned long long* ctr, int n) {
+  unsigned long long b = 0;
+  if (lane_id() == 0) b = atomicAdd(ctr, (unsigned long long)n);
+  return __shfl(b, 0);
+}
+// orders one wave's LDS accesses of different lanes
+__device__ inline void wave_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
 }
 
-// CompressSpawnedList (Annihilation.F90:249-515) + FindResidualParticle
-// (:551-634): the head of each run of equal keys sums the run in sorted
-// (= emission, the sort is stable) order.
-template <typename K, int NW>
-__device__ inline bool key_eq(const K* a, const K* b) {
-  bool e = true;
-#pragma unroll
-  for (int w = 0; w < NW; ++w) e = e && (a[w] == b[w]);
-  return e;
-}
-
-// The merged (compressed) spawned list alone, for the explicit-list entry
-// point: run heads sum their runs as k_merge_annihilate does, and the list
-// goes to memory; no statistics (k_merge_annihilate counts them).
-template <int W, int R, typename K, int NW>
-__device__ __forceinline__ void k_merge_list_body(const Grid& g_, const DevSys& s, Counters* cnt, const K* skey, const uint32_t* sidx, const uint64_t* sp_rec, int64_t scap, uint64_t* u_key, double* u_sgn, uint32_t* u_flag, unsigned long long* u_count) {
-  if (cnt->halt) return;
-  __shared__ ListStage<W, R> ls;
-  stage_init(&ls.st);
-  const int S = R == 1 ? 1 : s.S;
-  int64_t n = (int64_t)cnt->n_spawned;
-  if (n > scap) n = scap;
-  int64_t trips = grid_trips(g_, n);
-  for (int64_t t = 0; t < trips; ++t) {
-    int64_t i = grid_elem(g_, t);
-    bool keep = false;
-    double sum[R];
-    uint32_t flag = 0;
-    uint64_t key[W];
-    if (i < n) {
-      const K* ki = skey + i * NW;
-      bool head = true;
-      if (i > 0) head = !key_eq<K, NW>(ki, skey + (i - 1) * NW);
-      if (head) {
-        int64_t j = i + 1;
-        while (j < n && key_eq<K, NW>(ki, skey + j * NW)) ++j;
-        const uint64_t* kd = sp_rec + (size_t)sidx[i] * s.rec_words;
-#pragma unroll
-        for (int w = 0; w < W; ++w) key[w] = kd[w];
-        for (int r = 0; r < S; ++r) sum[r] = 0.0;
-        for (int64_t q = i; q < j; ++q) {
-          const uint64_t* rq = sp_rec + (size_t)sidx[q] * s.rec_words;
-          uint32_t inf = rec_info<W>(s, rq);
-          int r = (int)(inf & 0xFFu);
-          double nv = rec_val<W>(s, rq);
-          double cv = sum[r];
-          if (j == i + 1) {
-            if (inf & kInfoInit) flag |= 1u << r;
-          } else if (s.t_init) {
-            if ((fabs(cv) > 1.e-12 && fabs(nv) > 1.e-12) || (inf & kInfoInit)) flag |= 1u << r;
-          }
-          sum[r] = cv + nv;
-        }
-        if (j == i + 1) {
-          keep = !(fabs(sum[rec_info<W>(s, kd) & 0xFFu]) < 1.e-12);
+// the table slot of each todo lane's key (one record per lane): inserted if
+// absent.  won: this lane inserted it; -1: the table is full of other keys.
+// Every lane probes slot by slot, so either all records of a determinant find
+// its slot in a round or none does.
+template <int W, int R>
+__device__ inline int merge_slot(MergeTab<W, R>* tb, bool todo, const uint64_t* key, uint32_t first, bool& won) {
+  constexpr int T = MergeTab<W, R>::kSize;
+  int slot = (int)first, found = -1, probes = 0;
+  won = false;
+  while (__ballot(todo)) {
+    if (todo) {
+      bool next = false;
+      if constexpr (W == 1) {
+        const uint64_t old = atomicCAS((unsigned long long*)&tb->key[slot], kTabEmpty, (unsigned long long)key[0]);
+        if (old == kTabEmpty || old == key[0]) {
+          found = slot;
+          won = old == kTabEmpty;
+          todo = false;
         } else {
-          double tot = 0.0;
-          for (int r = 0; r < S; ++r) tot += fabs(sum[r]);
-          keep = tot > 1.e-12;
-        }
-      }
-    }
-    list_push<W, R>(&ls, keep, key, sum, flag, S);
-    list_flush<W, R>(&ls, u_count, u_key, u_sgn, u_flag, S, false);
-  }
-  list_flush<W, R>(&ls, u_count, u_key, u_sgn, u_flag, S, true);
-}
-template <int W, int R, typename K, int NW>
-__global__ void __launch_bounds__(kBlock) k_merge_list(DevSys s, Counters* cnt, const K* skey, const uint32_t* sidx, const uint64_t* sp_rec, int64_t scap, uint64_t* u_key, double* u_sgn, uint32_t* u_flag, unsigned long long* u_count) {
-  k_merge_list_body<W, R, K, NW>(hw_grid(), s, cnt, skey, sidx, sp_rec, scap, u_key, u_sgn, u_flag, u_count);
-}
-
-// CompressSpawnedList (Annihilation.F90:249-515) + FindResidualParticle
-// (:551-634), then AnnihilateSpawnedParts (:965-1352), in one pass over the
-// sorted spawns: the head of each run of equal keys sums the run in sorted
-// (= emission, the sort is stable) order, then looks its determinant up in the
-// walker hash; found determinants are updated in place (each key is owned by
-// one lane), absent ones go to the new list.  The lookups of one wave overlap
-// the record gathers of the others, and the merged list never goes to memory.
-template <int W, int R, typename K, int NW>
-__device__ __forceinline__ void k_merge_annihilate_body(const Grid& g_, const DevSys& s, const Walk& wk, Counters* cnt, double* part, const K* skey, const uint32_t* sidx, const uint64_t* sp_rec, int64_t scap, uint64_t* n_key, double* n_sgn, uint32_t* n_flag, const IterParams* prm) {
-  if (cnt->halt) return;
-  const uint32_t iter = prm->iter;
-  __shared__ double acc_lds[kStatStride];
-  __shared__ ListStage<W, R> ls;
-  __shared__ FreeStage fs;
-  __shared__ unsigned int blk_unique;
-  BlockStats bs{acc_lds};
-  bs.zero();
-  stage_init(&ls.st);
-  stage_init(&fs.st);
-  if (threadIdx.x == 0) blk_unique = 0;
-  const int S = R == 1 ? 1 : s.S;
-  int64_t n = (int64_t)cnt->n_spawned;
-  if (n > scap) n = scap;
-  int64_t trips = grid_trips(g_, n);
-  double ann[R], st_ab[R], st_an[R], st_rm[R], st_bn[R];
-  for (int r = 0; r < S; ++r) ann[r] = st_ab[r] = st_an[r] = st_rm[r] = st_bn[r] = 0.0;
-  for (int64_t t = 0; t < trips; ++t) {
-    int64_t i = grid_elem(g_, t);
-    bool keep = false;
-    double ss[R];
-    uint32_t sflag = 0;
-    uint64_t key[W];
-    if (i < n) {
-      const K* ki = skey + i * NW;
-      bool head = true;
-      if (i > 0) head = !key_eq<K, NW>(ki, skey + (i - 1) * NW);
-      if (head) {
-        int64_t j = i + 1;
-        while (j < n && key_eq<K, NW>(ki, skey + j * NW)) ++j;
-        const uint64_t* kd = sp_rec + (size_t)sidx[i] * s.rec_words;
-#pragma unroll
-        for (int w = 0; w < W; ++w) key[w] = kd[w];
-        for (int r = 0; r < S; ++r) ss[r] = 0.0;
-        if (j == i + 1) {
-          uint32_t inf = rec_info<W>(s, kd);
-          int r = (int)(inf & 0xFFu);
-          ss[r] = rec_val<W>(s, kd);
-          if (inf & kInfoInit) sflag |= 1u << r;
-          keep = !(fabs(ss[r]) < 1.e-12);
-        } else {
-          for (int64_t q = i; q < j; ++q) {
-            const uint64_t* rq = sp_rec + (size_t)sidx[q] * s.rec_words;
-            uint32_t inf = rec_info<W>(s, rq);
-            int r = (int)(inf & 0xFFu);
-            double nv = rec_val<W>(s, rq);
-            double cv = ss[r];
-            if (s.t_init) {
-              if ((fabs(cv) > 1.e-12 && fabs(nv) > 1.e-12) || (inf & kInfoInit)) sflag |= 1u << r;
-            }
-            if (cv * nv < 0.0) {
-              double x = fabs(cv), y = fabs(nv);
-              ann[r] += 2.0 * (x < y ? x : y);
-            }
-            ss[r] = cv + nv;
-          }
-          double tot = 0.0;
-          for (int r = 0; r < S; ++r) tot += fabs(ss[r]);
-          keep = tot > 1.e-12;
-        }
-      }
-    }
-    unsigned int nk = (unsigned int)wave_count(keep);
-    if (nk && lane_id() == 0) atomicAdd(&blk_unique, nk);
-    bool isnew = false, rm = false;
-    int64_t pos = -1;
-    if (keep) {
-      int64_t home = find_walker_hash<W>(key, s.rh, s.L) - 1;
-      pos = hash_lookup<W>(wk, key, home, cnt);
-      if (pos >= 0) {
-        double cs[R];
-        double tot = 0.0;
-        for (int r = 0; r < S; ++r) { cs[r] = wk.sgn(pos, r); tot += fabs(cs[r]); }
-        bool determ = (wk.flags(pos) & kFlagCore) != 0;
-        if (tot >= 1.e-12 || determ) {
-          for (int r = 0; r < S; ++r) {
-            double prod = cs[r] * ss[r];
-            if (fabs(cs[r]) < 1.0e-12 && s.t_init && !((sflag >> r) & 1u) && !determ) {
-              st_ab[r] += fabs(ss[r]);
-              ss[r] = 0.0;
-            }
-            if (prod < 0.0) {
-              double x = fabs(cs[r]), y = fabs(ss[r]);
-              st_an[r] += 2.0 * (x < y ? x : y);
-            }
-          }
-          bool occ = false;
-          for (int r = 0; r < S; ++r) {
-            cs[r] = ss[r] + cs[r];
-            wk.sgn(pos, r) = cs[r];
-            occ = occ || !(fabs(cs[r]) < 1.e-12);
-          }
-          rm = !determ && !occ;
+          next = true;
         }
       } else {
-        if (s.t_init)
-          for (int r = 0; r < S; ++r)
-            if (!((sflag >> r) & 1u)) {
-              st_ab[r] += fabs(ss[r]);
-              ss[r] = 0.0;
-            }
-        bool occ = false;
-        for (int r = 0; r < S; ++r) occ = occ || !(fabs(ss[r]) < 1.e-12);
-        if (occ) {
-          // stochRoundSpawn (Annihilation.F90:1354-1418)
-          double thr = s.occ_thresh;
-          for (int r = 0; r < S; ++r) {
-            if (fabs(ss[r]) > 1.e-12 && fabs(ss[r]) < thr) {
-              double pRemove = 1.0 - fabs(ss[r]) / thr;
-              double u, dummy;
-              draw2<W>(s.seed, key, iter, r, 0, 4, u, dummy);
-              if (pRemove > u) {
-                st_rm[r] += fabs(ss[r]);
-                ss[r] = 0.0;
-              } else {
-                st_bn[r] += thr - fabs(ss[r]);
-                ss[r] = ss[r] >= 0.0 ? thr : -thr;
-              }
-            }
+        const uint32_t t = __hip_atomic_load(&tb->tag[slot], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        if (t & kTagKey) {
+          if (det_eq<W>(&tb->key[slot * W], key)) {
+            found = slot;
+            todo = false;
+          } else {
+            next = true;
           }
-          occ = false;
-          for (int r = 0; r < S; ++r) occ = occ || !(fabs(ss[r]) < 1.e-12);
-          isnew = occ;
-        }
+        } else if (!(t & kTagTaken) && atomicCAS(&tb->tag[slot], 0u, kTagTaken) == 0u) {
+#pragma unroll
+          for (int w = 0; w < W; ++w) tb->key[slot * W + w] = key[w];
+          __threadfence_block();
+          atomicOr(&tb->tag[slot], kTagKey);
+          found = slot;
+          won = true;
+          todo = false;
+        }  // else claimed by a lane of this step, whose key is there at the next
+      }
+      if (next) {
+        slot = (slot + 1) & (T - 1);
+        if (++probes == T) todo = false;
       }
     }
-    remove_dets<W>(wk, &fs, rm, pos);
-    list_push<W, R>(&ls, isnew, key, ss, sflag & 0xFFFFu, S);
-    free_flush(wk, cnt, &fs, false);
-    list_flush<W, R>(&ls, &cnt->n_new, n_key, n_sgn, n_flag, S, false);
   }
-  free_flush(wk, cnt, &fs, true);
-  list_flush<W, R>(&ls, &cnt->n_new, n_key, n_sgn, n_flag, S, true);
-  for (int r = 0; r < S; ++r) {
-    bs.add(soff(F_NABORTED, r), st_ab[r]);
-    bs.add(soff(F_NANNIHIL, r), st_an[r] + ann[r]);
-    bs.add(soff(F_NREMOVED, r), st_rm[r]);
-    bs.add(soff(F_NBORN, r), st_bn[r]);
+  return found;
+}
+
+// LIST: only the merged list is written (the explicit-list entry point), the
+// bins stay as they are and nothing is counted
+template <int W, int R, bool LIST>
+__device__ __forceinline__ void k_merge_body(const Grid& g_, const DevSys& s, const Walk& wk, Counters* cnt, double* part, const Bins& bins, uint64_t* n_key, double* n_sgn, uint32_t* n_flag, unsigned long long* n_ctr, const IterParams* prm) {
+  constexpr int kWaves = kBlock / kWave;
+  const uint32_t nb = cnt->nbins, cap = cnt->bin_cap, sh = cnt->bin_shift;
+  if (cnt->halt || g_.b * kWaves >= (int64_t)nb) return;
+  constexpr int T = MergeTab<W, R>::kSize;
+  constexpr int kCap = WaveStage<W, R>::kCap;
+  __shared__ MergeTab<W, R> tabs[kWaves];
+  __shared__ WaveStage<W, R> stages[kWaves];
+  __shared__ double acc_lds[LIST ? 1 : kStatStride];
+  __shared__ uint32_t tail_n[kWaves][2];
+  __shared__ unsigned long long tail_base[2];
+  __shared__ unsigned int blk_unique;
+  const uint32_t iter = LIST ? 0u : prm->iter;
+  const int wv = threadIdx.x / kWave, lane = lane_id();
+  MergeTab<W, R>* tb = &tabs[wv];
+  WaveStage<W, R>* ws = &stages[wv];
+  BlockStats bs{acc_lds};
+  if constexpr (!LIST) bs.zero();
+  if (threadIdx.x == 0) blk_unique = 0;
+  for (int i = lane; i < T; i += kWave) {
+    for (int w = 0; w < W; ++w) tb->key[i * W + w] = kTabEmpty;
+    for (int r = 0; r < R; ++r) tb->sum[i * R + r] = 0.0;
+    tb->tag[i] = 0;
   }
   __syncthreads();
-  if (threadIdx.x == 0 && blk_unique)
-    atomicAdd(&cnt->uniq_part[g_.b % Counters::kSpread].v, (unsigned long long)blk_unique);
-  bs.flush(part, g_.b);
+  const int S = R == 1 ? 1 : s.S;
+  int n_list = 0, n_free = 0;  // staged (wave-uniform)
+  unsigned int uniq = 0;
+  double ann[R], st_ab[R], st_an[R], st_rm[R], st_bn[R];
+  for (int r = 0; r < S; ++r) ann[r] = st_ab[r] = st_an[r] = st_rm[r] = st_bn[r] = 0.0;
+  // The wave's bins, 64 counters per load; the records of the next bin are on
+  // their way while a bin's determinants are looked up.
+  const int64_t nwaves = g_.nb * kWaves;
+  const int64_t first_seg = g_.b * kWaves + wv;
+  uint32_t my_c = 0;  // lane l: records of bin seg0 + l * nwaves
+  int64_t seg0 = first_seg - kWave * nwaves;
+  uint64_t have = 0;  // bins of this group of 64 not yet taken that hold records
+  auto next_bin = [&](int64_t& seg, uint32_t& c_all) -> bool {
+    while (have == 0) {
+      seg0 += kWave * nwaves;
+      if (seg0 >= (int64_t)nb) return false;
+      const int64_t mine = seg0 + lane * nwaves;
+      my_c = mine < (int64_t)nb ? bins.count[(size_t)mine << sh] : 0u;
+      if (!LIST && my_c) bins.count[(size_t)mine << sh] = 0;
+      have = __ballot(my_c != 0);
+    }
+    const int l = ctz64(have);
+    have &= have - 1;
+    seg = seg0 + l * nwaves;
+    c_all = __shfl(my_c, l);
+    return true;
+  };
+  struct Rec {  // a lane's record
+    uint64_t key[W];
+    double v;
+    uint32_t inf;
+  };
+  auto load_rec = [&](const uint64_t* r, bool on) {
+    Rec q;
+#pragma unroll
+    for (int w = 0; w < W; ++w) q.key[w] = on ? r[w] : 0ull;
+    q.v = on ? rec_val<W>(s, r) : 0.0;
+    q.inf = on ? rec_info<W>(s, r) : 0u;
+    return q;
+  };
+  int64_t seg = 0, seg_n = 0;
+  uint32_t c_all = 0, c_n = 0;
+  Rec rec_n;
+  bool more = next_bin(seg_n, c_n);
+  if (more) rec_n = load_rec(bins.rec + ((size_t)seg_n * cap + lane) * s.rec_words, (uint32_t)lane < (c_n < cap ? c_n : cap));
+  while (more) {
+    seg = seg_n;
+    c_all = c_n;
+    const Rec rec_0 = rec_n;
+    more = next_bin(seg_n, c_n);
+    if (more) rec_n = load_rec(bins.rec + ((size_t)seg_n * cap + lane) * s.rec_words, (uint32_t)lane < (c_n < cap ? c_n : cap));
+    const int64_t c = c_all < cap ? c_all : cap;
+    int64_t csp = c, total = c;  // the bin's records, its area's, the overflow list's
+    if (c_all > cap) {
+      const uint32_t a = bins.scount[seg % kSpill];
+      csp += a < bins.spill_cap ? a : bins.spill_cap;
+      total = csp + (a > bins.spill_cap ? (int64_t)cnt->n_ovf : 0);
+    }
+    uint64_t* spill_rec = bins.spill + (size_t)(seg % kSpill) * bins.spill_cap * s.rec_words;
+    uint64_t* seg_rec = bins.rec + (size_t)seg * cap * s.rec_words;
+    bool again = false;  // records are left for another round
+    do {
+      const bool first_round = !again;
+      again = false;
+      int nu = 0;
+      for (int64_t i0 = 0; i0 < total; i0 += kWave) {
+        const int64_t i = i0 + lane;
+        bool act = i < total;
+        uint64_t* rec = i < c ? seg_rec + i * s.rec_words
+                      : i < csp ? spill_rec + (i - c) * s.rec_words : bins.ovf + (i - csp) * s.rec_words;
+        const Rec q = i0 == 0 && first_round && act && i < c ? rec_0 : load_rec(rec, act);
+        const uint64_t* key = q.key;
+        const double v = q.v;
+        const uint32_t inf = q.inf;
+        uint32_t frac = 0;
+        if (act) {
+          const uint32_t h = bin_hash<W>(key);
+          frac = h * nb;  // the position inside the bin
+          if (i >= c) act = bin_of(h, nb) == (uint32_t)seg;
+          if (!first_round) act = act && (inf & kInfoLeft);
+        }
+        bool won;
+        const int slot = merge_slot<W, R>(tb, act, key, frac >> (T == 128 ? 25 : 26), won);
+        const bool left = act && slot < 0;
+        if (left && first_round) rec_mark<W>(s, rec, true);
+        if (act && !left && !first_round) rec_mark<W>(s, rec, false);
+        again = again || __ballot(left) != 0;
+        if (act && !left) {
+          // the record joins its determinant, in order of arrival
+          const int r = (int)(inf & 0xFFu);
+          const double cv = atomicAdd(&tb->sum[slot * R + r], v);
+          uint32_t t = won ? 0u : kTagMulti;
+          if ((inf & kInfoInit) || (s.t_init && fabs(cv) > 1.e-12 && fabs(v) > 1.e-12)) t |= 1u << r;
+          if (t) atomicOr(&tb->tag[slot], t);
+          if (cv * v < 0.0) {
+            const double x = fabs(cv), y = fabs(v);
+            ann[r] += 2.0 * (x < y ? x : y);
+          }
+        }
+        const uint64_t wm = __ballot(won);
+        if (won) tb->list[nu + popc64(wm & lanemask_lt())] = (uint8_t)slot;
+        nu += popc64(wm);
+      }
+      wave_sync();
+      // the merged determinants, one per lane
+      for (int u0 = 0; u0 < nu; u0 += kWave) {
+        const bool act = u0 + lane < nu;
+        uint64_t key[W];
+        double ss[R];
+        uint32_t tag = 0;
+        if (act) {
+          const int slot = tb->list[u0 + lane];
+#pragma unroll
+          for (int w = 0; w < W; ++w) {
+            key[w] = tb->key[slot * W + w];
+            tb->key[slot * W + w] = kTabEmpty;
+          }
+          for (int r = 0; r < S; ++r) {
+            ss[r] = tb->sum[slot * R + r];
+            tb->sum[slot * R + r] = 0.0;
+          }
+          tag = tb->tag[slot];
+          tb->tag[slot] = 0;
+        }
+        const bool multi = (tag & kTagMulti) != 0;
+        // a single record carries its flag as it is, several only under the
+        // initiator approximation
+        const uint32_t sflag = multi && !s.t_init ? 0u : tag & 0xFFFFu;
+        bool keep = false;
+        if (act) {
+          double tot = 0.0;
+          for (int r = 0; r < S; ++r) tot += fabs(ss[r]);
+          keep = multi ? tot > 1.e-12 : !(tot < 1.e-12);
+        }
+        uniq += (unsigned int)wave_count(keep);
+        bool isnew = false, rm = false;
+        int64_t pos = -1;
+        if (LIST) {
+          isnew = keep;
+        } else if (keep) {
+          int64_t home = find_walker_hash<W>(key, s.rh, s.L) - 1;
+          pos = hash_lookup<W>(wk, key, home, cnt);
+          if (pos >= 0) {
+            double cs[R];  // the walkers there
+            double tot = 0.0;
+            for (int r = 0; r < S; ++r) { cs[r] = wk.sgn(pos, r); tot += fabs(cs[r]); }
+            bool determ = (wk.flags(pos) & kFlagCore) != 0;
+            if (tot >= 1.e-12 || determ) {
+              for (int r = 0; r < S; ++r) {
+                double prod = cs[r] * ss[r];
+                if (fabs(cs[r]) < 1.0e-12 && s.t_init && !((sflag >> r) & 1u) && !determ) {
+                  st_ab[r] += fabs(ss[r]);
+                  ss[r] = 0.0;
+                }
+                if (prod < 0.0) {
+                  double x = fabs(cs[r]), y = fabs(ss[r]);
+                  st_an[r] += 2.0 * (x < y ? x : y);
+                }
+              }
+              bool occ = false;
+              for (int r = 0; r < S; ++r) {
+                cs[r] = ss[r] + cs[r];
+                wk.sgn(pos, r) = cs[r];
+                occ = occ || !(fabs(cs[r]) < 1.e-12);
+              }
+              rm = !determ && !occ;
+            }
+          } else {
+            if (s.t_init)
+              for (int r = 0; r < S; ++r)
+                if (!((sflag >> r) & 1u)) {
+                  st_ab[r] += fabs(ss[r]);
+                  ss[r] = 0.0;
+                }
+            bool occ = false;
+            for (int r = 0; r < S; ++r) occ = occ || !(fabs(ss[r]) < 1.e-12);
+            if (occ) {
+              // stochRoundSpawn (Annihilation.F90:1354-1418)
+              double thr = s.occ_thresh;
+              for (int r = 0; r < S; ++r) {
+                if (fabs(ss[r]) > 1.e-12 && fabs(ss[r]) < thr) {
+                  double pRemove = 1.0 - fabs(ss[r]) / thr;
+                  double u, dummy;
+                  draw2<W>(s.seed, key, iter, r, 0, 4, u, dummy);
+                  if (pRemove > u) {
+                    st_rm[r] += fabs(ss[r]);
+                    ss[r] = 0.0;
+                  } else {
+                    st_bn[r] += thr - fabs(ss[r]);
+                    ss[r] = ss[r] >= 0.0 ? thr : -thr;
+                  }
+                }
+              }
+              occ = false;
+              for (int r = 0; r < S; ++r) occ = occ || !(fabs(ss[r]) < 1.e-12);
+              isnew = occ;
+            }
+          }
+          if (rm) {  // RemoveHashDet (load_balancer.fpp:631-644): the entry becomes a tombstone
+            const int64_t hp = wk.hpos(pos);
+            int32_t* sl = (int32_t*)(wk.htab + (size_t)(hp >> 2) * 8 * W + 4 * W);
+            sl[hp & 3] = kSlotTomb;
+            wk.flags(pos) |= kFlagRemoved;
+          }
+        }
+        const uint64_t nm = __ballot(isnew), fm = __ballot(rm);
+        if (nm && kCap == 0) {
+          const unsigned long long q = wave_reserve(n_ctr, popc64(nm)) + (unsigned long long)popc64(nm & lanemask_lt());
+          if (isnew) {
+#pragma unroll
+            for (int w = 0; w < W; ++w) n_key[q * W + w] = key[w];
+            for (int r = 0; r < S; ++r) n_sgn[q * S + r] = ss[r];
+            n_flag[q] = sflag;
+          }
+        } else if (nm) {
+          if (n_list + popc64(nm) > kCap) {
+            wave_sync();
+            wave_list_write<W, R>(ws, n_list, wave_reserve(n_ctr, n_list), n_key, n_sgn, n_flag, S);
+            wave_sync();
+            n_list = 0;
+          }
+          if (isnew) {
+            const int q = n_list + popc64(nm & lanemask_lt());
+#pragma unroll
+            for (int w = 0; w < W; ++w) ws->key[q * W + w] = key[w];
+            for (int r = 0; r < S; ++r) ws->sgn[q * R + r] = ss[r];
+            ws->flag[q] = sflag;
+          }
+          n_list += popc64(nm);
+        }
+        if (fm) {
+          if (n_free + popc64(fm) > 128) {
+            wave_sync();
+            wave_free_write<W, R>(wk, ws, n_free, wave_reserve(&cnt->free_tail, n_free));
+            wave_sync();
+            n_free = 0;
+          }
+          if (rm) ws->freed[n_free + popc64(fm & lanemask_lt())] = (int32_t)pos;
+          n_free += popc64(fm);
+        }
+      }
+      wave_sync();
+    } while (again);
+  }
+  // what is still staged: one reservation per block
+  if (lane == 0) {
+    tail_n[wv][0] = (uint32_t)n_list;
+    tail_n[wv][1] = (uint32_t)n_free;
+    if (uniq) atomicAdd(&blk_unique, uniq);
+  }
+  __syncthreads();
+  if (threadIdx.x < 2) {
+    unsigned int n = 0;
+    for (int q = 0; q < kWaves; ++q) n += tail_n[q][threadIdx.x];
+    if (n) tail_base[threadIdx.x] = atomicAdd(threadIdx.x ? &cnt->free_tail : n_ctr, (unsigned long long)n);
+  }
+  __syncthreads();
+  unsigned int before[2] = {0, 0};
+  for (int q = 0; q < wv; ++q) {
+    before[0] += tail_n[q][0];
+    before[1] += tail_n[q][1];
+  }
+  wave_list_write<W, R>(ws, n_list, tail_base[0] + before[0], n_key, n_sgn, n_flag, S);
+  if constexpr (!LIST) {
+    wave_free_write<W, R>(wk, ws, n_free, tail_base[1] + before[1]);
+    for (int r = 0; r < S; ++r) {
+      bs.add(soff(F_NABORTED, r), st_ab[r]);
+      bs.add(soff(F_NANNIHIL, r), st_an[r] + ann[r]);
+      bs.add(soff(F_NREMOVED, r), st_rm[r]);
+      bs.add(soff(F_NBORN, r), st_bn[r]);
+    }
+    if (threadIdx.x == 0 && blk_unique)
+      atomicAdd(&cnt->uniq_part[g_.b % Counters::kSpread].v, (unsigned long long)blk_unique);
+    bs.flush(part, g_.b);
+  }
 }
-template <int W, int R, typename K, int NW>
-__global__ void __launch_bounds__(kBlock) k_merge_annihilate(DevSys s, Walk wk, Counters* cnt, double* part, const K* skey, const uint32_t* sidx, const uint64_t* sp_rec, int64_t scap, uint64_t* n_key, double* n_sgn, uint32_t* n_flag, const IterParams* prm) {
-  k_merge_annihilate_body<W, R, K, NW>(hw_grid(), s, wk, cnt, part, skey, sidx, sp_rec, scap, n_key, n_sgn, n_flag, prm);
+template <int W, int R>
+__global__ void __launch_bounds__(kBlock, R <= 2 && W == 1 ? 5 : 1) k_merge_annihilate(DevSys s, Walk wk, Counters* cnt, double* part, Bins bins, uint64_t* n_key, double* n_sgn, uint32_t* n_flag, const IterParams* prm) {
+  k_merge_body<W, R, false>(hw_grid(), s, wk, cnt, part, bins, n_key, n_sgn, n_flag, &cnt->n_new, prm);
+}
+template <int W, int R>
+__global__ void __launch_bounds__(kBlock) k_merge_list(DevSys s, Walk wk, Counters* cnt, Bins bins, uint64_t* u_key, double* u_sgn, uint32_t* u_flag, unsigned long long* u_count) {
+  k_merge_body<W, R, true>(hw_grid(), s, wk, cnt, nullptr, bins, u_key, u_sgn, u_flag, u_count, nullptr);
 }
 
 // ------------------------------------------------------ semistochastic core
