@@ -191,11 +191,12 @@ __global__ void __launch_bounds__(kBlock) km_core_apply(const EngDev* __restrict
   k_core_apply_body<R>(g, a.s, a.wk, a.cnt, a.core_slot, a.core_y, a.ncore, a.part, a.s.S);
 }
 
-template <int W, int R>
+template <int W, int R, int GL>
 __global__ void __launch_bounds__(kBlock) km_insert(const EngDev* __restrict__ ed, const uint16_t* __restrict__ map) {
+  extern __shared__ double insert_dyn[];
   Grid g;
   const EngDev& a = eng_of(ed, map, kLkGrid, g);
-  k_insert_body<W, R>(g, a.s, a.wk, a.cnt, a.n_key, a.n_sgn, a.n_flag, &a.cnt->n_new);
+  k_insert_body<W, R, GL>(g, a.s, a.wk, a.cnt, a.n_key, a.n_sgn, a.n_flag, &a.cnt->n_new, insert_dyn);
 }
 
 template <int W, int R>

@@ -277,6 +277,8 @@ struct BatchGroup {
   bool singles = false;     // queued heat-bath singles (PCHB generator)
   int lanes = 4, pl = 4;    // heat-bath singles: lanes per attempt, orbitals per lane
   int items = 4;            // launch-shape knob of the set-up sorts
+  int ins_lanes = 1;        // lanes per new determinant, and a block's LDS for them
+  size_t ins_lds = 0;
   bool core = false, core_fp32 = false;
   // every engine of the group has the same core determinants: one projection
   // over the interleaved vectors X, Y of ccols columns (kernels in ngpu_batch.h)
@@ -551,6 +553,28 @@ void core_projection(ngpu_t* h) {
 template <int W>
 void check_chain(ngpu_t* h, bool gen);
 
+// lanes per diagonal element of a short list's new determinants (k_insert's
+// G), and a block's LDS for them: 16 while 48 KB hold the terms of 16
+// determinants, then 64; one without LDS when not even four fit 64 KB
+int insert_lanes(const ngpu_t* h) {
+  if (h->sys.model == NGPU_MODEL_HUBBARD) return 1;
+  const int b = 8 * diag_lds(h->ds);
+  return 16 * b <= 48 * 1024 ? 16 : 4 * b <= 64 * 1024 ? 64 : 1;
+}
+size_t insert_lds(const ngpu_t* h, int lanes) {
+  return lanes == 1 ? 0 : 8 * (size_t)diag_lds(h->ds) * (size_t)(kBlock / lanes);
+}
+
+// AddNewHashDet of the new list (n_new determinants) into the walker table
+template <int W, int R>
+void insert_new(ngpu_t* h, int stage) {
+  const int G = insert_lanes(h);
+  auto kern = G == 1 ? k_insert<W, R, 1> : G == 16 ? k_insert<W, R, 16> : k_insert<W, R, 64>;
+  launch_lds(h, stage, stage, kern, dim3(h->nb_grid), dim3(kBlock), insert_lds(h, G), h->ds, h->wk, h->cnt,
+             (const uint64_t*)h->n_key, (const double*)h->n_sgn, (const uint32_t*)h->n_flag,
+             (const unsigned long long*)&h->cnt->n_new);
+}
+
 template <int W, int R>
 void annihilation_chain(ngpu_t* h, bool with_core, bool list_out = false) {
   // the projected core amplitudes join the walkers before the spawns do, as
@@ -560,9 +584,7 @@ void annihilation_chain(ngpu_t* h, bool with_core, bool list_out = false) {
            dim3(kBlock), h->ds, h->wk, (const Counters*)h->cnt, (const int64_t*)h->core_slot, (const double*)h->core_y,
            h->ncore, h->dpart);
   merge<W, R>(h, list_out);
-  launch(h, 7, 7, k_insert<W, R>, dim3(h->nb_grid), dim3(kBlock), h->ds, h->wk, h->cnt,
-         (const uint64_t*)h->n_key, (const double*)h->n_sgn, (const uint32_t*)h->n_flag,
-         (const unsigned long long*)&h->cnt->n_new);
+  insert_new<W, R>(h, 7);
   launch(h, 8, 8, k_stats<W, R>, dim3(h->nb_grid), dim3(kBlock), h->ds, h->wk, h->cnt, h->dpart,
          (const IterParams*)h->dparams);
   launch(h, -1, -1, k_end_iter, dim3(1), dim3(kBlock), h->dout, h->dpart, h->dcyc, h->cnt,
@@ -1478,12 +1500,8 @@ int ngpu_upload_walkers(ngpu_t* h, const int64_t* rows, int64_t n) {
   hipLaunchKernelGGL(k_set_u32, dim3(1), dim3(1), 0, h->stream, &h->cnt->err, 0u);
   hipLaunchKernelGGL(k_set_count, dim3(1), dim3(1), 0, h->stream, &h->cnt->n_fail, 0ull);
   hipLaunchKernelGGL(k_set_u32, dim3(1), dim3(1), 0, h->stream, &h->cnt->ins_refused, 0u);
-  {
-    auto kern = h->W == 1 ? (h->S == 1 ? k_insert<1, 1> : k_insert<1, kMaxRep>)
-                          : (h->S == 1 ? k_insert<2, 1> : k_insert<2, kMaxRep>);
-    hipLaunchKernelGGL(kern, dim3(h->nb_grid), dim3(kBlock), 0, h->stream, h->ds, h->wk, h->cnt, h->n_key,
-                       h->n_sgn, h->n_flag, &h->cnt->n_new);
-  }
+  if (h->W == 1) h->S == 1 ? insert_new<1, 1>(h, -1) : insert_new<1, kMaxRep>(h, -1);
+  else h->S == 1 ? insert_new<2, 1>(h, -1) : insert_new<2, kMaxRep>(h, -1);
   hipLaunchKernelGGL(k_post_insert, dim3(1), dim3(1), 0, h->stream, h->cnt, &h->cnt->n_new, h->wk.cap);
   if (h->W == 1) hash_upkeep<1>(h);
   else hash_upkeep<2>(h);
@@ -1868,9 +1886,7 @@ int set_core_impl(ngpu_t* h, int64_t ncore, bool fp32, int64_t* nnz_out) {
   dim3 gp((unsigned)std::min<int64_t>((ncore + kBlock - 1) / kBlock, h->nb_grid));
   hipLaunchKernelGGL(HIP_KERNEL_NAME(k_core_place<W>), gp, dim3(kBlock), 0, h->stream, h->ds, h->wk, h->cnt,
                      (const uint64_t*)h->core_keys, ncore, cflags, h->core_slot, h->n_key, h->n_sgn, h->n_flag);
-  hipLaunchKernelGGL(HIP_KERNEL_NAME(k_insert<W, R>), dim3(h->nb_grid), dim3(kBlock), 0, h->stream, h->ds, h->wk,
-                     h->cnt, (const uint64_t*)h->n_key, (const double*)h->n_sgn, (const uint32_t*)h->n_flag,
-                     (const unsigned long long*)&h->cnt->n_new);
+  insert_new<W, R>(h, -1);
   hipLaunchKernelGGL(k_post_insert, dim3(1), dim3(1), 0, h->stream, h->cnt, (const unsigned long long*)&h->cnt->n_new,
                      h->wk.cap);
   hash_upkeep<W>(h);
@@ -2626,6 +2642,14 @@ int build_groups(ngpu_batch* b) {
   for (BatchGroup& g : b->groups) {
     const size_t E = g.hs.size();
     if (E > 65535) return NGPU_ERR_ARG;
+    // the lanes of the engine that needs most (1: an engine past the LDS)
+    g.ins_lanes = 16;
+    for (ngpu_t* h : g.hs) {
+      const int l = insert_lanes(h);
+      g.ins_lanes = l == 1 || g.ins_lanes == 1 ? 1 : std::max(g.ins_lanes, l);
+    }
+    g.ins_lds = 0;
+    for (ngpu_t* h : g.hs) g.ins_lds = std::max(g.ins_lds, insert_lds(h, g.ins_lanes));
     int64_t wmax = 1;
     for (ngpu_t* h : g.hs) wmax = std::max<int64_t>(wmax, h->wk.cap);
     std::vector<EngDev> ed(E);
@@ -2778,7 +2802,9 @@ void group_chain_wr(BatchGroup& g) {
   else if (g.core)
     glaunch(h0, -1, -1, km_core_apply<R>, g.tot[kLkCore], kBlock, 0, ed, (const uint16_t*)m[kLkCore]);
   glaunch(h0, 6, 6, km_merge_annihilate<W, R>, g.tot[kLkMerge], kBlock, 0, ed, (const uint16_t*)m[kLkMerge]);
-  glaunch(h0, 7, 7, km_insert<W, R>, g.tot[kLkGrid], kBlock, 0, ed, (const uint16_t*)m[kLkGrid]);
+  auto ins = g.ins_lanes == 1 ? km_insert<W, R, 1> : g.ins_lanes == 16 ? km_insert<W, R, 16>
+           : km_insert<W, R, 64>;
+  glaunch(h0, 7, 7, ins, g.tot[kLkGrid], kBlock, g.ins_lds, ed, (const uint16_t*)m[kLkGrid]);
   glaunch(h0, 8, 8, km_stats<W, R>, g.tot[kLkGrid], kBlock, 0, ed, (const uint16_t*)m[kLkGrid]);
   glaunch(h0, -1, -1, km_end_iter, (int)g.hs.size(), kBlock, 0, ed);
 }

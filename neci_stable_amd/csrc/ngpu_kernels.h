@@ -1641,11 +1641,13 @@ __device__ inline unsigned long long wave_reserve(unsigned long long* ctr, int n
   if (lane_id() == 0) b = atomicAdd(ctr, (unsigned long long)n);
   return __shfl(b, 0);
 }
-// orders one wave's LDS accesses of different lanes
+// orders one wave's LDS accesses of different lanes: a wave's LDS operations
+// run in order, so only the compiler has to keep them so.  (A workgroup fence
+// would wait for every global access in flight, prefetches and stores too.)
 __device__ inline void wave_sync() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
   __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
 // the table slot of each todo lane's key (one record per lane): inserted if
@@ -1681,7 +1683,7 @@ __device__ inline int merge_slot(MergeTab<W, R>* tb, bool todo, const uint64_t* 
         } else if (!(t & kTagTaken) && atomicCAS(&tb->tag[slot], 0u, kTagTaken) == 0u) {
 #pragma unroll
           for (int w = 0; w < W; ++w) tb->key[slot * W + w] = key[w];
-          __threadfence_block();
+          wave_sync();
           atomicOr(&tb->tag[slot], kTagKey);
           found = slot;
           won = true;
@@ -2161,9 +2163,105 @@ __global__ void __launch_bounds__(kBlock) k_core_place(DevSys s, Walk wk, Counte
   k_core_place_body<W>(hw_grid(), s, wk, cnt, keys, ncore, cflags, core_slot, n_key, n_sgn, n_flag);
 }
 
-// AddNewHashDet (load_balancer.fpp:514-629) for the new list
-template <int W, int R>
-__device__ __forceinline__ void k_insert_body(const Grid& g_, const DevSys& s, const Walk& wk, Counters* cnt, const uint64_t* n_key, const double* n_sgn, const uint32_t* n_flag, const unsigned long long* n_ptr) {
+// Diagonal elements of new molecular determinants by a group of G lanes.
+// sltcnd_0's sums run over nel (nel - 1) / 2 pairs; on one lane their loads
+// were about 50 dependent round trips at 14 electrons and 150 at 26, and a
+// list of new determinants is too short to hide them.  Here the rows of pairs
+// are spread over the group: lane g sums the Coulomb terms of the electrons
+// g, g + G, ... with the electrons above them (each row's sum is its own in
+// sltcnd_0 too) and leaves the exchange terms, whose order the sum fixes, in
+// LDS; then three lanes add the one-electron terms, the rows and the exchange
+// terms, each list in sltcnd_0's order, so the value is sltcnd_0's to the last
+// bit.
+// LDS per determinant: nel one-electron terms, nel rows, the same-spin pairs.
+__host__ __device__ inline int diag_pairs(int na, int nb) { return na * (na - 1) / 2 + nb * (nb - 1) / 2; }
+__host__ __device__ inline int diag_lds(const DevSys& s) {  // doubles
+  return 2 * s.nel + diag_pairs(s.nalpha_ref, s.nbeta_ref);
+}
+template <int W, int G>
+__device__ inline double diag_group(const DevSys& s, const uint64_t* d, int g, double* lds) {
+  const uint64_t kA = 0xAAAAAAAAAAAAAAAAull;
+  int na = 0;
+#pragma unroll
+  for (int w = 0; w < W; ++w) na += popc64(d[w] & kA);
+  const int nel = s.nel, nb = nel - na, np = diag_pairs(na, nb);
+  const bool fits = np <= diag_pairs(s.nalpha_ref, s.nbeta_ref);  // else other spin counts than the run's
+  double *sing = lds, *rows = lds + nel, *ex = lds + 2 * nel;
+  wave_sync();
+  if (fits) {
+    for (int e = g; e < nel; e += G) {
+      const int o = select_orb<W>(d, ~0ull, e + 1), wi = (o - 1) >> 6, bit = (o - 1) & 63;
+      const bool beta = is_beta(o);
+      sing[e] = s.tmat[(size_t)(o - 1) * (s.nbasis + 1)];
+      // same-spin pairs of the electrons below this one
+      int a = 0;
+#pragma unroll
+      for (int w = 0; w < W; ++w) {
+        const uint64_t below = w < wi ? ~0ull : w == wi ? (1ull << bit) - 1ull : 0ull;
+        a += popc64(d[w] & below & kA);
+      }
+      const int b = e - a;
+      double* k = ex + a * (na - 1) - a * (a - 1) / 2 + b * (nb - 1) - b * (b - 1) / 2;
+      const double2* row = (const double2*)(s.jk0 + 2 * (size_t)(spat(o) - 1) * s.nsp);
+      double t = 0.0;
+#pragma unroll
+      for (int w = 0; w < W; ++w) {
+        uint64_t x = w < wi ? 0ull : w > wi ? d[w] : bit == 63 ? 0ull : d[w] & (~0ull << (bit + 1));
+        while (x) {  // eight pairs' (J, K) per round trip
+          constexpr int N = 8;
+          int oj[N], n = 0;
+          double2 v[N];
+#pragma unroll
+          for (int q = 0; q < N; ++q)
+            if (x) {
+              oj[q] = 64 * w + ctz64(x) + 1;
+              x &= x - 1;
+              n = q + 1;
+            }
+#pragma unroll
+          for (int q = 0; q < N; ++q) v[q] = q < n ? row[spat(oj[q]) - 1] : double2{0.0, 0.0};
+#pragma unroll
+          for (int q = 0; q < N; ++q)
+            if (q < n) {
+              t += v[q].x;
+              if (is_beta(oj[q]) == beta) *k++ = -v[q].y;
+            }
+        }
+      }
+      rows[e] = t;
+    }
+  }
+  wave_sync();
+  if (!fits) return diag_helement<W>(s, d);  // (group-uniform)
+  static_assert(G >= 3, "three lanes add the three lists");
+  const double* list = g == 0 ? sing : g == 1 ? rows : ex;
+  const int n = g == 0 ? nel : g == 1 ? nel - 1 : g == 2 ? np : 0;
+  double sum = 0.0;
+  for (int p = 0; p < n; p += 8) {
+    double v[8];
+#pragma unroll
+    for (int q = 0; q < 8; ++q) v[q] = p + q < n ? list[p + q] : 0.0;
+#pragma unroll
+    for (int q = 0; q < 8; ++q)
+      if (p + q < n) sum += v[q];
+  }
+  const int lead = lane_id() - g;
+  const double hel_sing = __shfl(sum, lead), hel_doub = __shfl(sum, lead + 1), hel_tmp = __shfl(sum, lead + 2);
+  return hel_doub + hel_tmp + hel_sing + s.ecore;
+}
+
+// AddNewHashDet (load_balancer.fpp:514-629) for the new list.  A wave takes D
+// determinants, one lane each for the hash entry and the walker row.  On a
+// short list (up to 8 per wave of the grid) the diagonal elements follow, by
+// groups of G lanes: its time is the length of one wave's instruction stream,
+// which the groups shorten (us per iteration, one lane before: 10e/20o, 700
+// new determinants 24 -> 13; two-word 26e/40o, 2.8e4 92 -> 49).  A long list
+// fills the lanes and is bound by issue and L1 gathers, which groups make
+// worse (14e/30o, 1.3e5: 55 with one lane, 56 with four, 102 with 16), so
+// there the lane sums its own.  G is 16, or 64 when a block's LDS does not
+// hold 16 determinants' terms; 1 for the lattice.
+template <int W, int R, int G>
+__device__ __forceinline__ void k_insert_body(const Grid& g_, const DevSys& s, const Walk& wk, Counters* cnt, const uint64_t* n_key, const double* n_sgn, const uint32_t* n_flag, const unsigned long long* n_ptr, double* lds) {
   if (cnt->halt) return;
   const int S = R == 1 ? 1 : s.S;
   int64_t nn = (int64_t)*n_ptr;
@@ -2186,34 +2284,64 @@ __device__ __forceinline__ void k_insert_body(const Grid& g_, const DevSys& s, c
     return;
   }
   unsigned long long my_reused = 0;
-  for (int64_t i = (int64_t)g_.b * blockDim.x + threadIdx.x; i < nn;
-       i += (int64_t)g_.nb * blockDim.x) {
-    int64_t slot = i < avail ? wk.freeq[(head + (unsigned long long)i) % (unsigned long long)wk.cap]
-                             : ns0 + (i - avail);
-    if (slot >= wk.cap) {
-      atomicOr(&cnt->err, 1u << NGPU_ERR_WALKERS_FULL);
-      atomicAdd(&cnt->n_fail, 1ull);
-      continue;
-    }
+  constexpr int kWaves = kBlock / kWave;
+  const int lane = lane_id(), wv = threadIdx.x / kWave;
+  const int64_t nwaves = g_.nb * kWaves;
+  const bool group = G > 1 && nn <= 8 * nwaves;
+  constexpr int kPer = kWave / G;  // determinants of a wave's group step
+  int64_t D = kWave;
+  if (group) {
+    D = ((nn + nwaves - 1) / nwaves + kPer - 1) / kPer * kPer;
+    if (D > kWave) D = kWave;
+  }
+  if (g_.b * kWaves * D >= nn) return;  // no determinant for this block
+  for (int64_t base = (g_.b * kWaves + wv) * D; base < nn; base += nwaves * D) {
+    const int64_t i = base + lane;
+    const bool act = lane < D && i < nn;
+    int64_t slot = -1;  // the determinant's row; -1: none
     uint64_t key[W];
 #pragma unroll
-    for (int w = 0; w < W; ++w) key[w] = n_key[i * W + w];
-    int64_t home = find_walker_hash<W>(key, s.rh, s.L) - 1;
-    bool reused = false;
-    int64_t hp = hash_insert<W>(wk, key, home, (int32_t)slot, reused);
-    my_reused += reused ? 1 : 0;
-    if (hp < 0) {
-      atomicOr(&cnt->err, 1u << NGPU_ERR_HASH_FULL);
-      atomicAdd(&cnt->n_fail, 1ull);
-      wk.flags(slot) = kFlagRemoved;
-    } else {
+    for (int w = 0; w < W; ++w) key[w] = act ? n_key[i * W + w] : s.ref[w];
+    if (act) {
+      slot = i < avail ? wk.freeq[(head + (unsigned long long)i) % (unsigned long long)wk.cap] : ns0 + (i - avail);
+      int64_t hp = -1;
+      if (slot >= wk.cap) {
+        atomicOr(&cnt->err, 1u << NGPU_ERR_WALKERS_FULL);
+        atomicAdd(&cnt->n_fail, 1ull);
+        slot = -1;
+      } else {
+        int64_t home = find_walker_hash<W>(key, s.rh, s.L) - 1;
+        bool reused = false;
+        hp = hash_insert<W>(wk, key, home, (int32_t)slot, reused);
+        my_reused += reused ? 1 : 0;
+        if (hp < 0) {
+          atomicOr(&cnt->err, 1u << NGPU_ERR_HASH_FULL);
+          atomicAdd(&cnt->n_fail, 1ull);
+          wk.flags(slot) = kFlagRemoved;
+          slot = -1;
+        }
+      }
+      if (slot >= 0) {
 #pragma unroll
-      for (int w = 0; w < W; ++w) wk.keys[slot * W + w] = key[w];
-      for (int r = 0; r < S; ++r) wk.sgn(slot, r) = n_sgn[i * S + r];
-      wk.flags(slot) = n_flag[i] & ~kFlagRemoved;
-      wk.diagH[slot] = diag_helement<W>(s, key) - s.hii;
-      wk.offdiagH[slot] = offdiag_helement<W>(s, key);
-      wk.hpos(slot) = hp;
+        for (int w = 0; w < W; ++w) wk.keys[slot * W + w] = key[w];
+        for (int r = 0; r < S; ++r) wk.sgn(slot, r) = n_sgn[i * S + r];
+        wk.flags(slot) = n_flag[i] & ~kFlagRemoved;
+        wk.hpos(slot) = hp;
+        wk.offdiagH[slot] = offdiag_helement<W>(s, key);
+        if (!group) wk.diagH[slot] = diag_helement<W>(s, key) - s.hii;
+      }
+    }
+    if constexpr (G > 1) {
+      const int n_here = group ? (int)(nn - base < D ? nn - base : D) : 0;
+      for (int r = 0; r < n_here; r += kPer) {  // wave-uniform
+        const int src = r + lane / G;           // the lane that holds this group's determinant
+        uint64_t k[W];
+#pragma unroll
+        for (int w = 0; w < W; ++w) k[w] = __shfl((unsigned long long)key[w], src);
+        const int64_t row = __shfl((long long)slot, src);
+        const double d = diag_group<W, G>(s, k, lane % G, lds + (size_t)(threadIdx.x / G) * diag_lds(s));
+        if (lane % G == 0 && row >= 0) wk.diagH[row] = d - s.hii;
+      }
     }
   }
   // one no-return atomic per wave that reused entries
@@ -2227,9 +2355,10 @@ __device__ __forceinline__ void k_insert_body(const Grid& g_, const DevSys& s, c
   if (threadIdx.x == 0 && blk_reused)
     atomicAdd(&cnt->reuse_part[g_.b % Counters::kSpread].v, (unsigned long long)blk_reused);
 }
-template <int W, int R>
+template <int W, int R, int G>
 __global__ void __launch_bounds__(kBlock) k_insert(DevSys s, Walk wk, Counters* cnt, const uint64_t* n_key, const double* n_sgn, const uint32_t* n_flag, const unsigned long long* n_ptr) {
-  k_insert_body<W, R>(hw_grid(), s, wk, cnt, n_key, n_sgn, n_flag, n_ptr);
+  extern __shared__ double insert_dyn[];
+  k_insert_body<W, R, G>(hw_grid(), s, wk, cnt, n_key, n_sgn, n_flag, n_ptr, insert_dyn);
 }
 
 // bookkeeping of k_insert: queued slots used, fresh slots appended (beyond
