@@ -104,7 +104,8 @@ __global__ void __launch_bounds__(kBlock, R <= 2 && W == 1 ? 5 : 1) km_merge_ann
                                                               const uint16_t* __restrict__ map) {
   Grid g;
   const EngDev& a = eng_of(ed, map, kLkMerge, g);
-  k_merge_body<W, R, false>(g, a.s, a.wk, a.cnt, a.part, a.bins, a.n_key, a.n_sgn, a.n_flag, &a.cnt->n_new, a.prm);
+  k_merge_body<W, R, false>(g, a.s, a.wk, a.cnt, a.part, a.bins, a.n_key, a.n_sgn, a.n_flag, &a.cnt->n_new, a.prm,
+                            stats_by_parts(a.s));
 }
 
 template <int R>
@@ -203,6 +204,7 @@ template <int W, int R>
 __global__ void __launch_bounds__(kBlock) km_stats(const EngDev* __restrict__ ed, const uint16_t* __restrict__ map) {
   Grid g;
   const EngDev& a = eng_of(ed, map, kLkGrid, g);
+  if (stats_by_parts(a.s)) return;
   k_stats_body<W, R>(g, a.s, a.wk, a.cnt, a.part, a.prm);
 }
 

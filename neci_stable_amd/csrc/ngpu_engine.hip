@@ -524,12 +524,12 @@ int merge_blocks(const ngpu_t* h) {
 // annihilation into the walker list (stage 6; stages 4 and 5, the sort and
 // the merge alone, are empty)
 template <int W, int R>
-void merge(ngpu_t* h, bool list_out) {
+void merge(ngpu_t* h, bool list_out, bool by_parts) {
   if (list_out)
     launch(h, -1, -1, k_merge_list<W, R>, dim3(merge_blocks(h)), dim3(kBlock), h->ds, h->wk, h->cnt, h->bins, h->u_key,
            h->u_sgn, h->u_flag, h->u_count);
   launch(h, 6, 6, k_merge_annihilate<W, R>, dim3(merge_blocks(h)), dim3(kBlock), h->ds, h->wk, h->cnt, h->dpart,
-         h->bins, h->n_key, h->n_sgn, h->n_flag, (const IterParams*)h->dparams);
+         h->bins, h->n_key, h->n_sgn, h->n_flag, (const IterParams*)h->dparams, by_parts ? 1 : 0);
 }
 
 // semistochastic projection of the core amplitudes (before spawning)
@@ -583,9 +583,11 @@ void annihilation_chain(ngpu_t* h, bool with_core, bool list_out = false) {
     launch(h, -1, -1, k_core_apply<R>, dim3((int)std::min<int64_t>((h->ncore + kBlock - 1) / kBlock, h->nb_grid)),
            dim3(kBlock), h->ds, h->wk, (const Counters*)h->cnt, (const int64_t*)h->core_slot, (const double*)h->core_y,
            h->ncore, h->dpart);
-  merge<W, R>(h, list_out);
+  // an explicit list has no prepass before it: its statistics take a pass
+  const bool by_parts = with_core && stats_by_parts(h->ds);
+  merge<W, R>(h, list_out, by_parts);
   insert_new<W, R>(h, 7);
-  launch(h, 8, 8, k_stats<W, R>, dim3(h->nb_grid), dim3(kBlock), h->ds, h->wk, h->cnt, h->dpart,
+  if (!by_parts) launch(h, 8, 8, k_stats<W, R>, dim3(h->nb_grid), dim3(kBlock), h->ds, h->wk, h->cnt, h->dpart,
          (const IterParams*)h->dparams);
   launch(h, -1, -1, k_end_iter, dim3(1), dim3(kBlock), h->dout, h->dpart, h->dcyc, h->cnt,
          h->scap, h->wk.cap, h->wk.L * (int64_t)kBucketEntries, (const IterParams*)h->dparams, h->bins.scount);
@@ -2805,7 +2807,9 @@ void group_chain_wr(BatchGroup& g) {
   auto ins = g.ins_lanes == 1 ? km_insert<W, R, 1> : g.ins_lanes == 16 ? km_insert<W, R, 16>
            : km_insert<W, R, 64>;
   glaunch(h0, 7, 7, ins, g.tot[kLkGrid], kBlock, g.ins_lds, ed, (const uint16_t*)m[kLkGrid]);
-  glaunch(h0, 8, 8, km_stats<W, R>, g.tot[kLkGrid], kBlock, 0, ed, (const uint16_t*)m[kLkGrid]);
+  bool pass = false;  // an engine whose statistics take a pass over its table
+  for (const ngpu_t* h : g.hs) pass = pass || !stats_by_parts(h->ds);
+  if (pass) glaunch(h0, 8, 8, km_stats<W, R>, g.tot[kLkGrid], kBlock, 0, ed, (const uint16_t*)m[kLkGrid]);
   glaunch(h0, -1, -1, km_end_iter, (int)g.hs.size(), kBlock, 0, ed);
 }
 

@@ -198,8 +198,8 @@ struct BlockStats {
     if (lane_id() == 0 && t > 0.0)
       atomicMax((unsigned long long*)&acc[i], (unsigned long long)__double_as_longlong(t));
   }
-  // into partial row blockIdx % kStatCopies (InstNoAtHF has a single writer,
-  // so summing the rows reproduces it)
+  // into partial row blockIdx % kStatCopies (InstNoAtHF has a single writer, or
+  // one writer and the changes after it, so summing the rows reproduces it)
   __device__ void flush(double* part, int64_t blk) {
     __syncthreads();
     double* g = part + (size_t)(blk % kStatCopies) * kStatStride;
@@ -506,6 +506,15 @@ __device__ inline int64_t grid_elem(const Grid& g, int64_t t) {
   return t * g.nb * blockDim.x + g.b * blockDim.x + threadIdx.x;
 }
 
+// ------------------------------------------------- incremental statistics
+// CalcHashTableStats's sums (TotParts, norm, occupied determinants, InstNoAtHF)
+// need a pass over the walker table only when that pass also rounds (real
+// coefficients) or when core amplitudes change outside the merge.  With
+// integer walkers the prepass sums what it leaves behind and the merge adds
+// what it changes, exactly (sums of integers), so k_stats is not launched:
+// 6 us of an iteration over 3e3 determinants, 25 us over 2.9e6.
+__host__ __device__ inline bool stats_by_parts(const DevSys& s) { return !s.t_real && s.ncore == 0; }
+
 // ------------------------------------------------------------- prepass
 // CalcParentFlag_det + SumEContrib + decide_num_to_spawn + walker_death for
 // every occupied slot (FciMCPar.F90:1294-1758, fcimc_helper.F90:518-802,
@@ -532,7 +541,9 @@ __device__ __forceinline__ void k_prepass_body(const Grid& g_, const DevSys& s, 
   chunk_of(g_, nslots, begin, end);
   int64_t my_att = 0, my_rm = 0;
   bool death_err = false;
-  LaneSum<R> a_idets, a_iwalk, a_ndets, a_nwalk, a_hf, a_doubs, a_enum, a_died, a_born, a_abort;
+  LaneSum<R> a_idets, a_iwalk, a_ndets, a_nwalk, a_hf, a_doubs, a_enum, a_died, a_born, a_abort, a_tot, a_norm;
+  LaneSum<1> a_occ;
+  const bool by_parts = stats_by_parts(s);
   for (int64_t base = begin; base < end; base += blockDim.x) {
     int64_t slot = base + threadIdx.x;
     bool valid = slot < end;
@@ -633,6 +644,17 @@ __device__ __forceinline__ void k_prepass_body(const Grid& g_, const DevSys& s, 
       a_abort.add(bs, soff(F_NABORTED, r), ab);
     }
     bool rm = occ && !(any_left || core);
+    if (by_parts) {  // what is left of the slot
+      bool left = live && core;
+      for (int r = 0; r < S; ++r) left = left || (!rm && !(fabs(cp[r]) < 1.e-12));
+      for (int r = 0; r < S; ++r) {
+        const double v = left ? cp[r] : 0.0;
+        a_tot.add(bs, soff(F_TOTPARTS, r), fabs(v));
+        a_norm.add(bs, soff(F_NORMSQ, r), v * v);
+        if (isref && left) bs.acc[soff(F_INSTHF, r)] = v;
+      }
+      a_occ.add(bs, X_NOCC, left ? 1.0 : 0.0);
+    }
     if (occ) {
       for (int r = 0; r < S; ++r) wk.sgn(slot, r) = rm ? 0.0 : cp[r];
       wk.flags(slot) = rm ? (f | kFlagRemoved) : f;
@@ -658,6 +680,11 @@ __device__ __forceinline__ void k_prepass_body(const Grid& g_, const DevSys& s, 
   a_died.done(bs, soff(F_NDIED, 0));
   a_born.done(bs, soff(F_NBORN, 0));
   a_abort.done(bs, soff(F_NABORTED, 0));
+  if (by_parts) {
+    a_tot.done(bs, soff(F_TOTPARTS, 0));
+    a_norm.done(bs, soff(F_NORMSQ, 0));
+    a_occ.done(bs, X_NOCC);
+  }
   int64_t tot;
   (void)block_exclusive_scan(my_att, red, tot);
   if (threadIdx.x == 0) blk_part[g_.b] = tot;
@@ -1702,7 +1729,7 @@ __device__ inline int merge_slot(MergeTab<W, R>* tb, bool todo, const uint64_t* 
 // LIST: only the merged list is written (the explicit-list entry point), the
 // bins stay as they are and nothing is counted
 template <int W, int R, bool LIST>
-__device__ __forceinline__ void k_merge_body(const Grid& g_, const DevSys& s, const Walk& wk, Counters* cnt, double* part, const Bins& bins, uint64_t* n_key, double* n_sgn, uint32_t* n_flag, unsigned long long* n_ctr, const IterParams* prm) {
+__device__ __forceinline__ void k_merge_body(const Grid& g_, const DevSys& s, const Walk& wk, Counters* cnt, double* part, const Bins& bins, uint64_t* n_key, double* n_sgn, uint32_t* n_flag, unsigned long long* n_ctr, const IterParams* prm, bool by_parts) {
   constexpr int kWaves = kBlock / kWave;
   const uint32_t nb = cnt->nbins, cap = cnt->bin_cap, sh = cnt->bin_shift;
   if (cnt->halt || g_.b * kWaves >= (int64_t)nb) return;
@@ -1730,8 +1757,9 @@ __device__ __forceinline__ void k_merge_body(const Grid& g_, const DevSys& s, co
   const int S = R == 1 ? 1 : s.S;
   int n_list = 0, n_free = 0;  // staged (wave-uniform)
   unsigned int uniq = 0;
-  double ann[R], st_ab[R], st_an[R], st_rm[R], st_bn[R];
-  for (int r = 0; r < S; ++r) ann[r] = st_ab[r] = st_an[r] = st_rm[r] = st_bn[r] = 0.0;
+  double ann[R], st_ab[R], st_an[R], st_rm[R], st_bn[R], d_tot[R], d_norm[R];
+  for (int r = 0; r < S; ++r) ann[r] = st_ab[r] = st_an[r] = st_rm[r] = st_bn[r] = d_tot[r] = d_norm[r] = 0.0;
+  int d_occ = 0;  // by_parts: changes of the statistics
   // The wave's bins, 64 counters per load; the records of the next bin are on
   // their way while a bin's determinants are looked up.
   const int64_t nwaves = g_.nb * kWaves;
@@ -1888,11 +1916,24 @@ __device__ __forceinline__ void k_merge_body(const Grid& g_, const DevSys& s, co
               }
               bool occ = false;
               for (int r = 0; r < S; ++r) {
+                if (by_parts) {
+                  d_tot[r] -= fabs(cs[r]);
+                  d_norm[r] -= cs[r] * cs[r];
+                  if (det_eq<W>(key, s.ref)) atomicAdd(&bs.acc[soff(F_INSTHF, r)], ss[r]);
+                }
                 cs[r] = ss[r] + cs[r];
                 wk.sgn(pos, r) = cs[r];
                 occ = occ || !(fabs(cs[r]) < 1.e-12);
               }
               rm = !determ && !occ;
+              if (by_parts) {
+                if (rm) d_occ -= 1;
+                for (int r = 0; r < S; ++r)
+                  if (!rm) {
+                    d_tot[r] += fabs(cs[r]);
+                    d_norm[r] += cs[r] * cs[r];
+                  }
+              }
             }
           } else {
             if (s.t_init)
@@ -1923,6 +1964,14 @@ __device__ __forceinline__ void k_merge_body(const Grid& g_, const DevSys& s, co
               occ = false;
               for (int r = 0; r < S; ++r) occ = occ || !(fabs(ss[r]) < 1.e-12);
               isnew = occ;
+              if (by_parts && isnew) {
+                d_occ += 1;
+                for (int r = 0; r < S; ++r) {
+                  d_tot[r] += fabs(ss[r]);
+                  d_norm[r] += ss[r] * ss[r];
+                  if (det_eq<W>(key, s.ref)) atomicAdd(&bs.acc[soff(F_INSTHF, r)], ss[r]);
+                }
+              }
             }
           }
           if (rm) {  // RemoveHashDet (load_balancer.fpp:631-644): the entry becomes a tombstone
@@ -1997,19 +2046,24 @@ __device__ __forceinline__ void k_merge_body(const Grid& g_, const DevSys& s, co
       bs.add(soff(F_NANNIHIL, r), st_an[r] + ann[r]);
       bs.add(soff(F_NREMOVED, r), st_rm[r]);
       bs.add(soff(F_NBORN, r), st_bn[r]);
+      if (by_parts) {
+        bs.add(soff(F_TOTPARTS, r), d_tot[r]);
+        bs.add(soff(F_NORMSQ, r), d_norm[r]);
+      }
     }
+    if (by_parts) bs.add(X_NOCC, (double)d_occ);
     if (threadIdx.x == 0 && blk_unique)
       atomicAdd(&cnt->uniq_part[g_.b % Counters::kSpread].v, (unsigned long long)blk_unique);
     bs.flush(part, g_.b);
   }
 }
 template <int W, int R>
-__global__ void __launch_bounds__(kBlock, R <= 2 && W == 1 ? 5 : 1) k_merge_annihilate(DevSys s, Walk wk, Counters* cnt, double* part, Bins bins, uint64_t* n_key, double* n_sgn, uint32_t* n_flag, const IterParams* prm) {
-  k_merge_body<W, R, false>(hw_grid(), s, wk, cnt, part, bins, n_key, n_sgn, n_flag, &cnt->n_new, prm);
+__global__ void __launch_bounds__(kBlock, R <= 2 && W == 1 ? 5 : 1) k_merge_annihilate(DevSys s, Walk wk, Counters* cnt, double* part, Bins bins, uint64_t* n_key, double* n_sgn, uint32_t* n_flag, const IterParams* prm, int by_parts) {
+  k_merge_body<W, R, false>(hw_grid(), s, wk, cnt, part, bins, n_key, n_sgn, n_flag, &cnt->n_new, prm, by_parts != 0);
 }
 template <int W, int R>
 __global__ void __launch_bounds__(kBlock) k_merge_list(DevSys s, Walk wk, Counters* cnt, Bins bins, uint64_t* u_key, double* u_sgn, uint32_t* u_flag, unsigned long long* u_count) {
-  k_merge_body<W, R, true>(hw_grid(), s, wk, cnt, nullptr, bins, u_key, u_sgn, u_flag, u_count, nullptr);
+  k_merge_body<W, R, true>(hw_grid(), s, wk, cnt, nullptr, bins, u_key, u_sgn, u_flag, u_count, nullptr, false);
 }
 
 // ------------------------------------------------------ semistochastic core
