@@ -351,12 +351,14 @@ __global__ void k_begin_iter(ngpu_iter_out_t* out, double* part, Counters* cnt, 
   }
 }
 
+constexpr int kEndThreads = 512;  // one pass over one replica's statistics
+
 // sum of the block-statistics rows, final counters of the iteration, then
 // accumulation into the cycle sums (ENumCyc, HFCyc, NoBorn, ... are cycle
 // accumulators in the reference too)
 __device__ __forceinline__ void end_iter_body(ngpu_iter_out_t* out, double* part, ngpu_iter_out_t* cyc, Counters* cnt,
                                               int64_t scap, int64_t cap, int64_t hash_entries, const IterParams* prm,
-                                              uint32_t* scount) {
+                                              uint32_t* scount, int S) {
   // halted: the output block keeps the failing iteration's statistics and
   // error, and nothing is added to the cycle
   if (cnt->halt) return;
@@ -385,18 +387,40 @@ __device__ __forceinline__ void end_iter_body(ngpu_iter_out_t* out, double* part
   }
   double* g = (double*)out;
   double* c = (double*)cyc;
-  for (int i = threadIdx.x; i < kStatStride; i += blockDim.x) {
-    bool is_max = stat_is_max(i);
+  // the statistics rows: kEndParts threads per field take kStatCopies /
+  // kEndParts rows each, all loads in one round trip.  Only the S replicas'
+  // fields are ever written.
+  __shared__ double sums[kStatStride];
+  constexpr int kEndParts = 8, kRows = kStatCopies / kEndParts;
+  const int nfields = F_NFIELDS * S + (kStatStride - S_NVALID);
+  for (int t = threadIdx.x; t < (nfields * kEndParts + kWave - 1) / kWave * kWave; t += blockDim.x) {
+    const int f = t / kEndParts, part0 = (t % kEndParts) * kRows;
+    const int i = f < F_NFIELDS * S ? soff(f / S, f % S) : S_NVALID + (f - F_NFIELDS * S);
+    const bool on = f < nfields, is_max = stat_is_max(i);
+    double x[kRows];
+#pragma unroll
+    for (int q = 0; q < kRows; ++q) x[q] = on ? part[(size_t)(part0 + q) * kStatStride + i] : 0.0;
     double v = 0.0;
-    for (int q = 0; q < kStatCopies; ++q) {
-      double x = part[(size_t)q * kStatStride + i];
-      part[(size_t)q * kStatStride + i] = 0.0;  // empty for the next iteration
-      v = is_max ? (x > v ? x : v) : v + x;
+#pragma unroll
+    for (int q = 0; q < kRows; ++q) {
+      if (on && x[q] != 0.0) part[(size_t)(part0 + q) * kStatStride + i] = 0.0;  // empty for the next iteration
+      v = is_max ? (x[q] > v ? x[q] : v) : v + x[q];
     }
+#pragma unroll
+    for (int o = 1; o < kEndParts; o <<= 1) {
+      const double y = __shfl_xor(v, o);
+      v = is_max ? (y > v ? y : v) : v + y;
+    }
+    if (on && part0 == 0) sums[i] = v;
+  }
+  __syncthreads();
+  for (int f = threadIdx.x; f < nfields; f += blockDim.x) {
+    const int i = f < F_NFIELDS * S ? soff(f / S, f % S) : S_NVALID + (f - F_NFIELDS * S);
+    const double v = sums[i];
     if (i == X_NOCC) cnt->n_occ = (unsigned long long)v;
     if (i >= S_NDOUBLE) continue;
     g[i] = v;
-    if (is_max) c[i] = c[i] > v ? c[i] : v;
+    if (stat_is_max(i)) c[i] = c[i] > v ? c[i] : v;
     else if (i >= soff(F_INSTHF, 0) && i < soff(F_INSTHF, kMaxRep)) c[i] = v;
     else c[i] += v;
   }
@@ -435,16 +459,16 @@ __device__ __forceinline__ void end_iter_body(ngpu_iter_out_t* out, double* part
     cnt->err = 0;
   }
 }
-__global__ void k_end_iter(ngpu_iter_out_t* out, double* part, ngpu_iter_out_t* cyc, Counters* cnt,
+__global__ void __launch_bounds__(kEndThreads) k_end_iter(ngpu_iter_out_t* out, double* part, ngpu_iter_out_t* cyc, Counters* cnt,
                            int64_t scap, int64_t cap, int64_t hash_entries, const IterParams* prm,
-                           uint32_t* scount) {
-  end_iter_body(out, part, cyc, cnt, scap, cap, hash_entries, prm, scount);
+                           uint32_t* scount, int S) {
+  end_iter_body(out, part, cyc, cnt, scap, cap, hash_entries, prm, scount, S);
 }
 // the end of the iteration of every engine of a batch group: one block each
-__global__ void km_end_iter(const EngDev* __restrict__ ed) {
+__global__ void __launch_bounds__(kEndThreads) km_end_iter(const EngDev* __restrict__ ed) {
   const EngDev& a = ed[blockIdx.x];
   end_iter_body(a.dout, a.part, a.dcyc, a.cnt, a.scap, a.wk.cap, a.wk.L * (int64_t)kBucketEntries, a.prm,
-                a.bins.scount);
+                a.bins.scount, a.s.S);
 }
 
 __global__ void k_reset_cycle(ngpu_iter_out_t* cyc) {
@@ -589,8 +613,8 @@ void annihilation_chain(ngpu_t* h, bool with_core, bool list_out = false) {
   insert_new<W, R>(h, 7);
   if (!by_parts) launch(h, 8, 8, k_stats<W, R>, dim3(h->nb_grid), dim3(kBlock), h->ds, h->wk, h->cnt, h->dpart,
          (const IterParams*)h->dparams);
-  launch(h, -1, -1, k_end_iter, dim3(1), dim3(kBlock), h->dout, h->dpart, h->dcyc, h->cnt,
-         h->scap, h->wk.cap, h->wk.L * (int64_t)kBucketEntries, (const IterParams*)h->dparams, h->bins.scount);
+  launch(h, -1, -1, k_end_iter, dim3(1), dim3(kEndThreads), h->dout, h->dpart, h->dcyc, h->cnt,
+         h->scap, h->wk.cap, h->wk.L * (int64_t)kBucketEntries, (const IterParams*)h->dparams, h->bins.scount, h->S);
   if (h->checks) check_chain<W>(h, with_core);
 }
 
@@ -2810,7 +2834,7 @@ void group_chain_wr(BatchGroup& g) {
   bool pass = false;  // an engine whose statistics take a pass over its table
   for (const ngpu_t* h : g.hs) pass = pass || !stats_by_parts(h->ds);
   if (pass) glaunch(h0, 8, 8, km_stats<W, R>, g.tot[kLkGrid], kBlock, 0, ed, (const uint16_t*)m[kLkGrid]);
-  glaunch(h0, -1, -1, km_end_iter, (int)g.hs.size(), kBlock, 0, ed);
+  glaunch(h0, -1, -1, km_end_iter, (int)g.hs.size(), kEndThreads, 0, ed);
 }
 
 void group_chain(BatchGroup& g) {

@@ -152,31 +152,60 @@ __device__ inline uint64_t lanemask_lt() {
   return l == 0 ? 0ull : (~0ull >> (64 - l));
 }
 
-// wave-aggregated append: returns the index for lanes with pred, -1 otherwise.
-// Must be reached by every active lane of the wave.
-__device__ inline long long wave_append(bool pred, unsigned long long* counter, int n = 1) {
-  uint64_t m = __ballot(pred);
-  if (m == 0) return -1;
-  int leader = __ffsll((unsigned long long)m) - 1;
-  unsigned long long base = 0;
-  if (lane_id() == leader) base = atomicAdd(counter, (unsigned long long)(popc64(m) * n));
-  base = __shfl(base, leader);
-  if (!pred) return -1;
-  return (long long)(base + (unsigned long long)(popc64(m & lanemask_lt()) * n));
+// A lane's value moved by DPP (row_shr within rows of 16, then the rows'
+// last lanes to the rows after them); lanes without a source get 0.  A wave
+// reduction by these is VALU code of a few dozen cycles; by ds_bpermute
+// shuffles it is six LDS round trips (0.3 us), which the 7 to 13 statistics
+// of a kernel made 2 to 4 us of each launch.
+template <int CTRL, int ROWS>
+__device__ inline uint32_t dpp_u32(uint32_t v) {
+  return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, ROWS, 0xF, CTRL < 0x140);
 }
-
+template <int CTRL, int ROWS>
+__device__ inline uint64_t dpp_u64(uint64_t v) {
+  return ((uint64_t)dpp_u32<CTRL, ROWS>((uint32_t)(v >> 32)) << 32) | dpp_u32<CTRL, ROWS>((uint32_t)v);
+}
+template <int CTRL, int ROWS>
+__device__ inline double dpp_f64(double v) {
+  return __longlong_as_double((long long)dpp_u64<CTRL, ROWS>((uint64_t)__double_as_longlong(v)));
+}
+constexpr int kRowShr = 0x110, kRowBcast15 = 0x142, kRowBcast31 = 0x143;
+// a value of one lane (wave-uniform index), to every lane
+__device__ inline uint32_t lane_value(uint32_t v, int l) { return (uint32_t)__builtin_amdgcn_readlane((int)v, l); }
+__device__ inline uint64_t lane_value(uint64_t v, int l) {
+  return ((uint64_t)lane_value((uint32_t)(v >> 32), l) << 32) | lane_value((uint32_t)v, l);
+}
+// inclusive sums over the lanes (every lane of the wave active)
+__device__ inline int64_t wave_scan(int64_t x) {
+  uint64_t v = (uint64_t)x;
+  v += dpp_u64<kRowShr + 1, 0xF>(v);
+  v += dpp_u64<kRowShr + 2, 0xF>(v);
+  v += dpp_u64<kRowShr + 4, 0xF>(v);
+  v += dpp_u64<kRowShr + 8, 0xF>(v);
+  v += dpp_u64<kRowBcast15, 0xA>(v);
+  v += dpp_u64<kRowBcast31, 0xC>(v);
+  return (int64_t)v;
+}
+// sum over the wave, to every lane
 __device__ inline double wave_sum(double v) {
-#pragma unroll
-  for (int o = kWave / 2; o > 0; o >>= 1) v += __shfl_xor(v, o);
-  return v;
+  v += dpp_f64<kRowShr + 1, 0xF>(v);
+  v += dpp_f64<kRowShr + 2, 0xF>(v);
+  v += dpp_f64<kRowShr + 4, 0xF>(v);
+  v += dpp_f64<kRowShr + 8, 0xF>(v);
+  v += dpp_f64<kRowBcast15, 0xA>(v);
+  v += dpp_f64<kRowBcast31, 0xC>(v);
+  return __longlong_as_double((long long)lane_value((uint64_t)__double_as_longlong(v), kWave - 1));
 }
+// maximum over the wave of values >= 0, to every lane
 __device__ inline double wave_max(double v) {
-#pragma unroll
-  for (int o = kWave / 2; o > 0; o >>= 1) {
-    double w = __shfl_xor(v, o);
-    v = w > v ? w : v;
-  }
-  return v;
+  auto up = [&](double w) { v = w > v ? w : v; };
+  up(dpp_f64<kRowShr + 1, 0xF>(v));
+  up(dpp_f64<kRowShr + 2, 0xF>(v));
+  up(dpp_f64<kRowShr + 4, 0xF>(v));
+  up(dpp_f64<kRowShr + 8, 0xF>(v));
+  up(dpp_f64<kRowBcast15, 0xA>(v));
+  up(dpp_f64<kRowBcast31, 0xC>(v));
+  return __longlong_as_double((long long)lane_value((uint64_t)__double_as_longlong(v), kWave - 1));
 }
 __device__ inline unsigned long long wave_count(bool p) { return (unsigned long long)popc64(__ballot(p)); }
 
@@ -231,7 +260,7 @@ __device__ inline int stage_push(bool pred, Stage* st) {
   int leader = __ffsll((unsigned long long)m) - 1;
   uint32_t b = 0;
   if (lane_id() == leader) b = atomicAdd(&st->n, (uint32_t)popc64(m));
-  b = __shfl(b, leader);
+  b = lane_value(b, leader);
   return pred ? (int)(b + (uint32_t)popc64(m & lanemask_lt())) : -1;
 }
 
@@ -443,8 +472,11 @@ __device__ inline uint64_t* bin_record(Counters* cnt, const Bins& bins, uint32_t
   return bins.ovf + (size_t)atomicAdd(&cnt->n_ovf, 1ull) * rec_words;
 }
 
+// this block's slots: whole waves, so that a small table does not
+// spread over more blocks than it fills (each pays its set-up and its
+// statistics' atomics) and every block starts on a line
 __device__ inline void chunk_of(const Grid& g, int64_t n, int64_t& begin, int64_t& end) {
-  int64_t chunk = (n + g.nb - 1) / g.nb;
+  int64_t chunk = ((n + g.nb - 1) / g.nb + kWave - 1) / kWave * kWave;
   begin = g.b * chunk;
   end = begin + chunk;
   if (end > n) end = n;
@@ -477,19 +509,16 @@ struct LaneMax {
 
 // block exclusive scan of one int64 per thread (blockDim = kBlock)
 __device__ inline int64_t block_exclusive_scan(int64_t v, int64_t* lds, int64_t& total) {
-  int lane = lane_id(), wv = threadIdx.x / kWave;
-  int64_t x = v;
-#pragma unroll
-  for (int o = 1; o < kWave; o <<= 1) {
-    int64_t y = __shfl_up(x, o);
-    if (lane >= o) x += y;
-  }
+  const int lane = lane_id(), wv = threadIdx.x / kWave;
+  const int64_t x = wave_scan(v);
   if (lane == kWave - 1) lds[wv] = x;
   __syncthreads();
   int64_t pre = 0, tot = 0;
+#pragma unroll
   for (int q = 0; q < kBlock / kWave; ++q) {
-    if (q < wv) pre += lds[q];
-    tot += lds[q];
+    const int64_t n = lds[q];
+    if (q < wv) pre += n;
+    tot += n;
   }
   __syncthreads();
   total = tot;
@@ -530,15 +559,19 @@ __device__ __forceinline__ void k_prepass_body(const Grid& g_, const DevSys& s, 
   const uint32_t iter = use_v ? v.iter : prm->iter;
   if (use_v && g_.b == 0 && threadIdx.x == 0) *prm = v;
   __shared__ double acc_lds[kStatStride];
-  __shared__ int64_t red[kBlock / kWave];
-  BlockStats bs{acc_lds};
-  bs.zero();
+  __shared__ int64_t red[2 * kBlock / kWave];
   const int S = R == 1 ? 1 : s.S;
   int64_t nslots = (int64_t)cnt->nslots;
   const bool rebuild = cnt->rebuild != 0;
   if (rebuild) hash_clear_part<W>(g_, wk);  // the attempt scan refills the table
   int64_t begin, end;
   chunk_of(g_, nslots, begin, end);
+  if (begin >= end) {  // no slots for this block
+    if (threadIdx.x == 0) blk_part[g_.b] = blk_rm[g_.b] = 0;
+    return;
+  }
+  BlockStats bs{acc_lds};
+  bs.zero();
   int64_t my_att = 0, my_rm = 0;
   bool death_err = false;
   LaneSum<R> a_idets, a_iwalk, a_ndets, a_nwalk, a_hf, a_doubs, a_enum, a_died, a_born, a_abort, a_tot, a_norm;
@@ -685,11 +718,22 @@ __device__ __forceinline__ void k_prepass_body(const Grid& g_, const DevSys& s, 
     a_norm.done(bs, soff(F_NORMSQ, 0));
     a_occ.done(bs, X_NOCC);
   }
-  int64_t tot;
-  (void)block_exclusive_scan(my_att, red, tot);
-  if (threadIdx.x == 0) blk_part[g_.b] = tot;
-  (void)block_exclusive_scan(my_rm, red, tot);
-  if (threadIdx.x == 0) blk_rm[g_.b] = tot;
+  my_att = wave_scan(my_att);
+  my_rm = wave_scan(my_rm);
+  if (lane_id() == kWave - 1) {
+    red[2 * (threadIdx.x / kWave)] = my_att;
+    red[2 * (threadIdx.x / kWave) + 1] = my_rm;
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    int64_t a = 0, f = 0;
+    for (int q = 0; q < kBlock / kWave; ++q) {
+      a += red[2 * q];
+      f += red[2 * q + 1];
+    }
+    blk_part[g_.b] = a;
+    blk_rm[g_.b] = f;
+  }
   bs.flush(part, g_.b);
 }
 template <int W, int R>
@@ -720,6 +764,9 @@ __device__ __forceinline__ void k_scan_apply_body(const Grid& g_, const DevSys& 
   }
   int64_t begin, end;
   chunk_of(g_, nslots, begin, end);
+  // the block of the last slots closes the scan; an empty table is block 0's
+  const bool last = end == nslots && (begin < end || (nslots == 0 && g_.b == 0));
+  if (begin >= end && !last) return;
   // this block's first attempt offset and first free-queue position: the
   // counts of the blocks before it.  The slots the prepass freed go, in slot
   // order, after the free queue's tail (the prepass appends nothing itself,
@@ -778,7 +825,7 @@ __device__ __forceinline__ void k_scan_apply_body(const Grid& g_, const DevSys& 
       run += tot;
     }
   }
-  if (g_.b == g_.nb - 1 && threadIdx.x == 0) {
+  if (last && threadIdx.x == 0) {
     att_off[nslots * S] = run;
     cnt->n_attempts = (unsigned long long)run;
     cnt->free_tail = tail0 + (unsigned long long)run_rm;
@@ -1081,6 +1128,8 @@ __device__ inline void spawn_attempt(const DevSys& s, const Walk& wk, Counters* 
 template <int W, int R, int G>
 __device__ __forceinline__ void k_spawn_body(const Grid& g_, const DevSys& s, const Walk& wk, Counters* cnt, double* part, const int64_t* att_off, const int64_t* tile_p, int64_t tcap, const uint8_t* pinfo, const Bins& bins, int64_t scap, int64_t* sq, const IterParams* prm) {
   if (cnt->halt) return;
+  const int64_t total = (int64_t)cnt->n_attempts;
+  if (g_.b * kBlock >= total) return;  // no attempts for this block
   const double tau = prm->tau;
   const uint32_t iter = prm->iter;
   __shared__ double acc_lds[kStatStride];
@@ -1090,7 +1139,6 @@ __device__ __forceinline__ void k_spawn_body(const Grid& g_, const DevSys& s, co
   bs.zero();
   stage_init(&ss.st);
   stage_init(&qs.st);
-  const int64_t total = (int64_t)cnt->n_attempts;
   const int64_t npairs = (int64_t)cnt->nslots * s.S;
   bool overflow = false;
   constexpr int mode = (G == kGenPchb || G == kGenPchbW) ? 1 : 0;
@@ -1225,6 +1273,9 @@ template <int W, int R, int PL, int G>
 __device__ __forceinline__ void k_spawn_singles_body(const Grid& g_, const DevSys& s, const Walk& wk, Counters* cnt, double* part, const uint8_t* pinfo, const Bins& bins, int64_t scap, const int64_t* sq, const IterParams* prm) {
   if (cnt->halt) return;
   constexpr int kGroups = kBlock / G;
+  int64_t nq = (int64_t)cnt->n_singles;
+  if (nq > scap) nq = scap;
+  if (g_.b * kGroups >= nq) return;  // no queued attempts for this block
   const double tau = prm->tau;
   const uint32_t iter = prm->iter;
   __shared__ double acc_lds[kStatStride];
@@ -1235,8 +1286,6 @@ __device__ __forceinline__ void k_spawn_singles_body(const Grid& g_, const DevSy
   bs.zero();
   stage_init(&ss.st);
   const int S = R == 1 ? 1 : s.S;
-  int64_t nq = (int64_t)cnt->n_singles;
-  if (nq > scap) nq = scap;
   bool overflow = false;
   SpawnAcc<R> acc;
   const int nsp = s.nbasis / 2;
@@ -1666,7 +1715,7 @@ __device__ inline void wave_free_write(const Walk& wk, const WaveStage<W, R>* ws
 __device__ inline unsigned long long wave_reserve(unsigned long long* ctr, int n) {
   unsigned long long b = 0;
   if (lane_id() == 0) b = atomicAdd(ctr, (unsigned long long)n);
-  return __shfl(b, 0);
+  return lane_value((uint64_t)b, 0);
 }
 // orders one wave's LDS accesses of different lanes: a wave's LDS operations
 // run in order, so only the compiler has to keep them so.  (A workgroup fence
@@ -1779,7 +1828,7 @@ __device__ __forceinline__ void k_merge_body(const Grid& g_, const DevSys& s, co
     const int l = ctz64(have);
     have &= have - 1;
     seg = seg0 + l * nwaves;
-    c_all = __shfl(my_c, l);
+    c_all = lane_value(my_c, l);
     return true;
   };
   struct Rec {  // a lane's record
@@ -2306,7 +2355,7 @@ __device__ inline double diag_group(const DevSys& s, const uint64_t* d, int g, d
 
 // AddNewHashDet (load_balancer.fpp:514-629) for the new list.  A wave takes D
 // determinants, one lane each for the hash entry and the walker row.  On a
-// short list (up to 8 per wave of the grid) the diagonal elements follow, by
+// short list (up to kShortList) the diagonal elements follow, by
 // groups of G lanes: its time is the length of one wave's instruction stream,
 // which the groups shorten (us per iteration, one lane before: 10e/20o, 700
 // new determinants 24 -> 13; two-word 26e/40o, 2.8e4 92 -> 49).  A long list
@@ -2314,6 +2363,7 @@ __device__ inline double diag_group(const DevSys& s, const uint64_t* d, int g, d
 // worse (14e/30o, 1.3e5: 55 with one lane, 56 with four, 102 with 16), so
 // there the lane sums its own.  G is 16, or 64 when a block's LDS does not
 // hold 16 determinants' terms; 1 for the lattice.
+constexpr int64_t kShortList = 32768;
 template <int W, int R, int G>
 __device__ __forceinline__ void k_insert_body(const Grid& g_, const DevSys& s, const Walk& wk, Counters* cnt, const uint64_t* n_key, const double* n_sgn, const uint32_t* n_flag, const unsigned long long* n_ptr, double* lds) {
   if (cnt->halt) return;
@@ -2341,7 +2391,9 @@ __device__ __forceinline__ void k_insert_body(const Grid& g_, const DevSys& s, c
   constexpr int kWaves = kBlock / kWave;
   const int lane = lane_id(), wv = threadIdx.x / kWave;
   const int64_t nwaves = g_.nb * kWaves;
-  const bool group = G > 1 && nn <= 8 * nwaves;
+  // short: at most kShortList determinants on the chip, the engine's share of
+  // them by its share of a batch launch
+  const bool group = G > 1 && nn * (int64_t)gridDim.x <= kShortList * g_.nb;
   constexpr int kPer = kWave / G;  // determinants of a wave's group step
   int64_t D = kWave;
   if (group) {
@@ -2457,6 +2509,10 @@ __global__ void k_post_insert(Counters* cnt, const unsigned long long* n_ptr, in
 template <int W, int R>
 __device__ __forceinline__ void k_stats_body(const Grid& g_, const DevSys& s, const Walk& wk, Counters* cnt, double* part, const IterParams* prm) {
   if (cnt->halt) return;
+  unsigned long long used, ns;
+  slots_after_insert(cnt, cnt->n_new, wk.cap, used, ns);  // the bookkeeping applies it later
+  const int64_t nslots = (int64_t)ns;
+  if (g_.b * blockDim.x >= nslots) return;  // no slots for this block
   const uint32_t iter = prm->iter;
   __shared__ double acc_lds[kStatStride];
   __shared__ FreeStage fs;
@@ -2464,9 +2520,6 @@ __device__ __forceinline__ void k_stats_body(const Grid& g_, const DevSys& s, co
   bs.zero();
   stage_init(&fs.st);
   const int S = R == 1 ? 1 : s.S;
-  unsigned long long used, ns;
-  slots_after_insert(cnt, cnt->n_new, wk.cap, used, ns);  // the bookkeeping applies it later
-  const int64_t nslots = (int64_t)ns;
   unsigned long long my_occ = 0;
   double tp[R], nq[R], rmv[R], bn[R];
   for (int r = 0; r < S; ++r) tp[r] = nq[r] = rmv[r] = bn[r] = 0.0;
