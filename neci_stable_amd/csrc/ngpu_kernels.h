@@ -483,28 +483,28 @@ __device__ inline void chunk_of(const Grid& g, int64_t n, int64_t& begin, int64_
   if (begin > n) begin = n;
 }
 
-// Per-lane statistic accumulator of one field: a register when the kernel is
-// built for one replica (the field index is then the same in every trip), the
-// block's LDS row otherwise.  add() and done() are wave-wide calls.
+// Per-lane statistic accumulator of one field: registers when the kernel is
+// built for one or two replicas (the replica of a call is then known at
+// compile time), the block's LDS row otherwise.  add() and done() are
+// wave-wide calls.
 template <int R>
 struct LaneSum {
-  double v = 0.0;
+  double v[R <= 2 ? R : 1] = {0.0};
   __device__ void add(BlockStats& bs, int i, double x) {
-    if constexpr (R == 1) v += x; else bs.add(i, x);
+    if constexpr (R == 1) v[0] += x;
+    else if constexpr (R == 2) v[i & (kMaxRep - 1)] += x;
+    else bs.add(i, x);
   }
   __device__ void done(BlockStats& bs, int i) {
-    if constexpr (R == 1) bs.add(i, v);
+    if constexpr (R <= 2)
+#pragma unroll
+      for (int r = 0; r < R; ++r) bs.add(i + r, v[r]);
   }
 };
-template <int R>
 struct LaneMax {
   double v = 0.0;
-  __device__ void add(BlockStats& bs, int i, double x) {
-    if constexpr (R == 1) v = x > v ? x : v; else bs.max(i, x);
-  }
-  __device__ void done(BlockStats& bs, int i) {
-    if constexpr (R == 1) bs.max(i, v);
-  }
+  __device__ void add(double x) { v = x > v ? x : v; }
+  __device__ void done(BlockStats& bs, int i) { bs.max(i, v); }
 };
 
 // block exclusive scan of one int64 per thread (blockDim = kBlock)
@@ -560,7 +560,7 @@ __device__ __forceinline__ void k_prepass_body(const Grid& g_, const DevSys& s, 
   if (use_v && g_.b == 0 && threadIdx.x == 0) *prm = v;
   __shared__ double acc_lds[kStatStride];
   __shared__ int64_t red[2 * kBlock / kWave];
-  const int S = R == 1 ? 1 : s.S;
+  const int S = R <= 2 ? R : s.S;
   int64_t nslots = (int64_t)cnt->nslots;
   const bool rebuild = cnt->rebuild != 0;
   if (rebuild) hash_clear_part<W>(g_, wk);  // the attempt scan refills the table
@@ -992,7 +992,7 @@ __device__ inline bool core_child(const DevSys& s, const Walk& wk, Counters* cnt
 template <int R>
 struct SpawnAcc {
   LaneSum<1> valid, invalid, bloomc1, bloomc2;
-  LaneMax<1> maxspawn, blooms1, blooms2;
+  LaneMax maxspawn, blooms1, blooms2;
   LaneSum<R> born, sing;
   __device__ void done(BlockStats& bs, int mode) {
     valid.done(bs, S_NVALID);
@@ -1026,7 +1026,7 @@ template <int W, int R, int G>
 __device__ inline void spawn_attempt(const DevSys& s, const Walk& wk, Counters* cnt, BlockStats& bs,
                                      SpawnAcc<R>& acc, const uint8_t* pinfo, bool active, int64_t p, uint32_t k,
                                      int mode, SpawnStage<W>* ss, QueueStage* qs, double tau, uint32_t iter) {
-  const int S = R == 1 ? 1 : s.S;
+  const int S = R <= 2 ? R : s.S;
   bool emit = false, queue = false;
   uint64_t child[W];
   double nspawn = 0.0, an = 0.0, raw = 0.0;
@@ -1099,7 +1099,7 @@ __device__ inline void spawn_attempt(const DevSys& s, const Walk& wk, Counters* 
   }
   acc.invalid.add(bs, S_NINVALID, invalid);
   acc.valid.add(bs, S_NVALID, valid);
-  acc.maxspawn.add(bs, S_MAXSPAWN, raw);
+  acc.maxspawn.add(raw);
   for (int rr = 0; rr < S; ++rr) {
     acc.born.add(bs, soff(F_NBORN, rr), rr == r ? an : 0.0);
     if (mode != 1) acc.sing.add(bs, soff(F_SPAWNSING, rr), (rr == r && ic == 1) ? an : 0.0);
@@ -1107,11 +1107,11 @@ __device__ inline void spawn_attempt(const DevSys& s, const Walk& wk, Counters* 
   bool bloom = emit && an > s.init_walk_no;
   if (mode != 2) {
     acc.bloomc2.add(bs, S_BLOOMC + 2, (bloom && ic == 2) ? 1.0 : 0.0);
-    acc.blooms2.add(bs, S_BLOOMS + 2, (bloom && ic == 2) ? an : 0.0);
+    acc.blooms2.add((bloom && ic == 2) ? an : 0.0);
   }
   if (mode != 1) {
     acc.bloomc1.add(bs, S_BLOOMC + 1, (bloom && ic == 1) ? 1.0 : 0.0);
-    acc.blooms1.add(bs, S_BLOOMS + 1, (bloom && ic == 1) ? an : 0.0);
+    acc.blooms1.add((bloom && ic == 1) ? an : 0.0);
   }
   int idx = stage_push(emit, &ss->st);
   if (emit) {
@@ -1285,7 +1285,7 @@ __device__ __forceinline__ void k_spawn_singles_body(const Grid& g_, const DevSy
   BlockStats bs{acc_lds};
   bs.zero();
   stage_init(&ss.st);
-  const int S = R == 1 ? 1 : s.S;
+  const int S = R <= 2 ? R : s.S;
   bool overflow = false;
   SpawnAcc<R> acc;
   const int nsp = s.nbasis / 2;
@@ -1414,14 +1414,14 @@ __device__ __forceinline__ void k_spawn_singles_body(const Grid& g_, const DevSy
       }
       acc.invalid.add(bs, S_NINVALID, invalid);
       acc.valid.add(bs, S_NVALID, valid);
-      acc.maxspawn.add(bs, S_MAXSPAWN, raw);
+      acc.maxspawn.add(raw);
       for (int rr2 = 0; rr2 < S; ++rr2) {
         acc.born.add(bs, soff(F_NBORN, rr2), rr2 == r ? an : 0.0);
         acc.sing.add(bs, soff(F_SPAWNSING, rr2), rr2 == r ? an : 0.0);
       }
       bool bloom = emit && an > s.init_walk_no;
       acc.bloomc1.add(bs, S_BLOOMC + 1, bloom ? 1.0 : 0.0);
-      acc.blooms1.add(bs, S_BLOOMS + 1, bloom ? an : 0.0);
+      acc.blooms1.add(bloom ? an : 0.0);
       int idx = stage_push(emit, &ss.st);
       if (emit) {
 #pragma unroll
@@ -1803,7 +1803,7 @@ __device__ __forceinline__ void k_merge_body(const Grid& g_, const DevSys& s, co
     tb->tag[i] = 0;
   }
   __syncthreads();
-  const int S = R == 1 ? 1 : s.S;
+  const int S = R <= 2 ? R : s.S;
   int n_list = 0, n_free = 0;  // staged (wave-uniform)
   unsigned int uniq = 0;
   double ann[R], st_ab[R], st_an[R], st_rm[R], st_bn[R], d_tot[R], d_norm[R];
@@ -2170,7 +2170,7 @@ __device__ __forceinline__ void k_core_apply_body(const Grid& g_, const DevSys& 
   __shared__ double acc_lds[kStatStride];
   BlockStats bs{acc_lds};
   bs.zero();
-  const int S = R == 1 ? 1 : s.S;
+  const int S = R <= 2 ? R : s.S;
   LaneSum<R> born, ann;
   int64_t trips = grid_trips(g_, ncore);
   for (int64_t t = 0; t < trips; ++t) {
@@ -2198,7 +2198,7 @@ __device__ __forceinline__ void k_core_apply_body(const Grid& g_, const DevSys& 
 }
 template <int R>
 __global__ void __launch_bounds__(kBlock) k_core_apply(DevSys s, Walk wk, const Counters* cnt, const int64_t* core_slot, const double* y, int64_t ncore, double* part) {
-  k_core_apply_body<R>(hw_grid(), s, wk, cnt, core_slot, y, ncore, part, R == 1 ? 1 : s.S);
+  k_core_apply_body<R>(hw_grid(), s, wk, cnt, core_slot, y, ncore, part, R <= 2 ? R : s.S);
 }
 
 // core Hamiltonian rows (calc_determ_hamil, fast_determ_hamil.F90:892-1548):
@@ -2367,7 +2367,7 @@ constexpr int64_t kShortList = 32768;
 template <int W, int R, int G>
 __device__ __forceinline__ void k_insert_body(const Grid& g_, const DevSys& s, const Walk& wk, Counters* cnt, const uint64_t* n_key, const double* n_sgn, const uint32_t* n_flag, const unsigned long long* n_ptr, double* lds) {
   if (cnt->halt) return;
-  const int S = R == 1 ? 1 : s.S;
+  const int S = R <= 2 ? R : s.S;
   int64_t nn = (int64_t)*n_ptr;
   // new det i takes the i-th queued free slot, past the queue a fresh slot
   // at the end of the table: positions follow from i, no atomics
@@ -2519,7 +2519,7 @@ __device__ __forceinline__ void k_stats_body(const Grid& g_, const DevSys& s, co
   BlockStats bs{acc_lds};
   bs.zero();
   stage_init(&fs.st);
-  const int S = R == 1 ? 1 : s.S;
+  const int S = R <= 2 ? R : s.S;
   unsigned long long my_occ = 0;
   double tp[R], nq[R], rmv[R], bn[R];
   for (int r = 0; r < S; ++r) tp[r] = nq[r] = rmv[r] = bn[r] = 0.0;
