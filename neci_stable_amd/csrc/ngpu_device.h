@@ -111,21 +111,24 @@ __host__ __device__ inline int excit_level(const uint64_t* a, const uint64_t* b)
   return c;
 }
 
-// rank-k (0-based) set bit of x, x has more than k bits set
+// rank-k (0-based) set bit of x, x has more than k bits set: the half that
+// holds it, then four bisections and a last bit on 32-bit words (half the
+// instructions of 64-bit shifts)
 __host__ __device__ inline int select64(uint64_t x, int k) {
-  int pos = 0;
-  int c = popc64(x & 0xFFFFFFFFull);
-  if (k >= c) { k -= c; x >>= 32; pos += 32; }
-  c = popc64(x & 0xFFFFull);
-  if (k >= c) { k -= c; x >>= 16; pos += 16; }
-  c = popc64(x & 0xFFull);
-  if (k >= c) { k -= c; x >>= 8; pos += 8; }
-  c = popc64(x & 0xFull);
-  if (k >= c) { k -= c; x >>= 4; pos += 4; }
-  c = popc64(x & 0x3ull);
-  if (k >= c) { k -= c; x >>= 2; pos += 2; }
-  c = (int)(x & 1ull);
-  if (k >= c) { pos += 1; }
+  const uint32_t lo = (uint32_t)x, hi = (uint32_t)(x >> 32);
+  int c = __builtin_popcount(lo);
+  bool up = k >= c;
+  uint32_t y = up ? hi : lo;
+  k -= up ? c : 0;
+  int pos = up ? 32 : 0;
+#pragma unroll
+  for (int h = 16; h >= 1; h >>= 1) {
+    c = __builtin_popcount(y & ((1u << h) - 1u));
+    up = k >= c;
+    y = up ? y >> h : y;
+    k -= up ? c : 0;
+    pos += up ? h : 0;
+  }
   return pos;
 }
 
@@ -147,6 +150,7 @@ __host__ __device__ inline int select_orb(const uint64_t* d, uint64_t mask, int 
 template <int W>
 __host__ __device__ inline int occ_between(const uint64_t* d, int a, int b) {
   int lo = a < b ? a : b, hi = a < b ? b : a;  // count bits lo+1 .. hi-1 (1-based)
+  if constexpr (W == 1) return popc64(d[0] & ((~0ull << lo) ^ (~0ull << (hi - 1))));  // orbitals 1..63
   int c = 0;
 #pragma unroll
   for (int w = 0; w < W; ++w) {
@@ -223,11 +227,13 @@ __host__ __device__ inline int64_t find_walker_hash(const uint64_t* d, const int
 }
 
 // --------------------------------------------------------- integrals
-// UMatInd_base (UMatCache.F90:257-303), real hermitian integrals, 1-based
-__host__ __device__ inline int64_t umat_ind(int i, int j, int k, int l) {
-  int64_t A = i > k ? ((int64_t)i * (i - 1)) / 2 + k : ((int64_t)k * (k - 1)) / 2 + i;
-  int64_t B = j > l ? ((int64_t)j * (j - 1)) / 2 + l : ((int64_t)l * (l - 1)) / 2 + j;
-  return A > B ? (A * (A - 1)) / 2 + B : (B * (B - 1)) / 2 + A;
+// UMatInd_base (UMatCache.F90:257-303), real hermitian integrals, 1-based.
+// At most 63 spatial orbitals: 2016 pairs, 2.03e6 entries, 32-bit arithmetic.
+__host__ __device__ inline uint32_t umat_ind(int i, int j, int k, int l) {
+  const uint32_t i1 = i > k ? i : k, k1 = i > k ? k : i, j1 = j > l ? j : l, l1 = j > l ? l : j;
+  const uint32_t A = i1 * (i1 - 1) / 2 + k1, B = j1 * (j1 - 1) / 2 + l1;
+  const uint32_t hi = A > B ? A : B, lo = A > B ? B : A;
+  return hi * (hi - 1) / 2 + lo;
 }
 
 __host__ __device__ inline bool is_beta(int orb) { return orb & 1; }
@@ -258,6 +264,10 @@ struct DevSys {
   // pairs, divided once on the host (the same IEEE quotients)
   int nalpha_ref, nbeta_ref;
   double pg_par_ref, pg_anti_ref;
+  // 1 / pparallel and 1 / (1 - pparallel) when both are powers of two (0.5),
+  // where multiplying is the same IEEE quotient; else 0
+  double pb_inv, pb_anti_inv;
+  double inv_nel;  // 1 / nel, divided once
   uint64_t ref[2];
   int64_t L;                   // walker hash buckets
   const int32_t* rh;           // RandomHash2
@@ -506,30 +516,50 @@ __device__ __host__ inline Excit gen_hubbard(const DevSys& s, const uint64_t* d,
   Excit ex{};
   int nel = s.nel;
   int elec = 1 + (int)(dr[0] * (double)nel);
-  double p_elec = 1.0 / (double)nel;
   int src = select_orb<W>(d, ~0ull, elec);
   int site = spat(src);
+  const int odd = is_beta(src) ? 1 : 0;
+  const int32_t* row = s.nbr + (site - 1) * s.maxnbr;
   double cum_sum = 0.0;
   double a = fabs(s.bhub);
-  for (int k = 0; k < s.maxnbr; ++k) {
-    int ns = s.nbr[(site - 1) * s.maxnbr + k];
+  constexpr int N = 4;  // neighbours loaded together; longer rows are read again below
+  int nb[N], n = 0;
+  bool more = true;
+#pragma unroll
+  for (int k = 0; k < N; ++k) nb[k] = k < s.maxnbr ? row[k] : 0;
+#pragma unroll
+  for (int k = 0; k < N; ++k) {
+    more = more && nb[k] != 0;  // a zero ends the row
+    if (more) {
+      n = k + 1;
+      if (!test_orb<W>(d, 2 * nb[k] - odd)) cum_sum += a;
+    }
+  }
+  for (int k = N; more && k < s.maxnbr; ++k) {
+    const int ns = row[k];
     if (ns == 0) break;
-    int orb = is_beta(src) ? 2 * ns - 1 : 2 * ns;
-    if (!test_orb<W>(d, orb)) cum_sum += a;
+    n = k + 1;
+    if (!test_orb<W>(d, 2 * ns - odd)) cum_sum += a;
   }
   if (cum_sum < kEps) return ex;
   double r = dr[1] * cum_sum;
   double cum = 0.0, prev = 0.0;
-  int orb = 0, k = 0;
-  for (; k < s.maxnbr; ++k) {
-    int ns = s.nbr[(site - 1) * s.maxnbr + k];
-    if (ns == 0) break;
-    int o = is_beta(src) ? 2 * ns - 1 : 2 * ns;
+  int orb = 0;
+  bool on = true;  // until the cumulated weight reaches r, or the last neighbour
+#pragma unroll
+  for (int k = 0; k < N; ++k) {
+    if (on && k < n) {
+      orb = 2 * nb[k] - odd;
+      prev = cum;
+      if (!test_orb<W>(d, orb)) cum += a;
+      on = cum < r;
+    }
+  }
+  for (int k = N; on && k < n; ++k) {
+    orb = 2 * row[k] - odd;
     prev = cum;
-    if (!test_orb<W>(d, o)) cum += a;
-    orb = o;
-    bool last = (k + 1 >= s.maxnbr) || s.nbr[(site - 1) * s.maxnbr + k + 1] == 0;
-    if (!(cum < r) || last) break;
+    if (!test_orb<W>(d, orb)) cum += a;
+    on = cum < r;
   }
   if (cum - prev == 0.0) return ex;
   double p_orb = (cum - prev) / cum_sum;
@@ -537,7 +567,7 @@ __device__ __host__ inline Excit gen_hubbard(const DevSys& s, const uint64_t* d,
   ex.e0 = src;
   ex.e1 = orb;
   ex.parity = single_parity<W>(d, src, orb);
-  ex.pgen = p_elec * p_orb;
+  ex.pgen = s.inv_nel * p_orb;
   return ex;
 }
 
@@ -634,41 +664,63 @@ template <int W>
 __device__ __host__ inline void pick_biased_elecs(const DevSys& s, const uint64_t* d, double r, int& o1,
                                                   int& o2, double& pgen) {
   const uint64_t kA = 0xAAAAAAAAAAAAAAAAull, kB = 0x5555555555555555ull;
-  int nalpha = 0, nbeta = 0;
+  int nalpha = 0;
 #pragma unroll
-  for (int w = 0; w < W; ++w) { nalpha += popc64(d[w] & kA); nbeta += popc64(d[w] & kB); }
-  int aa = nalpha * (nalpha - 1) / 2, bb = nbeta * (nbeta - 1) / 2;
-  int par = aa + bb, ab = nalpha * nbeta;
-  double pb = s.pparallel;
+  for (int w = 0; w < W; ++w) nalpha += popc64(d[w] & kA);
+  const int nbeta = s.nel - nalpha;  // every determinant has nel electrons
+  const int aa = nalpha * (nalpha - 1) / 2, bb = nbeta * (nbeta - 1) / 2;
+  const int par = aa + bb, ab = nalpha * nbeta;
+  const double pb = s.pparallel;
   o1 = o2 = 0;
   pgen = 0.0;
   if (r < pb ? par == 0 : ab == 0) return;  // no pair of the drawn spin type
-  const bool ref_counts = nalpha == s.nalpha_ref && nbeta == s.nbeta_ref;
+  const bool ref_counts = nalpha == s.nalpha_ref;
+  // the electrons as ranks k1, k2 among the set bits of masks m1, m2: selected
+  // once for both spin types
+  uint64_t m1, m2;
+  int k1, k2;
   if (r < pb) {
-    r = (r / pb) * (double)par;
-    int idx = (int)floor(r);
-    uint64_t mask = kA;
-    if (idx >= aa) { idx -= aa; mask = kB; }
+    r = (s.pb_inv != 0.0 ? r * s.pb_inv : r / pb) * (double)par;
+    int idx = (int)r;
+    const bool beta = idx >= aa;
+    if (beta) idx -= aa;
+    m1 = m2 = beta ? kB : kA;
     // the smallest n1 >= 2 with n1 (n1 - 1) / 2 > idx: the root of the
-    // quadratic, then one integer correction each way
-    int n1 = (int)floorf(0.5f * (1.0f + sqrtf(8.0f * (float)idx + 1.0f))) + 1;
+    // quadratic (to an ulp), then one integer correction each way
+#ifdef __HIP_DEVICE_COMPILE__
+    const float root = __builtin_amdgcn_sqrtf(8.0f * (float)idx + 1.0f);
+#else
+    const float root = sqrtf(8.0f * (float)idx + 1.0f);
+#endif
+    int n1 = (int)(0.5f * (1.0f + root)) + 1;
     if (n1 < 2) n1 = 2;
     if (n1 * (n1 - 1) / 2 <= idx) ++n1;
     if (n1 > 2 && (n1 - 1) * (n1 - 2) / 2 > idx) --n1;
-    int n2 = idx + 1 - ((n1 - 1) * (n1 - 2)) / 2;
-    o1 = select_orb<W>(d, mask, n2);
-    o2 = select_orb<W>(d, mask, n1);
+    k1 = idx - ((n1 - 1) * (n1 - 2)) / 2;
+    k2 = n1 - 1;
     pgen = ref_counts ? s.pg_par_ref : pb / (double)par;
   } else {
     pgen = ref_counts ? s.pg_anti_ref : (1.0 - pb) / (double)ab;
-    r = ((r - pb) / (1.0 - pb)) * (double)ab;
-    int idx = (int)floor(r);
-    int na = 1 + idx % nalpha;
-    int nb = 1 + (int)floor((double)idx / (double)nalpha);
-    int oa = select_orb<W>(d, kA, na), ob = select_orb<W>(d, kB, nb);
-    o1 = oa < ob ? oa : ob;
-    o2 = oa < ob ? ob : oa;
+    r = (s.pb_anti_inv != 0.0 ? (r - pb) * s.pb_anti_inv : (r - pb) / (1.0 - pb)) * (double)ab;
+    const int idx = (int)r;
+    // idx = nb nalpha + na, the quotient from its float reciprocal (idx < 2^12)
+    // and one correction each way
+#ifdef __HIP_DEVICE_COMPILE__
+    int q = (int)((float)idx * __builtin_amdgcn_rcpf((float)nalpha));
+#else
+    int q = (int)((float)idx * (1.0f / (float)nalpha));
+#endif
+    int rem = idx - q * nalpha;
+    if (rem < 0) { rem += nalpha; --q; }
+    if (rem >= nalpha) { rem -= nalpha; ++q; }
+    m1 = kA;
+    m2 = kB;
+    k1 = rem;
+    k2 = q;
   }
+  const int oa = select_orb<W>(d, m1, k1 + 1), ob = select_orb<W>(d, m2, k2 + 1);
+  o1 = oa < ob ? oa : ob;
+  o2 = oa < ob ? ob : oa;
 }
 
 // GAS_doubles_PCHB_spinorb_gen_exc (gasci_pchb_doubles_spinorb_fastweighted.fpp:131-244)
@@ -1183,7 +1235,7 @@ __device__ __host__ inline void apply_excit(const uint64_t* d, const Excit& ex, 
 
 // stochastic_round_r (lib/util_mod.fpp:207-224)
 __device__ __host__ inline double stochastic_round(double x, double r) {
-  double i = (double)(int64_t)x;
+  double i = trunc(x) + 0.0;  // INT(x); + 0.0: no negative zero
   double res = x - i;
   if (fabs(res) >= 1.0e-12)
     if (fabs(res) > r) i = i + (x >= 0.0 ? 1.0 : -1.0);
@@ -1210,7 +1262,7 @@ __device__ __host__ inline double attempt_create(const DevSys& s, double tau, do
 __device__ __host__ inline double attempt_die(bool real_coeff, double fac, double absc, double r) {
   if (real_coeff) return fac * absc;
   double rat = fac * absc;
-  double nd = (double)(int64_t)rat;
+  double nd = trunc(rat) + 0.0;
   rat = rat - nd;
   if (fabs(rat) > r) nd = nd + (rat >= 0.0 ? 1.0 : -1.0);
   return nd;

@@ -1154,6 +1154,7 @@ int ngpu_create(ngpu_t** out, const ngpu_sys_t* sys) {
   h->ds.seed = sys->seed;
   h->ds.L = sys->n_hash_buckets;
   h->ds.pdoubles = 1.0;
+  h->ds.inv_nel = 1.0 / (double)sys->nel;
   h->ds.spawn_fp32 = 0;
   h->ds.rec_words = kRecWords;
   if (rc == NGPU_OK) {
@@ -1327,6 +1328,10 @@ static void update_pair_probs(ngpu_t* h) {
   const double pb = h->ds.pparallel;
   h->ds.pg_par_ref = par > 0 ? pb / (double)par : 0.0;
   h->ds.pg_anti_ref = ab > 0 ? (1.0 - pb) / (double)ab : 0.0;
+  int e = 0;
+  const bool exact = pb > 0.0 && pb < 1.0 && std::frexp(pb, &e) == 0.5 && std::frexp(1.0 - pb, &e) == 0.5;
+  h->ds.pb_inv = exact ? 1.0 / pb : 0.0;
+  h->ds.pb_anti_inv = exact ? 1.0 / (1.0 - pb) : 0.0;
 }
 
 int ngpu_set_excitgen_pchb(ngpu_t* h, int32_t singles, int32_t particles, int32_t holes, double psingles,
