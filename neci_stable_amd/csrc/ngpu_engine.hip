@@ -172,6 +172,10 @@ struct ngpu_engine {
   int single_lanes = 4;  // lanes per heat-bath single attempt (4, 8 or 16)
   int nb_merge = 0;      // blocks of the merge-annihilation kernel (0: nb_grid)
   int n_cu = 256, max_chunk = 4096;
+  // blocks of the spawning kernels a compute unit holds (spawn_blocks)
+  const void* occ_kern[2] = {nullptr, nullptr};
+  size_t occ_lds[2] = {0, 0};
+  int occ[2] = {4, 4};
   hipStream_t stream = nullptr;
   DevSys ds{};
   Walk wk{};
@@ -428,6 +432,8 @@ __device__ __forceinline__ void end_iter_body(ngpu_iter_out_t* out, double* part
   }
   __syncthreads();
   if (threadIdx.x == 0) {
+    // checkValidSpawnedList (fcimc_helper.F90:483-510)
+    if (cnt->n_spawned > (unsigned long long)scap) cnt->err |= 1u << NGPU_ERR_SPAWN_FULL;
     out->tot_walkers = (int64_t)cnt->n_occ;
     out->n_attempts = (int64_t)cnt->n_attempts;
     int64_t ns = (int64_t)cnt->n_spawned;
@@ -636,6 +642,25 @@ void by_shape(int W, int S, F f) {
 template <typename F>
 void by_shape(const ngpu_t* h, F f) { by_shape(h->W, h->S, f); }
 
+// Blocks of the two spawning kernels (which = 0: k_spawn, 1: the queued
+// singles): as many as the chip holds at once, times grid_blocks over its
+// default of four per compute unit.  Their waves split the attempts evenly, so
+// a block too many is a second round of a few blocks, and one too few an idle
+// slot: at 14e/30o and 5e6 walkers, singles at three per compute unit (160
+// VGPRs) 135 us against 174 at four, k_spawn at five (91 VGPRs) 169 against
+// 177 at four and 204 at six.
+template <typename F>
+int spawn_blocks(ngpu_t* h, int which, F kern, size_t lds) {
+  if (h->occ_kern[which] != (const void*)kern || h->occ_lds[which] != lds) {
+    int n = 0;
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, (const void*)kern, kBlock, lds) != hipSuccess || n < 1) n = 4;
+    h->occ_kern[which] = (const void*)kern;
+    h->occ_lds[which] = lds;
+    h->occ[which] = n;
+  }
+  return std::max(64, (int)((int64_t)h->occ[which] * h->nb_grid / 4));
+}
+
 // the generator instance of an engine's spawn kernel
 int gen_of(const ngpu_t* h) {
   if (h->sys.model == NGPU_MODEL_HUBBARD) return kGenHubbard;
@@ -655,7 +680,7 @@ void iterate_chain(ngpu_t* h) {
   auto spawn = gen == kGenHubbard ? k_spawn<W, R, kGenHubbard>
              : gen == kGenUniform ? k_spawn<W, R, kGenUniform>
              : gen == kGenPchbW ? k_spawn<W, R, kGenPchbW> : k_spawn<W, R, kGenPchb>;
-  launch(h, 2, 2, spawn, dim3(h->nb_grid), dim3(kBlock), h->ds, h->wk, h->cnt, h->dpart,
+  launch(h, 2, 2, spawn, dim3(spawn_blocks(h, 0, spawn, 0)), dim3(kBlock), h->ds, h->wk, h->cnt, h->dpart,
          (const int64_t*)h->att_off, (const int64_t*)h->tile_p, h->tcap, (const uint8_t*)h->pinfo, h->bins,
          h->scap, h->sq, (const IterParams*)h->dparams);
   if (h->sys.model == NGPU_MODEL_MOLECULAR && !h->ds.uniform) {
@@ -671,7 +696,7 @@ void iterate_chain(ngpu_t* h) {
               : nsp <= 16 ? k_spawn_singles<W, R, 4, 4> : nsp <= 20 ? k_spawn_singles<W, R, 5, 4>
               : nsp <= 32 ? k_spawn_singles<W, R, 8, 4> : nsp <= 40 ? k_spawn_singles<W, R, 10, 4>
               : k_spawn_singles<W, R, 16, 4>;
-    launch_lds(h, 3, 3, kern, dim3(h->nb_grid), dim3(kBlock), lds, h->ds, h->wk, h->cnt, h->dpart,
+    launch_lds(h, 3, 3, kern, dim3(spawn_blocks(h, 1, kern, lds)), dim3(kBlock), lds, h->ds, h->wk, h->cnt, h->dpart,
                (const uint8_t*)h->pinfo, h->bins, h->scap, (const int64_t*)h->sq,
                (const IterParams*)h->dparams);
   }
@@ -1096,7 +1121,7 @@ int ngpu_create(ngpu_t** out, const ngpu_sys_t* sys) {
   fail(dalloc(&h->blk_rm, (size_t)h->max_chunk));
   // tiles of attempts with a recorded first parent: attempts up to 4x the
   // spawn capacity (beyond it the spawn kernel searches the offsets itself)
-  h->tcap = (4 * scap) / kBlock + 2;
+  h->tcap = (4 * scap) / kWave + 2;
   fail(dalloc(&h->tile_p, (size_t)h->tcap));
   {
     // one bin per kBinFill expected records, at most one per 64 of the
@@ -1107,6 +1132,7 @@ int ngpu_create(ngpu_t** out, const ngpu_sys_t* sys) {
     bn.cap = scap + 16 * (int64_t)bn.maxb;
     bn.words = std::max<uint32_t>(bn.maxb, (uint32_t)std::min<int64_t>(32 * (int64_t)bn.maxb, 1 << 19));
     bn.spill_cap = (uint32_t)(scap / 2 / kSpill + 1);
+    bn.ovf_cap = scap;
     fail(dalloc(&bn.rec, (size_t)bn.cap * kRecWords));
     fail(dalloc(&bn.spill, (size_t)bn.spill_cap * kSpill * kRecWords));
     fail(dalloc(&bn.ovf, (size_t)scap * kRecWords));

@@ -209,6 +209,20 @@ __device__ inline double wave_max(double v) {
 }
 __device__ inline unsigned long long wave_count(bool p) { return (unsigned long long)popc64(__ballot(p)); }
 
+__device__ inline unsigned long long wave_reserve(unsigned long long* ctr, int n) {
+  unsigned long long b = 0;
+  if (lane_id() == 0) b = atomicAdd(ctr, (unsigned long long)n);
+  return lane_value((uint64_t)b, 0);
+}
+// orders one wave's LDS accesses of different lanes: a wave's LDS operations
+// run in order, so only the compiler has to keep them so.  (A workgroup fence
+// would wait for every global access in flight, prefetches and stores too.)
+__device__ inline void wave_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // Block-local statistics in LDS.  Every add/max is a wave-wide call (all 64
 // lanes, inactive lanes passing 0): the wave reduces with shuffles and one lane
 // updates LDS, so no LDS address is contended by more than one lane per wave.
@@ -432,6 +446,7 @@ struct Bins {
   uint32_t* count;   // records of bin b at [b << bin_shift], emptied by the merge
   uint32_t* scount;  // records sent to each area, emptied at the iteration's end
   int64_t cap;
+  int64_t ovf_cap;   // the spawn capacity
   uint32_t spill_cap;
   uint32_t maxb;     // most bins
   uint32_t words;    // length of count
@@ -464,12 +479,15 @@ __device__ inline uint32_t bin_hash(const uint64_t* d) {
 __device__ inline uint32_t bin_of(uint32_t h, uint32_t nb) { return (uint32_t)(((uint64_t)h * nb) >> 32); }
 
 // where the record with place pos of bin b goes
+// (null: the overflow list is full, which takes more records than the spawn
+// capacity; the iteration's end reports those)
 __device__ inline uint64_t* bin_record(Counters* cnt, const Bins& bins, uint32_t b, uint32_t pos, uint32_t cap,
                                        int rec_words) {
   if (pos < cap) return bins.rec + ((size_t)b * cap + pos) * rec_words;
   const uint32_t a = b % kSpill, p = atomicAdd(&bins.scount[a], 1u);
   if (p < bins.spill_cap) return bins.spill + ((size_t)a * bins.spill_cap + p) * rec_words;
-  return bins.ovf + (size_t)atomicAdd(&cnt->n_ovf, 1ull) * rec_words;
+  const unsigned long long o = atomicAdd(&cnt->n_ovf, 1ull);
+  return o < (unsigned long long)bins.ovf_cap ? bins.ovf + (size_t)o * rec_words : nullptr;
 }
 
 // this block's slots: whole waves, so that a small table does not
@@ -742,8 +760,24 @@ __global__ void __launch_bounds__(kBlock) k_prepass(DevSys s, Walk wk, Counters*
 }
 
 
+// the tiles that begin among the v attempts from o on, of pair i
+__device__ inline void tile_mark(int64_t* tile_p, int64_t tcap, int64_t o, int64_t v, int64_t i) {
+  for (int64_t t = (o + kWave - 1) / kWave; t * kWave < o + v && t < tcap; ++t) tile_p[t] = i;
+}
+// pairs of many attempts (a reference of 2e5 walkers holds 3e3 tiles) are
+// marked by the whole wave; wave-wide call
+constexpr int64_t kTileRun = 16 * kWave;
+__device__ inline void tile_mark_runs(int64_t* tile_p, int64_t tcap, int64_t o, int64_t v, int64_t i) {
+  for (uint64_t m = __ballot(v > kTileRun); m; m &= m - 1) {
+    const int l = ctz64(m);
+    const int64_t lo = (int64_t)lane_value((uint64_t)o, l), lv = (int64_t)lane_value((uint64_t)v, l);
+    const int64_t li = (int64_t)lane_value((uint64_t)i, l);
+    for (int64_t t = (lo + kWave - 1) / kWave + lane_id(); t * kWave < lo + lv && t < tcap; t += kWave) tile_p[t] = li;
+  }
+}
+
 // attempt offsets per (slot, replica) pair, same chunking as k_prepass; also
-// the parent pair of the first attempt of every kBlock-attempt tile (the
+// the parent pair of the first attempt of every kWave-attempt tile (the
 // spawn kernel's tiles), written by the pair whose attempts contain it.  When
 // a rebuild is due, also the refill of the walker hash that the prepass
 // cleared, before any lookup of the iteration.
@@ -793,10 +827,11 @@ __device__ __forceinline__ void k_scan_apply_body(const Grid& g_, const DevSys& 
       }
       int64_t tot;
       int64_t pre = block_exclusive_scan(v | (f << kPackShift), red, tot);
+      const int64_t o = run + (pre & ((1ll << kPackShift) - 1));
+      tile_mark_runs(tile_p, tcap, o, v, i);
       if (i < end) {
-        int64_t o = run + (pre & ((1ll << kPackShift) - 1));
         att_off[i] = o;
-        for (int64_t t = (o + kBlock - 1) / kBlock; t * kBlock < o + v && t < tcap; ++t) tile_p[t] = i;
+        if (v <= kTileRun) tile_mark(tile_p, tcap, o, v, i);
         if (f) wk.freeq[(tail0 + (unsigned long long)(run_rm + (pre >> kPackShift))) % (unsigned long long)wk.cap] = i;
       }
       run += tot & ((1ll << kPackShift) - 1);
@@ -817,10 +852,11 @@ __device__ __forceinline__ void k_scan_apply_body(const Grid& g_, const DevSys& 
       int64_t v = i < pe ? att_cnt[i] : 0;
       int64_t tot;
       int64_t pre = block_exclusive_scan(v, red, tot);
+      const int64_t o = run + pre;
+      tile_mark_runs(tile_p, tcap, o, v, i);
       if (i < pe) {
-        int64_t o = run + pre;
         att_off[i] = o;
-        for (int64_t t = (o + kBlock - 1) / kBlock; t * kBlock < o + v && t < tcap; ++t) tile_p[t] = i;
+        if (v <= kTileRun) tile_mark(tile_p, tcap, o, v, i);
       }
       run += tot;
     }
@@ -851,19 +887,20 @@ __device__ inline int64_t parent_pair(const int64_t* att_off, int64_t lo, int64_
   return lo;
 }
 
-// LDS stages of the spawned list and of the queued single-excitation attempts
-constexpr int kSpawnStage = 576;
-constexpr int kParentWindow = 512;  // attempt offsets of one tile's parents staged in LDS
-constexpr int kQueueStage = 512;
+// One wave's LDS stages of its spawned records and of the single-excitation
+// attempts it queues.  Waves stage and flush on their own: the spawning
+// kernels have no block barrier between their set-up and their statistics, so
+// a wave that waits for its gathers holds up no other.
+constexpr int kParentWindow = 4096;  // pairs of a tile's window, holes included; longer ones are bisected
+constexpr int kSpawnStage = 128;     // flushed past 64
 template <int W>
 struct SpawnStage {
-  Stage st;
   uint64_t key[kSpawnStage * W];
   double val[kSpawnStage];
   uint32_t info[kSpawnStage];
 };
+constexpr int kQueueStage = 256;  // flushed past 192: one device atomic on the queue's counter each
 struct QueueStage {  // queued attempts as (parent pair, attempt number)
-  Stage st;
   int64_t p[kQueueStage];
   uint32_t k[kQueueStage];
 };
@@ -910,40 +947,32 @@ __device__ inline void rec_mark(const DevSys& s, uint64_t* r, bool on) {
   r[w] = on ? r[w] | bit : r[w] & ~bit;
 }
 
-// block-wide: drain staged spawns into their bins when due.  A thread's
-// counter atomics are all issued before the first of its records is written.
+// the wave's n staged spawns into their bins, at most two a lane; the counter
+// atomics are issued before the first record is written
 template <int W>
-__device__ inline void spawn_flush(SpawnStage<W>* ss, Counters* cnt, const Bins& bins, int64_t scap, bool force,
-                                   bool& overflow, const DevSys& s) {
-  uint32_t n;
-  unsigned long long base;
-  if (!stage_flush_begin(&ss->st, &cnt->n_spawned, kSpawnStage, force, n, base)) return;
+__device__ inline void spawn_flush(const SpawnStage<W>* ss, int n, Counters* cnt, const Bins& bins, const DevSys& s) {
+  wave_sync();
   const uint32_t nb = cnt->nbins, cap = cnt->bin_cap, sh = cnt->bin_shift;
-  constexpr int kPer = (kSpawnStage + kBlock - 1) / kBlock;
-  uint32_t bin[kPer], pos[kPer];
+  const int lane = lane_id();
+  uint32_t bin[2], pos[2];
 #pragma unroll
-  for (int j = 0; j < kPer; ++j) {
-    const uint32_t i = threadIdx.x + j * kBlock;
-    pos[j] = 0xFFFFFFFFu;
-    bin[j] = 0;
+  for (int j = 0; j < 2; ++j) {
+    const int i = lane + j * kWave;
+    bin[j] = pos[j] = 0;
     if (i < n) {
-      if (base + i < (unsigned long long)scap) {
-        bin[j] = bin_of(bin_hash<W>(ss->key + i * W), nb);
-        pos[j] = atomicAdd(&bins.count[(size_t)bin[j] << sh], 1u);
-      } else {
-        overflow = true;
-      }
+      bin[j] = bin_of(bin_hash<W>(ss->key + i * W), nb);
+      pos[j] = atomicAdd(&bins.count[(size_t)bin[j] << sh], 1u);
     }
   }
 #pragma unroll
-  for (int j = 0; j < kPer; ++j) {
-    const uint32_t i = threadIdx.x + j * kBlock;
-    if (pos[j] != 0xFFFFFFFFu) {
+  for (int j = 0; j < 2; ++j) {
+    const int i = lane + j * kWave;
+    if (i < n) {
       uint64_t* r = bin_record(cnt, bins, bin[j], pos[j], cap, s.rec_words);
-      rec_store<W>(s, r, ss->key + i * W, ss->val[i], ss->info[i]);
+      if (r) rec_store<W>(s, r, ss->key + i * W, ss->val[i], ss->info[i]);
     }
   }
-  stage_flush_end(&ss->st);
+  wave_sync();
 }
 
 // an explicit spawned list (n dense records) into the bins
@@ -954,26 +983,20 @@ __global__ void __launch_bounds__(kBlock) k_bin_list(DevSys s, Counters* cnt, co
     const uint64_t* q = list + i * s.rec_words;
     const uint32_t bin = bin_of(bin_hash<W>(q), nb), pos = atomicAdd(&bins.count[(size_t)bin << sh], 1u);
     uint64_t* r = bin_record(cnt, bins, bin, pos, cap, s.rec_words);
-    for (int w = 0; w < s.rec_words; ++w) r[w] = q[w];
+    if (r)
+      for (int w = 0; w < s.rec_words; ++w) r[w] = q[w];
   }
 }
 __global__ void k_set_bins(Counters* cnt, Bins bins, int64_t n) { set_bins(cnt, bins, (double)n); }
 
-__device__ inline void queue_flush(QueueStage* qs, Counters* cnt, int64_t* sq, int64_t scap, bool force,
+// the wave's n staged attempts to the queue from base on
+__device__ inline void queue_write(const QueueStage* qs, int n, unsigned long long base, int64_t* sq, int64_t scap,
                                    bool& overflow) {
-  uint32_t n;
-  unsigned long long base;
-  if (!stage_flush_begin(&qs->st, &cnt->n_singles, kQueueStage, force, n, base)) return;
-  for (uint32_t i = threadIdx.x; i < n; i += blockDim.x) {
-    unsigned long long d = base + i;
-    if (d < (unsigned long long)scap) {
-      sq[2 * d] = qs->p[i];
-      sq[2 * d + 1] = (int64_t)qs->k[i];
-    } else {
-      overflow = true;
-    }
+  for (int i = lane_id(); i < n; i += kWave) {
+    const unsigned long long d = base + (unsigned long long)i;
+    if (d < (unsigned long long)scap) *(longlong2*)(sq + 2 * d) = longlong2{qs->p[i], (int64_t)qs->k[i]};
+    else overflow = true;
   }
-  stage_flush_end(&qs->st);
 }
 
 // is_core_state (semi_stoch_procs.F90:590-605) of the child of an excitation:
@@ -1025,7 +1048,8 @@ constexpr int kGenHubbard = 0, kGenPchb = 1, kGenUniform = 2, kGenPchbW = 3;
 template <int W, int R, int G>
 __device__ inline void spawn_attempt(const DevSys& s, const Walk& wk, Counters* cnt, BlockStats& bs,
                                      SpawnAcc<R>& acc, const uint8_t* pinfo, bool active, int64_t p, uint32_t k,
-                                     int mode, SpawnStage<W>* ss, QueueStage* qs, double tau, uint32_t iter) {
+                                     int mode, SpawnStage<W>* ss, int& n_ss, QueueStage* qs, int& n_qs, double tau,
+                                     uint32_t iter) {
   const int S = R <= 2 ? R : s.S;
   bool emit = false, queue = false;
   uint64_t child[W];
@@ -1092,10 +1116,14 @@ __device__ inline void spawn_attempt(const DevSys& s, const Walk& wk, Counters* 
       }
     }
   }
-  int qi = qs ? stage_push(queue, &qs->st) : -1;
-  if (queue) {
-    qs->p[qi] = p;
-    qs->k[qi] = k;
+  if (mode == 1) {
+    const uint64_t m = __ballot(queue);
+    if (queue) {
+      const int qi = n_qs + popc64(m & lanemask_lt());
+      qs->p[qi] = p;
+      qs->k[qi] = k;
+    }
+    n_qs += popc64(m);
   }
   acc.invalid.add(bs, S_NINVALID, invalid);
   acc.valid.add(bs, S_NVALID, valid);
@@ -1113,13 +1141,15 @@ __device__ inline void spawn_attempt(const DevSys& s, const Walk& wk, Counters* 
     acc.bloomc1.add(bs, S_BLOOMC + 1, (bloom && ic == 1) ? 1.0 : 0.0);
     acc.blooms1.add((bloom && ic == 1) ? an : 0.0);
   }
-  int idx = stage_push(emit, &ss->st);
+  const uint64_t em = __ballot(emit);
   if (emit) {
+    const int idx = n_ss + popc64(em & lanemask_lt());
 #pragma unroll
     for (int w = 0; w < W; ++w) ss->key[idx * W + w] = child[w];
     ss->val[idx] = nspawn;
     ss->info[idx] = info;
   }
+  n_ss += popc64(em);
 }
 
 // all attempts: Hubbard spawns directly; molecular doubles spawn here while
@@ -1132,70 +1162,100 @@ __device__ __forceinline__ void k_spawn_body(const Grid& g_, const DevSys& s, co
   if (g_.b * kBlock >= total) return;  // no attempts for this block
   const double tau = prm->tau;
   const uint32_t iter = prm->iter;
+  constexpr int kWaves = kBlock / kWave;
+  constexpr int mode = (G == kGenPchb || G == kGenPchbW) ? 1 : 0;
   __shared__ double acc_lds[kStatStride];
-  __shared__ SpawnStage<W> ss;
-  __shared__ QueueStage qs;
+  __shared__ SpawnStage<W> sstages[kWaves];
+  __shared__ QueueStage qstages[mode == 1 ? kWaves : 1];
+  __shared__ uint32_t parents[kBlock];
+  __shared__ uint32_t tail_n[kWaves];
+  __shared__ unsigned long long tail_base;
+  __shared__ unsigned int blk_spawned;
   BlockStats bs{acc_lds};
+  if (threadIdx.x == 0) blk_spawned = 0;
   bs.zero();
-  stage_init(&ss.st);
-  stage_init(&qs.st);
+  const int wv = threadIdx.x / kWave, lane = lane_id();
+  SpawnStage<W>* ss = &sstages[wv];
+  QueueStage* qs = &qstages[mode == 1 ? wv : 0];
+  uint32_t* par = parents + wv * kWave;
+  int n_ss = 0, n_qs = 0;     // staged (wave-uniform)
+  unsigned int spawned = 0;
   const int64_t npairs = (int64_t)cnt->nslots * s.S;
   bool overflow = false;
-  constexpr int mode = (G == kGenPchb || G == kGenPchbW) ? 1 : 0;
   SpawnAcc<R> acc;
-  __shared__ int64_t pb[2];
-  __shared__ int64_t woff[kParentWindow];
-  int64_t trips = grid_trips(g_, total);
-  for (int64_t t = 0; t < trips; ++t) {
-    int64_t a = grid_elem(g_, t);
-    // the block's attempts are the consecutive tile a0 .. a0+kBlock-1: its
-    // parents lie between the tile's first parent and the next tile's
-    int64_t a0 = grid_elem(g_, t) - threadIdx.x;
-    int64_t tile = a0 / kBlock;
-    if (threadIdx.x == 0) {
-      int64_t lo = 0, hi = 0;
-      if (a0 < total) {
-        bool more = a0 + kBlock < total;
-        if (tile + 1 < tcap) {
-          lo = tile_p[tile];
-          hi = more ? tile_p[tile + 1] : npairs - 1;
-        } else {  // beyond the tile table: full searches
-          int64_t a1 = (more ? a0 + kBlock : total) - 1;
-          lo = parent_pair(att_off, 0, npairs - 1, a0);
-          hi = parent_pair(att_off, lo, npairs - 1, a1);
-        }
-      }
-      pb[0] = lo;
-      pb[1] = hi;
+  // tiles of 64 consecutive attempts, one per wave and trip
+  const int64_t stride = g_.nb * kBlock;
+  for (int64_t a0 = g_.b * kBlock + wv * kWave; a0 < total; a0 += stride) {
+    const int64_t a = a0 + lane, tile = a0 / kWave;
+    // the tile's parents lie between its first attempt's and the next tile's
+    const bool more = a0 + kWave < total, act = a < total;
+    int64_t lo, hi;
+    if (tile + 1 < tcap) {
+      lo = tile_p[tile];
+      hi = more ? tile_p[tile + 1] : npairs - 1;
+    } else {  // beyond the tile table: full searches
+      lo = parent_pair(att_off, 0, npairs - 1, a0);
+      hi = parent_pair(att_off, lo, npairs - 1, (more ? a0 + kWave : total) - 1);
     }
-    __syncthreads();
-    const int64_t lo = pb[0], hi = pb[1];
-    const int64_t nw = hi - lo + 1;
-    bool act = a < total;
     int64_t p = 0;
     uint32_t k = 0;
-    if (a0 < total && nw <= kParentWindow) {  // block-uniform: search the window in LDS
-      for (int64_t i = threadIdx.x; i < nw; i += blockDim.x) woff[i] = att_off[lo + i];
-      __syncthreads();
-      if (act) {
-        int64_t l = 0, h = nw - 1;
-        while (l < h) {
-          int64_t mid = (l + h + 1) >> 1;
-          if (woff[mid] <= a) l = mid; else h = mid - 1;
-        }
-        p = lo + l;
-        k = (uint32_t)(a - woff[l]);
+    if (hi - lo < kParentWindow) {
+      // each pair of the window marks its first attempt in the tile (of pairs
+      // at the same place the last one, which has the attempts), and a maximum
+      // over the lanes below spreads the marks
+      par[lane] = 0;
+      wave_sync();
+      for (int64_t i = lane; i <= hi - lo; i += kWave) {
+        const int64_t o = att_off[lo + i] - a0;
+        if (o < kWave) atomicMax(&par[o > 0 ? o : 0], (uint32_t)i);
       }
+      wave_sync();
+      uint32_t v = par[lane];
+      auto up = [&](uint32_t w) { v = w > v ? w : v; };
+      up(dpp_u32<kRowShr + 1, 0xF>(v));
+      up(dpp_u32<kRowShr + 2, 0xF>(v));
+      up(dpp_u32<kRowShr + 4, 0xF>(v));
+      up(dpp_u32<kRowShr + 8, 0xF>(v));
+      up(dpp_u32<kRowBcast15, 0xA>(v));
+      up(dpp_u32<kRowBcast31, 0xC>(v));
+      if (act) p = lo + v;
     } else if (act) {
       p = parent_pair(att_off, lo, hi, a);
-      k = (uint32_t)(a - att_off[p]);
     }
-    spawn_attempt<W, R, G>(s, wk, cnt, bs, acc, pinfo, act, p, k, mode, &ss, &qs, tau, iter);
-    spawn_flush<W>(&ss, cnt, bins, scap, false, overflow, s);
-    if (mode == 1) queue_flush(&qs, cnt, sq, scap, false, overflow);
+    if (act) k = (uint32_t)(a - att_off[p]);
+    const int before = n_ss;
+    spawn_attempt<W, R, G>(s, wk, cnt, bs, acc, pinfo, act, p, k, mode, ss, n_ss, qs, n_qs, tau, iter);
+    spawned += (unsigned int)(n_ss - before);
+    if (n_ss > kSpawnStage - kWave) {
+      spawn_flush<W>(ss, n_ss, cnt, bins, s);
+      n_ss = 0;
+    }
+    if (mode == 1 && n_qs > kQueueStage - kWave) {
+      wave_sync();
+      queue_write(qs, n_qs, wave_reserve(&cnt->n_singles, n_qs), sq, scap, overflow);
+      wave_sync();
+      n_qs = 0;
+    }
   }
-  spawn_flush<W>(&ss, cnt, bins, scap, true, overflow, s);
-  if (mode == 1) queue_flush(&qs, cnt, sq, scap, true, overflow);
+  if (n_ss) spawn_flush<W>(ss, n_ss, cnt, bins, s);
+  // what is still queued: one reservation per block
+  if (lane == 0) {
+    if (spawned) atomicAdd(&blk_spawned, spawned);
+    tail_n[wv] = (uint32_t)n_qs;
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    if (blk_spawned) atomicAdd(&cnt->n_spawned, (unsigned long long)blk_spawned);
+    unsigned int n = 0;
+    for (int q = 0; q < kWaves; ++q) n += tail_n[q];
+    if (mode == 1 && n) tail_base = atomicAdd(&cnt->n_singles, (unsigned long long)n);
+  }
+  if (mode == 1) {
+    __syncthreads();
+    unsigned int before = 0;
+    for (int q = 0; q < wv; ++q) before += tail_n[q];
+    queue_write(qs, n_qs, tail_base + before, sq, scap, overflow);
+  }
   if (overflow) atomicOr(&cnt->err, 1u << NGPU_ERR_SPAWN_FULL);
   acc.done(bs, mode);
   bs.flush(part, g_.b);
@@ -1279,14 +1339,18 @@ __device__ __forceinline__ void k_spawn_singles_body(const Grid& g_, const DevSy
   const double tau = prm->tau;
   const uint32_t iter = prm->iter;
   __shared__ double acc_lds[kStatStride];
-  __shared__ SpawnStage<W> ss;
+  constexpr int kWaves = kBlock / kWave;
+  __shared__ SpawnStage<W> sstages[kWaves];
+  __shared__ unsigned int blk_spawned;
+  if (threadIdx.x == 0) blk_spawned = 0;
+  SpawnStage<W>* ss = &sstages[threadIdx.x / kWave];
+  int n_ss = 0;  // staged (wave-uniform)
+  unsigned int spawned = 0;
   // per group: the signed H(src -> b) of its attempt, then their running sums
   extern __shared__ double hv_dyn[];
   BlockStats bs{acc_lds};
   bs.zero();
-  stage_init(&ss.st);
   const int S = R <= 2 ? R : s.S;
-  bool overflow = false;
   SpawnAcc<R> acc;
   const int nsp = s.nbasis / 2;
   const int mcount = (nsp + G - 1) / G;  // wave-uniform
@@ -1296,144 +1360,148 @@ __device__ __forceinline__ void k_spawn_singles_body(const Grid& g_, const DevSy
   const bool leader = g == 0;
   double* myv = hv_dyn + (size_t)gl * 2 * nsp;
   double* mycum = myv + nsp;
-  const int64_t groups = (int64_t)g_.nb * kGroups;
-  const int64_t grp = (int64_t)g_.b * kGroups + gl;
-  const int64_t trips = (nq + groups - 1) / groups;
-  for (int64_t t = 0; t < trips; ++t) {
-    // blocks whose groups are all past the queue skip the attempt (block-
-    // uniform, so the body's barrier is reached by all of the block or none)
-    if (t * groups + (int64_t)g_.b * kGroups < nq) {
-      int64_t q = t * groups + grp;
-      bool act = q < nq;
-      int64_t p = act ? sq[2 * q] : 0;
-      uint32_t k = act ? (uint32_t)sq[2 * q + 1] : 0u;
-      int64_t slot = p / S;
-      int r = (int)(p - slot * S);
-      uint64_t key[W];
+  constexpr int kPer = kWave / G;  // attempts of a wave's trip
+  const int64_t nwaves = g_.nb * kWaves;
+  for (int64_t q0 = (g_.b * kWaves + threadIdx.x / kWave) * kPer; q0 < nq; q0 += nwaves * kPer) {
+    const int64_t q = q0 + lane_id() / G;
+    const bool act = q < nq;
+    int64_t p = act ? sq[2 * q] : 0;
+    uint32_t k = act ? (uint32_t)sq[2 * q + 1] : 0u;
+    int64_t slot = p / S;
+    int r = (int)(p - slot * S);
+    uint64_t key[W];
 #pragma unroll
-      for (int w = 0; w < W; ++w) key[w] = act ? wk.keys[slot * W + w] : s.ref[w];  // idle groups: any valid det
-      // lane g < 3 draws Philox block g+1, all three in one pass of the wave;
-      // d1 = dsel (purpose 1), d5 = spawn rounding (purpose 2, second value),
-      // d2 = dorb (purpose 3, first)
-      static_assert(G >= 3, "three lanes of a group draw the attempt's Philox blocks");
-      double ua = 0.0, ub = 0.0;
-      if (g < 3) draw2<W>(s.seed, key, iter, r, k, (uint32_t)(g + 1), ua, ub);
-      const double d1 = __shfl(ub, gbase + 0);
-      const double d5 = __shfl(ub, gbase + 1);
-      const double d2 = __shfl(ua, gbase + 2);
-      int elec = 1 + (int)floor(d1 * (double)s.nel);
-      int src = select_orb<W>(key, ~0ull, elec);
-      int a = spat(src), off = is_beta(src) ? 1 : 0;
-      const double* row = s.jk + (size_t)2 * (a - 1) * nsp * nsp;
-      const double* frow = s.fref + (size_t)(src - 1) * nsp;
-      double v[PL];
+    for (int w = 0; w < W; ++w) key[w] = act ? wk.keys[slot * W + w] : s.ref[w];  // idle groups: any valid det
+    // lane g < 3 draws Philox block g+1, all three in one pass of the wave;
+    // d1 = dsel (purpose 1), d5 = spawn rounding (purpose 2, second value),
+    // d2 = dorb (purpose 3, first)
+    static_assert(G >= 3, "three lanes of a group draw the attempt's Philox blocks");
+    double ua = 0.0, ub = 0.0;
+    if (g < 3) draw2<W>(s.seed, key, iter, r, k, (uint32_t)(g + 1), ua, ub);
+    const double d1 = __shfl(ub, gbase + 0);
+    const double d5 = __shfl(ub, gbase + 1);
+    const double d2 = __shfl(ua, gbase + 2);
+    int elec = 1 + (int)floor(d1 * (double)s.nel);
+    int src = select_orb<W>(key, ~0ull, elec);
+    int a = spat(src), off = is_beta(src) ? 1 : 0;
+    const double* row = s.jk + (size_t)2 * (a - 1) * nsp * nsp;
+    const double* frow = s.fref + (size_t)(src - 1) * nsp;
+    double v[PL];
 #pragma unroll
-      for (int m = 0; m < PL; ++m) v[m] = (m < mcount && g + m * G < nsp) ? frow[g + m * G] : 0.0;
-      // the orbitals the parent occupies beyond the reference, then the
-      // reference's orbitals the parent lacks (hb_weight's order)
+    for (int m = 0; m < PL; ++m) v[m] = (m < mcount && g + m * G < nsp) ? frow[g + m * G] : 0.0;
+    // the orbitals the parent occupies beyond the reference, then the
+    // reference's orbitals the parent lacks (hb_weight's order)
 #pragma unroll
-      for (int w = 0; w < W; ++w) {
-        uint64_t x = key[w] & ~s.ref[w];
-        if ((src - 1) >> 6 == w) x &= ~(1ull << ((src - 1) & 63));
-        hb_corr<PL, G>(x, 64 * w, row, nsp, g, mcount, true, src, v);
-      }
+    for (int w = 0; w < W; ++w) {
+      uint64_t x = key[w] & ~s.ref[w];
+      if ((src - 1) >> 6 == w) x &= ~(1ull << ((src - 1) & 63));
+      hb_corr<PL, G>(x, 64 * w, row, nsp, g, mcount, true, src, v);
+    }
 #pragma unroll
-      for (int w = 0; w < W; ++w) {
-        uint64_t x = s.ref[w] & ~key[w];
-        if ((src - 1) >> 6 == w) x &= ~(1ull << ((src - 1) & 63));
-        hb_corr<PL, G>(x, 64 * w, row, nsp, g, mcount, false, src, v);
-      }
+    for (int w = 0; w < W; ++w) {
+      uint64_t x = s.ref[w] & ~key[w];
+      if ((src - 1) >> 6 == w) x &= ~(1ull << ((src - 1) & 63));
+      hb_corr<PL, G>(x, 64 * w, row, nsp, g, mcount, false, src, v);
+    }
 #pragma unroll
-      for (int m = 0; m < PL; ++m) {
-        int b = g + m * G + 1;
-        if (m < mcount && b <= nsp) {
-          int orb = 2 * b - off;
-          myv[b - 1] = test_orb<W>(key, orb) ? 0.0 : v[m];
-        }
-      }
-      __syncthreads();
-      // the normalisation, keeping the running sums (every lane of the group
-      // writes the same values, and reads its own writes below); then the
-      // first b whose running sum reaches r, by bisection over those sums:
-      // the running sums of a second sweep in the same order are the same
-      // values, so this is its selection (the last b when none reaches r)
-      double cum_sum = 0.0;
-      for (int b = 0; b < nsp; ++b) {
-        cum_sum += fabs(myv[b]);
-        mycum[b] = cum_sum;
-      }
-      double rr = d2 * cum_sum;
-      int lo = 0, hi = nsp - 1;
-      while (lo < hi) {
-        const int mid = (lo + hi) >> 1;
-        if (!(mycum[mid] < rr)) hi = mid;
-        else lo = mid + 1;
-      }
-      const int bsel = lo + 1;
-      const double vsel = myv[lo];
-      const double cpt = fabs(vsel);
-      bool mine_att = act && leader;
-      bool emit = false;
-      uint64_t child[W];
-      double nspawn = 0.0, an = 0.0, raw = 0.0, valid = 0.0, invalid = 0.0;
-      uint32_t info = 0;
-      bool cancel = false;
-      if (mine_att && s.ncore && (pinfo[p] & 4) && !(fabs(cum_sum) <= kEps || cpt == 0.0)) {
-        Excit ex{};
-        ex.ic = 1;
-        ex.e0 = src;
-        ex.e1 = 2 * bsel - off;
-        cancel = core_child<W>(s, wk, cnt, key, ex);  // from and to the core space
-      }
-      if (mine_att) {
-        if (fabs(cum_sum) <= kEps || cpt == 0.0) {
-          invalid = 1.0;
-        } else if (cancel) {
-          valid = 1.0;
-        } else {
-          valid = 1.0;
-          int tgt = 2 * bsel - off;
-          double pg = cpt / cum_sum;
-          pg = pg / (double)s.nel;
-          pg = pg * s.psingles;
-          double hel = single_parity<W>(key, src, tgt) ? -vsel : vsel;  // the weight's own sum
-          uint8_t pi = pinfo[p];
-          double wsign = (pi & 1) ? -1.0 : 1.0;
-          nspawn = attempt_create(s, tau, hel, pg, wsign, d5, raw);
-          raw = fabs(raw);
-          if (fabs(nspawn) > kEps) {
-            emit = true;
-            an = fabs(nspawn);
-#pragma unroll
-            for (int w = 0; w < W; ++w) child[w] = key[w];
-            flip_orb<W>(child, src);
-            flip_orb<W>(child, tgt);
-            info = (uint32_t)r | ((s.t_init && (pi & 2)) ? kInfoInit : 0u);
-          }
-        }
-      }
-      acc.invalid.add(bs, S_NINVALID, invalid);
-      acc.valid.add(bs, S_NVALID, valid);
-      acc.maxspawn.add(raw);
-      for (int rr2 = 0; rr2 < S; ++rr2) {
-        acc.born.add(bs, soff(F_NBORN, rr2), rr2 == r ? an : 0.0);
-        acc.sing.add(bs, soff(F_SPAWNSING, rr2), rr2 == r ? an : 0.0);
-      }
-      bool bloom = emit && an > s.init_walk_no;
-      acc.bloomc1.add(bs, S_BLOOMC + 1, bloom ? 1.0 : 0.0);
-      acc.blooms1.add(bloom ? an : 0.0);
-      int idx = stage_push(emit, &ss.st);
-      if (emit) {
-#pragma unroll
-        for (int w = 0; w < W; ++w) ss.key[idx * W + w] = child[w];
-        ss.val[idx] = nspawn;
-        ss.info[idx] = info;
+    for (int m = 0; m < PL; ++m) {
+      int b = g + m * G + 1;
+      if (m < mcount && b <= nsp) {
+        int orb = 2 * b - off;
+        myv[b - 1] = test_orb<W>(key, orb) ? 0.0 : v[m];
       }
     }
-    spawn_flush<W>(&ss, cnt, bins, scap, false, overflow, s);  // its barriers also order the reuse of hv
+    wave_sync();
+    // the normalisation, keeping the running sums (every lane of the group
+    // writes the same values, and reads its own writes below); then the
+    // first b whose running sum reaches r, by bisection over those sums:
+    // the running sums of a second sweep in the same order are the same
+    // values, so this is its selection (the last b when none reaches r)
+    double cum_sum = 0.0;
+    for (int b = 0; b < nsp; ++b) {
+      cum_sum += fabs(myv[b]);
+      mycum[b] = cum_sum;
+    }
+    double rr = d2 * cum_sum;
+    int lo = 0, hi = nsp - 1;
+    while (lo < hi) {
+      const int mid = (lo + hi) >> 1;
+      if (!(mycum[mid] < rr)) hi = mid;
+      else lo = mid + 1;
+    }
+    const int bsel = lo + 1;
+    const double vsel = myv[lo];
+    const double cpt = fabs(vsel);
+    bool mine_att = act && leader;
+    bool emit = false;
+    uint64_t child[W];
+    double nspawn = 0.0, an = 0.0, raw = 0.0, valid = 0.0, invalid = 0.0;
+    uint32_t info = 0;
+    bool cancel = false;
+    if (mine_att && s.ncore && (pinfo[p] & 4) && !(fabs(cum_sum) <= kEps || cpt == 0.0)) {
+      Excit ex{};
+      ex.ic = 1;
+      ex.e0 = src;
+      ex.e1 = 2 * bsel - off;
+      cancel = core_child<W>(s, wk, cnt, key, ex);  // from and to the core space
+    }
+    if (mine_att) {
+      if (fabs(cum_sum) <= kEps || cpt == 0.0) {
+        invalid = 1.0;
+      } else if (cancel) {
+        valid = 1.0;
+      } else {
+        valid = 1.0;
+        int tgt = 2 * bsel - off;
+        double pg = cpt / cum_sum;
+        pg = pg / (double)s.nel;
+        pg = pg * s.psingles;
+        double hel = single_parity<W>(key, src, tgt) ? -vsel : vsel;  // the weight's own sum
+        uint8_t pi = pinfo[p];
+        double wsign = (pi & 1) ? -1.0 : 1.0;
+        nspawn = attempt_create(s, tau, hel, pg, wsign, d5, raw);
+        raw = fabs(raw);
+        if (fabs(nspawn) > kEps) {
+          emit = true;
+          an = fabs(nspawn);
+#pragma unroll
+          for (int w = 0; w < W; ++w) child[w] = key[w];
+          flip_orb<W>(child, src);
+          flip_orb<W>(child, tgt);
+          info = (uint32_t)r | ((s.t_init && (pi & 2)) ? kInfoInit : 0u);
+        }
+      }
+    }
+    acc.invalid.add(bs, S_NINVALID, invalid);
+    acc.valid.add(bs, S_NVALID, valid);
+    acc.maxspawn.add(raw);
+    for (int rr2 = 0; rr2 < S; ++rr2) {
+      acc.born.add(bs, soff(F_NBORN, rr2), rr2 == r ? an : 0.0);
+      acc.sing.add(bs, soff(F_SPAWNSING, rr2), rr2 == r ? an : 0.0);
+    }
+    bool bloom = emit && an > s.init_walk_no;
+    acc.bloomc1.add(bs, S_BLOOMC + 1, bloom ? 1.0 : 0.0);
+    acc.blooms1.add(bloom ? an : 0.0);
+    const uint64_t em = __ballot(emit);
+    if (emit) {
+      const int idx = n_ss + popc64(em & lanemask_lt());
+#pragma unroll
+      for (int w = 0; w < W; ++w) ss->key[idx * W + w] = child[w];
+      ss->val[idx] = nspawn;
+      ss->info[idx] = info;
+    }
+    n_ss += popc64(em);
+    spawned += (unsigned int)popc64(em);
+    if (n_ss > kSpawnStage - kWave) {
+      spawn_flush<W>(ss, n_ss, cnt, bins, s);
+      n_ss = 0;
+    }
+    wave_sync();  // the next attempts reuse the weights' LDS
   }
-  spawn_flush<W>(&ss, cnt, bins, scap, true, overflow, s);
-  if (overflow) atomicOr(&cnt->err, 1u << NGPU_ERR_SPAWN_FULL);
+  if (n_ss) spawn_flush<W>(ss, n_ss, cnt, bins, s);
+  if (spawned && lane_id() == 0) atomicAdd(&blk_spawned, spawned);
+  __syncthreads();
+  if (threadIdx.x == 0 && blk_spawned) atomicAdd(&cnt->n_spawned, (unsigned long long)blk_spawned);
   acc.done(bs, 2);
   bs.flush(part, g_.b);
 }
@@ -1712,20 +1780,6 @@ __device__ inline void wave_free_write(const Walk& wk, const WaveStage<W, R>* ws
   for (int i = lane_id(); i < n; i += kWave)
     wk.freeq[(base + (unsigned long long)i) % (unsigned long long)wk.cap] = ws->freed[i];
 }
-__device__ inline unsigned long long wave_reserve(unsigned long long* ctr, int n) {
-  unsigned long long b = 0;
-  if (lane_id() == 0) b = atomicAdd(ctr, (unsigned long long)n);
-  return lane_value((uint64_t)b, 0);
-}
-// orders one wave's LDS accesses of different lanes: a wave's LDS operations
-// run in order, so only the compiler has to keep them so.  (A workgroup fence
-// would wait for every global access in flight, prefetches and stores too.)
-__device__ inline void wave_sync() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 // the table slot of each todo lane's key (one record per lane): inserted if
 // absent.  won: this lane inserted it; -1: the table is full of other keys.
 // Every lane probes slot by slot, so either all records of a determinant find
@@ -1860,7 +1914,7 @@ __device__ __forceinline__ void k_merge_body(const Grid& g_, const DevSys& s, co
     if (c_all > cap) {
       const uint32_t a = bins.scount[seg % kSpill];
       csp += a < bins.spill_cap ? a : bins.spill_cap;
-      total = csp + (a > bins.spill_cap ? (int64_t)cnt->n_ovf : 0);
+      total = csp + (a > bins.spill_cap ? (int64_t)(cnt->n_ovf < (unsigned long long)bins.ovf_cap ? cnt->n_ovf : bins.ovf_cap) : 0);
     }
     uint64_t* spill_rec = bins.spill + (size_t)(seg % kSpill) * bins.spill_cap * s.rec_words;
     uint64_t* seg_rec = bins.rec + (size_t)seg * cap * s.rec_words;
