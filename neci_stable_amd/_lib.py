@@ -87,7 +87,10 @@ class IterOutT(ctypes.Structure):
     ]
 
     def to_dict(self, nrep):
-        d = {f: np.array(getattr(self, f)[:nrep]) for f in REPLICA_FIELDS}
+        # the replica fields are consecutive rows of MAX_REPLICAS doubles: one copy of the block
+        rows = np.frombuffer(self, dtype=np.float64, count=len(REPLICA_FIELDS) * MAX_REPLICAS)
+        rows = rows.reshape(len(REPLICA_FIELDS), MAX_REPLICAS)[:, :nrep].copy()
+        d = dict(zip(REPLICA_FIELDS, rows))
         for f in ["n_valid_excits", "n_invalid_excits", "max_cyc_spawn", "tot_walkers",
                   "n_attempts", "n_spawned", "n_unique", "n_new", "err"]:
             d[f] = getattr(self, f)
