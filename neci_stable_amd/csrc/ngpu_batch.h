@@ -91,12 +91,12 @@ __global__ void __launch_bounds__(kBlock) km_spawn(const EngDev* __restrict__ ed
                         a.scap, a.sq, a.prm);
 }
 
-template <int W, int R, int PL, int G>
+template <int W, int R, int PP, int G>
 __global__ void __launch_bounds__(kBlock) km_spawn_singles(const EngDev* __restrict__ ed,
                                                            const uint16_t* __restrict__ map) {
   Grid g;
   const EngDev& a = eng_of(ed, map, kLkGrid, g);
-  k_spawn_singles_body<W, R, PL, G>(g, a.s, a.wk, a.cnt, a.part, a.pinfo, a.bins, a.scap, a.sq, a.prm);
+  k_spawn_singles_body<W, R, PP, G>(g, a.s, a.wk, a.cnt, a.part, a.pinfo, a.bins, a.scap, a.sq, a.prm);
 }
 
 template <int W, int R>

@@ -296,6 +296,9 @@ struct DevSys {
   // heat-bath singles: (U(a,j,b,j), U(a,j,j,b)) at jk[2*(((a-1)*nsp + j-1)*nsp + b-1)]
   // for spatial a, j, b; copies of UMAT entries, rows contiguous in b
   const double* jk;
+  // the same by rows: row (a-1, j-1) holds the U(a,j,b,j) of all b, then the
+  // U(a,j,j,b), each nsp rounded up to even (16-byte rows)
+  const double* jkrow;
   // diagonal elements: (U(i,j,i,j), U(i,j,j,i)) at jk0[2*((i-1)*nsp + j-1)]
   const double* jk0;
   // heat-bath single weights relative to the reference determinant:

@@ -231,6 +231,7 @@ struct ngpu_engine {
   double* d_tmat = nullptr;
   double* d_umat = nullptr;
   double* d_jk = nullptr;
+  double* d_jkrow = nullptr;
   double* d_jk0 = nullptr;
   double* d_fref = nullptr;  // reference-relative heat-bath single weights
   AliasEnt* d_ab_tab = nullptr;
@@ -288,7 +289,7 @@ struct BatchGroup {
   bool two = false;         // every engine has two replicas
   int gen = 0;              // kGenHubbard, kGenPchb or kGenUniform
   bool singles = false;     // queued heat-bath singles (PCHB generator)
-  int lanes = 4, pl = 4;    // heat-bath singles: lanes per attempt, orbitals per lane
+  int lanes = 4, pp = 2;    // heat-bath singles: lanes per attempt, orbital pairs per lane
   int items = 4;            // launch-shape knob of the set-up sorts
   int ins_lanes = 1;        // lanes per new determinant, and a block's LDS for them
   size_t ins_lds = 0;
@@ -675,6 +676,9 @@ int spawn_blocks(ngpu_t* h, int which, F kern, size_t lds) {
   return std::max(64, (int)((int64_t)h->occ[which] * h->nb_grid / 4));
 }
 
+// the queued singles' lists of differing orbitals
+size_t singles_lds(const ngpu_t* h) { return (size_t)kBlock * singles_list(h->sys.nel, h->sys.nbasis); }
+
 // the generator instance of an engine's spawn kernel
 int gen_of(const ngpu_t* h) {
   if (h->sys.model == NGPU_MODEL_HUBBARD) return kGenHubbard;
@@ -699,17 +703,15 @@ void iterate_chain(ngpu_t* h) {
          h->scap, h->sq, (const IterParams*)h->dparams);
   if (h->sys.model == NGPU_MODEL_MOLECULAR && !h->ds.uniform) {
     const int nsp = h->sys.nbasis / 2;
-    // G lanes per attempt, PL >= nsp / G orbitals per lane
+    // G lanes per attempt, PP >= nsp / 2G pairs of orbitals per lane
     const int G = h->single_lanes;
-    const size_t lds = 2 * sizeof(double) * (size_t)(kBlock / G) * nsp;  // weights and running sums
-    auto kern = G == 16 ? (nsp <= 16 ? k_spawn_singles<W, R, 1, 16> : nsp <= 32 ? k_spawn_singles<W, R, 2, 16>
-                           : k_spawn_singles<W, R, 4, 16>)
-              : G == 8 ? (nsp <= 16 ? k_spawn_singles<W, R, 2, 8> : nsp <= 24 ? k_spawn_singles<W, R, 3, 8>
-                          : nsp <= 32 ? k_spawn_singles<W, R, 4, 8> : nsp <= 40 ? k_spawn_singles<W, R, 5, 8>
-                          : k_spawn_singles<W, R, 8, 8>)
-              : nsp <= 16 ? k_spawn_singles<W, R, 4, 4> : nsp <= 20 ? k_spawn_singles<W, R, 5, 4>
-              : nsp <= 32 ? k_spawn_singles<W, R, 8, 4> : nsp <= 40 ? k_spawn_singles<W, R, 10, 4>
-              : k_spawn_singles<W, R, 16, 4>;
+    const size_t lds = singles_lds(h);
+    auto kern = G == 16 ? (nsp <= 32 ? k_spawn_singles<W, R, 1, 16> : k_spawn_singles<W, R, 2, 16>)
+              : G == 8 ? (nsp <= 16 ? k_spawn_singles<W, R, 1, 8> : nsp <= 32 ? k_spawn_singles<W, R, 2, 8>
+                          : nsp <= 48 ? k_spawn_singles<W, R, 3, 8> : k_spawn_singles<W, R, 4, 8>)
+              : nsp <= 16 ? k_spawn_singles<W, R, 2, 4> : nsp <= 24 ? k_spawn_singles<W, R, 3, 4>
+              : nsp <= 32 ? k_spawn_singles<W, R, 4, 4> : nsp <= 40 ? k_spawn_singles<W, R, 5, 4>
+              : nsp <= 48 ? k_spawn_singles<W, R, 6, 4> : k_spawn_singles<W, R, 8, 4>;
     launch_lds(h, 3, 3, kern, dim3(spawn_blocks(h, 1, kern, lds)), dim3(kBlock), lds, h->ds, h->wk, h->cnt, h->dpart,
                (const uint8_t*)h->pinfo, h->bins, h->scap, (const int64_t*)h->sq,
                (const IterParams*)h->dparams);
@@ -1220,7 +1222,7 @@ int ngpu_destroy(ngpu_t* h) {
   void* ptrs[] = {h->wk.keys, h->wk.st, h->wk.diagH, h->wk.offdiagH, h->wk.freeq,
                   h->wk.htab, h->att_cnt, h->att_off, h->pinfo, h->blk_part, h->blk_rm, h->bins.rec,
                   h->bins.spill, h->bins.ovf, h->bins.count, h->bins.scount, h->l_rec, h->hist, h->digit_tot, h->sq, h->n_key,
-                  h->n_sgn, h->n_flag, h->u_key, h->u_sgn, h->u_flag, h->u_count, h->cnt, h->dout, h->dpart, h->dcyc, h->own_params, h->d_rh, h->d_nbr, h->d_tmat, h->d_umat, h->d_jk, h->d_jk0, h->d_fref, h->d_chk, h->tile_p, h->core_keys, h->core_slot, h->core_rowptr, h->core_cols,
+                  h->n_sgn, h->n_flag, h->u_key, h->u_sgn, h->u_flag, h->u_count, h->cnt, h->dout, h->dpart, h->dcyc, h->own_params, h->d_rh, h->d_nbr, h->d_tmat, h->d_umat, h->d_jk, h->d_jkrow, h->d_jk0, h->d_fref, h->d_chk, h->tile_p, h->core_keys, h->core_slot, h->core_rowptr, h->core_cols,
                   h->core_vals, h->core_x, h->core_y, h->d_ab_tab,
                   h->d_ab_prob, h->d_ab_ok, h->d_j_tab, h->d_j_prob, h->d_j_ok, h->d_ab_tgt, h->d_i_tab, h->d_i_prob,
                   h->d_a_tab, h->d_a_prob, h->d_a_ok, h->d_b_tab, h->d_b_prob, h->d_b_ok};
@@ -1287,15 +1289,21 @@ int ngpu_set_integrals(ngpu_t* h, const double* tmat2d, const double* umat, int6
   if (int rc = table_upload(&h->d_tmat, tmat2d, nt)) return rc;
   if (int rc = table_upload(&h->d_umat, umat, (size_t)umat_len)) return rc;
   {
-    // (Coulomb, exchange) rows of the heat-bath single-excitation weights
-    std::vector<double> jk((size_t)nsp * nsp * nsp * 2);
+    // (Coulomb, exchange) rows of the heat-bath single-excitation weights; the
+    // singles' lanes past nsp read beyond the last row, less than 64 values
+    const size_t rs = (size_t)((nsp + 1) & ~1);
+    std::vector<double> jk((size_t)nsp * nsp * nsp * 2), rows((size_t)nsp * nsp * rs * 2 + 64);
     for (int a = 1; a <= nsp; ++a)
       for (int j = 1; j <= nsp; ++j)
         for (int b = 1; b <= nsp; ++b) {
           size_t e = 2 * (((size_t)(a - 1) * nsp + (j - 1)) * nsp + (b - 1));
           jk[e] = umat[umat_ind(a, j, b, j) - 1];
           jk[e + 1] = umat[umat_ind(a, j, j, b) - 1];
+          const size_t r = 2 * rs * ((size_t)(a - 1) * nsp + (j - 1)) + (b - 1);
+          rows[r] = jk[e];
+          rows[r + rs] = jk[e + 1];
         }
+    if (int rc = table_upload(&h->d_jkrow, rows.data(), rows.size())) return rc;
     if (int rc = table_upload(&h->d_jk, jk.data(), jk.size())) return rc;
     // (J, K) pairs of the diagonal elements
     std::vector<double> jk0((size_t)nsp * nsp * 2);
@@ -1310,6 +1318,7 @@ int ngpu_set_integrals(ngpu_t* h, const double* tmat2d, const double* umat, int6
   h->ds.tmat = h->d_tmat;
   h->ds.umat = h->d_umat;
   h->ds.jk = h->d_jk;
+  h->ds.jkrow = h->d_jkrow;
   h->ds.jk0 = h->d_jk0;
   h->ds.nsp = (int)nsp;
   h->ds.ecore = ecore;
@@ -2634,13 +2643,12 @@ int ngpu_set_graph(ngpu_t* h, int32_t on) {
 extern "C++" {
 namespace {
 
-// orbitals per lane of the heat-bath singles for lanes G and nsp spatial orbitals
-int singles_pl(int G, int nsp) {
-  if (G == 16) return nsp <= 16 ? 1 : nsp <= 32 ? 2 : 4;
-  if (G == 8) return nsp <= 16 ? 2 : nsp <= 24 ? 3 : nsp <= 32 ? 4 : nsp <= 40 ? 5 : 8;
-  return nsp <= 16 ? 4 : nsp <= 20 ? 5 : nsp <= 32 ? 8 : nsp <= 40 ? 10 : 16;
+// pairs of orbitals per lane of the heat-bath singles for lanes G and nsp spatial orbitals
+int singles_pp(int G, int nsp) {
+  if (G == 16) return nsp <= 32 ? 1 : 2;
+  if (G == 8) return nsp <= 16 ? 1 : nsp <= 32 ? 2 : nsp <= 48 ? 3 : 4;
+  return nsp <= 16 ? 2 : nsp <= 24 ? 3 : nsp <= 32 ? 4 : nsp <= 40 ? 5 : nsp <= 48 ? 6 : 8;
 }
-
 
 // an engine's group: same kernel instances and launch knobs
 BatchGroup group_of(const ngpu_t* h) {
@@ -2650,7 +2658,7 @@ BatchGroup group_of(const ngpu_t* h) {
   g.gen = gen_of(h);
   g.singles = g.gen == kGenPchb || g.gen == kGenPchbW;
   g.lanes = h->single_lanes;
-  g.pl = singles_pl(h->single_lanes, h->sys.nbasis / 2);
+  g.pp = singles_pp(h->single_lanes, h->sys.nbasis / 2);
   g.items = h->radix_items;
   g.core = h->ncore > 0;
   g.core_fp32 = h->core_fp32;
@@ -2659,7 +2667,7 @@ BatchGroup group_of(const ngpu_t* h) {
 }
 
 bool same_group(const BatchGroup& a, const BatchGroup& b) {
-  return a.W == b.W && a.S == b.S && a.gen == b.gen && a.lanes == b.lanes && a.pl == b.pl && a.items == b.items &&
+  return a.W == b.W && a.S == b.S && a.gen == b.gen && a.lanes == b.lanes && a.pp == b.pp && a.items == b.items &&
          a.core == b.core && a.core_fp32 == b.core_fp32 && a.rec_words == b.rec_words;
 }
 
@@ -2832,10 +2840,11 @@ void group_spawn(BatchGroup& g) {
           (const uint16_t*)g.d_map[kLkGrid]);
 }
 
-template <int W, int R, int PL, int GL>
-void group_singles(BatchGroup& g, int nsp) {
-  const size_t lds = 2 * sizeof(double) * (size_t)(kBlock / GL) * nsp;  // weights and running sums
-  glaunch(g.hs[0], 3, 3, km_spawn_singles<W, R, PL, GL>, g.tot[kLkGrid], kBlock, lds, (const EngDev*)g.d_ed,
+template <int W, int R, int PP, int GL>
+void group_singles(BatchGroup& g) {
+  size_t lds = 0;
+  for (const ngpu_t* h : g.hs) lds = std::max(lds, singles_lds(h));
+  glaunch(g.hs[0], 3, 3, km_spawn_singles<W, R, PP, GL>, g.tot[kLkGrid], kBlock, lds, (const EngDev*)g.d_ed,
           (const uint16_t*)g.d_map[kLkGrid]);
 }
 
@@ -2869,21 +2878,19 @@ void group_chain_wr(BatchGroup& g) {
   else if (g.gen == kGenPchbW) group_spawn<W, R, kGenPchbW>(g);
   else group_spawn<W, R, kGenPchb>(g);
   if (g.singles) {
-    const int nsp = h0->sys.nbasis / 2;
-    switch (g.lanes * 100 + g.pl) {
-      case 1601: group_singles<W, R, 1, 16>(g, nsp); break;
-      case 1602: group_singles<W, R, 2, 16>(g, nsp); break;
-      case 1604: group_singles<W, R, 4, 16>(g, nsp); break;
-      case 802: group_singles<W, R, 2, 8>(g, nsp); break;
-      case 803: group_singles<W, R, 3, 8>(g, nsp); break;
-      case 804: group_singles<W, R, 4, 8>(g, nsp); break;
-      case 805: group_singles<W, R, 5, 8>(g, nsp); break;
-      case 808: group_singles<W, R, 8, 8>(g, nsp); break;
-      case 404: group_singles<W, R, 4, 4>(g, nsp); break;
-      case 405: group_singles<W, R, 5, 4>(g, nsp); break;
-      case 408: group_singles<W, R, 8, 4>(g, nsp); break;
-      case 410: group_singles<W, R, 10, 4>(g, nsp); break;
-      default: group_singles<W, R, 16, 4>(g, nsp); break;
+    switch (g.lanes * 10 + g.pp) {
+      case 161: group_singles<W, R, 1, 16>(g); break;
+      case 162: group_singles<W, R, 2, 16>(g); break;
+      case 81: group_singles<W, R, 1, 8>(g); break;
+      case 82: group_singles<W, R, 2, 8>(g); break;
+      case 83: group_singles<W, R, 3, 8>(g); break;
+      case 84: group_singles<W, R, 4, 8>(g); break;
+      case 42: group_singles<W, R, 2, 4>(g); break;
+      case 43: group_singles<W, R, 3, 4>(g); break;
+      case 44: group_singles<W, R, 4, 4>(g); break;
+      case 45: group_singles<W, R, 5, 4>(g); break;
+      case 46: group_singles<W, R, 6, 4>(g); break;
+      default: group_singles<W, R, 8, 4>(g); break;
     }
   }
   if (g.core && g.shared_core)

@@ -169,7 +169,8 @@ template <int CTRL, int ROWS>
 __device__ inline double dpp_f64(double v) {
   return __longlong_as_double((long long)dpp_u64<CTRL, ROWS>((uint64_t)__double_as_longlong(v)));
 }
-constexpr int kRowShr = 0x110, kRowBcast15 = 0x142, kRowBcast31 = 0x143;
+constexpr int kRowShr = 0x110, kRowMirror = 0x140, kRowHalfMirror = 0x141, kRowBcast15 = 0x142, kRowBcast31 = 0x143,
+              kRowNewbcast = 0x150;
 // a value of one lane (wave-uniform index), to every lane
 __device__ inline uint32_t lane_value(uint32_t v, int l) { return (uint32_t)__builtin_amdgcn_readlane((int)v, l); }
 __device__ inline uint64_t lane_value(uint64_t v, int l) {
@@ -1265,201 +1266,298 @@ __global__ void __launch_bounds__(kBlock) k_spawn(DevSys s, Walk wk, Counters* c
   k_spawn_body<W, R, G>(hw_grid(), s, wk, cnt, part, att_off, tile_p, tcap, pinfo, bins, scap, sq, prm);
 }
 
-// Queued single excitations (molecular, heat-bath singles), G lanes per
-// attempt (G = 4, 8 or 16, a launch-shape choice).  gen_single_heatbath's two
-// sequential sweeps need the weight |hb_weight(src -> b)| of every same-spin
-// orbital b; lane g of a group evaluates the orbitals b = g+1, g+1+G, ...:
-// the reference-relative element fref[src][b] (one contiguous row), then the
-// (Coulomb, exchange) pairs jk[a][j][b] of the orbitals j in which the parent
-// and the reference differ (contiguous in b, so a group's loads for one j are
-// one contiguous run), added in hb_weight's order, and stores it in LDS; both
-// sweeps then run in ascending b over LDS on every lane of the group, so the
-// selected orbital, pgen and the spawn's element (the selected weight, signed)
-// are bit-identical to the one-lane generator.
-// The attempt's three Philox blocks are spread over the group's lanes and
-// shared.  More lanes per attempt shorten each attempt's chain of loads
-// (measured at 20 spatial orbitals: 1, 2 and 4 lanes took 116, 64 and 46 us
-// for 1e5 attempts); fewer lanes would repeat the sequential sweeps on fewer
-// lanes.
+// Queued single excitations (molecular, heat-bath singles).  A wave takes up to
+// 64 attempts a trip.  What an attempt needs once (queue entry, draws, source,
+// element, spawn, statistics) runs with one lane per attempt; the weights
+// |hb_weight(src -> b)| of every same-spin orbital b, ~20 times as long, with G
+// lanes per attempt (G = 4, 8 or 16, a launch-shape choice), 64/G attempts a
+// round: lane g takes every G-th pair of neighbouring orbitals b, the
+// reference-relative element fref[src][b], then the Coulomb and (of the same
+// spin) exchange rows of the orbitals j in which the parent and the reference
+// differ, 16 bytes a lane and a group's loads one contiguous run, added in
+// hb_weight's order.  The loads' lanes bound the kernel, so rows that are not
+// needed (exchange of the other spin, the second of an odd list) are masked.
+//  gen_single_heatbath's two sequential sweeps run over
+// the group's registers by DPP broadcasts, in ascending b, so the selected
+// orbital, pgen and the spawn's element (the selected weight, signed) are
+// bit-identical to the one-lane generator.  The differing orbitals wait in LDS
+// as a byte list per attempt, so a round's loop is as long as its longest list
+// of both signs.
+// Measured (a whole attempt on its G lanes, sums through LDS, interleaved
+// (Coulomb, exchange) pairs before; us): 14e/30o at 5e6 walkers 139 -> 115,
+// 26e/40o 131 -> 81, 10e/20o 32 -> 30, 2e3 attempts 13.3 -> 12.  Of the 24 at
+// 14e/30o the masks of rows not needed are 38, without them the dense lanes
+// alone had cost 14: the loads keep the address units busy 80% of the time.
+// Eight lanes per attempt take 124 and 101, sixteen 150 and 132.
 
-// Adds sign * (U(a,j,b,j) - [same spin] U(a,j,j,b)) into v for the orbitals j
-// of x (ascending, src removed), two orbitals per step so that both pairs'
-// loads are in flight before the ordered additions.
-template <int PL, int G>
-__device__ inline void hb_corr(uint64_t x, int base, const double* row, int nsp, int g, int mcount, bool plus,
-                               int src, double* v) {
-  while (x) {
-    int o1 = base + ctz64(x) + 1;
-    x &= x - 1;
-    bool two = x != 0;
-    int o2 = two ? base + ctz64(x) + 1 : o1;
-    if (two) x &= x - 1;
-    const bool s1 = ((o1 ^ src) & 1) == 0, s2 = ((o2 ^ src) & 1) == 0;
-    const double2* r1 = (const double2*)(row + (size_t)2 * (spat(o1) - 1) * nsp) + g;
-    const double2* r2 = (const double2*)(row + (size_t)2 * (spat(o2) - 1) * nsp) + g;
-    double2 a1[PL], a2[PL];
-#pragma unroll
-    for (int m = 0; m < PL; ++m) {
-      bool in = m < mcount && g + m * G < nsp;
-      a1[m] = in ? r1[m * G] : double2{0.0, 0.0};
-      a2[m] = (in && two) ? r2[m * G] : double2{0.0, 0.0};
+// a group's lanes exchange by DPP: lane I's value, and the sum over the lanes
+// of values of which at most one is not 0 (or of small counts)
+template <int G, int I>
+__device__ inline uint32_t group_lane(uint32_t v) {
+  if constexpr (G == 4) return dpp_u32<I * 0x55, 0xF>(v);
+  else if constexpr (G == 16) return dpp_u32<kRowNewbcast + I, 0xF>(v);
+  else {
+    const uint32_t lo = dpp_u32<kRowNewbcast + I, 0xF>(v), hi = dpp_u32<kRowNewbcast + 8 + I, 0xF>(v);
+    return (threadIdx.x & 8) ? hi : lo;
+  }
+}
+template <int G>
+__device__ inline uint32_t group_sum(uint32_t v) {
+  v += dpp_u32<0xB1, 0xF>(v);  // quads: lanes 1 0 3 2, then 2 3 0 1
+  v += dpp_u32<0x4E, 0xF>(v);
+  if constexpr (G >= 8) v += dpp_u32<kRowHalfMirror, 0xF>(v);
+  if constexpr (G >= 16) v += dpp_u32<kRowMirror, 0xF>(v);
+  return v;
+}
+template <int G, int I>
+__device__ inline double group_lane(double v) {
+  const uint64_t u = (uint64_t)__double_as_longlong(v);
+  const uint64_t w = ((uint64_t)group_lane<G, I>((uint32_t)(u >> 32)) << 32) | group_lane<G, I>((uint32_t)u);
+  return __longlong_as_double((long long)w);
+}
+// cum += |v[0]|, |v[1]| of the lanes I = 0..G-1 of the group in order; mine:
+// the sums after this lane's own
+template <int G, int I>
+__device__ inline void group_cum(const double* v, int g, double& cum, double* mine) {
+  if constexpr (I < G) {
+    const double c0 = cum + fabs(group_lane<G, I>(v[0]));
+    cum = c0 + fabs(group_lane<G, I>(v[1]));
+    if (g == I) {
+      mine[0] = c0;
+      mine[1] = cum;
     }
-#pragma unroll
-    for (int m = 0; m < PL; ++m) {
-      if (m < mcount && g + m * G < nsp) {
-        if (plus) {
-          v[m] += a1[m].x;
-          if (s1) v[m] -= a1[m].y;
-          if (two) {
-            v[m] += a2[m].x;
-            if (s2) v[m] -= a2[m].y;
-          }
-        } else {
-          v[m] -= a1[m].x;
-          if (s1) v[m] += a1[m].y;
-          if (two) {
-            v[m] -= a2[m].x;
-            if (s2) v[m] += a2[m].y;
-          }
-        }
-      }
-    }
+    group_cum<G, I + 1>(v, g, cum, mine);
   }
 }
 
-// PL: spatial orbitals per lane (nsp <= G*PL); dynamic LDS holds the
-// (kBlock/G)*nsp values of the block's attempts
-template <int W, int R, int PL, int G>
+// bytes of an attempt's list: orbital-1, and 0x80 for one that the parent lacks
+__host__ __device__ inline int singles_list(int nel, int nbasis) {
+  const int m = 2 * (nel < nbasis - nel ? nel : nbasis - nel);
+  return m < 8 ? 8 : (m + 7) & ~7;
+}
+
+// a wave's attempts between the two divisions of its lanes
+template <int W>
+struct SingleStage {
+  uint64_t key[W * kWave];
+  double a[kWave];       // selection uniform, then the normalisation
+  double v[kWave];       // the selected signed weight
+  double round[kWave];   // the spawn's rounding uniform
+  uint32_t meta[kWave];  // source | replica << 8 | parent bits << 16
+  uint32_t n[kWave];     // differing orbitals, then the selected b - 1
+};
+
+// PP: pairs of spatial orbitals per lane (nsp <= 2*G*PP); dynamic LDS holds the lists
+template <int W, int R, int PP, int G>
 __device__ __forceinline__ void k_spawn_singles_body(const Grid& g_, const DevSys& s, const Walk& wk, Counters* cnt, double* part, const uint8_t* pinfo, const Bins& bins, int64_t scap, const int64_t* sq, const IterParams* prm) {
   if (cnt->halt) return;
-  constexpr int kGroups = kBlock / G;
+  constexpr int kWaves = kBlock / kWave;
+  constexpr int kPer = kWave / G;  // attempts of a round
   int64_t nq = (int64_t)cnt->n_singles;
   if (nq > scap) nq = scap;
-  if (g_.b * kGroups >= nq) return;  // no queued attempts for this block
+  // rounds of a trip: as few as give every wave the same number of trips
+  const int64_t nwaves = g_.nb * kWaves;
+  const int64_t trips = (nq + nwaves * kWave - 1) / (nwaves * kWave);
+  const int rounds = nq > 0 ? (int)((nq + nwaves * trips * kPer - 1) / (nwaves * trips * kPer)) : 1;
+  const int per = rounds * kPer;
+  if (g_.b * kWaves * per >= nq) return;  // no queued attempts for this block
   const double tau = prm->tau;
   const uint32_t iter = prm->iter;
   __shared__ double acc_lds[kStatStride];
-  constexpr int kWaves = kBlock / kWave;
   __shared__ SpawnStage<W> sstages[kWaves];
+  __shared__ SingleStage<W> qstages[kWaves];
   __shared__ unsigned int blk_spawned;
+  extern __shared__ uint64_t lists_dyn[];
   if (threadIdx.x == 0) blk_spawned = 0;
-  SpawnStage<W>* ss = &sstages[threadIdx.x / kWave];
+  const int wv = threadIdx.x / kWave, lane = lane_id();
+  SpawnStage<W>* ss = &sstages[wv];
+  SingleStage<W>* st = &qstages[wv];
   int n_ss = 0;  // staged (wave-uniform)
   unsigned int spawned = 0;
-  // per group: the signed H(src -> b) of its attempt, then their running sums
-  extern __shared__ double hv_dyn[];
   BlockStats bs{acc_lds};
   bs.zero();
   const int S = R <= 2 ? R : s.S;
   SpawnAcc<R> acc;
   const int nsp = s.nbasis / 2;
-  const int mcount = (nsp + G - 1) / G;  // wave-uniform
-  const int g = threadIdx.x % G;
-  const int gl = threadIdx.x / G;        // group within the block
-  const int gbase = lane_id() - lane_id() % G;
-  const bool leader = g == 0;
-  double* myv = hv_dyn + (size_t)gl * 2 * nsp;
-  double* mycum = myv + nsp;
-  constexpr int kPer = kWave / G;  // attempts of a wave's trip
-  const int64_t nwaves = g_.nb * kWaves;
-  for (int64_t q0 = (g_.b * kWaves + threadIdx.x / kWave) * kPer; q0 < nq; q0 += nwaves * kPer) {
-    const int64_t q = q0 + lane_id() / G;
-    const bool act = q < nq;
-    int64_t p = act ? sq[2 * q] : 0;
-    uint32_t k = act ? (uint32_t)sq[2 * q + 1] : 0u;
-    int64_t slot = p / S;
-    int r = (int)(p - slot * S);
-    uint64_t key[W];
+  const int rs = (nsp + 1) & ~1;  // stride of the Coulomb and exchange rows
+  const int g = lane % G;
+  const int lw = singles_list(s.nel, s.nbasis) / 8;
+  uint64_t* lists = lists_dyn + (size_t)wv * kWave * lw;
+  for (int64_t q0 = (g_.b * kWaves + wv) * per; q0 < nq; q0 += nwaves * per) {
+    const int64_t left = nq - q0;
+    const bool act = lane < per && lane < left;
+    {
+      // idle lanes: any valid determinant, no differing orbitals
+      uint64_t key[W];
+      int64_t p = 0;
+      uint32_t k = 0;
+      if (act) {
+        p = sq[2 * (q0 + lane)];
+        k = (uint32_t)sq[2 * (q0 + lane) + 1];
+      }
+      const int64_t slot = p / S;
+      const int r = (int)(p - slot * S);
 #pragma unroll
-    for (int w = 0; w < W; ++w) key[w] = act ? wk.keys[slot * W + w] : s.ref[w];  // idle groups: any valid det
-    // lane g < 3 draws Philox block g+1, all three in one pass of the wave;
-    // d1 = dsel (purpose 1), d5 = spawn rounding (purpose 2, second value),
-    // d2 = dorb (purpose 3, first)
-    static_assert(G >= 3, "three lanes of a group draw the attempt's Philox blocks");
-    double ua = 0.0, ub = 0.0;
-    if (g < 3) draw2<W>(s.seed, key, iter, r, k, (uint32_t)(g + 1), ua, ub);
-    const double d1 = __shfl(ub, gbase + 0);
-    const double d5 = __shfl(ub, gbase + 1);
-    const double d2 = __shfl(ua, gbase + 2);
-    int elec = 1 + (int)floor(d1 * (double)s.nel);
-    int src = select_orb<W>(key, ~0ull, elec);
-    int a = spat(src), off = is_beta(src) ? 1 : 0;
-    const double* row = s.jk + (size_t)2 * (a - 1) * nsp * nsp;
-    const double* frow = s.fref + (size_t)(src - 1) * nsp;
-    double v[PL];
+      for (int w = 0; w < W; ++w) key[w] = act ? wk.keys[slot * W + w] : s.ref[w];
+      const uint32_t pi = act ? pinfo[p] : 0u;
+      double d0, d1, d2, d3, d4, d5;
+      draw2<W>(s.seed, key, iter, r, k, 1, d0, d1);
+      draw2<W>(s.seed, key, iter, r, k, 2, d3, d5);
+      draw2<W>(s.seed, key, iter, r, k, 3, d2, d4);
+      const int src = select_orb<W>(key, ~0ull, 1 + (int)floor(d1 * (double)s.nel));
 #pragma unroll
-    for (int m = 0; m < PL; ++m) v[m] = (m < mcount && g + m * G < nsp) ? frow[g + m * G] : 0.0;
-    // the orbitals the parent occupies beyond the reference, then the
-    // reference's orbitals the parent lacks (hb_weight's order)
+      for (int w = 0; w < W; ++w) st->key[w * kWave + lane] = key[w];
+      st->a[lane] = d2;
+      st->round[lane] = d5;
+      st->meta[lane] = (uint32_t)src | ((uint32_t)r << 8) | (pi << 16);
+      // the orbitals the parent occupies beyond the reference, then the
+      // reference's orbitals the parent lacks (hb_weight's order)
+      uint8_t* list = (uint8_t*)(lists + (size_t)lane * lw);
+      uint32_t n = 0;
 #pragma unroll
-    for (int w = 0; w < W; ++w) {
-      uint64_t x = key[w] & ~s.ref[w];
-      if ((src - 1) >> 6 == w) x &= ~(1ull << ((src - 1) & 63));
-      hb_corr<PL, G>(x, 64 * w, row, nsp, g, mcount, true, src, v);
+      for (int w = 0; w < 2 * W; ++w) {
+        const int ww = w % W;
+        uint64_t x = w < W ? key[ww] & ~s.ref[ww] : s.ref[ww] & ~key[ww];
+        if ((src - 1) >> 6 == ww) x &= ~(1ull << ((src - 1) & 63));
+        while (x) {
+          list[n++] = (uint8_t)((64 * ww + ctz64(x)) | (w < W ? 0 : 0x80));
+          x &= x - 1;
+        }
+      }
+      st->n[lane] = n;
     }
+    wave_sync();
+    const int live = left < per ? (int)left : per;
+    for (int t0 = 0; t0 < live; t0 += kPer) {
+      const int j = t0 + lane / G;
+      const int src = (int)(st->meta[j] & 0xFF), n = (int)st->n[j];
+      const uint32_t spin = (uint32_t)(src - 1) & 1u;
+      const double* frow = s.fref + (size_t)(src - 1) * nsp;
+      const double* row = s.jkrow + (size_t)2 * rs * nsp * ((src - 1) >> 1) + 2 * g;
+      double v[2 * PP];
 #pragma unroll
-    for (int w = 0; w < W; ++w) {
-      uint64_t x = s.ref[w] & ~key[w];
-      if ((src - 1) >> 6 == w) x &= ~(1ull << ((src - 1) & 63));
-      hb_corr<PL, G>(x, 64 * w, row, nsp, g, mcount, false, src, v);
-    }
+      for (int m = 0; m < 2 * PP; ++m) {
+        const int b = 2 * (g + m / 2 * G) + m % 2;
+        v[m] = b < nsp ? frow[b] : 0.0;
+      }
+      // two orbitals per step so that both rows' loads are in flight before
+      // the ordered additions.  (Loads past a row's end stay in the table,
+      // which is padded, and their values are dropped below.)
+      const uint64_t* list = lists + (size_t)j * lw;
+      uint64_t chunk = 0;
+      for (int i = 0; i < n; i += 2) {
+        if ((i & 7) == 0) chunk = list[i >> 3];
+        const uint32_t e1 = (uint32_t)chunk & 0xFF, e2 = (uint32_t)(chunk >> 8) & 0xFF;
+        chunk >>= 16;
+        const bool two = i + 1 < n;
+        const bool x1 = (e1 & 1u) == spin, x2 = two && (e2 & 1u) == spin;
+        const double* r1 = row + (size_t)(2 * rs) * ((e1 & 0x7F) >> 1);
+        const double* r2 = row + (size_t)(2 * rs) * ((e2 & 0x7F) >> 1);
+        double2 j1[PP], k1[PP], j2[PP], k2[PP];
 #pragma unroll
-    for (int m = 0; m < PL; ++m) {
-      int b = g + m * G + 1;
-      if (m < mcount && b <= nsp) {
-        int orb = 2 * b - off;
-        myv[b - 1] = test_orb<W>(key, orb) ? 0.0 : v[m];
+        for (int m = 0; m < PP; ++m) j1[m] = *(const double2*)(r1 + 2 * G * m);
+        if (x1) {
+#pragma unroll
+          for (int m = 0; m < PP; ++m) k1[m] = *(const double2*)(r1 + rs + 2 * G * m);
+        }
+        if (two) {
+#pragma unroll
+          for (int m = 0; m < PP; ++m) j2[m] = *(const double2*)(r2 + 2 * G * m);
+        }
+        if (x2) {
+#pragma unroll
+          for (int m = 0; m < PP; ++m) k2[m] = *(const double2*)(r2 + rs + 2 * G * m);
+        }
+        // +-1: the products are exact, so these are the plain sums
+        const double s1 = (e1 & 0x80) ? -1.0 : 1.0, s2 = (e2 & 0x80) ? -1.0 : 1.0;
+        auto add = [&](double f, const double2* a) {
+#pragma unroll
+          for (int m = 0; m < PP; ++m) {
+            v[2 * m] = fma(f, a[m].x, v[2 * m]);
+            v[2 * m + 1] = fma(f, a[m].y, v[2 * m + 1]);
+          }
+        };
+        add(s1, j1);
+        if (x1) add(-s1, k1);
+        if (two) add(s2, j2);
+        if (x2) add(-s2, k2);
+      }
+      // occupied targets and the lanes' orbitals past the last have no weight
+      {
+        uint64_t key[W];
+#pragma unroll
+        for (int w = 0; w < W; ++w) key[w] = st->key[w * kWave + j];
+#pragma unroll
+        for (int m = 0; m < 2 * PP; ++m) {
+          // orbital-1 = 4G (m/2) + the rest, which is below 4G, and that divides 64
+          const int o = 4 * G * (m / 2), rest = 4 * g + 2 * (m % 2) + (int)spin;
+          const bool occ = o / 64 < W && (key[o / 64 < W ? o / 64 : 0] >> (o % 64 + rest)) & 1;
+          if (2 * (g + m / 2 * G) + m % 2 >= nsp || occ) v[m] = 0.0;
+        }
+      }
+      // the normalisation in ascending b, then the first b whose running sum
+      // reaches r (the last b when none does): the running sums of a second
+      // sweep in the same order are the same values, and they do not fall, so
+      // that b is the number of sums below r
+      double cum = 0.0, own[2 * PP];
+#pragma unroll
+      for (int m = 0; m < 2 * PP; m += 2) {
+        own[m] = own[m + 1] = 0.0;
+        group_cum<G, 0>(v + m, g, cum, own + m);
+      }
+      const double rr = st->a[j] * cum;
+      uint32_t below = 0;
+#pragma unroll
+      for (int m = 0; m < 2 * PP; ++m)
+        below += (2 * (g + m / 2 * G) + m % 2 < nsp && own[m] < rr) ? 1u : 0u;
+      below = group_sum<G>(below);
+      if (below > (uint32_t)(nsp - 1)) below = (uint32_t)(nsp - 1);
+      uint64_t sel = 0;
+#pragma unroll
+      for (int m = 0; m < 2 * PP; ++m)
+        sel = (uint32_t)(2 * (g + m / 2 * G) + m % 2) == below ? (uint64_t)__double_as_longlong(v[m]) : sel;
+      sel = ((uint64_t)group_sum<G>((uint32_t)(sel >> 32)) << 32) | group_sum<G>((uint32_t)sel);
+      if (g == 0) {
+        st->a[j] = cum;
+        st->v[j] = __longlong_as_double((long long)sel);
+        st->n[j] = below;
       }
     }
     wave_sync();
-    // the normalisation, keeping the running sums (every lane of the group
-    // writes the same values, and reads its own writes below); then the
-    // first b whose running sum reaches r, by bisection over those sums:
-    // the running sums of a second sweep in the same order are the same
-    // values, so this is its selection (the last b when none reaches r)
-    double cum_sum = 0.0;
-    for (int b = 0; b < nsp; ++b) {
-      cum_sum += fabs(myv[b]);
-      mycum[b] = cum_sum;
-    }
-    double rr = d2 * cum_sum;
-    int lo = 0, hi = nsp - 1;
-    while (lo < hi) {
-      const int mid = (lo + hi) >> 1;
-      if (!(mycum[mid] < rr)) hi = mid;
-      else lo = mid + 1;
-    }
-    const int bsel = lo + 1;
-    const double vsel = myv[lo];
-    const double cpt = fabs(vsel);
-    bool mine_att = act && leader;
     bool emit = false;
-    uint64_t child[W];
+    uint64_t key[W], child[W];
     double nspawn = 0.0, an = 0.0, raw = 0.0, valid = 0.0, invalid = 0.0;
     uint32_t info = 0;
-    bool cancel = false;
-    if (mine_att && s.ncore && (pinfo[p] & 4) && !(fabs(cum_sum) <= kEps || cpt == 0.0)) {
-      Excit ex{};
-      ex.ic = 1;
-      ex.e0 = src;
-      ex.e1 = 2 * bsel - off;
-      cancel = core_child<W>(s, wk, cnt, key, ex);  // from and to the core space
-    }
-    if (mine_att) {
-      if (fabs(cum_sum) <= kEps || cpt == 0.0) {
+    int r = 0;
+    if (act) {
+#pragma unroll
+      for (int w = 0; w < W; ++w) key[w] = st->key[w * kWave + lane];
+      const uint32_t meta = st->meta[lane], pi = meta >> 16;
+      const int src = (int)(meta & 0xFF);
+      const int tgt = 2 * (int)st->n[lane] + 2 - (is_beta(src) ? 1 : 0);
+      const double cum_sum = st->a[lane], vsel = st->v[lane], cpt = fabs(vsel);
+      r = (int)((meta >> 8) & 0xFF);
+      const bool none = fabs(cum_sum) <= kEps || cpt == 0.0;
+      bool cancel = false;
+      if (!none && s.ncore && (pi & 4)) {
+        Excit ex{};
+        ex.ic = 1;
+        ex.e0 = src;
+        ex.e1 = tgt;
+        cancel = core_child<W>(s, wk, cnt, key, ex);  // from and to the core space
+      }
+      if (none) {
         invalid = 1.0;
       } else if (cancel) {
         valid = 1.0;
       } else {
         valid = 1.0;
-        int tgt = 2 * bsel - off;
         double pg = cpt / cum_sum;
         pg = pg / (double)s.nel;
         pg = pg * s.psingles;
         double hel = single_parity<W>(key, src, tgt) ? -vsel : vsel;  // the weight's own sum
-        uint8_t pi = pinfo[p];
         double wsign = (pi & 1) ? -1.0 : 1.0;
-        nspawn = attempt_create(s, tau, hel, pg, wsign, d5, raw);
+        nspawn = attempt_create(s, tau, hel, pg, wsign, st->round[lane], raw);
         raw = fabs(raw);
         if (fabs(nspawn) > kEps) {
           emit = true;
@@ -1496,18 +1594,18 @@ __device__ __forceinline__ void k_spawn_singles_body(const Grid& g_, const DevSy
       spawn_flush<W>(ss, n_ss, cnt, bins, s);
       n_ss = 0;
     }
-    wave_sync();  // the next attempts reuse the weights' LDS
+    wave_sync();  // the next attempts reuse the LDS
   }
   if (n_ss) spawn_flush<W>(ss, n_ss, cnt, bins, s);
-  if (spawned && lane_id() == 0) atomicAdd(&blk_spawned, spawned);
+  if (spawned && lane == 0) atomicAdd(&blk_spawned, spawned);
   __syncthreads();
   if (threadIdx.x == 0 && blk_spawned) atomicAdd(&cnt->n_spawned, (unsigned long long)blk_spawned);
   acc.done(bs, 2);
   bs.flush(part, g_.b);
 }
-template <int W, int R, int PL, int G>
-__global__ void __launch_bounds__(kBlock) k_spawn_singles(DevSys s, Walk wk, Counters* cnt, double* part, const uint8_t* pinfo, Bins bins, int64_t scap, const int64_t* sq, const IterParams* prm) {
-  k_spawn_singles_body<W, R, PL, G>(hw_grid(), s, wk, cnt, part, pinfo, bins, scap, sq, prm);
+template <int W, int R, int PP, int G>
+__global__ void __launch_bounds__(kBlock, PP <= 3 ? 4 : PP <= 5 ? 3 : 2) k_spawn_singles(DevSys s, Walk wk, Counters* cnt, double* part, const uint8_t* pinfo, Bins bins, int64_t scap, const int64_t* sq, const IterParams* prm) {
+  k_spawn_singles_body<W, R, PP, G>(hw_grid(), s, wk, cnt, part, pinfo, bins, scap, sq, prm);
 }
 
 // ---------------------------------------------------------- radix sort
