@@ -797,6 +797,30 @@ struct DrawSeq {
     }
     return (j & 1) ? c1 : c0;
   }
+  // The next uniforms without taking them: at most four, those of d1..d4 that
+  // are left or what two blocks hold; returns how many.
+  __device__ __host__ int peek(double* v) const {
+    if (n < 4) {
+      v[0] = n == 0 ? d1 : n == 1 ? d2 : n == 2 ? d3 : d4;
+      v[1] = n == 0 ? d2 : n == 1 ? d3 : d4;
+      v[2] = n == 0 ? d3 : d4;
+      v[3] = d4;
+      return 4 - n;
+    }
+    const int j = n - 4;
+    const uint64_t dh = det_hash64<W>(key);
+    const U4 c{(uint32_t)dh, (uint32_t)(dh >> 32), iter, (k << 3) | 6u};
+    const uint32_t b = (uint32_t)(j >> 1) + 1;
+    const U4 o = philox4x32_10(c, seed, (uint32_t)rep | (b << 8));
+    const U4 q = philox4x32_10(c, seed, (uint32_t)rep | ((b + 1) << 8));
+    const bool odd = j & 1;
+    const double x0 = u01(o.x, o.y), x1 = u01(o.z, o.w), x2 = u01(q.x, q.y), x3 = u01(q.z, q.w);
+    v[0] = odd ? x1 : x0;
+    v[1] = odd ? x2 : x1;
+    v[2] = odd ? x3 : x2;
+    v[3] = x3;
+    return odd ? 3 : 4;
+  }
 };
 
 // ------------------------------------------ weighted PCHB particles and holes
@@ -856,12 +880,31 @@ __device__ __host__ inline int constrained_draw(const AliasEnt* tab, const doubl
       }
     return 0;
   }
-  for (int t = 0; t < kMaxRedraw; ++t) {
-    double pa;
-    const int tgt = alias_sample(tab, n, u.next(), pa) + 1;
-    if (!test_orb<W>(set, tgt)) continue;
-    p = prob[tgt - 1] / renorm;
-    return p == 0.0 ? 0 : tgt;
+  // Up to four draws a step, their table entries in flight together; the draws
+  // up to the first hit are taken.  A wave loops as long as its unluckiest
+  // lane, and a step is a Philox block (0.3 us) and a gather each.
+  for (int t = 0; t < kMaxRedraw;) {
+    double r[4];
+    int m = u.peek(r), hit = 0;
+    if (m > kMaxRedraw - t) m = kMaxRedraw - t;
+    int tgt[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      double pa;
+      tgt[q] = alias_sample(tab, n, r[q], pa) + 1;
+    }
+    int used = m;
+#pragma unroll
+    for (int q = 3; q >= 0; --q)
+      if (q < m && test_orb<W>(set, tgt[q])) {
+        hit = tgt[q];
+        used = q + 1;
+      }
+    u.n += used;
+    t += used;
+    if (!hit) continue;
+    p = prob[hit - 1] / renorm;
+    return p == 0.0 ? 0 : hit;
   }
   return 0;
 }

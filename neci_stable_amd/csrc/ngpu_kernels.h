@@ -1153,6 +1153,12 @@ __device__ inline void spawn_attempt(const DevSys& s, const Walk& wk, Counters* 
   n_ss += popc64(em);
 }
 
+// generators whose attempts loop over draws: at 2e4 attempts of the weighted
+// one (8e/16o) a wave of 16 attempts and the draws by four take 41 us of 52;
+// eight attempts a wave take 45 with eight values of a sum in flight
+template <int G>
+constexpr bool kSplitTiles = G == kGenUniform || G == kGenPchbW;
+
 // all attempts: Hubbard spawns directly; molecular doubles spawn here while
 // singles (the heat-bath list is ~20x longer per attempt) go to a queue so that
 // waves do not idle on a few long lanes
@@ -1160,10 +1166,14 @@ template <int W, int R, int G>
 __device__ __forceinline__ void k_spawn_body(const Grid& g_, const DevSys& s, const Walk& wk, Counters* cnt, double* part, const int64_t* att_off, const int64_t* tile_p, int64_t tcap, const uint8_t* pinfo, const Bins& bins, int64_t scap, int64_t* sq, const IterParams* prm) {
   if (cnt->halt) return;
   const int64_t total = (int64_t)cnt->n_attempts;
-  if (g_.b * kBlock >= total) return;  // no attempts for this block
+  constexpr int kWaves = kBlock / kWave;
+  // waves per tile of 64 attempts: with few attempts a wave takes a part of a
+  // tile, as long loops run to the longest of its lanes
+  const int64_t twaves = g_.nb * kWaves, tiles = (total + kWave - 1) / kWave;
+  const int sub = !kSplitTiles<G> ? 1 : 4 * tiles <= twaves ? 4 : 2 * tiles <= twaves ? 2 : 1;
+  if (g_.b * kWaves >= tiles * sub) return;  // no attempts for this block
   const double tau = prm->tau;
   const uint32_t iter = prm->iter;
-  constexpr int kWaves = kBlock / kWave;
   constexpr int mode = (G == kGenPchb || G == kGenPchbW) ? 1 : 0;
   __shared__ double acc_lds[kStatStride];
   __shared__ SpawnStage<W> sstages[kWaves];
@@ -1184,12 +1194,12 @@ __device__ __forceinline__ void k_spawn_body(const Grid& g_, const DevSys& s, co
   const int64_t npairs = (int64_t)cnt->nslots * s.S;
   bool overflow = false;
   SpawnAcc<R> acc;
-  // tiles of 64 consecutive attempts, one per wave and trip
-  const int64_t stride = g_.nb * kBlock;
-  for (int64_t a0 = g_.b * kBlock + wv * kWave; a0 < total; a0 += stride) {
-    const int64_t a = a0 + lane, tile = a0 / kWave;
+  // tiles of 64 consecutive attempts, one (or a part of one) per wave and trip
+  for (int64_t t0 = g_.b * kWaves + wv; t0 < tiles * sub; t0 += twaves) {
+    const int64_t tile = sub == 1 ? t0 : t0 / sub, a0 = tile * kWave, a = a0 + lane;
     // the tile's parents lie between its first attempt's and the next tile's
-    const bool more = a0 + kWave < total, act = a < total;
+    const bool more = a0 + kWave < total;
+    const bool act = a < total && (sub == 1 || (lane * sub) / kWave == (int)(t0 - tile * sub));
     int64_t lo, hi;
     if (tile + 1 < tcap) {
       lo = tile_p[tile];
