@@ -40,11 +40,13 @@ HBM_PEAK_GBS = 8000.0
 
 
 def sort_key(nbasis, nel):
-    """(bytes per key, 8-bit passes through global memory) of the spawn sort:
-    for the 32-bit colex-rank key (C(nbasis, nel) fits 32 bits and its
-    binomial table the engine's LDS copy) the top-byte pass and the segment
-    sort's read and write, counted as two passes; else the determinant words,
-    one LSD pass per 8 bits."""
+    """(bytes per key, 8-bit passes through global memory) of a sort of the
+    spawned list, the algorithmic reference of compressing it (the engine's
+    bins take its place, and its sort stage is empty): for the 32-bit
+    colex-rank key (C(nbasis, nel) fits 32 bits and its binomial table the
+    engine's LDS copy) a top-byte pass and a segment sort's read and write,
+    counted as two passes; else the determinant words, one LSD pass per 8
+    bits."""
     import math
     if nel is not None and math.comb(nbasis, nel) <= 2 ** 32 and nbasis * (nel + 1) <= 512:
         return 4, 2

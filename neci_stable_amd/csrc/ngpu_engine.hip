@@ -661,9 +661,9 @@ void by_shape(const ngpu_t* h, F f) { by_shape(h->W, h->S, f); }
 // singles): as many as the chip holds at once, times grid_blocks over its
 // default of four per compute unit.  Their waves split the attempts evenly, so
 // a block too many is a second round of a few blocks, and one too few an idle
-// slot: at 14e/30o and 5e6 walkers, singles at three per compute unit (160
-// VGPRs) 135 us against 174 at four, k_spawn at five (91 VGPRs) 169 against
-// 177 at four and 204 at six.
+// slot: at 14e/30o and 5e6 walkers k_spawn at five per compute unit (91 VGPRs)
+// took 165 us against 182 at four and 195 at six, the singles at three (161
+// VGPRs) 116 us against 143 at two and 124 at four.
 template <typename F>
 int spawn_blocks(ngpu_t* h, int which, F kern, size_t lds) {
   if (h->occ_kern[which] != (const void*)kern || h->occ_lds[which] != lds) {
