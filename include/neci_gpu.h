@@ -310,7 +310,7 @@ int ngpu_batch_iterate(ngpu_batch_t *b, const ngpu_iter_in_t *ins);
 int ngpu_batch_destroy(ngpu_batch_t *b);
 /* The batch's launch groups: engines whose iteration chains use the same
    kernel instances (determinant words, replica layout, excitation generator,
-   sort path, spawn-record and core precision, launch knobs).  Every kernel of
+   spawn-record and core precision, launch knobs).  Every kernel of
    the chain is ONE launch for all the engines of a group, each engine taking
    a share of its blocks in proportion to its walker capacity; the groups run
    concurrently, each on its own stream.  group_of_engine[i] receives engine

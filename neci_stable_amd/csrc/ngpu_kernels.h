@@ -7,7 +7,7 @@
 //                it frees; clears the walker hash when a rebuild is due
 //   k_scan_apply exclusive scan of attempt counts -> attempt offsets; the
 //                freed slots into the free queue; the hash refill of a rebuild
-//   k_spawn      per attempt: parent by binary search, excitation, H_ij,
+//   k_spawn      per attempt: parent from the scan's tile marks, excitation, H_ij,
 //                stochastic rounding, spawn records staged in LDS and written
 //                into the bins of their determinants' hashes; heat-bath
 //                singles are queued for k_spawn_singles
@@ -15,6 +15,8 @@
 //                LDS, then hash lookup, add/abort/remove
 //   k_insert     new dets: slot from the free queue, bucketed open-addressing insert
 //   k_stats      per slot: occupied-threshold rounding, TotParts, norm, HF pop
+//                (only with real coefficients or a core; whole-number runs sum
+//                them in the prepass and the merge)
 //   (k_end_iter in the engine: slot and hash bookkeeping, statistics sums)
 #pragma once
 #include "ngpu_device.h"
