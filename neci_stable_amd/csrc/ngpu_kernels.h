@@ -483,7 +483,8 @@ __device__ inline uint32_t bin_of(uint32_t h, uint32_t nb) { return (uint32_t)((
 
 // where the record with place pos of bin b goes
 // (null: the overflow list is full, which takes more records than the spawn
-// capacity; the iteration's end reports those)
+// capacity; the merge takes nothing from such a list and the iteration's end
+// reports it)
 __device__ inline uint64_t* bin_record(Counters* cnt, const Bins& bins, uint32_t b, uint32_t pos, uint32_t cap,
                                        int rec_words) {
   if (pos < cap) return bins.rec + ((size_t)b * cap + pos) * rec_words;
@@ -1946,6 +1947,17 @@ __device__ __forceinline__ void k_merge_body(const Grid& g_, const DevSys& s, co
   constexpr int kWaves = kBlock / kWave;
   const uint32_t nb = cnt->nbins, cap = cnt->bin_cap, sh = cnt->bin_shift;
   if (cnt->halt || g_.b * kWaves >= (int64_t)nb) return;
+  // checkValidSpawnedList (fcimc_helper.F90:483-510) stops between spawning
+  // and annihilation when the list is past its capacity: no record is merged,
+  // the iteration's end reports it.  The bins, spill areas and overflow list
+  // together hold 2.75 times the capacity, the new list max(capacity,
+  // MaxWalkers) rows; past this line the new determinants are no more than
+  // the capacity, so that no append needs a bound of its own.
+  if (!LIST && cnt->n_spawned > (unsigned long long)bins.ovf_cap) {
+    for (int64_t b = g_.b * blockDim.x + threadIdx.x; b < (int64_t)nb; b += g_.nb * blockDim.x)
+      bins.count[(size_t)b << sh] = 0;
+    return;
+  }
   constexpr int T = MergeTab<W, R>::kSize;
   constexpr int kCap = WaveStage<W, R>::kCap;
   __shared__ MergeTab<W, R> tabs[kWaves];
