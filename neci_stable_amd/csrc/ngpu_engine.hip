@@ -359,6 +359,7 @@ __global__ void k_begin_iter(ngpu_iter_out_t* out, double* part, Counters* cnt, 
     cnt->n_fail = 0;
     cnt->ins_refused = 0;
     cnt->err = 0;
+    cnt->prev_spawned = cnt->prev_attempts = 0;  // other walkers: their spawning rate is not known
     out->tot_walkers = 0;
     out->n_attempts = out->n_spawned = out->n_unique = out->n_new = 0;
     out->err = 0;

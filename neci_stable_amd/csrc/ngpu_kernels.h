@@ -87,8 +87,9 @@ struct alignas(256) Counters {
   unsigned int nbins;
   unsigned int bin_cap;
   unsigned int bin_shift;
-  // spawned records and attempts of the previous iteration: the expected
-  // number of records sizes the bins (speed only, results do not depend on it)
+  // spawned records and attempts of the previous iteration (no attempts after
+  // an upload or an explicit list): the expected number of records sizes the
+  // bins (speed only, results do not depend on it)
   unsigned long long prev_spawned, prev_attempts;
   alignas(256) unsigned long long free_tail;
   alignas(256) unsigned long long n_spawned;
@@ -456,6 +457,12 @@ struct Bins {
 };
 // records per bin aimed at: a wave merges up to 64 in one pass over its lanes
 constexpr int kBinFill = 44;
+// The least number of spawns expected is attempts / kMinRate.  A bin's merge
+// takes (its determinants / 128) rounds over its records, so without a bound
+// on a bin's records one iteration's time grows with the square of the list;
+// with this one a bin holds kBinFill * kMinRate records at most when every
+// attempt spawns, 22 rounds.  Empty bins cost a 64th of a load each.
+constexpr int kMinRate = 64;
 
 __device__ inline void set_bins(Counters* cnt, const Bins& b, double expect) {
   double nb = expect * (1.0 / kBinFill) + 1.0;
@@ -870,9 +877,11 @@ __device__ __forceinline__ void k_scan_apply_body(const Grid& g_, const DevSys& 
     cnt->n_attempts = (unsigned long long)run;
     cnt->free_tail = tail0 + (unsigned long long)run_rm;
     cnt->rm_pre = (unsigned long long)run_rm;
-    // spawns expected at the previous iteration's rate per attempt
-    set_bins(cnt, bins, cnt->prev_attempts ? (double)run * ((double)cnt->prev_spawned / (double)cnt->prev_attempts)
-                                           : 0.5 * (double)run);
+    // spawns expected at the previous iteration's rate per attempt, and no
+    // fewer than one in kMinRate attempts: a larger time step, another shift or
+    // an iteration that happened to spawn nothing says little about this one
+    const double per = cnt->prev_attempts ? (double)cnt->prev_spawned / (double)cnt->prev_attempts : 0.5;
+    set_bins(cnt, bins, (double)run * (per > 1.0 / kMinRate ? per : 1.0 / kMinRate));
   }
 }
 template <int W>
