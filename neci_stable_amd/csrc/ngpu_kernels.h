@@ -1955,6 +1955,7 @@ template <int W, int R, bool LIST>
 __device__ __forceinline__ void k_merge_body(const Grid& g_, const DevSys& s, const Walk& wk, Counters* cnt, double* part, const Bins& bins, uint64_t* n_key, double* n_sgn, uint32_t* n_flag, unsigned long long* n_ctr, const IterParams* prm, bool by_parts) {
   constexpr int kWaves = kBlock / kWave;
   const uint32_t nb = cnt->nbins, cap = cnt->bin_cap, sh = cnt->bin_shift;
+  const unsigned long long spawned = LIST ? 0ull : cnt->n_spawned;  // in the same round trip
   if (cnt->halt || g_.b * kWaves >= (int64_t)nb) return;
   // checkValidSpawnedList (fcimc_helper.F90:483-510) stops between spawning
   // and annihilation when the list is past its capacity: no record is merged,
@@ -1962,7 +1963,7 @@ __device__ __forceinline__ void k_merge_body(const Grid& g_, const DevSys& s, co
   // together hold 2.75 times the capacity, the new list max(capacity,
   // MaxWalkers) rows; past this line the new determinants are no more than
   // the capacity, so that no append needs a bound of its own.
-  if (!LIST && cnt->n_spawned > (unsigned long long)bins.ovf_cap) {
+  if (spawned > (unsigned long long)bins.ovf_cap) {
     for (int64_t b = g_.b * blockDim.x + threadIdx.x; b < (int64_t)nb; b += g_.nb * blockDim.x)
       bins.count[(size_t)b << sh] = 0;
     return;
