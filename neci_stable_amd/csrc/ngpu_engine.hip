@@ -373,7 +373,8 @@ constexpr int kEndThreads = 512;  // one pass over one replica's statistics
 // accumulators in the reference too)
 __device__ __forceinline__ void end_iter_body(ngpu_iter_out_t* out, double* part, ngpu_iter_out_t* cyc, Counters* cnt,
                                               int64_t scap, int64_t cap, int64_t hash_entries, const IterParams* prm,
-                                              uint32_t* scount, int S) {
+                                              uint32_t* scount, int S, const NewList& nl) {
+  const bool refused = nl.W && cnt->n_fail != 0;  // in the same round trip as halt
   // halted: the output block keeps the failing iteration's statistics and
   // error, and nothing is added to the cycle
   if (cnt->halt) return;
@@ -400,6 +401,7 @@ __device__ __forceinline__ void end_iter_body(ngpu_iter_out_t* out, double* part
       n_unique = (unsigned long long)u;
     }
   }
+  if (refused) uncount_refused(nl, cnt, part, S);
   double* g = (double*)out;
   double* c = (double*)cyc;
   // the statistics rows: kEndParts threads per field take kStatCopies /
@@ -478,14 +480,15 @@ __device__ __forceinline__ void end_iter_body(ngpu_iter_out_t* out, double* part
 }
 __global__ void __launch_bounds__(kEndThreads) k_end_iter(ngpu_iter_out_t* out, double* part, ngpu_iter_out_t* cyc, Counters* cnt,
                            int64_t scap, int64_t cap, int64_t hash_entries, const IterParams* prm,
-                           uint32_t* scount, int S) {
-  end_iter_body(out, part, cyc, cnt, scap, cap, hash_entries, prm, scount, S);
+                           uint32_t* scount, int S, NewList nl) {
+  end_iter_body(out, part, cyc, cnt, scap, cap, hash_entries, prm, scount, S, nl);
 }
 // the end of the iteration of every engine of a batch group: one block each
-__global__ void __launch_bounds__(kEndThreads) km_end_iter(const EngDev* __restrict__ ed) {
+__global__ void __launch_bounds__(kEndThreads) km_end_iter(const EngDev* __restrict__ ed, int W) {
   const EngDev& a = ed[blockIdx.x];
+  const NewList nl{a.n_key, a.n_sgn, a.n_flag, a.s.ref[0], a.s.ref[1], stats_by_parts(a.s) ? W : 0};
   end_iter_body(a.dout, a.part, a.dcyc, a.cnt, a.scap, a.wk.cap, a.wk.L * (int64_t)kBucketEntries, a.prm,
-                a.bins.scount, a.s.S);
+                a.bins.scount, a.s.S, nl);
 }
 
 // the last iteration's statistics, the cycle's sums and the sticky error to
@@ -619,7 +622,7 @@ void insert_new(ngpu_t* h, int stage) {
   const int G = insert_lanes(h);
   auto kern = G == 1 ? k_insert<W, R, 1> : G == 16 ? k_insert<W, R, 16> : k_insert<W, R, 64>;
   launch_lds(h, stage, stage, kern, dim3(h->nb_grid), dim3(kBlock), insert_lds(h, G), h->ds, h->wk, h->cnt,
-             (const uint64_t*)h->n_key, (const double*)h->n_sgn, (const uint32_t*)h->n_flag,
+             (const uint64_t*)h->n_key, (const double*)h->n_sgn, h->n_flag,
              (const unsigned long long*)&h->cnt->n_new);
 }
 
@@ -638,7 +641,8 @@ void annihilation_chain(ngpu_t* h, bool with_core, bool list_out = false) {
   if (!by_parts) launch(h, 8, 8, k_stats<W, R>, dim3(h->nb_grid), dim3(kBlock), h->ds, h->wk, h->cnt, h->dpart,
          (const IterParams*)h->dparams);
   launch(h, -1, -1, k_end_iter, dim3(1), dim3(kEndThreads), h->dout, h->dpart, h->dcyc, h->cnt,
-         h->scap, h->wk.cap, h->wk.L * (int64_t)kBucketEntries, (const IterParams*)h->dparams, h->bins.scount, h->S);
+         h->scap, h->wk.cap, h->wk.L * (int64_t)kBucketEntries, (const IterParams*)h->dparams, h->bins.scount, h->S,
+         NewList{h->n_key, h->n_sgn, h->n_flag, h->ds.ref[0], h->ds.ref[1], by_parts ? W : 0});
   if (h->checks) check_chain<W>(h, with_core);
 }
 
@@ -2906,7 +2910,7 @@ void group_chain_wr(BatchGroup& g) {
   bool pass = false;  // an engine whose statistics take a pass over its table
   for (const ngpu_t* h : g.hs) pass = pass || !stats_by_parts(h->ds);
   if (pass) glaunch(h0, 8, 8, km_stats<W, R>, g.tot[kLkGrid], kBlock, 0, ed, (const uint16_t*)m[kLkGrid]);
-  glaunch(h0, -1, -1, km_end_iter, (int)g.hs.size(), kEndThreads, 0, ed);
+  glaunch(h0, -1, -1, km_end_iter, (int)g.hs.size(), kEndThreads, 0, ed, W);
 }
 
 void group_chain(BatchGroup& g) {

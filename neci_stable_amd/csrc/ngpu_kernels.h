@@ -572,6 +572,33 @@ __device__ inline int64_t grid_elem(const Grid& g, int64_t t) {
 // what it changes, exactly (sums of integers), so k_stats is not launched:
 // 6 us of an iteration over 3e3 determinants, 25 us over 2.9e6.
 __host__ __device__ inline bool stats_by_parts(const DevSys& s) { return !s.t_real && s.ncore == 0; }
+// The merge counts a new determinant before k_insert has placed it: what the
+// insertion refused (the iteration ends in an error) is taken out again by the
+// iteration's end, so that the statistics are those of the kept walker list.
+// The new list as the end of an iteration sees it; W = 0: not by parts
+struct NewList {
+  const uint64_t* key;
+  const double* sgn;
+  const uint32_t* flag;
+  uint64_t ref0, ref1;
+  int W;
+};
+__device__ inline void uncount_refused(const NewList& nl, const Counters* cnt, double* part, int S) {
+  const int64_t nn = (int64_t)cnt->n_new;
+  const bool all = cnt->ins_refused != 0;
+  for (int64_t i = threadIdx.x; i < nn; i += blockDim.x) {
+    if (!all && !(nl.flag[i] & kFlagRemoved)) continue;
+    const bool isref = nl.key[i * nl.W] == nl.ref0 && (nl.W == 1 || nl.key[i * nl.W + 1] == nl.ref1);
+    atomicAdd(&part[X_NOCC], -1.0);
+    for (int r = 0; r < S; ++r) {
+      const double v = nl.sgn[i * S + r];
+      atomicAdd(&part[soff(F_TOTPARTS, r)], -fabs(v));
+      atomicAdd(&part[soff(F_NORMSQ, r)], -(v * v));
+      if (isref) atomicAdd(&part[soff(F_INSTHF, r)], -v);
+    }
+  }
+  __syncthreads();
+}
 
 // ------------------------------------------------------------- prepass
 // CalcParentFlag_det + SumEContrib + decide_num_to_spawn + walker_death for
@@ -2549,9 +2576,11 @@ __device__ inline double diag_group(const DevSys& s, const uint64_t* d, int g, d
 // worse (14e/30o, 1.3e5: 55 with one lane, 56 with four, 102 with 16), so
 // there the lane sums its own.  G is 16, or 64 when a block's LDS does not
 // hold 16 determinants' terms; 1 for the lattice.
+// A determinant that is refused, in an iteration that ends in an error, has
+// its list entry marked (kFlagRemoved).
 constexpr int64_t kShortList = 32768;
 template <int W, int R, int G>
-__device__ __forceinline__ void k_insert_body(const Grid& g_, const DevSys& s, const Walk& wk, Counters* cnt, const uint64_t* n_key, const double* n_sgn, const uint32_t* n_flag, const unsigned long long* n_ptr, double* lds) {
+__device__ __forceinline__ void k_insert_body(const Grid& g_, const DevSys& s, const Walk& wk, Counters* cnt, const uint64_t* n_key, const double* n_sgn, uint32_t* n_flag, const unsigned long long* n_ptr, double* lds) {
   if (cnt->halt) return;
   const int S = R <= 2 ? R : s.S;
   int64_t nn = (int64_t)*n_ptr;
@@ -2600,6 +2629,7 @@ __device__ __forceinline__ void k_insert_body(const Grid& g_, const DevSys& s, c
       if (slot >= wk.cap) {
         atomicOr(&cnt->err, 1u << NGPU_ERR_WALKERS_FULL);
         atomicAdd(&cnt->n_fail, 1ull);
+        n_flag[i] = kFlagRemoved;
         slot = -1;
       } else {
         int64_t home = find_walker_hash<W>(key, s.rh, s.L) - 1;
@@ -2610,6 +2640,7 @@ __device__ __forceinline__ void k_insert_body(const Grid& g_, const DevSys& s, c
           atomicOr(&cnt->err, 1u << NGPU_ERR_HASH_FULL);
           atomicAdd(&cnt->n_fail, 1ull);
           wk.flags(slot) = kFlagRemoved;
+          n_flag[i] = kFlagRemoved;
           slot = -1;
         }
       }
@@ -2648,7 +2679,7 @@ __device__ __forceinline__ void k_insert_body(const Grid& g_, const DevSys& s, c
     atomicAdd(&cnt->reuse_part[g_.b % Counters::kSpread].v, (unsigned long long)blk_reused);
 }
 template <int W, int R, int G>
-__global__ void __launch_bounds__(kBlock) k_insert(DevSys s, Walk wk, Counters* cnt, const uint64_t* n_key, const double* n_sgn, const uint32_t* n_flag, const unsigned long long* n_ptr) {
+__global__ void __launch_bounds__(kBlock) k_insert(DevSys s, Walk wk, Counters* cnt, const uint64_t* n_key, const double* n_sgn, uint32_t* n_flag, const unsigned long long* n_ptr) {
   extern __shared__ double insert_dyn[];
   k_insert_body<W, R, G>(hw_grid(), s, wk, cnt, n_key, n_sgn, n_flag, n_ptr, insert_dyn);
 }
