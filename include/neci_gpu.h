@@ -280,12 +280,13 @@ int ngpu_set_graph(ngpu_t *h, int32_t on);
 /* Launch shape, the knobs of the autotuner (neci_stable_amd/autotune.py):
    blocks of the chunked kernels (prepass, attempt scan; 64 to 16 per compute
    unit), blocks of the grid-stride kernels (insert, statistics; 64 to 64 per
-   compute unit; the spawning kernels run as many as the chip holds, times this
-   value over its default of four per compute unit), elements per thread of a radix tile (2, 4 or 8; the
-   sorts of the core space's set-up), lanes per heat-bath single attempt
-   (4, 8 or 16) and blocks of the merge-annihilation kernel (64 to 64 per
-   compute unit).  0 keeps a value.  Results do not
-   depend on the shape (the kernels' outputs are independent of how work is
+   compute unit; an engine's own spawning kernels run as many as the chip
+   holds, times this value over its default of four per compute unit), lanes
+   per heat-bath single attempt (4, 8 or 16) and blocks of the
+   merge-annihilation kernel (64 to 64 per compute unit).  radix_items (2, 4 or
+   8) is kept and read back but shapes nothing: it set the tile of the spawned
+   list's sort, whose place the spawn bins took.  0 keeps a value.  Results do
+   not depend on the shape (the kernels' outputs are independent of how work is
    split; only the storage order of new determinants may differ).  No
    counterpart in the reference. */
 int ngpu_set_launch_shape(ngpu_t *h, int32_t chunk_blocks, int32_t grid_blocks, int32_t radix_items,

@@ -174,7 +174,7 @@ struct ngpu_engine {
   int W = 1, S = 1;
   int nb_chunk = 1024;  // blocks of the chunked kernels (prepass, scans, radix)
   int nb_grid = 1024;   // blocks of the grid-stride kernels
-  int radix_items = 4;  // elements per thread of a radix tile (2, 4 or 8)
+  int radix_items = 4;  // a launch-shape value kept for its readers: no kernel has a choice of radix tiles left
   int single_lanes = 4;  // lanes per heat-bath single attempt (4, 8 or 16)
   int nb_merge = 0;      // blocks of the merge-annihilation kernel (0: nb_grid)
   int n_cu = 256, max_chunk = 4096;
@@ -290,7 +290,6 @@ struct BatchGroup {
   int gen = 0;              // kGenHubbard, kGenPchb or kGenUniform
   bool singles = false;     // queued heat-bath singles (PCHB generator)
   int lanes = 4, pp = 2;    // heat-bath singles: lanes per attempt, orbital pairs per lane
-  int items = 4;            // launch-shape knob of the set-up sorts
   int ins_lanes = 1;        // lanes per new determinant, and a block's LDS for them
   size_t ins_lds = 0;
   bool core = false, core_fp32 = false;
@@ -2664,7 +2663,6 @@ BatchGroup group_of(const ngpu_t* h) {
   g.singles = g.gen == kGenPchb || g.gen == kGenPchbW;
   g.lanes = h->single_lanes;
   g.pp = singles_pp(h->single_lanes, h->sys.nbasis / 2);
-  g.items = h->radix_items;
   g.core = h->ncore > 0;
   g.core_fp32 = h->core_fp32;
   g.rec_words = h->ds.rec_words;
@@ -2672,7 +2670,7 @@ BatchGroup group_of(const ngpu_t* h) {
 }
 
 bool same_group(const BatchGroup& a, const BatchGroup& b) {
-  return a.W == b.W && a.S == b.S && a.gen == b.gen && a.lanes == b.lanes && a.pp == b.pp && a.items == b.items &&
+  return a.W == b.W && a.S == b.S && a.gen == b.gen && a.lanes == b.lanes && a.pp == b.pp &&
          a.core == b.core && a.core_fp32 == b.core_fp32 && a.rec_words == b.rec_words;
 }
 
