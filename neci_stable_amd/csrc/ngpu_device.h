@@ -1279,9 +1279,21 @@ __device__ __host__ inline void apply_excit(const uint64_t* d, const Excit& ex, 
   }
 }
 
+// INT(x) of the reference, as a 64-bit integer gives it: one instruction while
+// it fits (+ 0.0: no negative zero), the conversion itself for NaN (0) and for
+// what no 64-bit integer holds (the largest or smallest ones)
+__device__ __host__ inline double int_part(double x) {
+  double i = trunc(x) + 0.0;
+  if (__builtin_expect(!(fabs(x) < 9223372036854775808.0), 0)) {
+    asm volatile("");  // a branch, not the conversion's ten instructions in every call
+    i = (double)(int64_t)x;
+  }
+  return i;
+}
+
 // stochastic_round_r (lib/util_mod.fpp:207-224)
 __device__ __host__ inline double stochastic_round(double x, double r) {
-  double i = trunc(x) + 0.0;  // INT(x); + 0.0: no negative zero
+  double i = int_part(x);
   double res = x - i;
   if (fabs(res) >= 1.0e-12)
     if (fabs(res) > r) i = i + (x >= 0.0 ? 1.0 : -1.0);
@@ -1308,7 +1320,7 @@ __device__ __host__ inline double attempt_create(const DevSys& s, double tau, do
 __device__ __host__ inline double attempt_die(bool real_coeff, double fac, double absc, double r) {
   if (real_coeff) return fac * absc;
   double rat = fac * absc;
-  double nd = trunc(rat) + 0.0;
+  double nd = int_part(rat);
   rat = rat - nd;
   if (fabs(rat) > r) nd = nd + (rat >= 0.0 ? 1.0 : -1.0);
   return nd;
