@@ -441,7 +441,8 @@ __device__ inline void hash_refill_part(const Grid& g, const DevSys& s, const Wa
 // very often, or a spawned list near its capacity) sends its further records
 // to one of kSpill spill areas, a full area to the overflow list; the wave of
 // a bin that spilled searches them for its own.  Order within a bin is the
-// order of arrival: the merge's sums do not depend on it beyond FP64 rounding.
+// order of arrival (of an explicit list, the list's): the merge's sums do not
+// depend on it beyond FP64 rounding.
 constexpr uint32_t kSpill = 1024;
 struct Bins {
   uint64_t* rec;     // cap records, bin_cap to each bin
@@ -464,21 +465,30 @@ constexpr int kBinFill = 44;
 // attempt spawns, 22 rounds.  Empty bins cost a 64th of a load each.
 constexpr int kMinRate = 64;
 
-__device__ inline void set_bins(Counters* cnt, const Bins& b, double expect) {
+// the number of bins for a list of the expected length, the records each holds
+// and the log2 distance of their counters
+struct BinPlan {
+  uint32_t nbins, cap, shift;
+};
+__host__ __device__ inline BinPlan bin_plan(const Bins& b, double expect) {
   double nb = expect * (1.0 / kBinFill) + 1.0;
   const uint32_t n = nb < (double)b.maxb ? (uint32_t)nb : b.maxb;
   uint32_t sh = 0;
   while (sh < 5 && ((uint64_t)n << (sh + 1)) <= b.words) ++sh;
   const int64_t c = b.cap / n;
-  cnt->nbins = n;
-  cnt->bin_cap = (uint32_t)(c < 0x7FFFFFFF ? c : 0x7FFFFFFF);
-  cnt->bin_shift = sh;
+  return BinPlan{n, (uint32_t)(c < 0x7FFFFFFF ? c : 0x7FFFFFFF), sh};
+}
+__host__ __device__ inline void set_bins(Counters* cnt, const Bins& b, double expect) {
+  const BinPlan p = bin_plan(b, expect);
+  cnt->nbins = p.nbins;
+  cnt->bin_cap = p.cap;
+  cnt->bin_shift = p.shift;
 }
 
 // hash of a determinant: the high word picks the bin, its fraction inside the
 // bin the first slot of the merge's table
 template <int W>
-__device__ inline uint32_t bin_hash(const uint64_t* d) {
+__host__ __device__ inline uint32_t bin_hash(const uint64_t* d) {
   uint64_t h = d[0] * 0x9E3779B97F4A7C15ull;
   if constexpr (W == 2) {
     h += (d[1] ^ (d[1] >> 29)) * 0xBF58476D1CE4E5B9ull;
@@ -486,7 +496,7 @@ __device__ inline uint32_t bin_hash(const uint64_t* d) {
   }
   return (uint32_t)(h >> 32);
 }
-__device__ inline uint32_t bin_of(uint32_t h, uint32_t nb) { return (uint32_t)(((uint64_t)h * nb) >> 32); }
+__host__ __device__ inline uint32_t bin_of(uint32_t h, uint32_t nb) { return (uint32_t)(((uint64_t)h * nb) >> 32); }
 
 // where the record with place pos of bin b goes
 // (null: the overflow list is full, which takes more records than the spawn
@@ -1015,16 +1025,24 @@ __device__ inline void spawn_flush(const SpawnStage<W>* ss, int n, Counters* cnt
   wave_sync();
 }
 
-// an explicit spawned list (n dense records) into the bins
+// An explicit spawned list (n dense records) into the bins, each record at the
+// place the host chose for it: places in list order, so that a wave reads a
+// determinant's records, and sums them, in the order of the list.  Places count
+// through the bins' records, the spill areas and the overflow list.
 template <int W>
-__global__ void __launch_bounds__(kBlock) k_bin_list(DevSys s, Counters* cnt, const uint64_t* list, int64_t n, Bins bins) {
-  const uint32_t nb = cnt->nbins, cap = cnt->bin_cap, sh = cnt->bin_shift;
+__global__ void __launch_bounds__(kBlock) k_bin_list(DevSys s, Counters* cnt, const uint64_t* list, const int64_t* place, int64_t n, Bins bins) {
+  const uint32_t nb = cnt->nbins, sh = cnt->bin_shift;
+  const int64_t spill0 = bins.cap, ovf0 = spill0 + (int64_t)kSpill * bins.spill_cap;
   for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
     const uint64_t* q = list + i * s.rec_words;
-    const uint32_t bin = bin_of(bin_hash<W>(q), nb), pos = atomicAdd(&bins.count[(size_t)bin << sh], 1u);
-    uint64_t* r = bin_record(cnt, bins, bin, pos, cap, s.rec_words);
-    if (r)
-      for (int w = 0; w < s.rec_words; ++w) r[w] = q[w];
+    const int64_t p = place[i];
+    const uint32_t bin = bin_of(bin_hash<W>(q), nb);
+    atomicAdd(&bins.count[(size_t)bin << sh], 1u);
+    if (p >= spill0) atomicAdd(&bins.scount[bin % kSpill], 1u);
+    if (p >= ovf0) atomicAdd(&cnt->n_ovf, 1ull);
+    uint64_t* r = p < spill0 ? bins.rec + p * s.rec_words
+                : p < ovf0 ? bins.spill + (p - spill0) * s.rec_words : bins.ovf + (p - ovf0) * s.rec_words;
+    for (int w = 0; w < s.rec_words; ++w) r[w] = q[w];
   }
 }
 __global__ void k_set_bins(Counters* cnt, Bins bins, int64_t n) { set_bins(cnt, bins, (double)n); }
