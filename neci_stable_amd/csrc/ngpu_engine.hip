@@ -3418,7 +3418,7 @@ int ngpu_annihilate(ngpu_t* h, uint32_t iter, const int64_t* sdet, const double*
     for (int64_t i = 0; i < n; ++i) {
       uint64_t* r = rec.data() + (size_t)i * rw;
       for (int w = 0; w < W; ++w) r[w] = (uint64_t)sdet[i * W + w];
-      const uint64_t info = sinfo[i];
+      const uint64_t info = sinfo[i] & (0xFFu | kInfoInit);  // the merge marks records in the other bits
       if (h->ds.spawn_fp32) {  // FP32 amplitudes: each value rounded to nearest on entry
         float f = (float)sval[i];
         uint32_t fb;

@@ -2,7 +2,9 @@
 summed in the order of the list, so that the merged list is the same to the
 last bit on every call (CompressSpawnedList sums a sorted list front to back).
 Lists short and long, spread and crowded into a few bins whose records spill
-into their areas and the overflow list, and longer than one step of the upload."""
+into their areas and the overflow list, and longer than one step of the upload.
+Only bits 0 to 8 of the info word mean anything (include/neci_gpu.h): others
+change nothing."""
 import numpy as np
 import pytest
 
@@ -50,3 +52,17 @@ def test_sums_in_list_order(kind, system, nrep, fp32):
         np.testing.assert_array_equal(got[0], want[0])
         np.testing.assert_array_equal(got[1], want[1])
         eng.close()
+
+
+@pytest.mark.parametrize("kind", ["crowded", "spread"])
+def test_other_bits_of_the_info_word_mean_nothing(kind):
+    from neci_stable_amd.engine import Engine
+    spec, sdet, sval, sinfo = _case(kind, "one", 2, False)
+    out = []
+    for extra in (0, 0xFFFFFE00):
+        eng = Engine(spec)
+        a, md, ms, mf = eng.annihilate(3, sdet, sval, sinfo | np.uint32(extra))
+        out.append(sort_walkers(md, ms, mf) + (a["n_unique"], a["n_new"]))
+        eng.close()
+    for x, y in zip(*out):
+        np.testing.assert_array_equal(x, y)
