@@ -221,9 +221,9 @@ struct ngpu_engine {
   double* u_sgn = nullptr;
   uint32_t* u_flag = nullptr;
   unsigned long long* u_count = nullptr;
-  // its input list, kListChunk dense records at a time, and their places
-  uint64_t* l_rec = nullptr;
-  int64_t* l_place = nullptr;
+  // its input list on the way: dense records, then their places (pinned)
+  uint64_t* l_buf[2] = {nullptr, nullptr};
+  hipEvent_t l_read[2] = {nullptr, nullptr};  // the kernel has read the buffer
   uint64_t* n_key = nullptr;
   double* n_sgn = nullptr;
   uint32_t* n_flag = nullptr;
@@ -1227,7 +1227,7 @@ int ngpu_destroy(ngpu_t* h) {
   if (h->stream) (void)hipStreamSynchronize(h->stream);
   void* ptrs[] = {h->wk.keys, h->wk.st, h->wk.diagH, h->wk.offdiagH, h->wk.freeq,
                   h->wk.htab, h->att_cnt, h->att_off, h->pinfo, h->blk_part, h->blk_rm, h->bins.rec,
-                  h->bins.spill, h->bins.ovf, h->bins.count, h->bins.scount, h->l_rec, h->l_place, h->hist, h->digit_tot, h->sq, h->n_key,
+                  h->bins.spill, h->bins.ovf, h->bins.count, h->bins.scount, h->hist, h->digit_tot, h->sq, h->n_key,
                   h->n_sgn, h->n_flag, h->u_key, h->u_sgn, h->u_flag, h->u_count, h->cnt, h->dout, h->dpart, h->dcyc, h->own_params, h->d_rh, h->d_nbr, h->d_tmat, h->d_umat, h->d_jk, h->d_jkrow, h->d_jk0, h->d_fref, h->d_chk, h->tile_p, h->core_keys, h->core_slot, h->core_rowptr, h->core_cols,
                   h->core_vals, h->core_x, h->core_y, h->d_ab_tab,
                   h->d_ab_prob, h->d_ab_ok, h->d_j_tab, h->d_j_prob, h->d_j_ok, h->d_ab_tgt, h->d_i_tab, h->d_i_prob,
@@ -1236,6 +1236,10 @@ int ngpu_destroy(ngpu_t* h) {
   if (h->hout) (void)hipHostFree(h->hout);
   if (h->hcnt) (void)hipHostFree(h->hcnt);
   if (h->hcyc) (void)hipHostFree(h->hcyc);
+  for (int q = 0; q < 2; ++q) {
+    if (h->l_buf[q]) (void)hipHostFree(h->l_buf[q]);
+    if (h->l_read[q]) (void)hipEventDestroy(h->l_read[q]);
+  }
   if (h->ev_ok)
     for (int q = 0; q < kEvRing; ++q)
       for (int s = 0; s < kStages; ++s)
@@ -3360,28 +3364,29 @@ int ngpu_attempt_create_batch(ngpu_t* h, const double* hel, const double* pgen, 
 
 extern "C++" {
 namespace {
-// an explicit list passes through this many records of device memory at a time
-constexpr int64_t kListChunk = 1 << 18;
+// An explicit list passes through this many records at a time: the host fills
+// one of two pinned buffers of them while the kernel reads the other.  (us per
+// call at 1e5 and 1e6 records, one pageable copy of the whole list: 664, 7581.)
+constexpr int64_t kListChunk = 1 << 15;
 
-// The places of an explicit list's n records in list order: record i follows
+// The places of an explicit list's records in list order: a record follows
 // the records of its bin that stand before it in the list, first in the bin,
-// then in the bin's spill area, then in the overflow list.  n is at most the
-// spawn capacity, which the overflow list holds alone.
-template <int W>
-std::vector<int64_t> list_places(const Bins& b, const std::vector<uint64_t>& rec, int64_t n, int rec_words) {
-  const BinPlan p = bin_plan(b, (double)n);
-  std::vector<uint32_t> count(p.nbins, 0), spilled(kSpill, 0);
-  std::vector<int64_t> place((size_t)n);
-  const int64_t spill0 = b.cap, ovf0 = spill0 + (int64_t)kSpill * b.spill_cap;
+// then in the bin's spill area, then in the overflow list.  The list is no
+// longer than the spawn capacity, which the overflow list holds alone.
+struct ListPlaces {
+  Bins b;
+  BinPlan p;
+  std::vector<uint32_t> count, spilled;
   int64_t over = 0;
-  for (int64_t i = 0; i < n; ++i) {
-    const uint32_t bin = bin_of(bin_hash<W>(rec.data() + (size_t)i * rec_words), p.nbins), a = bin % kSpill;
-    if (count[bin] < p.cap) place[i] = (int64_t)bin * p.cap + count[bin]++;
-    else if (spilled[a] < b.spill_cap) place[i] = spill0 + (int64_t)a * b.spill_cap + spilled[a]++;
-    else place[i] = ovf0 + over++;
+  ListPlaces(const Bins& bins, int64_t n)
+      : b(bins), p(bin_plan(bins, (double)n)), count(p.nbins, 0), spilled(kSpill, 0) {}
+  int64_t next(uint32_t hash) {
+    const uint32_t bin = bin_of(hash, p.nbins), a = bin % kSpill;
+    if (count[bin] < p.cap) return (int64_t)bin * p.cap + count[bin]++;
+    if (spilled[a] < b.spill_cap) return b.cap + (int64_t)a * b.spill_cap + spilled[a]++;
+    return b.cap + (int64_t)kSpill * b.spill_cap + over++;
   }
-  return place;
-}
+};
 }  // namespace
 }
 
@@ -3407,45 +3412,46 @@ int ngpu_annihilate(ngpu_t* h, uint32_t iter, const int64_t* sdet, const double*
     HIP_OK(hipMalloc((void**)&h->u_flag, (size_t)h->scap * 4));
     HIP_OK(hipMalloc((void**)&h->u_count, 8));
   }
+  const int rw = h->ds.rec_words;
   const int64_t chunk = std::min<int64_t>(h->scap, kListChunk);
-  if (!h->l_rec) HIP_OK(hipMalloc((void**)&h->l_rec, (size_t)chunk * kRecWords * 8));
-  if (!h->l_place) HIP_OK(hipMalloc((void**)&h->l_place, (size_t)chunk * 8));
-  std::vector<uint64_t> rec;
-  std::vector<int64_t> place;
-  if (n) {
-    const int rw = h->ds.rec_words;
-    rec.assign((size_t)n * rw, 0);
-    for (int64_t i = 0; i < n; ++i) {
-      uint64_t* r = rec.data() + (size_t)i * rw;
-      for (int w = 0; w < W; ++w) r[w] = (uint64_t)sdet[i * W + w];
-      const uint64_t info = sinfo[i] & (0xFFu | kInfoInit);  // the merge marks records in the other bits
-      if (h->ds.spawn_fp32) {  // FP32 amplitudes: each value rounded to nearest on entry
-        float f = (float)sval[i];
-        uint32_t fb;
-        memcpy(&fb, &f, 4);
-        r[W] = (info << 32) | fb;
-      } else {
-        uint64_t vb;
-        memcpy(&vb, &sval[i], 8);
-        r[2] = vb;
-        r[3] = info;
-      }
-    }
-    place = W == 1 ? list_places<1>(h->bins, rec, n, rw) : list_places<2>(h->bins, rec, n, rw);
+  for (int q = 0; q < 2; ++q) {
+    if (!h->l_read[q]) HIP_OK(hipEventCreateWithFlags(&h->l_read[q], hipEventDisableTiming));
+    if (!h->l_buf[q])
+      HIP_OK(hipHostMalloc((void**)&h->l_buf[q], (size_t)chunk * (kRecWords + 1) * 8, hipHostMallocDefault));
   }
+  ListPlaces places(h->bins, n);
   hipLaunchKernelGGL(k_begin_iter, dim3(1), dim3(kBlock), 0, h->stream, h->dout, h->dpart, h->cnt, h->dparams,
                      IterParams{}, 0);
   hipLaunchKernelGGL(k_set_count, dim3(1), dim3(1), 0, h->stream, &h->cnt->n_spawned, (unsigned long long)n);
   hipLaunchKernelGGL(k_set_count, dim3(1), dim3(1), 0, h->stream, h->u_count, 0ull);
   hipLaunchKernelGGL(k_set_bins, dim3(1), dim3(1), 0, h->stream, h->cnt, h->bins, n);
-  for (int64_t i = 0; i < n; i += chunk) {
-    const int64_t m = std::min(chunk, n - i);
-    const int rw = h->ds.rec_words;
-    HIP_OK(hipMemcpyAsync(h->l_rec, rec.data() + (size_t)i * rw, (size_t)m * rw * 8, hipMemcpyHostToDevice, h->stream));
-    HIP_OK(hipMemcpyAsync(h->l_place, place.data() + i, (size_t)m * 8, hipMemcpyHostToDevice, h->stream));
+  for (int64_t i0 = 0; i0 < n; i0 += chunk) {
+    const int64_t m = std::min(chunk, n - i0);
+    const int q = (int)(i0 / chunk % 2);
+    if (i0 >= 2 * chunk) HIP_OK(hipEventSynchronize(h->l_read[q]));
+    uint64_t* place = h->l_buf[q] + (size_t)m * rw;
+    for (int64_t i = 0; i < m; ++i) {
+      uint64_t* r = h->l_buf[q] + (size_t)i * rw;
+      const uint64_t* d = (const uint64_t*)sdet + (i0 + i) * W;
+      const double v = sval[i0 + i];
+      for (int w = 0; w < W; ++w) r[w] = d[w];
+      const uint64_t info = sinfo[i0 + i] & (0xFFu | kInfoInit);  // the merge marks records in the other bits
+      if (h->ds.spawn_fp32) {  // FP32 amplitudes: each value rounded to nearest on entry
+        float f = (float)v;
+        uint32_t fb;
+        memcpy(&fb, &f, 4);
+        r[W] = (info << 32) | fb;
+      } else {
+        if (W == 1) r[1] = 0;
+        memcpy(&r[2], &v, 8);
+        r[3] = info;
+      }
+      place[i] = (uint64_t)places.next(W == 1 ? bin_hash<1>(d) : bin_hash<2>(d));
+    }
     auto kern = W == 1 ? k_bin_list<1> : k_bin_list<2>;
-    hipLaunchKernelGGL(kern, dim3(grid_for(m)), dim3(kBlock), 0, h->stream, h->ds, h->cnt, (const uint64_t*)h->l_rec,
-                       (const int64_t*)h->l_place, m, h->bins);
+    hipLaunchKernelGGL(kern, dim3(grid_for(m)), dim3(kBlock), 0, h->stream, h->ds, h->cnt,
+                       (const uint64_t*)h->l_buf[q], (const int64_t*)place, m, h->bins);
+    HIP_OK(hipEventRecord(h->l_read[q], h->stream));
   }
   bool p = h->prof;
   h->prof = false;
