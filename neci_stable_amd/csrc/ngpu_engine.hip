@@ -227,6 +227,7 @@ struct ngpu_engine {
   uint64_t* n_key = nullptr;
   double* n_sgn = nullptr;
   uint32_t* n_flag = nullptr;
+  NewList* d_nl = nullptr;  // the same for the iteration's end, with the reference
   // system tables
   int32_t* d_rh = nullptr;
   int32_t* d_nbr = nullptr;
@@ -374,8 +375,8 @@ constexpr int kEndThreads = 512;  // one pass over one replica's statistics
 // accumulators in the reference too)
 __device__ __forceinline__ void end_iter_body(ngpu_iter_out_t* out, double* part, ngpu_iter_out_t* cyc, Counters* cnt,
                                               int64_t scap, int64_t cap, int64_t hash_entries, const IterParams* prm,
-                                              uint32_t* scount, int S, const NewList& nl) {
-  const bool refused = nl.W && cnt->n_fail != 0;  // in the same round trip as halt
+                                              uint32_t* scount, int S, const NewList* nl) {
+  const bool refused = nl && cnt->n_fail != 0;  // in the same round trip as halt
   // halted: the output block keeps the failing iteration's statistics and
   // error, and nothing is added to the cycle
   if (cnt->halt) return;
@@ -402,7 +403,7 @@ __device__ __forceinline__ void end_iter_body(ngpu_iter_out_t* out, double* part
       n_unique = (unsigned long long)u;
     }
   }
-  if (refused) uncount_refused(nl, cnt, part, S);
+  if (__builtin_expect(refused, 0)) uncount_refused(*nl, cnt, part, S);
   double* g = (double*)out;
   double* c = (double*)cyc;
   // the statistics rows: kEndParts threads per field take kStatCopies /
@@ -481,15 +482,15 @@ __device__ __forceinline__ void end_iter_body(ngpu_iter_out_t* out, double* part
 }
 __global__ void __launch_bounds__(kEndThreads) k_end_iter(ngpu_iter_out_t* out, double* part, ngpu_iter_out_t* cyc, Counters* cnt,
                            int64_t scap, int64_t cap, int64_t hash_entries, const IterParams* prm,
-                           uint32_t* scount, int S, NewList nl) {
+                           uint32_t* scount, int S, const NewList* nl) {
   end_iter_body(out, part, cyc, cnt, scap, cap, hash_entries, prm, scount, S, nl);
 }
 // the end of the iteration of every engine of a batch group: one block each
 __global__ void __launch_bounds__(kEndThreads) km_end_iter(const EngDev* __restrict__ ed, int W) {
   const EngDev& a = ed[blockIdx.x];
-  const NewList nl{a.n_key, a.n_sgn, a.n_flag, a.s.ref[0], a.s.ref[1], stats_by_parts(a.s) ? W : 0};
+  const NewList nl{a.n_key, a.n_sgn, a.n_flag, a.s.ref[0], a.s.ref[1], W};
   end_iter_body(a.dout, a.part, a.dcyc, a.cnt, a.scap, a.wk.cap, a.wk.L * (int64_t)kBucketEntries, a.prm,
-                a.bins.scount, a.s.S, nl);
+                a.bins.scount, a.s.S, stats_by_parts(a.s) ? &nl : nullptr);
 }
 
 // the last iteration's statistics, the cycle's sums and the sticky error to
@@ -643,7 +644,7 @@ void annihilation_chain(ngpu_t* h, bool with_core, bool list_out = false) {
          (const IterParams*)h->dparams);
   launch(h, -1, -1, k_end_iter, dim3(1), dim3(kEndThreads), h->dout, h->dpart, h->dcyc, h->cnt,
          h->scap, h->wk.cap, h->wk.L * (int64_t)kBucketEntries, (const IterParams*)h->dparams, h->bins.scount, h->S,
-         NewList{h->n_key, h->n_sgn, h->n_flag, h->ds.ref[0], h->ds.ref[1], by_parts ? W : 0});
+         by_parts ? (const NewList*)h->d_nl : nullptr);
   if (h->checks) check_chain<W>(h, with_core);
 }
 
@@ -1168,6 +1169,7 @@ int ngpu_create(ngpu_t** out, const ngpu_sys_t* sys) {
   fail(dalloc(&h->n_key, (size_t)ncap * W));
   fail(dalloc(&h->n_sgn, (size_t)ncap * S));
   fail(dalloc(&h->n_flag, (size_t)ncap));
+  fail(dalloc(&h->d_nl, 1));
   fail(dalloc(&h->cnt, 1));
   fail(dalloc(&h->dout, 1));
   fail(dalloc(&h->dpart, (size_t)kStatCopies * kStatStride));
@@ -1228,7 +1230,7 @@ int ngpu_destroy(ngpu_t* h) {
   void* ptrs[] = {h->wk.keys, h->wk.st, h->wk.diagH, h->wk.offdiagH, h->wk.freeq,
                   h->wk.htab, h->att_cnt, h->att_off, h->pinfo, h->blk_part, h->blk_rm, h->bins.rec,
                   h->bins.spill, h->bins.ovf, h->bins.count, h->bins.scount, h->hist, h->digit_tot, h->sq, h->n_key,
-                  h->n_sgn, h->n_flag, h->u_key, h->u_sgn, h->u_flag, h->u_count, h->cnt, h->dout, h->dpart, h->dcyc, h->own_params, h->d_rh, h->d_nbr, h->d_tmat, h->d_umat, h->d_jk, h->d_jkrow, h->d_jk0, h->d_fref, h->d_chk, h->tile_p, h->core_keys, h->core_slot, h->core_rowptr, h->core_cols,
+                  h->n_sgn, h->n_flag, h->d_nl, h->u_key, h->u_sgn, h->u_flag, h->u_count, h->cnt, h->dout, h->dpart, h->dcyc, h->own_params, h->d_rh, h->d_nbr, h->d_tmat, h->d_umat, h->d_jk, h->d_jkrow, h->d_jk0, h->d_fref, h->d_chk, h->tile_p, h->core_keys, h->core_slot, h->core_rowptr, h->core_cols,
                   h->core_vals, h->core_x, h->core_y, h->d_ab_tab,
                   h->d_ab_prob, h->d_ab_ok, h->d_j_tab, h->d_j_prob, h->d_j_ok, h->d_ab_tgt, h->d_i_tab, h->d_i_prob,
                   h->d_a_tab, h->d_a_prob, h->d_a_ok, h->d_b_tab, h->d_b_prob, h->d_b_ok};
@@ -1587,6 +1589,8 @@ int ngpu_set_reference(ngpu_t* h, const int64_t* ilut_ref, double hii) {
   h->ds.ref[0] = (uint64_t)ilut_ref[0];
   h->ds.ref[1] = h->W > 1 ? (uint64_t)ilut_ref[1] : 0;
   h->ds.hii = hii;
+  const NewList nl{h->n_key, h->n_sgn, h->n_flag, h->ds.ref[0], h->ds.ref[1], h->W};
+  HIP_OK(hipMemcpy(h->d_nl, &nl, sizeof nl, hipMemcpyHostToDevice));
   h->have_ref = true;
   update_pair_probs(h);
   return refresh_fref(h);

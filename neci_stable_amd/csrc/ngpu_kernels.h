@@ -585,7 +585,9 @@ __host__ __device__ inline bool stats_by_parts(const DevSys& s) { return !s.t_re
 // The merge counts a new determinant before k_insert has placed it: what the
 // insertion refused (the iteration ends in an error) is taken out again by the
 // iteration's end, so that the statistics are those of the kept walker list.
-// The new list as the end of an iteration sees it; W = 0: not by parts
+// The new list as the end of an iteration sees it, in device memory: only an
+// iteration that refused something reads it, and a longer argument block cost
+// every one 0.5 us.
 struct NewList {
   const uint64_t* key;
   const double* sgn;
