@@ -86,8 +86,8 @@ __device__ __forceinline__ EngDev eng_of(const EngDev* __restrict__ ed, const ui
   NGPU_GLOBAL(wk.freeq);
   NGPU_GLOBAL(cnt); NGPU_GLOBAL(part); NGPU_GLOBAL(att_cnt); NGPU_GLOBAL(att_off); NGPU_GLOBAL(pinfo);
   NGPU_GLOBAL(blk_part); NGPU_GLOBAL(blk_rm); NGPU_GLOBAL(tile_p);
-  NGPU_GLOBAL(bins.rec); NGPU_GLOBAL(bins.spill); NGPU_GLOBAL(bins.ovf); NGPU_GLOBAL(bins.count);
-  NGPU_GLOBAL(bins.scount);
+  NGPU_GLOBAL(bins.rec); NGPU_GLOBAL(bins.ovf); NGPU_GLOBAL(bins.next); NGPU_GLOBAL(bins.head);
+  NGPU_GLOBAL(bins.count);
   NGPU_GLOBAL(sq); NGPU_GLOBAL(n_key); NGPU_GLOBAL(n_sgn); NGPU_GLOBAL(n_flag); NGPU_GLOBAL(prm);
   NGPU_GLOBAL(core_slot); NGPU_GLOBAL(core_rowptr); NGPU_GLOBAL(core_cols); NGPU_GLOBAL(core_x); NGPU_GLOBAL(core_y);
 #undef NGPU_GLOBAL

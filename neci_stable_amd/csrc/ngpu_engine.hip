@@ -5,7 +5,9 @@
 #include <algorithm>
 #include <cmath>
 #include <cstdio>
+#include <cstdlib>
 #include <cstring>
+#include <memory>
 #include <mutex>
 #include <type_traits>
 #include <vector>
@@ -221,7 +223,7 @@ struct ngpu_engine {
   double* u_sgn = nullptr;
   uint32_t* u_flag = nullptr;
   unsigned long long* u_count = nullptr;
-  // its input list on the way: dense records, then their places (pinned)
+  // its input list on the way: dense records, then their places and links (pinned)
   uint64_t* l_buf[2] = {nullptr, nullptr};
   hipEvent_t l_read[2] = {nullptr, nullptr};  // the kernel has read the buffer
   uint64_t* n_key = nullptr;
@@ -361,7 +363,7 @@ __global__ void k_begin_iter(ngpu_iter_out_t* out, double* part, Counters* cnt, 
     cnt->n_fail = 0;
     cnt->ins_refused = 0;
     cnt->err = 0;
-    cnt->prev_spawned = cnt->prev_attempts = 0;  // other walkers: their spawning rate is not known
+    cnt->prev_spawned = cnt->prev_attempts = cnt->prev_unique = 0;  // other walkers: their spawning rate is not known
     out->tot_walkers = 0;
     out->n_attempts = out->n_spawned = out->n_unique = out->n_new = 0;
     out->err = 0;
@@ -375,13 +377,12 @@ constexpr int kEndThreads = 512;  // one pass over one replica's statistics
 // accumulators in the reference too)
 __device__ __forceinline__ void end_iter_body(ngpu_iter_out_t* out, double* part, ngpu_iter_out_t* cyc, Counters* cnt,
                                               int64_t scap, int64_t cap, int64_t hash_entries, const IterParams* prm,
-                                              uint32_t* scount, int S, const NewList* nl) {
+                                              int S, const NewList* nl) {
   const bool refused = nl && cnt->n_fail != 0;  // in the same round trip as halt
   // halted: the output block keeps the failing iteration's statistics and
   // error, and nothing is added to the cycle
   if (cnt->halt) return;
   __shared__ unsigned long long n_unique;
-  for (uint32_t i = threadIdx.x; i < kSpill; i += blockDim.x) scount[i] = 0;
   if (threadIdx.x < kWave) {
     // the spread per-block counts, one line per lane, summed across the wave
     const int l = threadIdx.x;
@@ -469,6 +470,7 @@ __device__ __forceinline__ void end_iter_body(ngpu_iter_out_t* out, double* part
     }
     cnt->prev_spawned = (unsigned long long)out->n_spawned;
     cnt->prev_attempts = cnt->n_attempts;
+    cnt->prev_unique = n_unique;
     // the counters the next iteration appends to start from zero (the chain
     // has no separate reset launch)
     cnt->n_spawned = 0;
@@ -482,15 +484,15 @@ __device__ __forceinline__ void end_iter_body(ngpu_iter_out_t* out, double* part
 }
 __global__ void __launch_bounds__(kEndThreads) k_end_iter(ngpu_iter_out_t* out, double* part, ngpu_iter_out_t* cyc, Counters* cnt,
                            int64_t scap, int64_t cap, int64_t hash_entries, const IterParams* prm,
-                           uint32_t* scount, int S, const NewList* nl) {
-  end_iter_body(out, part, cyc, cnt, scap, cap, hash_entries, prm, scount, S, nl);
+                           int S, const NewList* nl) {
+  end_iter_body(out, part, cyc, cnt, scap, cap, hash_entries, prm, S, nl);
 }
 // the end of the iteration of every engine of a batch group: one block each
 __global__ void __launch_bounds__(kEndThreads) km_end_iter(const EngDev* __restrict__ ed, int W) {
   const EngDev& a = ed[blockIdx.x];
   const NewList nl{a.n_key, a.n_sgn, a.n_flag, a.s.ref[0], a.s.ref[1], W};
   end_iter_body(a.dout, a.part, a.dcyc, a.cnt, a.scap, a.wk.cap, a.wk.L * (int64_t)kBucketEntries, a.prm,
-                a.bins.scount, a.s.S, stats_by_parts(a.s) ? &nl : nullptr);
+                a.s.S, stats_by_parts(a.s) ? &nl : nullptr);
 }
 
 // the last iteration's statistics, the cycle's sums and the sticky error to
@@ -643,7 +645,7 @@ void annihilation_chain(ngpu_t* h, bool with_core, bool list_out = false) {
   if (!by_parts) launch(h, 8, 8, k_stats<W, R>, dim3(h->nb_grid), dim3(kBlock), h->ds, h->wk, h->cnt, h->dpart,
          (const IterParams*)h->dparams);
   launch(h, -1, -1, k_end_iter, dim3(1), dim3(kEndThreads), h->dout, h->dpart, h->dcyc, h->cnt,
-         h->scap, h->wk.cap, h->wk.L * (int64_t)kBucketEntries, (const IterParams*)h->dparams, h->bins.scount, h->S,
+         h->scap, h->wk.cap, h->wk.L * (int64_t)kBucketEntries, (const IterParams*)h->dparams, h->S,
          by_parts ? (const NewList*)h->d_nl : nullptr);
   if (h->checks) check_chain<W>(h, with_core);
 }
@@ -1149,18 +1151,17 @@ int ngpu_create(ngpu_t** out, const ngpu_sys_t* sys) {
   {
     // one bin per kBinFill expected records, at most one per 64 of the
     // capacity; their regions hold the whole capacity and 16 records' slack
-    // each, so that even lists near it spill little
+    // each, so that even lists near it overflow little
     Bins& bn = h->bins;
     bn.maxb = (uint32_t)std::max<int64_t>(1, std::min<int64_t>(scap / 64, 1 << 20));
     bn.cap = scap + 16 * (int64_t)bn.maxb;
     bn.words = std::max<uint32_t>(bn.maxb, (uint32_t)std::min<int64_t>(32 * (int64_t)bn.maxb, 1 << 19));
-    bn.spill_cap = (uint32_t)(scap / 2 / kSpill + 1);
     bn.ovf_cap = scap;
     fail(dalloc(&bn.rec, (size_t)bn.cap * kRecWords));
-    fail(dalloc(&bn.spill, (size_t)bn.spill_cap * kSpill * kRecWords));
     fail(dalloc(&bn.ovf, (size_t)scap * kRecWords));
+    fail(dalloc(&bn.next, (size_t)scap));
+    fail(dalloc(&bn.head, (size_t)bn.maxb * kBinChains));
     fail(dalloc(&bn.count, (size_t)bn.words));
-    fail(dalloc(&bn.scount, (size_t)kSpill));
   }
   fail(dalloc(&h->hist, (size_t)h->max_chunk * kRadixBins));
   fail(dalloc(&h->digit_tot, (size_t)kRadixBins));
@@ -1183,7 +1184,6 @@ int ngpu_create(ngpu_t** out, const ngpu_sys_t* sys) {
     fail(hipMemsetAsync(wk.htab, 0xFF, (size_t)wk.L * 8 * W * sizeof(uint64_t), h->stream));
     fail(hipMemsetAsync(h->cnt, 0, sizeof(Counters), h->stream));
     fail(hipMemsetAsync(h->bins.count, 0, (size_t)h->bins.words * 4, h->stream));
-    fail(hipMemsetAsync(h->bins.scount, 0, kSpill * 4, h->stream));
     fail(hipMemsetAsync(h->dout, 0, sizeof(ngpu_iter_out_t), h->stream));
     fail(hipMemsetAsync(h->dpart, 0, sizeof(double) * kStatCopies * kStatStride, h->stream));
     fail(hipMemsetAsync(h->dcyc, 0, sizeof(ngpu_iter_out_t), h->stream));
@@ -1229,7 +1229,7 @@ int ngpu_destroy(ngpu_t* h) {
   if (h->stream) (void)hipStreamSynchronize(h->stream);
   void* ptrs[] = {h->wk.keys, h->wk.st, h->wk.diagH, h->wk.offdiagH, h->wk.freeq,
                   h->wk.htab, h->att_cnt, h->att_off, h->pinfo, h->blk_part, h->blk_rm, h->bins.rec,
-                  h->bins.spill, h->bins.ovf, h->bins.count, h->bins.scount, h->hist, h->digit_tot, h->sq, h->n_key,
+                  h->bins.ovf, h->bins.next, h->bins.head, h->bins.count, h->hist, h->digit_tot, h->sq, h->n_key,
                   h->n_sgn, h->n_flag, h->d_nl, h->u_key, h->u_sgn, h->u_flag, h->u_count, h->cnt, h->dout, h->dpart, h->dcyc, h->own_params, h->d_rh, h->d_nbr, h->d_tmat, h->d_umat, h->d_jk, h->d_jkrow, h->d_jk0, h->d_fref, h->d_chk, h->tile_p, h->core_keys, h->core_slot, h->core_rowptr, h->core_cols,
                   h->core_vals, h->core_x, h->core_y, h->d_ab_tab,
                   h->d_ab_prob, h->d_ab_ok, h->d_j_tab, h->d_j_prob, h->d_j_ok, h->d_ab_tgt, h->d_i_tab, h->d_i_prob,
@@ -3375,20 +3375,26 @@ constexpr int64_t kListChunk = 1 << 15;
 
 // The places of an explicit list's records in list order: a record follows
 // the records of its bin that stand before it in the list, first in the bin,
-// then in the bin's spill area, then in the overflow list.  The list is no
-// longer than the spawn capacity, which the overflow list holds alone.
+// then in the bin's chains.  The list is no longer than the spawn capacity,
+// which the overflow list holds alone.
 struct ListPlaces {
   Bins b;
   BinPlan p;
-  std::vector<uint32_t> count, spilled;
+  // records of each bin, and the last record (+ 1) of each chain; pages of them
+  // that no record touches are never there
+  std::unique_ptr<uint32_t, void (*)(void*)> count, tail;
   int64_t over = 0;
   ListPlaces(const Bins& bins, int64_t n)
-      : b(bins), p(bin_plan(bins, (double)n)), count(p.nbins, 0), spilled(kSpill, 0) {}
-  int64_t next(uint32_t hash) {
-    const uint32_t bin = bin_of(hash, p.nbins), a = bin % kSpill;
-    if (count[bin] < p.cap) return (int64_t)bin * p.cap + count[bin]++;
-    if (spilled[a] < b.spill_cap) return b.cap + (int64_t)a * b.spill_cap + spilled[a]++;
-    return b.cap + (int64_t)kSpill * b.spill_cap + over++;
+      : b(bins), p(bin_plan(bins, (double)n, (double)n)), count((uint32_t*)calloc(p.nbins, 4), free),
+        tail((uint32_t*)calloc((size_t)p.nbins * kBinChains, 4), free) {}
+  int64_t next(uint32_t hash, int64_t* link) {
+    const uint32_t bin = bin_of(hash, p.nbins), at = count.get()[bin]++;
+    if (at < p.cap) return (int64_t)bin * p.cap + at;
+    const int64_t chain = (int64_t)bin * kBinChains + (at - p.cap) % kBinChains;
+    uint32_t& last = tail.get()[chain];
+    *link = last ? (int64_t)last - 1 : kChainHead + chain;
+    last = (uint32_t)++over;
+    return b.cap + over - 1;
   }
 };
 }  // namespace
@@ -3421,9 +3427,10 @@ int ngpu_annihilate(ngpu_t* h, uint32_t iter, const int64_t* sdet, const double*
   for (int q = 0; q < 2; ++q) {
     if (!h->l_read[q]) HIP_OK(hipEventCreateWithFlags(&h->l_read[q], hipEventDisableTiming));
     if (!h->l_buf[q])
-      HIP_OK(hipHostMalloc((void**)&h->l_buf[q], (size_t)chunk * (kRecWords + 1) * 8, hipHostMallocDefault));
+      HIP_OK(hipHostMalloc((void**)&h->l_buf[q], (size_t)chunk * (kRecWords + 2) * 8, hipHostMallocDefault));
   }
   ListPlaces places(h->bins, n);
+  if (!places.count || !places.tail) return NGPU_ERR_HIP;  // no host memory
   hipLaunchKernelGGL(k_begin_iter, dim3(1), dim3(kBlock), 0, h->stream, h->dout, h->dpart, h->cnt, h->dparams,
                      IterParams{}, 0);
   hipLaunchKernelGGL(k_set_count, dim3(1), dim3(1), 0, h->stream, &h->cnt->n_spawned, (unsigned long long)n);
@@ -3450,11 +3457,11 @@ int ngpu_annihilate(ngpu_t* h, uint32_t iter, const int64_t* sdet, const double*
         memcpy(&r[2], &v, 8);
         r[3] = info;
       }
-      place[i] = (uint64_t)places.next(W == 1 ? bin_hash<1>(d) : bin_hash<2>(d));
+      place[i] = (uint64_t)places.next(W == 1 ? bin_hash<1>(d) : bin_hash<2>(d), (int64_t*)place + m + i);
     }
     auto kern = W == 1 ? k_bin_list<1> : k_bin_list<2>;
     hipLaunchKernelGGL(kern, dim3(grid_for(m)), dim3(kBlock), 0, h->stream, h->ds, h->cnt,
-                       (const uint64_t*)h->l_buf[q], (const int64_t*)place, m, h->bins);
+                       (const uint64_t*)h->l_buf[q], (const int64_t*)place, (const int64_t*)place + m, m, h->bins);
     HIP_OK(hipEventRecord(h->l_read[q], h->stream));
   }
   bool p = h->prof;

@@ -89,8 +89,8 @@ struct alignas(256) Counters {
   unsigned int bin_shift;
   // spawned records and attempts of the previous iteration (no attempts after
   // an upload or an explicit list): the expected number of records sizes the
-  // bins (speed only, results do not depend on it)
-  unsigned long long prev_spawned, prev_attempts;
+  // bins (speed only, results do not depend on it); and its unique ones
+  unsigned long long prev_spawned, prev_attempts, prev_unique;
   alignas(256) unsigned long long free_tail;
   alignas(256) unsigned long long n_spawned;
   alignas(256) unsigned long long n_singles;  // queued single-excitation attempts
@@ -439,20 +439,24 @@ __device__ inline void hash_refill_part(const Grid& g, const DevSys& s, const Wa
 // array has (an address, and so a line, takes one atomic in about 12 ns, and
 // scattered ones run at 25 G/s).  A bin that is full (one determinant spawned
 // very often, or a spawned list near its capacity) sends its further records
-// to one of kSpill spill areas, a full area to the overflow list; the wave of
-// a bin that spilled searches them for its own.  Order within a bin is the
+// to the overflow list, which holds the spawn capacity; they hang in
+// kBinChains chains of the bin, by their place in it, and the bin's wave
+// follows one chain a lane.  So a bin's records cost time in proportion to
+// their number wherever they are.  (Areas that the waves of all bins
+// that spilled searched for their own records took a time quadratic in the
+// list: 5.0e6 spawns on 6.2e4 determinants filling the list merged in 101 ms,
+// where the sort had taken 12.)  Order within a bin is the
 // order of arrival (of an explicit list, the list's): the merge's sums do not
 // depend on it beyond FP64 rounding.
-constexpr uint32_t kSpill = 1024;
+constexpr uint32_t kBinChains = 64;
 struct Bins {
   uint64_t* rec;     // cap records, bin_cap to each bin
-  uint64_t* spill;   // kSpill areas of spill_cap records, area b % kSpill for bin b
   uint64_t* ovf;     // overflow list (the spawn capacity)
+  uint32_t* next;    // of an overflow record, the one behind it in its chain
+  uint32_t* head;    // kBinChains per bin; never emptied, as chains are followed by length
   uint32_t* count;   // records of bin b at [b << bin_shift], emptied by the merge
-  uint32_t* scount;  // records sent to each area, emptied at the iteration's end
   int64_t cap;
   int64_t ovf_cap;   // the spawn capacity
-  uint32_t spill_cap;
   uint32_t maxb;     // most bins
   uint32_t words;    // length of count
 };
@@ -465,21 +469,33 @@ constexpr int kBinFill = 44;
 // attempt spawns, 22 rounds.  Empty bins cost a 64th of a load each.
 constexpr int kMinRate = 64;
 
-// the number of bins for a list of the expected length, the records each holds
-// and the log2 distance of their counters
+// the number of bins for a list of the expected length and number of
+// determinants, the records each holds and the log2 distance of their counters
 struct BinPlan {
   uint32_t nbins, cap, shift;
 };
-__host__ __device__ inline BinPlan bin_plan(const Bins& b, double expect) {
+// What a bin's load differs from the mean by is whole determinants with all
+// their records: a share 1 / sqrt(l) of it for l determinants a bin.  A list of
+// many records per determinant close to the capacity takes fewer bins, up to
+// kBinFill determinants in each, so that five such shares fit what is left of
+// the room (taken as 1.5 times the capacity: a bin has 1.25 times its share and
+// overflows a little for nothing).  Otherwise most of its records would take
+// the chains: 5.1e6 spawns on 6.0e4 uneven determinants, the list full, merge
+// in 0.40 ms with bins by records alone and in 0.30 ms with these.
+__host__ __device__ inline BinPlan bin_plan(const Bins& b, double expect, double dets) {
   double nb = expect * (1.0 / kBinFill) + 1.0;
+  const double spare = 1.5 * (double)b.ovf_cap - expect;  // (room / list - 1) list
+  const double l = spare > 0.0 && 25.0 * expect * expect < kBinFill * spare * spare
+                       ? 25.0 * expect * expect / (spare * spare) : (double)kBinFill;
+  if (nb * l > dets + l) nb = dets / l + 1.0;
   const uint32_t n = nb < (double)b.maxb ? (uint32_t)nb : b.maxb;
   uint32_t sh = 0;
   while (sh < 5 && ((uint64_t)n << (sh + 1)) <= b.words) ++sh;
   const int64_t c = b.cap / n;
   return BinPlan{n, (uint32_t)(c < 0x7FFFFFFF ? c : 0x7FFFFFFF), sh};
 }
-__host__ __device__ inline void set_bins(Counters* cnt, const Bins& b, double expect) {
-  const BinPlan p = bin_plan(b, expect);
+__host__ __device__ inline void set_bins(Counters* cnt, const Bins& b, double expect, double dets) {
+  const BinPlan p = bin_plan(b, expect, dets);
   cnt->nbins = p.nbins;
   cnt->bin_cap = p.cap;
   cnt->bin_shift = p.shift;
@@ -498,17 +514,15 @@ __host__ __device__ inline uint32_t bin_hash(const uint64_t* d) {
 }
 __host__ __device__ inline uint32_t bin_of(uint32_t h, uint32_t nb) { return (uint32_t)(((uint64_t)h * nb) >> 32); }
 
-// where the record with place pos of bin b goes
+// overflow record o, the k-th past the end of bin b, into its chain; its place
 // (null: the overflow list is full, which takes more records than the spawn
 // capacity; the merge takes nothing from such a list and the iteration's end
 // reports it)
-__device__ inline uint64_t* bin_record(Counters* cnt, const Bins& bins, uint32_t b, uint32_t pos, uint32_t cap,
-                                       int rec_words) {
-  if (pos < cap) return bins.rec + ((size_t)b * cap + pos) * rec_words;
-  const uint32_t a = b % kSpill, p = atomicAdd(&bins.scount[a], 1u);
-  if (p < bins.spill_cap) return bins.spill + ((size_t)a * bins.spill_cap + p) * rec_words;
-  const unsigned long long o = atomicAdd(&cnt->n_ovf, 1ull);
-  return o < (unsigned long long)bins.ovf_cap ? bins.ovf + (size_t)o * rec_words : nullptr;
+__device__ inline uint64_t* bin_overflow(const Bins& bins, uint32_t b, uint32_t k, unsigned long long o,
+                                         int rec_words) {
+  if (o >= (unsigned long long)bins.ovf_cap) return nullptr;
+  bins.next[o] = atomicExch(&bins.head[(size_t)b * kBinChains + k % kBinChains], (uint32_t)o);
+  return bins.ovf + (size_t)o * rec_words;
 }
 
 // this block's slots: whole waves, so that a small table does not
@@ -920,7 +934,10 @@ __device__ __forceinline__ void k_scan_apply_body(const Grid& g_, const DevSys& 
     // fewer than one in kMinRate attempts: a larger time step, another shift or
     // an iteration that happened to spawn nothing says little about this one
     const double per = cnt->prev_attempts ? (double)cnt->prev_spawned / (double)cnt->prev_attempts : 0.5;
-    set_bins(cnt, bins, (double)run * (per > 1.0 / kMinRate ? per : 1.0 / kMinRate));
+    const double expect = (double)run * (per > 1.0 / kMinRate ? per : 1.0 / kMinRate);
+    // of that, determinants: the previous iteration's share, by the same bound
+    const double share = cnt->prev_spawned ? (double)cnt->prev_unique / (double)cnt->prev_spawned : 1.0;
+    set_bins(cnt, bins, expect, expect * (share > 1.0 / kMinRate ? share : 1.0 / kMinRate));
   }
 }
 template <int W>
@@ -1019,10 +1036,14 @@ __device__ inline void spawn_flush(const SpawnStage<W>* ss, int n, Counters* cnt
 #pragma unroll
   for (int j = 0; j < 2; ++j) {
     const int i = lane + j * kWave;
-    if (i < n) {
-      uint64_t* r = bin_record(cnt, bins, bin[j], pos[j], cap, s.rec_words);
-      if (r) rec_store<W>(s, r, ss->key + i * W, ss->val[i], ss->info[i]);
+    const bool over = i < n && pos[j] >= cap;
+    uint64_t* r = i < n && !over ? bins.rec + ((size_t)bin[j] * cap + pos[j]) * s.rec_words : nullptr;
+    if (const uint64_t om = __ballot(over)) {
+      const unsigned long long base = wave_reserve(&cnt->n_ovf, popc64(om));
+      if (over)
+        r = bin_overflow(bins, bin[j], pos[j] - cap, base + (unsigned long long)popc64(om & lanemask_lt()), s.rec_words);
     }
+    if (r) rec_store<W>(s, r, ss->key + i * W, ss->val[i], ss->info[i]);
   }
   wave_sync();
 }
@@ -1030,24 +1051,28 @@ __device__ inline void spawn_flush(const SpawnStage<W>* ss, int n, Counters* cnt
 // An explicit spawned list (n dense records) into the bins, each record at the
 // place the host chose for it: places in list order, so that a wave reads a
 // determinant's records, and sums them, in the order of the list.  Places count
-// through the bins' records, the spill areas and the overflow list.
+// through the bins' records and the overflow list; an overflow record's link is
+// the one before it in its chain, or, past kChainHead, the chain it begins.
+constexpr int64_t kChainHead = 1ll << 40;
 template <int W>
-__global__ void __launch_bounds__(kBlock) k_bin_list(DevSys s, Counters* cnt, const uint64_t* list, const int64_t* place, int64_t n, Bins bins) {
+__global__ void __launch_bounds__(kBlock) k_bin_list(DevSys s, Counters* cnt, const uint64_t* list, const int64_t* place, const int64_t* link, int64_t n, Bins bins) {
   const uint32_t nb = cnt->nbins, sh = cnt->bin_shift;
-  const int64_t spill0 = bins.cap, ovf0 = spill0 + (int64_t)kSpill * bins.spill_cap;
   for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
     const uint64_t* q = list + i * s.rec_words;
     const int64_t p = place[i];
     const uint32_t bin = bin_of(bin_hash<W>(q), nb);
     atomicAdd(&bins.count[(size_t)bin << sh], 1u);
-    if (p >= spill0) atomicAdd(&bins.scount[bin % kSpill], 1u);
-    if (p >= ovf0) atomicAdd(&cnt->n_ovf, 1ull);
-    uint64_t* r = p < spill0 ? bins.rec + p * s.rec_words
-                : p < ovf0 ? bins.spill + (p - spill0) * s.rec_words : bins.ovf + (p - ovf0) * s.rec_words;
+    uint64_t* r = bins.rec + p * s.rec_words;
+    if (p >= bins.cap) {
+      const int64_t o = p - bins.cap, l = link[i];
+      if (l >= kChainHead) bins.head[l - kChainHead] = (uint32_t)o;
+      else bins.next[l] = (uint32_t)o;
+      r = bins.ovf + o * s.rec_words;
+    }
     for (int w = 0; w < s.rec_words; ++w) r[w] = q[w];
   }
 }
-__global__ void k_set_bins(Counters* cnt, Bins bins, int64_t n) { set_bins(cnt, bins, (double)n); }
+__global__ void k_set_bins(Counters* cnt, Bins bins, int64_t n) { set_bins(cnt, bins, (double)n, (double)n); }
 
 // the wave's n staged attempts to the queue from base on
 __device__ inline void queue_write(const QueueStage* qs, int n, unsigned long long base, int64_t* sq, int64_t scap,
@@ -1356,7 +1381,8 @@ __global__ void __launch_bounds__(kBlock) k_spawn(DevSys s, Walk wk, Counters* c
 // (Coulomb, exchange) pairs before; us): 14e/30o at 5e6 walkers 139 -> 115,
 // 26e/40o 131 -> 81, 10e/20o 32 -> 30, 2e3 attempts 13.3 -> 12.  Of the 24 at
 // 14e/30o the masks of rows not needed are 38, without them the dense lanes
-// alone had cost 14: the loads keep the address units busy 80% of the time.
+// alone had cost 14: the loads keep the address units busy for two thirds of
+// the time.
 // Eight lanes per attempt take 124 and 101, sixteen 150 and 132.
 
 // a group's lanes exchange by DPP: lane I's value, and the sum over the lanes
@@ -2006,8 +2032,8 @@ __device__ __forceinline__ void k_merge_body(const Grid& g_, const DevSys& s, co
   if (cnt->halt || g_.b * kWaves >= (int64_t)nb) return;
   // checkValidSpawnedList (fcimc_helper.F90:483-510) stops between spawning
   // and annihilation when the list is past its capacity: no record is merged,
-  // the iteration's end reports it.  The bins, spill areas and overflow list
-  // together hold 2.75 times the capacity, the new list max(capacity,
+  // the iteration's end reports it.  The bins and the overflow list together
+  // hold 2.25 times the capacity, the new list max(capacity,
   // MaxWalkers) rows; past this line the new determinants are no more than
   // the capacity, so that no append needs a bound of its own.
   if (spawned > (unsigned long long)bins.ovf_cap) {
@@ -2089,25 +2115,28 @@ __device__ __forceinline__ void k_merge_body(const Grid& g_, const DevSys& s, co
     more = next_bin(seg_n, c_n);
     if (more) rec_n = load_rec(bins.rec + ((size_t)seg_n * cap + lane) * s.rec_words, (uint32_t)lane < (c_n < cap ? c_n : cap));
     const int64_t c = c_all < cap ? c_all : cap;
-    int64_t csp = c, total = c;  // the bin's records, its area's, the overflow list's
-    if (c_all > cap) {
-      const uint32_t a = bins.scount[seg % kSpill];
-      csp += a < bins.spill_cap ? a : bins.spill_cap;
-      total = csp + (a > bins.spill_cap ? (int64_t)(cnt->n_ovf < (unsigned long long)bins.ovf_cap ? cnt->n_ovf : bins.ovf_cap) : 0);
-    }
-    uint64_t* spill_rec = bins.spill + (size_t)(seg % kSpill) * bins.spill_cap * s.rec_words;
+    const uint32_t over = c_all - (uint32_t)c;  // records in the bin's chains, and in this lane's
+    const uint32_t chain_n = (over + kBinChains - 1 - lane) / kBinChains;
+    static_assert(kBinChains == kWave, "a chain a lane");
+    const int64_t steps = (c + kWave - 1) / kWave, all_steps = steps + (over + kBinChains - 1) / kBinChains;
     uint64_t* seg_rec = bins.rec + (size_t)seg * cap * s.rec_words;
     bool again = false;  // records are left for another round
     do {
       const bool first_round = !again;
       again = false;
       int nu = 0;
-      for (int64_t i0 = 0; i0 < total; i0 += kWave) {
-        const int64_t i = i0 + lane;
-        bool act = i < total;
-        uint64_t* rec = i < c ? seg_rec + i * s.rec_words
-                      : i < csp ? spill_rec + (i - c) * s.rec_words : bins.ovf + (i - csp) * s.rec_words;
-        const Rec q = i0 == 0 && first_round && act && i < c ? rec_0 : load_rec(rec, act);
+      uint32_t link = 0;
+      for (int64_t st = 0; st < all_steps; ++st) {
+        const int64_t i = st * kWave + lane;
+        bool act = i < c;
+        uint64_t* rec = seg_rec + i * s.rec_words;
+        if (st >= steps) {  // the next record of the lane's chain
+          const uint32_t k = (uint32_t)(st - steps);
+          act = k < chain_n;
+          if (act) link = k == 0 ? bins.head[(size_t)seg * kBinChains + lane] : bins.next[link];
+          rec = bins.ovf + (size_t)link * s.rec_words;
+        }
+        const Rec q = st == 0 && first_round && act && i < c ? rec_0 : load_rec(rec, act);
         const uint64_t* key = q.key;
         const double v = q.v;
         const uint32_t inf = q.inf;
@@ -2115,7 +2144,6 @@ __device__ __forceinline__ void k_merge_body(const Grid& g_, const DevSys& s, co
         if (act) {
           const uint32_t h = bin_hash<W>(key);
           frac = h * nb;  // the position inside the bin
-          if (i >= c) act = bin_of(h, nb) == (uint32_t)seg;
           if (!first_round) act = act && (inf & kInfoLeft);
         }
         bool won;
@@ -2594,8 +2622,11 @@ __device__ inline double diag_group(const DevSys& s, const uint64_t* d, int g, d
 // new determinants 24 -> 13; two-word 26e/40o, 2.8e4 92 -> 49).  A long list
 // fills the lanes and is bound by issue and L1 gathers, which groups make
 // worse (14e/30o, 1.3e5: 55 with one lane, 56 with four, 102 with 16), so
-// there the lane sums its own.  G is 16, or 64 when a block's LDS does not
-// hold 16 determinants' terms; 1 for the lattice.
+// there the lane sums its own.  The line between them: at 32000 determinants
+// the groups take 21 us against 22 at 10 electrons, 25 against 32 at 14 and 55
+// against 115 at 26 (one lane takes 23, 31 and 120 for 33000), so it is right
+// for 10 electrons and early for 26.  G is 16, or 64 when a block's LDS does
+// not hold 16 determinants' terms; 1 for the lattice.
 // A determinant that is refused, in an iteration that ends in an error, has
 // its list entry marked (kFlagRemoved).
 constexpr int64_t kShortList = 32768;
