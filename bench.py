@@ -86,8 +86,8 @@ def algorithmic_bytes(stage, c, W=1, S=1, nbasis=40, psingles=0.1, nel=None, val
         return passes * Ns * (kb + 2 * (kb + 4))
     if stage == "merge":       # fused into the annihilate stage
         return 0.0
-    if stage == "annihilate":  # merge and annihilation in one pass: sorted keys + index, gathered value + info
-        #                        per spawn; per unique det one hash probe (K + 8) and its state row
+    if stage == "annihilate":  # merge and annihilation in one pass: key, place, value and info per spawn (a
+        #                        record); per unique det one hash probe (K + 8) and its state row
         #                        (S signs + flag word) read and written; new list written
         return Ns * (K + 4 + V + 4) + Nu * (K + 8) + Nu * 2 * (Sg + 8) + Nn * (K + Sg + 4)
     if stage == "insert":      # new list, free-queue entry, hash entry, walker row (key, signs, flags, 3x8)
