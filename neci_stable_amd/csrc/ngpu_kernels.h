@@ -1708,12 +1708,11 @@ __global__ void __launch_bounds__(kBlock, PP <= 3 ? 4 : PP <= 5 ? 3 : 2) k_spawn
 // histograms, a per-digit scan over blocks, stable block-local scatter.  The
 // set-up paths sort with it (the core space's selection and its connections).
 constexpr int kRadixBins = 256;  // digit values
-// radix tiles: IT elements per thread, IT*kBlock per tile (IT = 2, 4 or 8,
-// chosen per engine at run time)
+// radix tiles: IT elements per thread, IT*kBlock per tile
 
 // element range of this block in the histogram and scatter passes: whole
 // tiles, and no more blocks than there are tiles (blocks past the last tile
-// get an empty range), so that a small spawned list is not spread over more
+// get an empty range), so that a small list is not spread over more
 // blocks than it fills
 template <int IT>
 __device__ inline void radix_chunk(const Grid& g, int64_t n, int64_t& begin, int64_t& end) {
@@ -1729,7 +1728,7 @@ __device__ inline void radix_chunk(const Grid& g, int64_t n, int64_t& begin, int
 }
 
 // sort key: NW words of type K per element; FLIP compares word 0 as signed
-// DB-bit digit (DB = 8 or 10; kRadixBins is the largest digit range)
+// DB-bit digit (kRadixBins is the largest digit range)
 template <typename K, int NW, bool FLIP, int DB = 8>
 __device__ inline uint32_t radix_digit(const K* k, int word, int shift) {
   K x = k[word];
@@ -1738,7 +1737,8 @@ __device__ inline uint32_t radix_digit(const K* k, int word, int shift) {
 }
 
 template <typename K, int NW, bool FLIP, int IT, int DB>
-__device__ __forceinline__ void k_radix_hist_body(const Grid& g_, const K* keys, int kstride, const unsigned long long* n_ptr, int64_t ncap, int word, int shift, uint32_t* hist) {
+__global__ void __launch_bounds__(kBlock) k_radix_hist(const K* keys, int kstride, const unsigned long long* n_ptr, int64_t ncap, int word, int shift, uint32_t* hist) {
+  const Grid g_ = hw_grid();
   constexpr int RB = 1 << DB;
   __shared__ uint32_t h[RB];
   for (int i = threadIdx.x; i < RB; i += blockDim.x) h[i] = 0;
@@ -1752,13 +1752,10 @@ __device__ __forceinline__ void k_radix_hist_body(const Grid& g_, const K* keys,
   __syncthreads();
   for (int d = threadIdx.x; d < RB; d += blockDim.x) hist[(size_t)d * g_.nb + g_.b] = h[d];
 }
-template <typename K, int NW, bool FLIP, int IT, int DB>
-__global__ void __launch_bounds__(kBlock) k_radix_hist(const K* keys, int kstride, const unsigned long long* n_ptr, int64_t ncap, int word, int shift, uint32_t* hist) {
-  k_radix_hist_body<K, NW, FLIP, IT, DB>(hw_grid(), keys, kstride, n_ptr, ncap, word, shift, hist);
-}
 
 // one block per digit: exclusive scan of that digit's per-block counts
-__device__ __forceinline__ void k_radix_scan_body(const Grid& g_, uint32_t* hist, int nb, uint32_t* digit_tot) {
+__global__ void __launch_bounds__(kBlock) k_radix_scan(uint32_t* hist, int nb, uint32_t* digit_tot) {
+  const Grid g_ = hw_grid();
   __shared__ int64_t red[kBlock / kWave];
   uint32_t* row = hist + (size_t)g_.b * nb;
   int per = (nb + kBlock - 1) / kBlock;
@@ -1776,16 +1773,14 @@ __device__ __forceinline__ void k_radix_scan_body(const Grid& g_, uint32_t* hist
     }
   if (threadIdx.x == 0) digit_tot[g_.b] = (uint32_t)tot;
 }
-__global__ void __launch_bounds__(kBlock) k_radix_scan(uint32_t* hist, int nb, uint32_t* digit_tot) {
-  k_radix_scan_body(hw_grid(), hist, nb, digit_tot);
-}
 
 // Stable scatter of one digit, in tiles of IT*kBlock elements: the
 // tile is ranked by digit (ballot peers within a wave, LDS counts across waves
 // and rounds, in element order), reordered by digit in LDS, then written out
 // so that consecutive threads write consecutive positions of each digit's run.
 template <typename K, int NW, bool FLIP, int IT, int DB>
-__device__ __forceinline__ void k_radix_scatter_body(const Grid& g_, const K* kin, int kstride, const uint32_t* iin, K* kout, uint32_t* iout, const unsigned long long* n_ptr, int64_t ncap, int word, int shift, const uint32_t* hist, const uint32_t* digit_tot) {
+__global__ void __launch_bounds__(kBlock) k_radix_scatter(const K* kin, int kstride, const uint32_t* iin, K* kout, uint32_t* iout, const unsigned long long* n_ptr, int64_t ncap, int word, int shift, const uint32_t* hist, const uint32_t* digit_tot) {
+  const Grid g_ = hw_grid();
   constexpr int RB = 1 << DB;          // digit values
   constexpr int DPT = RB / kBlock;     // digits owned by each thread (consecutive)
   constexpr int TILE = IT * kBlock;
@@ -1905,10 +1900,6 @@ __device__ __forceinline__ void k_radix_scatter_body(const Grid& g_, const K* ki
     }
     __syncthreads();
   }
-}
-template <typename K, int NW, bool FLIP, int IT, int DB>
-__global__ void __launch_bounds__(kBlock) k_radix_scatter(const K* kin, int kstride, const uint32_t* iin, K* kout, uint32_t* iout, const unsigned long long* n_ptr, int64_t ncap, int word, int shift, const uint32_t* hist, const uint32_t* digit_tot) {
-  k_radix_scatter_body<K, NW, FLIP, IT, DB>(hw_grid(), kin, kstride, iin, kout, iout, n_ptr, ncap, word, shift, hist, digit_tot);
 }
 
 // ------------------------------------------------------------- merging
