@@ -3416,12 +3416,12 @@ int ngpu_annihilate(ngpu_t* h, uint32_t iter, const int64_t* sdet, const double*
   HIP_OK(hipMemcpy(h->hcnt, h->cnt, sizeof(Counters), hipMemcpyDeviceToHost));
   if (h->hcnt->halt) return err_from_mask(h->hcnt->halt);
   const int W = h->W, S = h->S;
-  if (!h->u_key) {  // the merged list is kept only for this entry point
-    HIP_OK(hipMalloc((void**)&h->u_key, (size_t)h->scap * W * 8));
-    HIP_OK(hipMalloc((void**)&h->u_sgn, (size_t)h->scap * S * 8));
-    HIP_OK(hipMalloc((void**)&h->u_flag, (size_t)h->scap * 4));
-    HIP_OK(hipMalloc((void**)&h->u_count, 8));
-  }
+  // the merged list is kept only for this entry point (each buffer by itself:
+  // a call after one that ran out of memory finds what is missing)
+  if (!h->u_key) HIP_OK(hipMalloc((void**)&h->u_key, (size_t)h->scap * W * 8));
+  if (!h->u_sgn) HIP_OK(hipMalloc((void**)&h->u_sgn, (size_t)h->scap * S * 8));
+  if (!h->u_flag) HIP_OK(hipMalloc((void**)&h->u_flag, (size_t)h->scap * 4));
+  if (!h->u_count) HIP_OK(hipMalloc((void**)&h->u_count, 8));
   const int rw = h->ds.rec_words;
   const int64_t chunk = std::min<int64_t>(h->scap, kListChunk);
   for (int q = 0; q < 2; ++q) {
